@@ -1,0 +1,632 @@
+"""Workloads of this framework: the calls a program makes that serves models with block-quantized weights.
+
+A case is a dict with an "op" and its sizes:
+
+  linear   f32 rows times a packed weight (`axq_gemv_f32` on device memory): one linear of a model on 1 to 64 activations
+  gemm     bf16 rows times a packed weight (`axq_gemm_bf16`): a linear of a prompt
+  codec    `axq_quantize` of a tensor and `axq_dequantize` of a packed one: what a loader does with every tensor
+  prompt   `DecoderModel.forward_tokens` on a fresh sequence: a prompt up to the logits behind it
+  decode   `DecoderModel.forward` token by token behind a context, the logits of every step
+  batch    one prompt forked to several sequences (`copy_sequence`), then `forward_batch` steps: parallel sampling, serving
+
+The models are the LLaMA/Mistral shape (`QuantizedLlama`), and the Lakulix and Gemosun kinds of described layers
+(`StackModel`).  Weights are normal, rounded to the block type by the torch code below; everything comes from the seed.
+"""
+import ctypes
+import math
+
+import numpy as np
+import torch
+
+from axonml_amd import stack
+from axonml_amd._lib import MEM_DEVICE
+from axonml_amd.decode import QuantizedLlama
+from axonml_amd.quant import DeviceWeight, QuantType, default_context
+
+DEV = "cuda"
+VOCAB = 32000
+BYTES = {"Q8_0": 34 / 32, "Q4_0": 18 / 32, "Q4_1": 20 / 32, "Q5_0": 22 / 32, "Q5_1": 24 / 32, "Q4_K": 144 / 256, "Q5_K": 176 / 256,
+         "Q6_K": 210 / 256, "F16": 2, "BF16": 2}
+BLOCKS = ("Q4_K", "Q4_K", "Q4_K", "Q5_K", "Q6_K", "Q8_0", "Q4_0", "Q4_1", "Q5_0", "Q5_1")  # Q4_K is what most files hold
+
+
+def listed():
+    return [
+        # the largest linear of a 7B model on one token: the smallest call, bound by latency and HBM
+        dict(name="linear_1", op="linear", type="Q4_K", n=14336, k=4096, rows=1, bias=False),
+        # its way back, on a few tokens that do not fill a tile, with a bias
+        dict(name="linear_21", op="linear", type="Q4_0", n=4096, k=11008, rows=21, bias=True),
+        # a long prompt's linear in the most used type, and an odd one in a type with a minimum
+        dict(name="gemm_2048", op="gemm", type="Q4_K", n=14336, k=4096, rows=2048),
+        dict(name="gemm_509", op="gemm", type="Q5_1", n=4096, k=4096, rows=509),
+        # a tensor on its way into and out of the packed form, with a tail that fills no block
+        dict(name="codec", op="codec", type="Q8_0", numel=4096 * 11008 + 21),
+        # a chat with a 7B model: the prompt, then token after token
+        dict(name="prompt_512", op="prompt", model="llama", type="Q4_K", width=4096, layers=32, tokens=512),
+        dict(name="decode_1", op="decode", model="llama", type="Q4_K", width=4096, layers=32, context=512, steps=8),
+        # the same model serving several: a few sequences, and as many as it takes
+        dict(name="batch_8", op="batch", model="llama", type="Q4_K", width=4096, layers=32, context=128, steps=4, sequences=8),
+        dict(name="batch_64", op="batch", model="llama", type="Q4_K", width=4096, layers=32, context=128, steps=4, sequences=64),
+        # described layers with bfloat16 weights: a prompt of each kind, and a reply
+        dict(name="lakulix_prompt", op="prompt", model="lakulix", width=2048, layers=4, tokens=2048),
+        dict(name="gemosun_prompt", op="prompt", model="gemosun", width=2048, layers=3, tokens=2001),
+        dict(name="gemosun_decode", op="decode", model="gemosun", width=2048, layers=3, context=1200, steps=8),
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    op = rng.choice(("linear", "linear", "gemm", "codec", "prompt", "decode", "batch", "batch", "prompt"))
+    if op in ("linear", "gemm"):
+        t = rng.choice(BLOCKS + ("BF16", "F16"))
+        k = 256 * _log(rng, 4, 56)
+        if t not in ("Q4_K", "Q5_K", "Q6_K") and rng.random() < 0.2:
+            k += 64 * rng.randint(-3, -1)  # rows that are no whole superblocks
+        n = rng.choice((_log(rng, 256, 32000), 16 * _log(rng, 16, 2000)))
+        if op == "linear":
+            return dict(op=op, type=t, n=n, k=k, rows=rng.choice((1, 1, rng.randint(2, 8), _log(rng, 2, 64))), bias=rng.random() < 0.5)
+        return dict(op=op, type=t, n=min(n, 14336), k=min(k, 4096), rows=rng.choice((_log(rng, 40, 2048), 128 * rng.randint(1, 16))))
+    if op == "codec":
+        return dict(op=op, type=rng.choice(BLOCKS), numel=_log(rng, 1 << 16, 45_000_000))
+    model = rng.choice(("llama", "llama", "llama", "lakulix", "gemosun")) if op != "batch" else "llama"
+    if model == "llama":
+        width = rng.choice((1024, 2048, 4096))
+        c = dict(op=op, model=model, type=rng.choice(BLOCKS), width=width, layers=rng.randint(2, 8))
+    else:
+        c = dict(op=op, model=model, width=rng.choice((1024, 2048)), layers=rng.randint(2, 4))
+    if op == "prompt":
+        return dict(c, tokens=_log(rng, 5, 2048))
+    if op == "decode":
+        return dict(c, context=0 if model == "lakulix" else _log(rng, 8, 1500), steps=rng.randint(4, 16))
+    return dict(c, context=_log(rng, 8, 600), steps=rng.randint(2, 6), sequences=rng.choice((rng.randint(2, 8), _log(rng, 2, 64), _log(rng, 9, 64))))
+
+
+# ----------------------------------------------------------------------------------------------- block types, in torch
+def _bytes(*parts):
+    return torch.cat([p.contiguous().view(torch.uint8).reshape(p.shape[0], -1) for p in parts], 1).reshape(-1)
+
+
+def _nibbles(lo, hi):
+    return (lo | (hi << 4)).to(torch.uint8)
+
+
+def _scales(s, m):
+    """Eight six-bit scales and minima of a superblock in twelve bytes."""
+    return torch.cat([s[:, :4] | ((s[:, 4:] >> 4) << 6), m[:, :4] | ((m[:, 4:] >> 4) << 6), (s[:, 4:] & 15) | ((m[:, 4:] & 15) << 4)], 1).to(torch.uint8)
+
+
+def pack(kind, w):
+    """f32 values, whole blocks, to (packed bytes, a function that gives the values they stand for in 64 bits)."""
+    w = w.reshape(-1)
+    if kind in ("BF16", "F16"):
+        h = w.to(torch.bfloat16 if kind == "BF16" else torch.float16)
+        return h.view(torch.uint8), lambda: h.double()
+    if kind in ("Q4_K", "Q5_K"):
+        top = 15 if kind == "Q4_K" else 31
+        b = w.view(-1, 8, 32)
+        lo = (-b.amin(2)).clamp_min(0)
+        step = (b.amax(2) + lo) / top
+        d, dm = (step.amax(1) / 63).half(), (lo.amax(1) / 63).half()
+        s, m = (torch.round(v / u.float()[:, None]).clamp(0, 63) for v, u in ((step, d), (lo, dm)))
+        ds, off = d.double()[:, None] * s, dm.double()[:, None] * m
+        q = torch.round((b + off.float()[..., None]) / ds.float()[..., None].clamp_min(1e-12)).clamp(0, top).to(torch.int32)
+        low = q & 15
+        parts = [d[:, None], dm[:, None], _scales(s.to(torch.int32), m.to(torch.int32))]
+        if kind == "Q5_K":
+            parts.append(((q >> 4) << torch.arange(8, device=w.device, dtype=torch.int32)[None, :, None]).sum(1).to(torch.uint8))
+        parts.append(_nibbles(low[:, 0::2], low[:, 1::2]).reshape(-1, 128))
+        return _bytes(*parts), lambda: (ds[..., None] * q - off[..., None]).reshape(-1)
+    if kind == "Q6_K":
+        b = w.view(-1, 16, 16)
+        step = b.abs().amax(2) / 31
+        d = (step.amax(1) / 127).half()
+        s = torch.round(step / d.float()[:, None]).clamp(1, 127)
+        ds = d.double()[:, None] * s
+        q = torch.round(b / ds.float()[..., None]).clamp(-32, 31).to(torch.int32)
+        u = (q + 32).view(-1, 2, 4, 32)
+        ql = torch.cat([_nibbles(u[:, :, 0] & 15, u[:, :, 2] & 15), _nibbles(u[:, :, 1] & 15, u[:, :, 3] & 15)], 2)
+        qh = ((u[:, :, 0] >> 4) | ((u[:, :, 1] >> 4) << 2) | ((u[:, :, 2] >> 4) << 4) | ((u[:, :, 3] >> 4) << 6)).to(torch.uint8)
+        return _bytes(ql.reshape(-1, 128), qh.reshape(-1, 64), s.to(torch.int8), d[:, None]), lambda: (ds[..., None] * q).reshape(-1)
+    b = w.view(-1, 32)
+    if kind in ("Q4_1", "Q5_1"):
+        top = 15 if kind == "Q4_1" else 31
+        m = b.amin(1, keepdim=True).half()
+        d = ((b.amax(1, keepdim=True) - m.float()) / top).half()
+        q = torch.round((b - m.float()) / d.float()).clamp(0, top).to(torch.int32)
+        head, centre = [d, m], 0
+    else:
+        half = {"Q8_0": 127, "Q4_0": 7, "Q5_0": 15}[kind]
+        d, m = (b.abs().amax(1, keepdim=True) / half).half(), None
+        q = torch.round(b / d.float()).clamp(-half - 1, half).to(torch.int32)
+        head, centre = [d], 0 if kind == "Q8_0" else half + 1
+
+    def values():
+        v = d.double() * q
+        return (v if m is None else v + m.double()).reshape(-1)
+    u = q + centre
+    if kind == "Q8_0":
+        return _bytes(d, q.clamp(-127, 127).to(torch.int8)), values
+    if kind in ("Q4_0", "Q4_1"):
+        return _bytes(*head, _nibbles(u[:, 0::2], u[:, 1::2])), values
+    qh = ((u >> 4) << torch.arange(32, device=w.device, dtype=torch.int32)).sum(1).to(torch.int32)
+    return _bytes(*head, qh[:, None], _nibbles(u[:, :16] & 15, u[:, 16:] & 15)), values
+
+
+# ---------------------------------------------------------------------------------------------------------- what is fed
+def _rng(seed):
+    return torch.Generator(device=DEV).manual_seed(int(seed))
+
+
+def _normal(g, *shape, std=1.0):
+    return torch.randn(*shape, generator=g, device=DEV) * std
+
+
+def _weight(g, n, k):
+    return _normal(g, n, k, std=0.02)
+
+
+def _upload(ctx, kind, n, k, packed):
+    torch.cuda.synchronize()
+    h = ctypes.c_void_p()
+    ctx.check(ctx.lib.axq_weight_upload(ctx.handle, int(QuantType[kind]), n, k, packed.data_ptr(), packed.numel(), MEM_DEVICE, ctypes.byref(h)))
+    return DeviceWeight(ctx, h, QuantType[kind], n, k)
+
+
+def _tokens(seed, *shape):
+    return np.random.default_rng([int(seed), 7]).integers(0, VOCAB, size=shape, dtype=np.int32)
+
+
+def _linear_inputs(case, seed):
+    g = _rng(seed)
+    w = _weight(g, case["n"], case["k"])
+    x = _normal(g, case["rows"], case["k"])
+    return w, x, _normal(g, case["n"]) if case.get("bias") else None
+
+
+def _codec_inputs(case, seed):
+    g = _rng(seed)
+    src = _normal(g, case["numel"], std=0.02)
+    return src, pack(case["type"], _normal(g, -(-case["numel"] // 256) * 256, std=0.02))
+
+
+def _llama_sizes(case):
+    w = case["width"]
+    heads, kv = w // 128, max(1, w // 512)
+    ff = w * 7 // 2
+    shapes = dict(q=(w, w), k=(kv * 128, w), v=(kv * 128, w), o=(w, w), gate=(ff, w), up=(ff, w), down=(w, ff))
+    return heads, kv, ff, shapes
+
+
+def _llama_tensors(case, seed):
+    """(layer, name, values) of a model in a fixed order; layer -1: embedding, final norm and head."""
+    g, w = _rng(seed), case["width"]
+    yield -1, "embed", _normal(g, VOCAB, w, std=0.5).half()
+    for layer in range(case["layers"]):
+        for name in ("norm0", "norm1"):
+            yield layer, name, 1 + _normal(g, w, std=0.1)
+        for name, (n, k) in _llama_sizes(case)[3].items():
+            yield layer, name, _weight(g, n, k)
+    yield -1, "norm0", 1 + _normal(g, w, std=0.1)
+    yield -1, "q", _weight(g, VOCAB, w)
+
+
+def _positions(case):
+    return case["tokens"] if case["op"] == "prompt" else case["context"] + case["steps"]
+
+
+def _llama(case, seed):
+    heads, kv, ff, _ = _llama_sizes(case)
+    ctx = default_context()
+    m = QuantizedLlama(ctx, vocab_size=VOCAB, hidden_size=case["width"], intermediate_size=ff, num_hidden_layers=case["layers"],
+                       num_attention_heads=heads, num_key_value_heads=kv, head_dim=128, max_position_embeddings=_positions(case) + 8,
+                       rms_norm_eps=1e-5, rope_theta=10000.0, sliding_window=0)
+    for layer, name, v in _llama_tensors(case, seed):
+        if name == "embed":
+            torch.cuda.synchronize()
+            ctx.check(ctx.lib.axq_model_set_embedding_f16(m.handle, v.data_ptr(), MEM_DEVICE))
+            ctx.synchronize()
+        elif name.startswith("norm"):
+            m.set_norm(layer, int(name[4:]), v.cpu().numpy())
+        else:
+            w = _upload(ctx, case["type"], *v.shape, pack(case["type"], v)[0])
+            m.set_linear(layer, name, w)
+            w.free()
+    return m
+
+
+# Described layers.  Lakulix: lightning, sigmoid attention with a feed-forward, time mixing, attention again.  Gemosun: a
+# dense layer, then mixtures of experts, all with windowed softmax attention over tokens and pooled blocks.
+def _layers(case):
+    w = case["width"]
+    heads, kv = w // 128, max(1, w // 512)
+    if case["model"] == "lakulix":
+        att = stack.LayerDescription(stack.ATTENTION, heads, 128, 128, kv_heads=kv, ff=w * 7 // 2, bias_rows=32, bias_max=128, scale=128 ** -0.5,
+                                     q_temp_every=1024, q_temp_coef=0.1)
+        kinds = (stack.LayerDescription(stack.LIGHTNING, heads, 128, 128), att, stack.LayerDescription(stack.WKV, w // 64, 64, 64, decay_rank=64), att)
+        return [kinds[i % 4] for i in range(case["layers"])]
+    mix = dict(kv_heads=kv, scale=128 ** -0.5, window=1024, pool=64, keys_as_values=1, head_gate=1, rot_dims=64, rot_base=10000.0,
+               rot_original=1024, rot_factor=4.0, rot_fast=32.0, rot_slow=1.0)
+    dense = stack.LayerDescription(stack.SOFTMAX, heads, 128, 128, ff=w * 7 // 2, ff_kind=stack.FF_GLU, **mix)
+    moe = stack.LayerDescription(stack.SOFTMAX, heads, 128, 128, ff=w, ff_kind=stack.FF_MOE, experts=16, top=4, groups=4, groups_keep=2, shared_ff=w, **mix)
+    return [dense] + [moe] * (case["layers"] - 1)
+
+
+def _stack_tensors(case, seed):
+    """(layer, name, values) of a model in a fixed order, linears bfloat16-exact; layer -1: outside the layers."""
+    g, w, soft = _rng(seed), case["width"], case["model"] == "gemosun"
+
+    def lin(n, k):
+        return _weight(g, n, k).bfloat16().float()
+
+    def norm(pre):
+        yield pre, 1 + _normal(g, w, std=0.1)
+        if not soft:
+            yield pre + ".b", _normal(g, w, std=0.1)
+            yield pre + ".alpha", torch.full((1,), 0.5, device=DEV)
+
+    def layer(i, l):
+        yield from norm("norm1")
+        hd, kd, hv, gv = l.heads * l.dim, l.kv_heads * l.dim, l.heads * l.vdim, l.kv_heads * l.vdim
+        if l.mixer == stack.SOFTMAX:
+            yield from (("mix.q", lin(hd, w)), ("mix.k", lin(kd, w)), ("mix.g", lin(l.heads, w)), ("mix.o", lin(w, hd)))
+            yield "dwa", torch.tensor([0.3 / (i + 1)] * (i + 1) + [0.7], device=DEV)
+        elif l.mixer == stack.ATTENTION:
+            yield from (("mix.q", lin(hd, w)), ("mix.k", lin(kd, w)), ("mix.v", lin(gv, w)), ("mix.o", lin(w, hv)))
+            yield from (("mix.q.norm", 1 + _normal(g, l.dim, std=0.1)), ("mix.k.norm", 1 + _normal(g, l.dim, std=0.1)))
+            yield from (("mix.pb", -6 + _normal(g, l.heads, std=0.5)), ("mix.rel", _normal(g, l.bias_rows, l.heads, std=0.5)))
+        elif l.mixer == stack.LIGHTNING:
+            yield from (("mix.q", lin(hd, w)), ("mix.k", lin(hd, w)), ("mix.v", lin(hv, w)), ("mix.g", lin(hv, w)), ("mix.o", lin(w, hv)))
+            yield "mix.norm", 1 + _normal(g, hv, std=0.1)
+            yield "mix.decay", torch.exp(-torch.exp2(-8.0 * (torch.arange(l.heads, device=DEV) + 1) / l.heads))
+        else:
+            for s in "rkvg":
+                yield "mix.mu." + s, torch.rand(w, generator=g, device=DEV)
+                yield "mix." + s, lin(hd, w)
+            yield from (("mix.mu.w", torch.rand(w, generator=g, device=DEV)), ("mix.w1", lin(l.decay_rank, w)), ("mix.w2", lin(hd, l.decay_rank)))
+            yield from (("mix.w0", -6 + 5 * torch.rand(hd, generator=g, device=DEV)), ("mix.u", _normal(g, l.heads, l.dim, std=0.5)))
+            yield from (("mix.norm", 1 + _normal(g, hd, std=0.1)), ("mix.o", lin(w, hd)))
+        if not l.ff:
+            return
+        yield from norm("norm2")
+        if l.ff_kind == stack.FF_POLY:
+            yield from (("mlp.up", lin(l.ff, w)), ("mlp.down", lin(w, l.ff)), ("mlp.act", torch.tensor([0.4, 0.3, 0.3, 0.01], device=DEV)))
+        elif l.ff_kind == stack.FF_GLU:
+            yield from (("mlp.gate", lin(l.ff, w)), ("mlp.up", lin(l.ff, w)), ("mlp.down", lin(w, l.ff)))
+        else:
+            yield "mlp.router", lin(l.experts, w)
+            for e in range(l.experts):
+                yield from ((f"mlp.e{e}.up", lin(l.ff, w)), (f"mlp.e{e}.down", lin(w, l.ff)))
+            yield from (("mlp.shared.up", lin(l.shared_ff, w)), ("mlp.shared.down", lin(w, l.shared_ff)), ("mlp.shared.sg", lin(1, w)))
+
+    yield -1, "embed", _normal(g, VOCAB, w)
+    if not soft:
+        yield -1, "pos", _normal(g, _positions(case) + 8, w, std=0.1)
+    for i, l in enumerate(_layers(case)):
+        yield from ((i, name, v) for name, v in layer(i, l))
+    yield from ((-1, name, v) for name, v in norm("final.norm"))
+    yield -1, "head", lin(VOCAB, w)
+
+
+def _stack(case, seed):
+    soft = case["model"] == "gemosun"
+    d = stack.StackDescription(vocab_size=VOCAB, width=case["width"], max_positions=_positions(case) + 8, layers=_layers(case), norm_eps=1e-5,
+                               logit_softcap=0.0 if soft else 30.0, norm=stack.NORM_LAYER if soft else stack.NORM_TANH, position_table=not soft,
+                               parallel=soft, depth_average=soft)
+    m = stack.StackModel(d, ctx=default_context())
+    for layer, name, v in _stack_tensors(case, seed):
+        if name == "embed":
+            torch.cuda.synchronize()
+            m.ctx.check(m.ctx.lib.axq_model_set_embedding_f32(m.handle, v.data_ptr(), MEM_DEVICE))
+            m.ctx.synchronize()
+        else:
+            m.set_tensor(layer, name, v.cpu().numpy())
+    return m
+
+
+# ------------------------------------------------------------------------------------------------------ prepare and run
+def prepare(case, seed):
+    ctx = default_context()
+    op = case["op"]
+    if op in ("linear", "gemm"):
+        w, x, bias = _linear_inputs(case, seed)
+        x = x if op == "linear" else x.bfloat16()
+        s = dict(op=op, ctx=ctx, x=x, bias=bias, y=torch.empty(case["rows"], case["n"], device=DEV))
+        s["w"] = _upload(ctx, case["type"], case["n"], case["k"], pack(case["type"], w)[0])
+        return s
+    if op == "codec":
+        src, (packed, _) = _codec_inputs(case, seed)
+        t = int(QuantType[case["type"]])
+        nbytes = ctx.lib.axq_packed_bytes(t, case["numel"])
+        torch.cuda.synchronize()
+        return dict(op=op, ctx=ctx, type=t, src=src, packed=packed, out=torch.empty(nbytes, dtype=torch.uint8, device=DEV), back=torch.empty_like(src))
+    m = _llama(case, seed) if case["model"] == "llama" else _stack(case, seed)
+    s = dict(op=op, model=m, case=case)
+    if op == "prompt":
+        s["tokens"] = _tokens(seed, case["tokens"])
+        return s
+    s["steps"] = _tokens(seed, case["steps"], case.get("sequences", 1))
+    if op == "batch":
+        m.set_batch(case["sequences"])
+    if case["context"]:
+        m.forward_tokens(_tokens(seed + 1, case["context"]), want_logits=False)
+    return s
+
+
+def run(s):
+    op = s["op"]
+    if op in ("linear", "gemm"):
+        ctx, x, y = s["ctx"], s["x"], s["y"]
+        if op == "linear":
+            bias = s["bias"].data_ptr() if s["bias"] is not None else None
+            ctx.check(ctx.lib.axq_gemv_f32(ctx.handle, s["w"].handle, x.data_ptr(), x.shape[0], bias, y.data_ptr(), MEM_DEVICE))
+        else:
+            ctx.check(ctx.lib.axq_gemm_bf16(ctx.handle, s["w"].handle, x.data_ptr(), x.shape[0], y.data_ptr(), MEM_DEVICE))
+        return y
+    if op == "codec":
+        ctx, n = s["ctx"], s["src"].numel()
+        ctx.check(ctx.lib.axq_quantize(ctx.handle, s["type"], s["src"].data_ptr(), n, s["out"].data_ptr(), MEM_DEVICE))
+        ctx.check(ctx.lib.axq_dequantize(ctx.handle, s["type"], s["packed"].data_ptr(), n, s["back"].data_ptr(), MEM_DEVICE))
+        return [s["out"], s["back"]]
+    m, c = s["model"], s["case"]
+    if op == "prompt":
+        m.reset()
+        return m.forward_tokens(s["tokens"])[1]
+    m.truncate(c["context"])
+    if op == "decode":
+        return [m.forward(t)[1] for t in s["steps"][:, 0]]
+    for i in range(1, c["sequences"]):
+        m.copy_sequence(0, i)
+    return [m.forward_batch(t)[1] for t in s["steps"]]
+
+
+# ------------------------------------------------------------------------------------------------- what a pass is worth
+def _model_work(case):
+    """(bytes of weights, flops of a token) of a model's layers, then of its head; bytes of a position's cache."""
+    w = case["width"]
+    if case["model"] == "llama":
+        per = sum(n * k for n, k in _llama_sizes(case)[3].values()) * case["layers"]
+        b = BYTES[case["type"]]
+        return per * b, 2 * per, VOCAB * w * b, 2 * VOCAB * w, case["layers"] * _llama_sizes(case)[1] * 128 * 4
+    all_, used, cache = 0, 0, 0
+    for l in _layers(case):
+        if l.mixer == stack.SOFTMAX:
+            n, cache = w * (2 * l.heads * l.dim + l.kv_heads * l.dim + l.heads), cache + l.kv_heads * l.dim * 4
+        elif l.mixer == stack.ATTENTION:
+            n, cache = w * (2 * l.heads * l.dim + 2 * l.kv_heads * l.dim), cache + l.kv_heads * l.dim * 4
+        else:
+            n = w * 5 * l.heads * l.dim + l.decay_rank * (w + l.heads * l.dim)
+        f = (3 if l.ff_kind == stack.FF_GLU else 2) * w * l.ff
+        if l.ff_kind == stack.FF_MOE:
+            all_ += 2 * w * (l.experts * l.ff + l.shared_ff) + w * l.experts
+            used += 2 * w * (l.top * l.ff + l.shared_ff) + w * l.experts
+        else:
+            all_, used = all_ + f, used + f
+        all_, used = all_ + n, used + n
+    if case["op"] == "decode":
+        all_ = used
+    return 2 * all_, 2 * used, 2 * VOCAB * w, 2 * VOCAB * w, cache
+
+
+def work(case):
+    op = case["op"]
+    if op in ("linear", "gemm"):
+        n, k, r = case["n"], case["k"], case["rows"]
+        return {"bytes": n * k * BYTES[case["type"]] + r * k * (4 if op == "linear" else 2) + 4 * r * n, "flops": 2 * n * k * r}
+    if op == "codec":
+        return {"bytes": 2 * case["numel"] * (4 + BYTES[case["type"]]), "flops": 0}
+    wb, wf, hb, hf, cache = _model_work(case)
+    if op == "prompt":
+        return {"bytes": wb + hb + 4 * VOCAB, "flops": wf * case["tokens"] + hf}
+    n, s = case["steps"], case.get("sequences", 1)
+    ctx = min(case["context"], 1024) if case["model"] == "gemosun" else case["context"]
+    return {"bytes": n * (wb + hb + s * (ctx * cache + 4 * VOCAB)), "flops": n * s * (wf + hf)}
+
+
+def tolerance(case):
+    if case["op"] == "codec":
+        return "exact"
+    if case["op"] in ("linear", "gemm"):
+        return {"rel": 4e-6}  # f32 sums of products that the block types and bf16 give exactly: 1e-7 to 4e-7 off 64 bits
+    if case["model"] == "llama":
+        return {"rel": 6e-3}  # f32 rows, an f16 cache of keys and values: up to 1.8e-3
+    return {"rel": 1e-2}      # bf16 rows through a few layers, now and then another expert: up to 2e-3
+
+
+# ------------------------------------------------------------------------------------------------ the same in 64 bits
+def _f64_llama(case, seed):
+    heads, kv, _, _ = _llama_sizes(case)
+    if case["op"] == "prompt":
+        tokens = _tokens(seed, case["tokens"])
+        pos, seq, want = np.arange(len(tokens)), np.zeros(len(tokens), int), [len(tokens) - 1]
+        forked = len(tokens)
+    else:
+        steps, forked = _tokens(seed, case["steps"], case.get("sequences", 1)), case["context"]
+        n, s = steps.shape
+        tokens = np.concatenate([_tokens(seed + 1, forked), steps.reshape(-1)])
+        pos = np.concatenate([np.arange(forked), forked + np.repeat(np.arange(n), s)])
+        seq = np.concatenate([np.zeros(forked, int), np.tile(np.arange(s), n)])
+        want = list(range(forked, len(tokens)))
+    p, sq = torch.tensor(pos, device=DEV), torch.tensor(seq, device=DEV)
+    sees = (p[None] <= p[:, None]) & ((p[None] < forked) | (sq[None] == sq[:, None]))
+    angle = p.double()[:, None] / (10000.0 ** (torch.arange(64, device=DEV).double() / 64))
+    cos, sin = angle.cos()[:, None], angle.sin()[:, None]
+
+    def rope(v):
+        a, b = v[..., :64], v[..., 64:]
+        return torch.cat([a * cos - b * sin, a * sin + b * cos], -1)
+
+    def rms(v, g):
+        return v / (v.square().mean(1, keepdim=True) + 1e-5).sqrt() * g
+
+    got, x, t = None, None, len(tokens)
+    for layer, name, v in _llama_tensors(case, seed):
+        if name not in ("embed", "norm0", "norm1"):
+            shape, v = v.shape, pack(case["type"], v)[1]()
+            v = v.view(shape).T
+        if name == "embed":
+            x = v[torch.tensor(tokens, device=DEV).long()].double()
+        elif name in ("norm0", "norm1"):
+            got = dict(got or {}, **{name: v.double()})
+        elif layer < 0:
+            logits = rms(x[torch.tensor(want, device=DEV)], got["norm0"]) @ v
+        elif name in "qkv":
+            got[name] = (rms(x, got["norm0"]) @ v).view(t, -1, 128)
+        elif name == "o":
+            q, k, val = rope(got["q"]), rope(got["k"]).repeat_interleave(heads // kv, 1), got["v"].repeat_interleave(heads // kv, 1)
+            out = torch.empty_like(q)
+            for h in range(heads):
+                sc = (q[:, h] @ k[:, h].T * 128 ** -0.5).masked_fill(~sees, -math.inf)
+                out[:, h] = sc.softmax(1) @ val[:, h]
+            x = x + out.reshape(t, -1) @ v
+            got["h"] = rms(x, got["norm1"])
+        elif name in ("gate", "up"):
+            got[name] = got["h"] @ v
+        else:
+            x = x + (torch.nn.functional.silu(got["gate"]) * got["up"]) @ v
+    if case["op"] == "prompt":
+        return logits[0]
+    logits = logits.view(*steps.shape, -1)
+    return [l[0] if case["op"] == "decode" else l for l in logits]
+
+
+def _f64_rotate(x, l, p):
+    n = l.rot_dims
+    f = l.rot_base ** (-2.0 * torch.arange(n // 2, device=DEV).double() / n)
+
+    def where(turns):
+        return n * math.log(l.rot_original / (2 * math.pi * turns)) / (2 * math.log(l.rot_base))
+    lo, hi = max(math.floor(where(l.rot_fast)), 0), min(math.ceil(where(l.rot_slow)), n - 1)
+    ramp = ((torch.arange(n // 2, device=DEV).double() - lo) / max(hi - lo, 0.001)).clamp(0, 1)
+    a = p.double()[:, None, None] * (f / l.rot_factor * ramp + f * (1 - ramp))
+    m = 0.1 * math.log(l.rot_factor) + 1
+    c, s = a.cos() * m, a.sin() * m
+    out = x.clone()
+    out[..., 0:n:2], out[..., 1:n:2] = x[..., 0:n:2] * c - x[..., 1:n:2] * s, x[..., 1:n:2] * c + x[..., 0:n:2] * s
+    return out
+
+
+def _f64_mixer(l, h, t):
+    """The mixers over all rows of one sequence, `t` giving a layer's tensors by name."""
+    rows, p = h.shape[0], torch.arange(h.shape[0], device=DEV)
+    back = p[:, None] - p[None]
+
+    def heads(name, n, d, x=h):
+        return (x @ t["mix." + name].T).view(rows, n, d)
+
+    def rms(v):
+        return v / (v.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+    rep = l.heads // l.kv_heads
+    if l.mixer == stack.SOFTMAX:
+        val = heads("k", l.kv_heads, l.dim)
+        q, k = _f64_rotate(heads("q", l.heads, l.dim), l, p), _f64_rotate(val, l, p)
+        nb = rows // l.pool
+        k, val = (torch.cat([v[:nb * l.pool].view(nb, l.pool, l.kv_heads, l.dim).mean(1), v]).repeat_interleave(rep, 1) for v in (k, val))
+        last = torch.arange(nb, device=DEV) * l.pool + l.pool - 1
+        sees = torch.cat([last[None] <= p[:, None] - l.window, (back >= 0) & (back < l.window)], 1)
+        gate = torch.sigmoid(h @ t["mix.g"].T)
+        out = torch.stack([(q[:, i] @ k[:, i].T * l.scale).masked_fill(~sees, -math.inf).softmax(1) @ val[:, i] * gate[:, i, None] for i in range(l.heads)], 1)
+        return out.reshape(rows, -1) @ t["mix.o"].T
+    if l.mixer == stack.ATTENTION:
+        q, k = rms(heads("q", l.heads, l.dim)) * t["mix.q.norm"], rms(heads("k", l.kv_heads, l.dim)) * t["mix.k.norm"]
+        q = q * (1 + l.q_temp_coef * torch.log(torch.floor((p.double() + 1) / l.q_temp_every) + 1))[:, None, None]
+        k, val = (v.repeat_interleave(rep, 1) for v in (k, heads("v", l.kv_heads, l.vdim)))
+        half, dist = l.bias_rows // 2, back.clamp_min(0)
+        v = torch.log(dist.clamp_min(1).double() / half) / math.log(l.bias_max / half) * (l.bias_rows - half)
+        v = torch.where((v - v.round()).abs() < 1e-9, v.round(), v.floor()).long() + half
+        bucket = torch.where(dist < half, dist, v.clamp_max(l.bias_rows - 1))
+        out = torch.stack([torch.sigmoid(q[:, i] @ k[:, i].T * l.scale + t["mix.rel"][bucket, i] + t["mix.pb"][0, i]).masked_fill(back < 0, 0) @ val[:, i]
+                           for i in range(l.heads)], 1)
+        return out.reshape(rows, -1) @ t["mix.o"].T
+    if l.mixer == stack.LIGHTNING:
+        silu = torch.nn.functional.silu
+        q, k, val = silu(heads("q", l.heads, l.dim)), silu(heads("k", l.heads, l.dim)), silu(heads("v", l.heads, l.vdim))
+        fade = torch.exp(back.clamp_min(0).double() * torch.log(t["mix.decay"][0])[:, None, None]).masked_fill(back < 0, 0)
+        out = torch.stack([(q[:, i] @ k[:, i].T * fade[i]) @ val[:, i] for i in range(l.heads)], 1)
+        return (rms(out.reshape(rows, -1)) * t["mix.norm"] * torch.sigmoid(h @ t["mix.g"].T)) @ t["mix.o"].T
+    prev = torch.cat([torch.zeros_like(h[:1]), h[:-1]])
+    m = {s: h + (prev - h) * t["mix.mu." + s] for s in "rkvgw"}
+    r, k, val = (heads(s, l.heads, l.dim, m[s]) for s in "rkv")
+    decay = torch.exp(-torch.exp(torch.tanh(m["w"] @ t["mix.w1"].T) @ t["mix.w2"].T + t["mix.w0"])).view(rows, l.heads, l.dim, 1)
+    state, u, out = torch.zeros(l.heads, l.dim, l.dim, dtype=torch.float64, device=DEV), t["mix.u"][..., None], torch.empty_like(r)
+    for i in range(rows):
+        kv = k[i][:, :, None] * val[i][:, None]
+        out[i] = ((state + u * kv) * r[i][:, :, None]).sum(1)
+        state = decay[i] * state + kv
+    return (rms(out).reshape(rows, -1) * t["mix.norm"] * torch.nn.functional.silu(m["g"] @ t["mix.g"].T)) @ t["mix.o"].T
+
+
+def _f64_ff(l, h, t):
+    if l.ff_kind == stack.FF_POLY:
+        z = h @ t["mlp.up"].T
+        a = t["mlp.act"][0]
+        z = sum(a[i] * z ** (i + 1) / ((z ** (i + 1)).square().mean(1, keepdim=True) + 1e-5).sqrt() for i in range(3)) + a[3]
+        return z @ t["mlp.down"].T
+    if l.ff_kind == stack.FF_GLU:
+        return (torch.nn.functional.gelu(h @ t["mlp.gate"].T, approximate="tanh") * (h @ t["mlp.up"].T)) @ t["mlp.down"].T
+    s = torch.sigmoid(h @ t["mlp.router"].T)
+    groups = s.view(len(h), l.groups, -1)
+    kept = torch.zeros(len(h), l.groups, dtype=torch.bool, device=DEV).scatter_(1, groups.topk(2, 2)[0].sum(2).topk(l.groups_keep, 1)[1], True)
+    top, at = s.masked_fill(~kept.repeat_interleave(groups.shape[2], 1), -1).topk(l.top, 1)
+    part = torch.zeros_like(s).scatter_(1, at, top / top.sum(1, keepdim=True))
+
+    def expert(pre, x):
+        return (x @ t[pre + ".up"].T).clamp_min(0).square() @ t[pre + ".down"].T
+    out = torch.sigmoid(h @ t["mlp.shared.sg"].T) * expert("mlp.shared", h)
+    for e in range(l.experts):
+        at = part[:, e].nonzero()[:, 0]
+        out[at] += part[at, e, None] * expert(f"mlp.e{e}", h[at])
+    return out
+
+
+def _f64_stack(case, seed):
+    if case["op"] == "prompt":
+        tokens, want = _tokens(seed, case["tokens"]), [case["tokens"] - 1]
+    else:
+        tokens = np.concatenate([_tokens(seed + 1, case["context"]), _tokens(seed, case["steps"], 1)[:, 0]])
+        want = list(range(case["context"], len(tokens)))
+    soft, layers = case["model"] == "gemosun", _layers(case)
+
+    def norm(x, t, name):
+        if not soft:
+            return torch.tanh(t[name + ".alpha"] * x) * t[name] + t[name + ".b"]
+        d = x - x.mean(1, keepdim=True)
+        return d / (d.square().mean(1, keepdim=True) + 1e-5).sqrt() * t[name]
+    x, results, t, at = None, [], {}, 0
+
+    def layer(x, l, t):
+        y = _f64_mixer(l, norm(x, t, "norm1"), t)
+        if soft:
+            results.append(x + y + _f64_ff(l, norm(x, t, "norm2"), t))
+            return sum(w * r for w, r in zip(t["dwa"][0], results))
+        x = x + y
+        return x + _f64_ff(l, norm(x, t, "norm2"), t) if l.ff else x
+    for i, name, v in _stack_tensors(case, seed):
+        if name == "embed":
+            x = v[torch.tensor(tokens, device=DEV).long()].double()
+            results.append(x)
+            continue
+        if name == "pos":
+            x = x + v[:len(tokens)].double()
+            continue
+        if i != at and t:  # a layer's tensors are complete
+            x, t = layer(x, layers[at], t), {}
+        at = i
+        t[name] = v.double() if v.dim() > 1 else v.double()[None]
+    logits = norm(x[torch.tensor(want, device=DEV)], t, "final.norm") @ t["head"].T
+    logits = logits if soft else 30 * torch.tanh(logits / 30)
+    return logits[0] if case["op"] == "prompt" else list(logits)
+
+
+def exact(case, seed):
+    op = case["op"]
+    if op == "codec":
+        return [None, _codec_inputs(case, seed)[1][1]()[:case["numel"]]]
+    if op in ("linear", "gemm"):
+        w, x, bias = _linear_inputs(case, seed)
+        x = (x if op == "linear" else x.bfloat16()).double()
+        y = x @ pack(case["type"], w)[1]().view(case["n"], case["k"]).T
+        return y if bias is None else y + bias.double()
+    return _f64_llama(case, seed) if case["model"] == "llama" else _f64_stack(case, seed)
