@@ -172,6 +172,7 @@ def _upload(ctx, kind, n, k, packed):
     torch.cuda.synchronize()
     h = ctypes.c_void_p()
     ctx.check(ctx.lib.axq_weight_upload(ctx.handle, int(QuantType[kind]), n, k, packed.data_ptr(), packed.numel(), MEM_DEVICE, ctypes.byref(h)))
+    ctx.synchronize()  # `packed` may be freed now
     return DeviceWeight(ctx, h, QuantType[kind], n, k)
 
 
