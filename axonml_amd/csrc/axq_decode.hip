@@ -912,6 +912,17 @@ bool all_layers_in_small_batch_reach(const axq_model *m, int nb) {
     return true;
 }
 
+// Fewest rows from which the layers' linears go through the GEMM: where all of them are superblock types as soon as the
+// small-batch GEMV would need a second pass over the weights, else PROMPT_GEMM_MIN where that GEMV is the alternative, and eight
+// where single-vector passes are.
+int gemm_rows_min(const axq_model *m, int nb) {
+    bool rows = true;
+    for (int l = 0; l < m->cfg.num_hidden_layers; l++)
+        for (const axq_weight *w : {m->w_qkv[l], m->w_o[l], m->w_gu[l], m->w_down[l], m->w_sep[0][l], m->w_sep[1][l], m->w_sep[2][l]})
+            rows = rows && (!w || axq_dev_rows_gemm_covers(w));
+    return rows ? AXQ_ROWS_GEMM_MIN : all_layers_in_small_batch_reach(m, nb) ? PROMPT_GEMM_MIN : PROMPT_BATCH;
+}
+
 template <class T>
 hipError_t dev_alloc(T **p, size_t count);
 
@@ -1141,7 +1152,7 @@ int feed_rows(axq_model *m, int seq, const int32_t *toks, int n, int pos0, int *
         r.mode = ROWS_NONE; r.toks = toks + i; r.per_seq = false; r.seq = seq; r.pos0 = pos0 + i; r.split_attn = false;
         // enough rows to fill GEMM tiles (fewer where the small-batch GEMV does not apply and single rows are the alternative)
         r.nb = left < m->prompt_chunk ? left : m->prompt_chunk;
-        if (allow >= 2 && r.nb >= (all_layers_in_small_batch_reach(m, left) ? PROMPT_GEMM_MIN : PROMPT_BATCH) &&
+        if (allow >= 2 && r.nb >= gemm_rows_min(m, left) &&
             rows_mode_covers(m, ROWS_GEMM, r.pos0 + r.nb, r.nb))
             r.mode = ROWS_GEMM;
         if (r.mode == ROWS_NONE) {
@@ -1183,9 +1194,10 @@ int run_batch_step(axq_model *m, int max_pos_now) {
     r.lds = prompt_attn_lds(m, r.split_attn ? 1 : m->fused_max);
     static const bool no_graph = getenv("AXQ_DECODE_GRAPH") && getenv("AXQ_DECODE_GRAPH")[0] == '0';
     int rc;
-    if (m->n_seq > PROMPT_BATCH && m->n_seq <= GEMV_GROUPS_MAX && all_layers_in_small_batch_reach(m, PROMPT_BATCH)) {
-        // a few more rows than the small-batch GEMV takes: groups of eight sequences, one after the other (three passes
-        // over the weights at 2.4 ms each still beat the GEMM's 8.5-10 ms at the 7B shape); plain launches
+    if (m->n_seq > PROMPT_BATCH && m->n_seq <= GEMV_GROUPS_MAX && m->n_seq < gemm_rows_min(m, PROMPT_BATCH) &&
+        all_layers_in_small_batch_reach(m, PROMPT_BATCH)) {
+        // a few more rows than the small-batch GEMV takes, and not all weights of superblock types: groups of eight sequences,
+        // one after the other; plain launches
         rc = AXQ_OK;
         for (int s = 0; s < m->n_seq && !rc; s += PROMPT_BATCH) {
             Rows g = r;

@@ -1,0 +1,867 @@
+// Rows times a packed weight of a superblock type: y[M, N] = x[M, K] * W[N, K]^T on v_mfma_f32_32x32x16_f16, for f32 rows
+// (nine of them up to a prompt) and bf16 rows.  The reference composition is dequantize_tensor -> f32 sgemm
+// (crates/axonml-quant/src/dequantize.rs:34-54, crates/axonml-core/src/backends/cpu.rs:566-598).
+//
+// Time of a call with f32 rows, Q4_K, before (groups of eight vectors, or two-stage operands in LDS) and now, us:
+//   rows            16          32          64
+//   28672 x 4096    40.5 28.0   81.5 35.9   61.8 54.0
+//   4096 x 4096     21.8 15.3   43.0 18.3   33.0 23.8
+//   4096 x 14336    32.0 26.2   63.2 31.0   63.9 40.0
+// What bounds it: at few rows the fixed parts (pre-pass, reduction and the launches around them: 14 us of the 4096 x 4096 calls) and
+// 0.35 us per step of barrier and LDS reads; at many the matrix pipe beside the vector instructions that make operands (2048 bf16 rows
+// x 14336: 320 us, 750 TFLOP/s), which overlap only in part.
+//
+// Numerics.  A bf16 row goes in as f16 under a power-of-two row scale (exact), an f32 row as two f16 rows, leading eleven
+// bits and remainder, whose results are added (22 bits).  A weight goes in without rounding:
+//   Q4_K, Q5_K   w = d (sc (q - C)) + (C d sc - dmin m), C = 8 or 16: sc (q - C) is an integer below 2^10, exact in f16, and is
+//                the operand; sums of them are in units of d.  A step's sum starts from zero and joins the total times d, or, where
+//                registers are short (more than 128 rows), the accumulators of a column hold the running sum and change their
+//                unit at a superblock boundary (one multiply per register and 256 k).  The offset, one number per sub-block of
+//                32, joins in the same unit as an f16 pair, against the sub-block's sum of x as an f16 pair: two products more
+//                per superblock.  Where dmin is so large beside d that the pair would leave f16's range, the unit is d times a
+//                power of two and the operands are divided by it (exact).
+//   Q6_K         w = d sc (q - 32): sc (q - 32) has 13 bits and goes in as two exact operands, sc times the multiple of eight
+//                and sc times the rest, two products per weight.
+// Centred codes because sums over uncentred ones cancel for rows with a mean.  Accumulation is f32 throughout.
+//
+// Shape.  A workgroup of eight waves; a wave computes 32 MI x 32 NJ outputs.  Four waves lie side by side along N; the other
+// factor of two is rows (WM = 2: 64 MI rows) or K (WM = 1: each four waves take half of the workgroup's superblocks, and the
+// two sums meet in LDS).  What the design turns on:
+//   - weights never pass through LDS as operands.  Their packed codes come into LDS as they are (global_load_lds, two K steps
+//     at a time, up to three such units ahead), a lane reads the 16 bytes it multiplies with and makes the B operand in registers:
+//     eleven vector instructions per eight Q4 codes ((w & 0x00F000F0) | 0x5400 is the f16 pair 64 + q, one packed multiply-add
+//     makes sc (q - 8) of it).  An operand written to LDS and read back costs four times the bytes, and binds conversion to
+//     the barrier.
+//   - x lies in memory in operand order (rows_prep_kernel): a wave's fragment is one kilobyte, lane after lane, so the copy
+//     into LDS is linear and the fragment reads are free of conflicts.
+//   - one barrier per K step of 64, in front of the step's last products: the next step's first fragments are requested
+//     behind it and arrive while those products run.
+#include <hip/hip_fp16.h>
+
+#include <type_traits>
+
+#include "axq_internal.h"
+
+namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float float16v __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_void;
+typedef const __attribute__((address_space(1))) void gbl_void;
+
+struct RowsArgs {
+    const uint8_t *codes, *meta, *qh;
+    uint32_t codes_pitch, meta_pitch, qh_pitch;
+    const _Float16 *xa;    // x in operand order: [tile of 32 rows][step of 64 k][t = 0..3][lane][8]
+    const _Float16 *xs;    // its sub-block sums: [tile][superblock][leading halves, remainders][lane][8]: sub-blocks 4 (lane / 32) .., twice
+    const float *rowscale; // [m]
+    float *y, *ypart;      // ypart: [splits][rows][n] unscaled sums (NULL: one workgroup covers all of K)
+    int m, n, k;           // m rows of xa; with `pair` rows 2t and 2t + 1 are the parts of row t, and y has m / 2 rows
+    int sb_per_split, pair;
+    const float *bias, *resid;
+};
+
+__device__ inline float h2f(uint32_t bits) { return (float)__builtin_bit_cast(_Float16, (unsigned short)bits); }
+__device__ inline half2v halfs(uint32_t v) { return __builtin_bit_cast(half2v, v); }
+__device__ inline uint32_t bits(half2v v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ inline half2v pk2(float v) { return __builtin_bit_cast(half2v, __builtin_amdgcn_cvt_pkrtz(v, v)); } // exact for what is put in
+__device__ inline half8 octet(const uint32_t (&o)[4]) { return __builtin_bit_cast(half8, u32x4{o[0], o[1], o[2], o[3]}); }
+
+template <int N>
+__device__ inline void wait_loads_and_lds() { // s_waitcnt vmcnt(N) lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(((N >> 4) << 14) | (7 << 4) | (N & 15));
+    asm volatile("" ::: "memory");
+}
+__device__ inline void barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// A lane of an operand of step j (0..3) of a superblock, product t (0..3): elements 64 j + 32 (t / 2) + 16 (lane / 32) + 8 (t % 2)
+// + {0, 2, 1, 3, 4, 6, 5, 7}: the order in which masks take code pairs out of a dword.
+//
+// A block type says
+//   PAIRS    32-byte pieces of a row's codes per unit of two steps; piece_src: the first byte of one, in row 0
+//   SIDE16, SIDE4   16-byte and 4-byte pieces of a row's superblock besides codes (scales, fifth bits); side_src
+//   Side, Raw       what a lane reads of them, and of the codes per step, from LDS
+//   make     the operand(s) of product t; PRODUCTS operands per weight; MIN: there is an offset term
+template <bool Q5>
+struct SuperQ45 {
+    static constexpr int PAIRS = 2, PRODUCTS = 1, SIDE16 = Q5 ? 3 : 1, SIDE4 = 0;
+    static constexpr bool MIN = true;
+    static constexpr float CENTRE = Q5 ? 16.0f : 8.0f;
+    struct Side { u32x4 h, b; };
+    struct Raw { u32x4 q; };
+    // piece p: the 16-byte halves p of two neighbouring pairs of sub-blocks (see q4k_code_offset)
+    __device__ static const uint8_t *piece_src(const RowsArgs &a, int unit, int p) {
+        const int pair = 2 * unit, slice = pair >> 6, left = (a.k >> 6) - (slice << 6), P = left < 64 ? left : 64;
+        return a.codes + (size_t)slice * 2048 + (size_t)(p * 16 * P + (pair & 63) * 16);
+    }
+    __device__ static uint32_t piece_pitch(const RowsArgs &a, int) { return a.codes_pitch; }
+    __device__ static const uint8_t *side_src(const RowsArgs &a, int sb, int c) { // the header, then the two halves of the fifth bits
+        return c == 0 ? a.meta + (size_t)sb * 16 : a.qh + (size_t)sb * 32 + (c - 1) * 16;
+    }
+    __device__ static uint32_t side_pitch(const RowsArgs &a, int c) { return c == 0 ? a.meta_pitch : a.qh_pitch; }
+    template <int N>
+    __device__ static void read_side(const uint8_t *stage, int row, int hh, int, Side &s) {
+        s.h = *reinterpret_cast<const u32x4 *>(stage + row * 16);
+        if constexpr (Q5) s.b = *reinterpret_cast<const u32x4 *>(stage + (1 + hh) * N * 16 + row * 16);
+    }
+    // u, the accumulators' unit for a superblock, inv = 1 / u and shrink = d / u: u = d 2^p, p = 0 unless dmin / d >= 64 (p <= 24:
+    // operands stay multiples of f16's smallest number); dmin where d = 0; 0 for a superblock of zeros
+    __device__ static void unit_of(const Side &s, float &u, float &inv, float &shrink) {
+        const float d = h2f(s.h[0] & 0xFFFFu), dm = h2f(s.h[0] >> 16);
+        auto expo = [](float v) { return (int)((__builtin_bit_cast(uint32_t, v) >> 23) & 0xFF); };
+        int p = expo(dm) - expo(d) - 5;
+        p = p < 0 ? 0 : (p > 24 ? 24 : p);
+        u = d == 0.f ? dm : d * __builtin_bit_cast(float, (uint32_t)(127 + p) << 23);
+        shrink = d == 0.f ? 0.f : __builtin_bit_cast(float, (uint32_t)(127 - p) << 23);
+        inv = 1.0f / (u == 0.f ? 1.0f : u);
+    }
+    // four of the offsets of a superblock, sub-blocks 4 hh .. 4 hh + 3, in units of u and times eight (their sums of x come times
+    // 1 / 8), |.| <= 8 (16 * 63 + 64 * 63): leading halves, then remainders
+    __device__ static half8 offsets(const Side &s, int hh, float inv) {
+        // C d sc - dmin m: both products exact (11 x 6 bits), so that their difference loses nothing where they nearly cancel
+        const float dc = CENTRE * h2f(s.h[0] & 0xFFFFu), dm = -h2f(s.h[0] >> 16), to_unit = 8.0f * inv;
+        const uint32_t sc = hh ? (s.h[3] & 0x0F0F0F0Fu) | ((s.h[1] >> 2) & 0x30303030u) : s.h[1] & 0x3F3F3F3Fu;
+        const uint32_t mn = hh ? ((s.h[3] >> 4) & 0x0F0F0F0Fu) | ((s.h[2] >> 2) & 0x30303030u) : s.h[2] & 0x3F3F3F3Fu;
+        uint32_t o[4];
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const float c0 = fmaf((float)((sc >> (16 * p)) & 0xFF), dc, (float)((mn >> (16 * p)) & 0xFF) * dm) * to_unit;
+            const float c1 = fmaf((float)((sc >> (16 * p + 8)) & 0xFF), dc, (float)((mn >> (16 * p + 8)) & 0xFF) * dm) * to_unit;
+            const half2v h = __builtin_bit_cast(half2v, __builtin_amdgcn_cvt_pkrtz(c0, c1)); // the leading eleven bits
+            o[p] = bits(h);
+            o[2 + p] = bits(half2v{(_Float16)(c0 - (float)h[0]), (_Float16)(c1 - (float)h[1])});
+        }
+        return octet(o);
+    }
+    __device__ static void read_raw(const uint8_t *tile, int col, int hh, int j, Raw &r) {
+        r.q = *reinterpret_cast<const u32x4 *>(tile + hh * 1024 + ((col * 2) + ((j & 1) ^ ((col >> 3) & 1))) * 16);
+    }
+    // per superblock: sub-block scales times shrink, two to a dword (2p low, 2p + 1 high), and -(64 + C) times them; both exact
+    // (72 * 63 = 8 * 567, 80 * 63 = 16 * 315)
+    struct Scales { half2v sc[4], off[4]; };
+    __device__ static void scales(const Side &s, float shrink, int, Scales &o) {
+        const uint32_t lo = s.h[1] & 0x3F3F3F3Fu, hi = (s.h[3] & 0x0F0F0F0Fu) | ((s.h[1] >> 2) & 0x30303030u); // sub-blocks 0..3, 4..7
+        const half2v k = {(_Float16)-1024.0f, (_Float16)-1024.0f}, f = pk2(shrink);
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            const uint32_t pair = __builtin_amdgcn_perm(0x64646464u, p < 2 ? lo : hi, (p & 1) ? 0x04030402u : 0x04010400u); // 1024 + scale
+            o.sc[p] = (halfs(pair) + k) * f;
+            o.off[p] = o.sc[p] * (_Float16)(-(64.0f + CENTRE));
+        }
+    }
+    __device__ static void make(const Raw &r, const Side &s, const Scales &c, uint32_t mask, int j, int t, half8 (&o)[1]) {
+        const half2v sc = (t >> 1) ? __builtin_shufflevector(c.sc[j], c.sc[j], 1, 1) : __builtin_shufflevector(c.sc[j], c.sc[j], 0, 0);
+        const half2v off = (t >> 1) ? __builtin_shufflevector(c.off[j], c.off[j], 1, 1) : __builtin_shufflevector(c.off[j], c.off[j], 0, 0);
+        uint32_t w[4];
+#pragma unroll
+        for (int d = 0; d < 2; d++) {
+            const uint32_t q = r.q[2 * (t & 1) + d];
+            // a code at bits 4..7 (4..8) of a half with 0x5400 is the f16 number 64 + q
+            uint32_t e = (((t >> 1) ? q : q << 4) & mask) | 0x54005400u, f = (((t >> 1) ? q >> 8 : q >> 4) & mask) | 0x54005400u;
+            if constexpr (Q5) {
+                const uint32_t b = s.b[2 * (t & 1) + d] >> (2 * j + (t >> 1)); // bit 0 of every byte
+                e |= (b & 0x00010001u) << 8;
+                f |= b & 0x01000100u;
+            }
+            w[2 * d] = bits(__builtin_elementwise_fma(halfs(e), sc, off));
+            w[2 * d + 1] = bits(__builtin_elementwise_fma(halfs(f), sc, off));
+        }
+        o[0] = octet(w);
+    }
+};
+
+struct SuperQ6 {
+    static constexpr int PAIRS = 3, PRODUCTS = 2, SIDE16 = 1, SIDE4 = 1;
+    static constexpr bool MIN = false;
+    struct Side { u32x4 sc; uint32_t d; };
+    struct Raw { u32x4 ql[2], qh; };
+    // a unit is half a superblock, 128 elements: pieces 0 and 1 its 64 bytes of low nibbles, piece 2 its 32 bytes of bit pairs
+    __device__ static const uint8_t *piece_src(const RowsArgs &a, int unit, int p) {
+        return p < 2 ? a.codes + (size_t)unit * 64 + p * 32 : a.qh + (size_t)unit * 32;
+    }
+    __device__ static uint32_t piece_pitch(const RowsArgs &a, int p) { return p < 2 ? a.codes_pitch : a.qh_pitch; }
+    __device__ static const uint8_t *side_src(const RowsArgs &a, int sb, int c) { // the scales; the d of this superblock and its neighbour
+        return c == 0 ? a.meta + (size_t)sb * 16 : a.meta + (size_t)(a.k >> 8) * 16 + (size_t)(sb & ~1) * 2;
+    }
+    __device__ static uint32_t side_pitch(const RowsArgs &a, int) { return a.meta_pitch; }
+    template <int N>
+    __device__ static void read_side(const uint8_t *stage, int row, int, int sb, Side &s) {
+        s.sc = *reinterpret_cast<const u32x4 *>(stage + row * 16);
+        s.d = (*reinterpret_cast<const uint32_t *>(stage + N * 16 + row * 4) >> (16 * (sb & 1))) & 0xFFFFu;
+    }
+    __device__ static void unit_of(const Side &s, float &u, float &inv, float &shrink) {
+        u = h2f(s.d);
+        inv = 1.0f / (u == 0.f ? 1.0f : u);
+        shrink = u == 0.f ? 0.f : 1.0f;
+    }
+    __device__ static void read_raw(const uint8_t *tile, int col, int hh, int, Raw &r) {
+        const uint8_t *at = tile + (col * 2 + (hh ^ ((col >> 3) & 1))) * 16;
+        r.ql[0] = *reinterpret_cast<const u32x4 *>(at);
+        r.ql[1] = *reinterpret_cast<const u32x4 *>(at + 1024);
+        r.qh = *reinterpret_cast<const u32x4 *>(at + 2048);
+    }
+    // this lane's scales, dword j = step j: sub-blocks 4 j + hh (low half) and 4 j + 2 + hh, as f16
+    struct Scales { half2v sc[4]; };
+    __device__ static void scales(const Side &s, float shrink, int hh, Scales &o) {
+        const half2v f = pk2(shrink);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t b = hh ? s.sc[j] >> 8 : s.sc[j];
+            o.sc[j] = half2v{(_Float16)(short)(int8_t)(b & 0xFF), (_Float16)(short)(int8_t)((b >> 16) & 0xFF)} * f;
+        }
+    }
+    // element byte l of the unit: nibble j % 2 of ql[t / 2], bits 2 (2 (j % 2) + t / 2) of qh
+    __device__ static void make(const Raw &r, const Side &, const Scales &c, uint32_t, int j, int t, half8 (&o)[2]) {
+        const half2v f = (t >> 1) ? __builtin_shufflevector(c.sc[j], c.sc[j], 1, 1) : __builtin_shufflevector(c.sc[j], c.sc[j], 0, 0);
+        const half2v c1 = {(_Float16)-1056.0f, (_Float16)-1056.0f}, c0 = {(_Float16)-1024.0f, (_Float16)-1024.0f};
+        uint32_t hi[4], lo[4];
+#pragma unroll
+        for (int d = 0; d < 2; d++) {
+            const int at = 2 * (t & 1) + d;
+            const uint32_t u = ((r.ql[t >> 1][at] >> (4 * (j & 1))) & 0x0F0F0F0Fu) | (((r.qh[at] >> (2 * (2 * (j & 1) + (t >> 1)))) & 0x03030303u) << 4);
+            const uint32_t v = u >> 8;
+            hi[2 * d] = bits((halfs((u & 0x00380038u) | 0x64006400u) + c1) * f);
+            hi[2 * d + 1] = bits((halfs((v & 0x00380038u) | 0x64006400u) + c1) * f);
+            lo[2 * d] = bits((halfs((u & 0x00070007u) | 0x64006400u) + c0) * f);
+            lo[2 * d + 1] = bits((halfs((v & 0x00070007u) | 0x64006400u) + c0) * f);
+        }
+        o[0] = octet(hi);
+        o[1] = octet(lo);
+    }
+};
+
+// Stages in LDS: NA K steps of x, NW units of codes, the sides and the sums of x of two superblocks.  Half of a group's waves
+// copy x, the other half codes and sides: a wave's waits are in order of its requests, and x, which comes from L2 shortly before
+// it is used, would otherwise wait for codes that were requested from memory for later.
+template <class T, int MI, int WM, int NJ>
+struct RowsTile {
+    static constexpr int KG = 2 / WM, GW = 4 * WM, CW = GW / 2;     // groups along K, waves of one, waves that copy x (and codes)
+    static constexpr int M = 32 * MI * WM, N = 128 * NJ;
+    static constexpr bool WHOLE = MI <= 2;                          // the fragments of a whole step ahead in registers
+    static constexpr int HB = T::PAIRS * 32;                        // code bytes of a row and unit
+    static constexpr int ABYTES = WM * MI * 4096, WBYTES = N * HB, SBYTES = T::MIN ? WM * MI * 2048 : 0; // of a group's stage
+    static constexpr int DBYTES = N * (16 * T::SIDE16 + 4 * T::SIDE4);
+    static constexpr int NA = WHOLE ? 3 : 2;
+    static constexpr int FIT = (160 * 1024 - KG * (NA * ABYTES + 2 * SBYTES + 2 * DBYTES)) / (KG * WBYTES), NW = FIT > 4 ? 4 : FIT;
+    static constexpr int MAIL = KG == 2 ? 8 * MI * NJ * 8 * 64 * 4 : 0; // the groups' exchange, which reuses the stages
+    static constexpr int STAGES = KG * (NA * ABYTES + NW * WBYTES + 2 * SBYTES + 2 * DBYTES), LDS = STAGES > MAIL ? STAGES : MAIL;
+    // a copying wave's requests: x of a step, sums of a superblock; codes of a unit, sides of a superblock (small ones some of them twice)
+    static constexpr int XL = 2 * MI, SL = T::MIN ? MI : 0, WT = 4 * NJ / CW, WL = WT * T::PAIRS;
+    static constexpr int D16 = (2 * NJ * T::SIDE16 + CW - 1) / CW, D4 = (2 * NJ * T::SIDE4 + CW - 1) / CW;
+    static constexpr int FIRST = 7 > 2 * NW - 1 ? 7 : 2 * NW - 1;
+    static_assert(NW >= 2 && WT * CW == 4 * NJ && NA <= FIRST, "stages");
+    // Behind barrier b: x of step b + NA and, where b % 4 = 1, the sums of superblock (b + 3) / 4; codes of unit (b + 1) / 2 + NW - 1
+    // where b is odd and the sides of superblock (b + 7) / 4 where b % 4 = 1.  In front of barrier g everything that is read
+    // behind it must have come (x and codes of step g + 1, at a superblock's end sums and sides of the next): how many of the wave's
+    // requests may still be under way then.
+    static constexpr int allowed_x(int g) {
+        int total = 0, need = 0;
+        g += 64;
+        for (int b = g - 60; b < g; b++) {
+            total += XL;
+            if (b + NA == g + 1) need = total;
+            if (b % 4 == 1) {
+                total += SL;
+                if (SL && g % 4 == 3 && b == g - 2 && total > need) need = total;
+            }
+        }
+        return total - need > 63 ? 63 : total - need;
+    }
+    static constexpr int allowed_w(int g) {
+        int total = 0, need = 0;
+        g += 64;
+        for (int b = g - 60; b < g; b++) {
+            if (b & 1) {
+                total += WL;
+                if ((g & 1) && b == g - 2 * (NW - 1)) need = total;
+            }
+            if (b % 4 == 1) {
+                total += D16 + D4;
+                if (g % 4 == 3 && b == g - 6 && total > need) need = total;
+            }
+        }
+        return (g & 1) == 0 || total - need > 63 ? 63 : total - need;
+    }
+};
+
+template <class T, int MI, int WM, int NJ>
+__global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
+    using Tile = RowsTile<T, MI, WM, NJ>;
+    constexpr int KG = Tile::KG, HB = Tile::HB, ABYTES = Tile::ABYTES, WBYTES = Tile::WBYTES, SBYTES = Tile::SBYTES, DBYTES = Tile::DBYTES, NA = Tile::NA, NW = Tile::NW;
+    extern __shared__ uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 31, hh = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = wave / Tile::GW, wi = wave % Tile::GW, wm = WM == 2 ? wi >> 2 : 0, wn = wave & 3;
+    const int nt = (a.n + Tile::N - 1) / Tile::N, total = (int)gridDim.x;
+    int tile = blockIdx.x;
+    if (total % 8 == 0) tile = (tile & 7) * (total >> 3) + (tile >> 3); // workgroups of one XCD share x tiles
+    const int mt0 = (tile / nt) * (WM * MI), n0 = (tile % nt) * Tile::N;
+    const int nsb_row = a.k >> 8, steps_row = a.k >> 6;
+    const int lo = (int)blockIdx.y * a.sb_per_split, hi = lo + a.sb_per_split < nsb_row ? lo + a.sb_per_split : nsb_row;
+    // superblocks of this group: `loops` is what every wave of the workgroup walks through, `mine` what this group multiplies
+    const int loops = (hi - lo + KG - 1) / KG, sb0 = lo + kg * loops;
+    const int mine = hi - sb0 < loops ? (hi - sb0 > 0 ? hi - sb0 : 0) : loops;
+    uint8_t *abase = lds + kg * NA * ABYTES, *wbase = lds + KG * NA * ABYTES + kg * NW * WBYTES;
+    uint8_t *sbase = lds + KG * (NA * ABYTES + NW * WBYTES) + kg * 2 * SBYTES, *dbase = sbase + (KG - kg) * 2 * SBYTES + kg * 2 * DBYTES;
+    const bool x_wave = wi < Tile::CW; // copies x, the others codes and sides
+    const int cw = x_wave ? wi : wi - Tile::CW;
+
+    // ---- copies into LDS (past the end of the row: its last step, unit or superblock again, which nobody looks at)
+    auto copy = [&](const void *src, uint8_t *dst) { __builtin_amdgcn_global_load_lds((gbl_void *)src, (lds_void *)dst, 16, 0, 0); };
+    auto in_order = [] { asm volatile("" ::: "memory"); }; // the waits in front of the barriers count on the order of the requests
+    auto copy_x = [&](int g, int at) { // x of step g of the group into the stage at byte `at`
+        int step = sb0 * 4 + g;
+        step = step < steps_row ? step : steps_row - 1;
+#pragma unroll
+        for (int q = 0; q < Tile::XL; q++) {
+            const int kb = cw * Tile::XL + q, mt = kb >> 2, t = kb & 3;
+            copy(a.xa + ((size_t)(mt0 + mt) * steps_row + step) * 2048 + t * 512 + lane * 8, abase + at + kb * 1024);
+        }
+        in_order();
+    };
+    auto copy_sums = [&](int sb) {
+        const int at = sb0 + sb < nsb_row ? sb0 + sb : nsb_row - 1;
+#pragma unroll
+        for (int q = 0; q < Tile::SL; q++) {
+            const int kb = cw * Tile::SL + q;
+            copy(a.xs + ((size_t)(mt0 + (kb >> 1)) * nsb_row + at) * 1024 + (kb & 1) * 512 + lane * 8, sbase + (sb & 1) * SBYTES + kb * 1024);
+        }
+        in_order();
+    };
+    // codes: lane -> (row of 32, 16-byte half of its piece): the halves of rows 8..15 and 24..31 change places, so that sixteen
+    // lanes that read the same half of consecutive rows touch all banks
+    const int cr = lane >> 1, cs = (lane & 1) ^ ((cr >> 3) & 1);
+    auto row_of = [&](int r) { return (uint32_t)(n0 + r < a.n ? r : a.n - 1 - n0); }; // row r of the tile; past the end the last one
+    auto copy_codes = [&](int u, int at) { // codes of unit u of the group
+        int unit = sb0 * 2 + u;
+        unit = unit < 2 * nsb_row ? unit : 2 * nsb_row - 1;
+#pragma unroll
+        for (int q = 0; q < Tile::WT; q++) {
+            const int ct = cw * Tile::WT + q; // column tile of 32 rows
+            const uint32_t row = row_of(ct * 32 + cr);
+#pragma unroll
+            for (int p = 0; p < T::PAIRS; p++)
+                copy(T::piece_src(a, unit, p) + (size_t)n0 * T::piece_pitch(a, p) + (row * T::piece_pitch(a, p) + cs * 16),
+                     wbase + at + ct * 32 * HB + p * 1024);
+        }
+        in_order();
+    };
+    auto copy_sides = [&](int sb) { // 64 rows of a piece at a time
+        const int at = sb0 + sb < nsb_row ? sb0 + sb : nsb_row - 1;
+        uint8_t *dst = dbase + (sb & 1) * DBYTES;
+#pragma unroll
+        for (int q = 0; q < Tile::D16; q++) {
+            const int ii = (cw + q * Tile::CW) % (2 * NJ * T::SIDE16), c = ii / (2 * NJ), r0 = ii % (2 * NJ) * 64;
+            copy(T::side_src(a, at, c) + (size_t)n0 * T::side_pitch(a, c) + row_of(r0 + lane) * T::side_pitch(a, c), dst + c * Tile::N * 16 + r0 * 16);
+        }
+#pragma unroll
+        for (int q = 0; q < Tile::D4; q++) {
+            const int r0 = (cw + q * Tile::CW) % (2 * NJ) * 64;
+            __builtin_amdgcn_global_load_lds((gbl_void *)(T::side_src(a, at, T::SIDE16) + (size_t)n0 * T::side_pitch(a, T::SIDE16) +
+                                                          row_of(r0 + lane) * T::side_pitch(a, T::SIDE16)),
+                                             (lds_void *)(dst + T::SIDE16 * Tile::N * 16 + r0 * 4), 4, 0, 0);
+        }
+        in_order();
+    };
+
+    // ---- products
+    float16v acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+    float unit[NJ], ratio[NJ], inv[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) unit[j] = 1.0f;
+    typename T::Side side[NJ], next_side[NJ];
+    typename T::Scales scales[NJ];
+    uint32_t mask; // in a vector register: an instruction takes one scalar operand, and (w & mask) | base has its base there
+    asm("v_mov_b32 %0, 0x00f000f0" : "=v"(mask));
+    auto read_sides = [&](int sb) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) T::template read_side<Tile::N>(dbase + (sb & 1) * DBYTES, (wn * NJ + j) * 32 + li, hh, sb0 + sb, next_side[j]);
+    };
+    auto new_side = [&](bool last = false) { // what the superblock in `side` asks for; where accumulators change their unit, they do with its first product
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            float u, shrink;
+            T::unit_of(side[j], u, inv[j], shrink);
+            T::scales(side[j], shrink, hh, scales[j]);
+            if (Tile::WHOLE) {
+                unit[j] = u;
+            } else {
+                const bool keep = u == 0.f || last; // behind the last superblock the accumulators stay as they are
+                ratio[j] = keep ? 1.0f : unit[j] / u;
+                unit[j] = keep ? unit[j] : u;
+            }
+        }
+    };
+    const uint8_t *my_x = abase + wm * MI * 4096 + lane * 16, *my_codes = wbase + wn * NJ * 32 * HB;
+    int a_rd = 0, w_rd = 0; // stage of the step, of the unit that is read next
+    auto read_x = [&](int t, half8 (&f)[MI]) {
+#pragma unroll
+        for (int i = 0; i < MI; i++) f[i] = *reinterpret_cast<const half8 *>(my_x + a_rd + i * 4096 + t * 1024);
+    };
+    auto read_codes = [&](int j4, typename T::Raw (&raw)[NJ]) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) T::read_raw(my_codes + w_rd + j * 32 * HB, li, hh, j4, raw[j]);
+    };
+    // behind the barrier of step 4 sb + J: the stages of that step have been read by everybody, and what the next one reads is there
+    auto meet = [&](int sb, auto step) {
+        constexpr int J = decltype(step)::value;
+        if (x_wave) {
+            wait_loads_and_lds<Tile::allowed_x(J)>();
+            barrier();
+            copy_x(4 * sb + J + NA, a_rd);
+            if (J == 1 && T::MIN) copy_sums(sb + 1);
+        } else {
+            wait_loads_and_lds<Tile::allowed_w(J)>();
+            barrier();
+            if (J & 1) copy_codes(2 * sb + (J >> 1) + NW, w_rd);
+            if (J == 1) copy_sides(sb + 2);
+        }
+        a_rd = a_rd == (NA - 1) * ABYTES ? 0 : a_rd + ABYTES;
+        if (J & 1) w_rd = w_rd == (NW - 1) * WBYTES ? 0 : w_rd + WBYTES;
+    };
+    auto change_unit = [&]() {
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int q = 0; q < 16; q++) acc[i][j][q] *= ratio[j];
+    };
+    auto make = [&](const typename T::Raw (&raw)[NJ], int j4, int t, half8 (&f)[NJ][T::PRODUCTS]) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) T::make(raw[j], side[j], scales[j], mask, j4, t, f[j]);
+    };
+    auto multiply = [&](const half8 (&x)[MI], const half8 (&w)[NJ][T::PRODUCTS]) {
+#pragma unroll
+        for (int pr = 0; pr < T::PRODUCTS; pr++)
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[i], w[j][pr], acc[i][j], 0, 0, 0);
+    };
+    auto add_offsets = [&](int sb, auto tile_j) { // of a column tile
+        if constexpr (T::MIN) {
+            constexpr int j = decltype(tile_j)::value;
+            const half8 o = T::offsets(side[j], hh, inv[j]);
+#pragma unroll
+            for (int i = 0; i < MI; i++) {
+                const uint8_t *x = sbase + (sb & 1) * SBYTES + (wm * MI + i) * 2048 + lane * 16;
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x), o, acc[i][j], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x + 1024), o, acc[i][j], 0, 0, 0);
+            }
+        }
+    };
+    using S0 = std::integral_constant<int, 0>; using S1 = std::integral_constant<int, 1>;
+    using S2 = std::integral_constant<int, 2>; using S3 = std::integral_constant<int, 3>;
+#pragma unroll
+    for (int b = -Tile::FIRST; b < 0; b++) { // the requests in front of the first step, in the order of the later ones
+        if (x_wave) {
+            if (b + NA >= 0) copy_x(b + NA, (b + NA) * ABYTES);
+            if (b == -3 && T::MIN) copy_sums(0);
+        } else {
+            if ((b & 1) && (b + 1) / 2 + NW - 1 >= 0) copy_codes((b + 1) / 2 + NW - 1, ((b + 1) / 2 + NW - 1) * WBYTES);
+            if (b == -7 || b == -3) copy_sides((b + 7) / 4);
+        }
+    }
+    if (x_wave) wait_loads_and_lds<Tile::allowed_x(3)>();
+    else wait_loads_and_lds<Tile::allowed_w(3)>();
+    barrier();
+    read_sides(0);
+    if constexpr (Tile::WHOLE) { // meet, request the next step's fragments, work on this step's
+        half8 af[2][4][MI];
+        typename T::Raw raw[2][NJ];
+        // a step's products start from zero and their sum joins the total times d: fewer of the additions that round are of the
+        // total's size.  Error against 64 bits, f32 rows of normal x, K = 1024 / 4096 / 14336, Q4_K: 1.0 / 1.1 / 1.25e-7 (a
+        // superblock's products in one sum: 1.3 / 1.4 / 1.45e-7; the two-stage kernel before it, from 40 rows on: 1.3 / 1.8 / 3.1e-7;
+        // the small-batch GEMV: 0.95 / 1.05 / 1.3e-7)
+        float16v sum[MI][NJ];
+        auto fold = [&]() {
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++)
+#pragma unroll
+                    for (int q = 0; q < 16; q++) {
+                        sum[i][j][q] = fmaf(acc[i][j][q], unit[j], sum[i][j][q]);
+                        acc[i][j][q] = 0.f;
+                    }
+        };
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) sum[i][j] = acc[i][j];
+        auto read_step = [&](int j4) {
+            read_codes(j4, raw[j4 & 1]);
+#pragma unroll
+            for (int t = 0; t < 4; t++) read_x(t, af[j4 & 1][t]);
+            asm volatile("" ::: "memory"); // requested here, not where they are used
+        };
+        auto step = [&](int sb, auto at) {
+            constexpr int J = decltype(at)::value;
+            meet(sb, at);
+            read_step((J + 1) & 3);
+            if (J == 3) read_sides(sb + 1); // looked at behind the next barrier
+            fold();
+            if (J == 0) {
+#pragma unroll
+                for (int j = 0; j < NJ; j++) side[j] = next_side[j];
+                new_side();
+            }
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                half8 bf[NJ][T::PRODUCTS];
+                make(raw[J & 1], J, t, bf);
+                multiply(af[J & 1][t], bf);
+            }
+            if constexpr (J >= 1 && J <= NJ) add_offsets(sb, std::integral_constant<int, J - 1>{});
+        };
+        read_step(0);
+        for (int sb = 0; sb < mine; sb++) {
+            step(sb, S0{}); step(sb, S1{}); step(sb, S2{}); step(sb, S3{});
+        }
+        fold();
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            unit[j] = 1.0f;
+#pragma unroll
+            for (int i = 0; i < MI; i++) acc[i][j] = sum[i][j];
+        }
+    } else { // a product's fragments ahead; the barrier in front of the step's last products
+        half8 af[2][MI], bf[2][NJ][T::PRODUCTS];
+        typename T::Raw raw[NJ];
+        auto step = [&](int sb, auto at) {
+            constexpr int J = decltype(at)::value;
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                if (t < 3) {
+                    read_x(t + 1, af[(t + 1) & 1]);
+                    make(raw, J, t + 1, bf[(t + 1) & 1]);
+                } else {
+                    meet(sb, at);
+                    read_codes((J + 1) & 3, raw);
+                    read_x(0, af[0]);
+                    if (J == 3) read_sides(sb + 1);
+                }
+                if (J == 0 && t == 0) change_unit();
+                multiply(af[t & 1], bf[t & 1]);
+                if constexpr (J >= 1 && J <= NJ)
+                    if (t == 1) add_offsets(sb, std::integral_constant<int, J - 1>{});
+                if (t == 3) {
+                    if (J == 3) {
+#pragma unroll
+                        for (int j = 0; j < NJ; j++) side[j] = next_side[j];
+                        new_side(sb + 1 >= mine);
+                    }
+                    make(raw, (J + 1) & 3, 0, bf[0]);
+                }
+            }
+        };
+        read_codes(0, raw);
+        read_x(0, af[0]);
+#pragma unroll
+        for (int j = 0; j < NJ; j++) side[j] = next_side[j];
+        new_side();
+        make(raw, 0, 0, bf[0]);
+        for (int sb = 0; sb < mine; sb++) {
+            step(sb, S0{}); step(sb, S1{}); step(sb, S2{}); step(sb, S3{});
+        }
+    }
+    for (int sb = mine; sb < loops; sb++) { // the other group has one more
+        meet(sb, S0{}); meet(sb, S1{}); meet(sb, S2{}); meet(sb, S3{});
+    }
+    wait_loads_and_lds<0>(); // nothing of this workgroup may still be on its way into LDS
+
+    // ---- results.  D layout: lane -> column li; register r -> row 8 (r / 4) + 4 (lane / 32) + r % 4
+    auto store = [&](int i, int j, int r, float v, float v2) { // v2: of row r + 1, where rows are pairs
+        const int gn = n0 + (wn * NJ + j) * 32 + li;
+        const int gm = (mt0 + wm * MI + i) * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
+        if (gm >= a.m || gn >= a.n) return;
+        const size_t row = (size_t)(a.pair ? gm >> 1 : gm), rows = (size_t)(a.pair ? a.m >> 1 : a.m);
+        if (a.pair) v += v2;
+        if (a.ypart) {
+            a.ypart[((size_t)blockIdx.y * rows + row) * a.n + gn] = v;
+        } else {
+            float out = v * a.rowscale[gm];
+            if (a.bias) out += a.bias[gn];
+            if (a.resid) out += a.resid[row * a.n + gn];
+            a.y[row * a.n + gn] = out;
+        }
+    };
+    const int step_r = a.pair ? 2 : 1;
+    if constexpr (KG == 2) { // a group finishes half of the registers and hands the other half over
+        barrier();
+        float *mail = reinterpret_cast<float *>(lds) + (kg * 4 + wn) * (MI * NJ * 8 * 64) + lane;
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int r = 0; r < 8; r++) mail[((i * NJ + j) * 8 + r) * 64] = (kg ? acc[i][j][r] : acc[i][j][r + 8]) * unit[j];
+        __syncthreads();
+        const float *got = reinterpret_cast<const float *>(lds) + ((1 - kg) * 4 + wn) * (MI * NJ * 8 * 64) + lane;
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                float v[8];
+#pragma unroll
+                for (int r = 0; r < 8; r++) v[r] = (kg ? acc[i][j][r + 8] : acc[i][j][r]) * unit[j] + got[((i * NJ + j) * 8 + r) * 64];
+#pragma unroll
+                for (int r = 0; r < 8; r++)
+                    if (r % step_r == 0) store(i, j, kg * 8 + r, v[r], v[r | 1]);
+            }
+    } else {
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    if (r % step_r == 0) store(i, j, r, acc[i][j][r] * unit[j], acc[i][j][r | 1] * unit[j]);
+    }
+}
+
+// Rows of x in operand order (see RowsArgs::xa, xs) under a power-of-two scale per row.  IN: 0 f32 rows, RMS-normalised where
+// norm_w is given ((x * inv_rms) * norm_w, RMSNorm::forward, llm/src/llama.rs:158-187); 1 f32 rows of 2 k gate/up values, four
+// and four, which become silu(gate) * up; 2 bf16 rows.  f32 rows become two rows each.  A workgroup per row, a thread per
+// eight elements; the row stays in registers (NC times 4096 elements) or, NC = 0, is read once per pass.
+template <int IN, int NC>
+__global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const float *norm_w, float eps, int k, _Float16 *xa, _Float16 *xs,
+                                                        float *rowscale) {
+    constexpr int HELD = NC > 0 ? NC : 1;
+    __shared__ float red[8];
+    const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, chunks = k >> 3;
+    float v[HELD][8];
+    auto load = [&](int c, float (&e)[8]) {
+        if (IN == 2) {
+            const u32x4 r = reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint16_t *>(x) + (size_t)row * k)[c];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                e[2 * i] = __builtin_bit_cast(float, r[i] << 16);
+                e[2 * i + 1] = __builtin_bit_cast(float, r[i] & 0xFFFF0000u);
+            }
+        } else if (IN == 1) {
+            const float4 *p = reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(x) + (size_t)row * 2 * k) + 4 * (size_t)c;
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const float4 g = p[2 * i], u = p[2 * i + 1];
+                e[4 * i] = (g.x * (1.0f / (1.0f + expf(-g.x)))) * u.x;
+                e[4 * i + 1] = (g.y * (1.0f / (1.0f + expf(-g.y)))) * u.y;
+                e[4 * i + 2] = (g.z * (1.0f / (1.0f + expf(-g.z)))) * u.z;
+                e[4 * i + 3] = (g.w * (1.0f / (1.0f + expf(-g.w)))) * u.w;
+            }
+        } else {
+            const float4 *p = reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(x) + (size_t)row * k) + 2 * (size_t)c;
+            const float4 l = p[0], h = p[1];
+            e[0] = l.x; e[1] = l.y; e[2] = l.z; e[3] = l.w; e[4] = h.x; e[5] = h.y; e[6] = h.z; e[7] = h.w;
+        }
+    };
+    // all threads go through `chunks` in steps of 512; `fn(e, c, i)`: e the elements of chunk c, the i-th of this thread
+    auto each = [&](bool first, auto fn) {
+        if constexpr (NC > 0) {
+#pragma unroll
+            for (int i = 0; i < NC; i++) {
+                const int c = i * 512 + tid;
+                if (first) {
+                    if (c < chunks) load(c, v[i]);
+                    else
+#pragma unroll
+                        for (int q = 0; q < 8; q++) v[i][q] = 0.f;
+                }
+                fn(v[i], c);
+            }
+        } else {
+            for (int c = tid; c < (chunks + 511) / 512 * 512; c += 512) {
+                float e[8];
+                if (c < chunks) load(c, e);
+                else
+#pragma unroll
+                    for (int q = 0; q < 8; q++) e[q] = 0.f;
+                fn(e, c);
+            }
+        }
+    };
+    float inv = 1.0f;
+    const bool norm = IN == 0 && norm_w;
+    bool first = true;
+    if (norm) {
+        float ss = 0.f;
+        each(true, [&](float (&e)[8], int) {
+#pragma unroll
+            for (int q = 0; q < 8; q++) ss = fmaf(e[q], e[q], ss);
+        });
+        first = false;
+#pragma unroll
+        for (int s = 32; s >= 1; s >>= 1) ss += __shfl_xor(ss, s);
+        if (lane == 0) red[wave] = ss;
+        __syncthreads();
+        ss = ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
+        __syncthreads();
+        inv = 1.0f / sqrtf(ss / (float)k + eps);
+    }
+    auto normed = [&](float (&e)[8], int c) {
+        if (!norm || c >= chunks) return;
+        const float4 l = reinterpret_cast<const float4 *>(norm_w)[2 * c], h = reinterpret_cast<const float4 *>(norm_w)[2 * c + 1];
+        e[0] = (e[0] * inv) * l.x; e[1] = (e[1] * inv) * l.y; e[2] = (e[2] * inv) * l.z; e[3] = (e[3] * inv) * l.w;
+        e[4] = (e[4] * inv) * h.x; e[5] = (e[5] * inv) * h.y; e[6] = (e[6] * inv) * h.z; e[7] = (e[7] * inv) * h.w;
+    };
+    uint32_t top = 0; // largest |v| as an integer: a NaN ranks above everything and is not dropped
+    each(first, [&](float (&e)[8], int c) {
+        normed(e, c); // the registers hold normed values from here on
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const uint32_t b = __builtin_bit_cast(uint32_t, e[q]) & 0x7FFFFFFFu;
+            top = b > top ? b : top;
+        }
+    });
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1) {
+        const uint32_t o = (uint32_t)__shfl_xor((int)top, s);
+        top = o > top ? o : top;
+    }
+    if (lane == 0) red[wave] = __builtin_bit_cast(float, top);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const uint32_t o = __builtin_bit_cast(uint32_t, red[i]);
+        top = o > top ? o : top;
+    }
+    // top in [2^e, 2^(e+1)) -> multiply by 2^(11 - e): a sum of 32 stays below 2^17; inf/nan rows are passed through unscaled
+    int eb = (int)(top >> 23);
+    if (eb == 0 || eb == 0xFF) eb = 127 + 11;
+    int sb = 127 + 11 - (eb - 127);
+    sb = sb < 1 ? 1 : (sb > 254 ? 254 : sb);
+    const float f = __builtin_bit_cast(float, (uint32_t)sb << 23);
+    constexpr int PARTS = IN == 2 ? 1 : 2;
+    const int r0 = row * PARTS, steps = k >> 6, nsb = k >> 8;
+    _Float16 *xt = xa + (size_t)(r0 >> 5) * steps * 2048, *st = xs + (size_t)(r0 >> 5) * nsb * 1024;
+    each(false, [&](float (&e)[8], int c) {
+        if (NC == 0) normed(e, c);
+        _Float16 p[2][8];
+        float sum[2] = {0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const float s = e[q] * f;
+            p[0][q] = (_Float16)s;
+            sum[0] += (float)p[0][q];
+            if (PARTS == 2) {
+                p[1][q] = (_Float16)(s - (float)p[0][q]);
+                sum[1] += (float)p[1][q];
+            }
+        }
+        // chunk c: step c / 8, product t, half of the lanes (see the order of elements above)
+        const int at = c & 7, t = (at >> 2) * 2 + (at & 1), h = (at >> 1) & 1;
+#pragma unroll
+        for (int part = 0; part < PARTS; part++) {
+            const int lrow = (r0 + part) & 31;
+            const _Float16 *s = p[part];
+            if (c < chunks)
+                *reinterpret_cast<half8 *>(xt + ((size_t)(c >> 3) * 4 + t) * 512 + (h * 32 + lrow) * 8) = half8{s[0], s[2], s[1], s[3], s[4], s[6], s[5], s[7]};
+            // the sum of 32 elements: four threads; times 1 / 8 it stays within f16's range
+            float g = sum[part];
+            g += __shfl_xor(g, 1);
+            g += __shfl_xor(g, 2);
+            if ((tid & 3) == 0 && c < chunks) {
+                g *= 1.0f / 8.0f;
+                const _Float16 ghi = (_Float16)g, glo = (_Float16)(g - (float)ghi);
+                const int sub = (c >> 2) & 7;
+                _Float16 *d = st + (size_t)(c >> 5) * 1024 + ((sub >> 2) * 32 + lrow) * 8 + (sub & 3);
+                d[0] = ghi; d[4] = ghi;
+                d[512] = glo; d[516] = glo;
+            }
+        }
+    });
+    if (tid < PARTS) rowscale[r0 + tid] = 1.0f / f;
+}
+
+template <class T, int MI, int WM, int NJ>
+int launch_tile(axq_ctx *ctx, const RowsArgs &a, int splits) {
+    using Tile = RowsTile<T, MI, WM, NJ>;
+    static std::atomic<uint64_t> lds_allowed{0};
+    if (int rc = axq_allow_lds(ctx, reinterpret_cast<const void *>(rows_gemm_kernel<T, MI, WM, NJ>), lds_allowed, Tile::LDS)) return rc;
+    const unsigned tiles = (unsigned)(((a.n + Tile::N - 1) / Tile::N) * ((a.m + Tile::M - 1) / Tile::M));
+    rows_gemm_kernel<T, MI, WM, NJ><<<dim3(tiles, (unsigned)splits), 512, Tile::LDS, ctx->stream>>>(a);
+    AXQ_LAUNCH_CHECK(ctx, "rows_gemm_kernel");
+    return AXQ_OK;
+}
+
+// The tile of a call.  Up to 32, 64 rows of operands (16, 32 f32 rows): one and two row tiles per wave and the two halves of the
+// waves on two parts of K, since a workgroup's time is then its number of steps.  65 to 128 rows: two times two row tiles (at
+// 64 f32 rows and Q4_K 28672 x 4096 2.5 us ahead of four row tiles per wave and split halves).  Above: 256 x 256 outputs.
+template <class T>
+int launch_rows(axq_ctx *ctx, const RowsArgs &a, int splits) {
+    if (a.m > 128) return launch_tile<T, 4, 2, 2>(ctx, a, splits);
+    if (a.m > 64) return launch_tile<T, 2, 2, 1>(ctx, a, splits);
+    if (a.m > 32) return launch_tile<T, 2, 1, 1>(ctx, a, splits);
+    return launch_tile<T, 1, 1, 1>(ctx, a, splits);
+}
+
+template <int IN>
+void launch_prep(hipStream_t st, const void *x, const float *norm_w, float eps, int rows, int k, _Float16 *xa, _Float16 *xs, float *rs) {
+    if (k <= 4096) rows_prep_kernel<IN, 1><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
+    else if (k <= 8192) rows_prep_kernel<IN, 2><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
+    else if (k <= 16384) rows_prep_kernel<IN, 4><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
+    else rows_prep_kernel<IN, 0><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
+}
+
+} // namespace
+
+bool axq_dev_rows_gemm_covers(const axq_weight *w) {
+    return (w->type == AXQ_Q4_K || w->type == AXQ_Q5_K || w->type == AXQ_Q6_K) && w->k % 256 == 0 && w->k <= INT32_MAX && w->n_rows <= INT32_MAX;
+}
+
+// Scratch: x in operand order | its sub-block sums | row scales | partial sums of a split K.
+int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, int rows, const float *norm_w, float eps, const float *bias,
+                      const float *resid, float *y) {
+    const int parts = in == AXQ_ROWS_BF16 ? 1 : 2, m = rows * parts, n = (int)w->n_rows, k = (int)w->k;
+    const int bm = m <= 32 ? 32 : m <= 64 ? 64 : m <= 128 ? 128 : 256;
+    const int nsb = k >> 8, cus = ctx->prop.multiProcessorCount, groups = m <= 64 ? 2 : 1;
+    const int bn = m <= 128 ? 128 : 256;
+    const long tiles = (long)((n + bn - 1) / bn) * ((m + bm - 1) / bm);
+    // K is split over as many workgroups as leave every group of waves a superblock, up to one workgroup per compute unit
+    int splits = (int)(cus / tiles);
+    if (splits > nsb / groups) splits = nsb / groups;
+    if (splits > 8) splits = 8;
+    if (splits < 2 || n % 4 != 0) splits = 1;
+    RowsArgs a;
+    a.sb_per_split = (nsb + splits - 1) / splits;
+    splits = (nsb + a.sb_per_split - 1) / a.sb_per_split;
+    const size_t mtiles = (size_t)(m + bm - 1) / bm * (bm / 32);
+    const size_t xa_bytes = mtiles * 32 * (size_t)k * 2, xs_bytes = mtiles * (size_t)nsb * 2048;
+    const size_t rs_bytes = axq_align_up((size_t)m * 4, 256), part_bytes = splits > 1 ? (size_t)splits * rows * (size_t)n * 4 : 0;
+    if (int rc = axq_gemm_reserve(ctx, xa_bytes + xs_bytes + rs_bytes + part_bytes)) return rc;
+    uint8_t *base = reinterpret_cast<uint8_t *>(ctx->gemm_scratch);
+    _Float16 *xa = reinterpret_cast<_Float16 *>(base), *xs = reinterpret_cast<_Float16 *>(base + xa_bytes);
+    float *rs = reinterpret_cast<float *>(base + xa_bytes + xs_bytes);
+    switch (in) {
+    case AXQ_ROWS_BF16: launch_prep<2>(ctx->stream, x, nullptr, 0.f, rows, k, xa, xs, rs); break;
+    case AXQ_ROWS_SWIGLU: launch_prep<1>(ctx->stream, x, nullptr, 0.f, rows, k, xa, xs, rs); break;
+    default: launch_prep<0>(ctx->stream, x, norm_w, eps, rows, k, xa, xs, rs); break;
+    }
+    a.codes = w->codes; a.meta = w->meta; a.qh = w->qh;
+    a.codes_pitch = (uint32_t)w->codes_pitch; a.meta_pitch = (uint32_t)w->meta_pitch; a.qh_pitch = (uint32_t)w->qh_pitch;
+    a.xa = xa; a.xs = xs; a.rowscale = rs; a.y = y;
+    a.ypart = splits > 1 ? reinterpret_cast<float *>(base + xa_bytes + xs_bytes + rs_bytes) : nullptr;
+    a.m = m; a.n = n; a.k = k; a.pair = parts == 2; a.bias = bias; a.resid = resid;
+    int rc;
+    switch (w->type) {
+    case AXQ_Q4_K: rc = launch_rows<SuperQ45<false>>(ctx, a, splits); break;
+    case AXQ_Q5_K: rc = launch_rows<SuperQ45<true>>(ctx, a, splits); break;
+    default: rc = launch_rows<SuperQ6>(ctx, a, splits); break;
+    }
+    if (rc || splits == 1) return rc;
+    return axq_gemm_reduce(ctx, a.ypart, rs, rows, n, splits, 1.0f, parts, bias, resid, y);
+}
