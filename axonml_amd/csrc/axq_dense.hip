@@ -302,10 +302,15 @@ int launch_gemv_mode(axq_ctx *ctx, GemvArgs &a) {
 
 // ---------------------------------------------------------------------------------------------------------------------
 // GEMM on bf16 rows: tiles of BM x BN, K in steps of 64, operands straight from memory into LDS (16 bytes per lane,
-// two stages).  Row r of a tile is 128 bytes of LDS whose 16-byte pieces are exchanged by r & 7 (the loads take the
-// permuted source address, the destination being fixed), so that the operand reads of eight rows use all banks.
+// two stages).  Row r of a tile is 128 bytes of LDS whose 16-byte pieces are exchanged by (r / 2) & 7 (the loads take the
+// permuted source address, the destination being fixed): sixteen lanes that read the same piece of consecutive rows touch all
+// 64 banks (exchanged by r & 7, rows r and r + 8 share theirs and every operand read takes twice as long).
 // The product is taken as D[row of x][row of W]: a lane's accumulators are one output column.
-// ---------------------------------------------------------------------------------------------------------------------
+// The barrier of a step stands in front of its last quarter of products: behind it the step after next is requested into the
+// stage that has just been read, and the next step's first operands, which arrive while those products run.
+// Tiles: 256 x 256 with eight waves of 128 x 64 (24 KB of operands per wave and 32 products, where 64 x 64 take 32) where that
+// gives the chip a round of work; 128 x 128 with four waves, two workgroups to a compute unit; the same with eight waves, four
+// to every other step (KG = 2), where there is no second workgroup; smaller ones where the tiles are few.
 struct GemmArgs {
     axq_parts parts;
     int m, k, ldx, mt, tiles;
@@ -348,12 +353,121 @@ __device__ inline int xcd_tile(int tiles) {
     return x * per + (x < rest ? x : rest) + (b >> 3);
 }
 
-template <int BM, int BN, bool GROUPED>
-__global__ void __launch_bounds__(256) dense_gemm_kernel(GemmArgs a) {
-    constexpr int MT = BM / 64, NT = BN / 64;          // 32 x 32 tiles of a wave (2 x 2 waves)
-    constexpr int AL = BM / 32, BL = BN / 32;          // 16-byte loads per thread and step
-    __shared__ __attribute__((aligned(16))) uint16_t lds[2][(BM + BN) * 64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
+// A wave's results on their way out, 32 rows at a time through a patch of LDS of its own: a lane then has four neighbouring columns
+// of a row (16-byte loads and stores), and bias, activation, residual and mean are a short loop.  (Straight from the accumulators,
+// an element at a time with every option asked for each, this was most of the kernel at K = 2048: 100 of 144 us at 2047 x 8192.)
+template <int MT, int NT, bool GROUPED>
+__device__ inline void write_tile(const axq_part &p, float cap, const f32x16 (&acc)[MT][NT], float *patch, int m_base, int m1, int n_base, int lane) {
+    constexpr int P = NT * 32 + 8; // row pitch: rows four apart lie half the banks apart
+    const int li = lane & 31;
+    const bool glu = NT == 2 && p.act == AXQ_ACT_GLU_GELU; // the wave's two column tiles are a group of gates and its ups
+    const int cols = glu ? p.n / 2 : p.n, n_first = glu ? n_base / 2 : n_base, quads = glu ? 8 : NT * 8, rows_at_once = 64 / quads;
+    const int row_l = lane / quads, quad = lane % quads, n = n_first + quad * 4;
+    const bool vec = ((p.ldy | cols) & 3) == 0 && ((reinterpret_cast<uintptr_t>(p.y) | reinterpret_cast<uintptr_t>(p.resid) | reinterpret_cast<uintptr_t>(p.bias) |
+                                                    reinterpret_cast<uintptr_t>(p.avg.out) | reinterpret_cast<uintptr_t>(p.avg.past) | p.avg.stride * 4) & 15) == 0;
+    auto load4 = [&](const float *q) {
+        if (vec) return *reinterpret_cast<const f32x4 *>(q);
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        for (int e = 0; e < 4; e++)
+            if (n + e < cols) v[e] = q[e];
+        return v;
+    };
+    const f32x4 bias = p.bias && n < cols ? load4(p.bias + n) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the last rows have been read
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) patch[acc_row(r, lane) * P + j * 32 + li] = acc[i][j][r];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (p.act != AXQ_ACT_NONE) { // in place, in a loop of its own: sixteen elements' code in each of the loops below is too much of it
+#pragma clang loop unroll(disable)
+            for (int r = row_l; r < 32; r += rows_at_once) {
+                f32x4 *at = reinterpret_cast<f32x4 *>(patch + r * P + quad * 4);
+                f32x4 v = *at;
+                if (glu) {
+                    const f32x4 up = at[8];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] = axq_gelu_tanh(v[e]) * up[e];
+                } else {
+                    v += bias;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] = axq_act(p.act, v[e], cap);
+                }
+                *at = v;
+            }
+        }
+#pragma clang loop unroll(disable)
+        for (int r0 = 0; r0 < 32; r0 += 4 * rows_at_once) { // four rows of a lane at a time: their loads are under way together
+            f32x4 v[4], o[4];
+            bool ok[4];
+            size_t at[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int r = r0 + q * rows_at_once + row_l, m = m_base + i * 32 + r;
+                ok[q] = m < m1 && n < cols;
+                at[q] = (size_t)m * p.ldy + n;
+                if (p.resid && ok[q]) o[q] = load4(p.resid + at[q]);
+                v[q] = *reinterpret_cast<const f32x4 *>(patch + r * P + quad * 4);
+                if (glu || p.act == AXQ_ACT_NONE) v[q] += bias;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                if (!ok[q]) continue;
+                if (p.scale) v[q] *= p.scale[at[q] / (size_t)p.ldy];
+                if (p.resid) v[q] += o[q];
+                if (vec && p.out16) {
+                    *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(p.y) + at[q]) =
+                        make_uint2(axq_to_bf16(v[q][0]) | (uint32_t)axq_to_bf16(v[q][1]) << 16, axq_to_bf16(v[q][2]) | (uint32_t)axq_to_bf16(v[q][3]) << 16);
+                } else if (vec) {
+                    *reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(p.y) + at[q]) = v[q];
+                } else {
+                    for (int e = 0; e < 4; e++)
+                        if (n + e < cols) {
+                            if (p.out16) reinterpret_cast<uint16_t *>(p.y)[at[q] + e] = axq_to_bf16(v[q][e]);
+                            else reinterpret_cast<float *>(p.y)[at[q] + e] = v[q][e];
+                        }
+                }
+            }
+            if (!GROUPED && p.avg.out) { // the mean over the layers (axq_average's sum)
+                f32x4 s[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) s[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int j = 0; j < p.avg.n; j++) {
+                    const float w = p.avg.w[j];
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        if (ok[q]) o[q] = load4(p.avg.past + j * p.avg.stride + at[q]);
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        for (int e = 0; e < 4; e++) s[q][e] = fmaf(w, o[q][e], s[q][e]);
+                }
+                const float w = p.avg.w[p.avg.n];
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    for (int e = 0; e < 4; e++)
+                        if (ok[q] && n + e < cols) p.avg.out[at[q] + e] = fmaf(w, v[q][e], s[q][e]);
+            }
+        }
+    }
+}
+
+constexpr int gemm_patch(int mt, int nt, int kg) {
+    const int rows = 32 * (nt * 32 + 8), mail = kg == 2 ? mt * nt * 16 * 64 : 0; // write_tile's rows; the other group's sums
+    return rows > mail ? rows : mail;
+}
+
+template <int BM, int BN, int WM, int WN, int KG, bool GROUPED>
+__global__ void __launch_bounds__(64 * WM * WN * KG, 2) dense_gemm_kernel(GemmArgs a) {
+    constexpr int MT = BM / 32 / WM, NT = BN / 32 / WN; // 32 x 32 tiles of a wave
+    constexpr int GW = WM * WN;                         // waves of a group along K
+    constexpr int AL = BM / 8 / GW, BL = BN / 8 / GW;   // 16-byte loads per thread and step
+    constexpr int STEP = (BM + BN) * 64;                // elements of a step's tile
+    constexpr int PATCH = gemm_patch(MT, NT, KG);       // floats of LDS that a wave's results pass through
+    extern __shared__ __attribute__((aligned(16))) uint16_t lds[]; // [stage][group][STEP]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kg = wave / GW, gw = wave % GW, wm = gw / WN, wn = gw % WN;
     const int tile = xcd_tile(a.tiles), ct = tile / a.mt;
     int m0 = (tile - ct * a.mt) * BM, m1 = a.m, pi = 0;
     size_t woff = 0;
@@ -366,25 +480,29 @@ __global__ void __launch_bounds__(256) dense_gemm_kernel(GemmArgs a) {
     const uint16_t *ga[AL], *gb[BL];
 #pragma unroll
     for (int i = 0; i < AL; i++) {
-        const int idx = (i * 4 + wave) * 64 + lane, r = idx >> 3, c = (idx & 7) ^ (r & 7);
+        const int idx = (i * GW + gw) * 64 + lane, r = idx >> 3, c = (idx & 7) ^ ((r >> 1) & 7);
         int row = m0 + r < m1 ? m0 + r : m1 - 1;
         if (GROUPED && a.g.src) row = a.g.src[row];
         ga[i] = x + (size_t)row * a.ldx + c * 8;
     }
 #pragma unroll
     for (int i = 0; i < BL; i++) {
-        const int idx = (i * 4 + wave) * 64 + lane, r = idx >> 3, c = (idx & 7) ^ (r & 7);
+        const int idx = (i * GW + gw) * 64 + lane, r = idx >> 3, c = (idx & 7) ^ ((r >> 1) & 7);
         const int row = n0 + r < p.n ? n0 + r : p.n - 1;
         gb[i] = p.w + woff + (size_t)row * p.ldw + c * 8;
     }
-    auto fetch = [&](int stage, int kt) {
-        uint16_t *la = lds[stage], *lb = la + BM * 64;
+    const int kts = a.k >> 6, its = (kts + KG - 1) / KG;
+    auto fetch = [&](int it) { // this group's step of iteration `it` (past the end the last one again, which nobody multiplies)
+        int kt = it * KG + kg;
+        kt = kt < kts ? kt : kts - 1;
+        uint16_t *la = lds + ((it & 1) * KG + kg) * STEP, *lb = la + BM * 64;
 #pragma unroll
         for (int i = 0; i < AL; i++)
-            __builtin_amdgcn_global_load_lds((gbl_void *)(ga[i] + kt * 64), (lds_void *)(la + (i * 4 + wave) * 512), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gbl_void *)(ga[i] + (size_t)kt * 64), (lds_void *)(la + (i * GW + gw) * 512), 16, 0, 0);
 #pragma unroll
         for (int i = 0; i < BL; i++)
-            __builtin_amdgcn_global_load_lds((gbl_void *)(gb[i] + kt * 64), (lds_void *)(lb + (i * 4 + wave) * 512), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gbl_void *)(gb[i] + (size_t)kt * 64), (lds_void *)(lb + (i * GW + gw) * 512), 16, 0, 0);
+        asm volatile("" ::: "memory");
     };
     f32x16 acc[MT][NT];
 #pragma unroll
@@ -394,63 +512,69 @@ __global__ void __launch_bounds__(256) dense_gemm_kernel(GemmArgs a) {
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
 
-    const int kts = a.k >> 6, li = lane & 31, lh = lane >> 5;
-    fetch(0, 0);
-    for (int kt = 0; kt < kts; kt++) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // this step's tile is in LDS ...
-        __syncthreads();                                  // ... of every wave, and nobody reads the other stage any more
-        if (kt + 1 < kts) fetch((kt + 1) & 1, kt + 1);
-        const uint16_t *la = lds[kt & 1], *lb = la + BM * 64;
+    const int li = lane & 31, lh = lane >> 5, sw = (li >> 1) & 7; // tiles of a wave start at multiples of 32 rows
+    const uint16_t *la = lds + kg * STEP + (wm * (BM / WM) + li) * 64, *lb = lds + kg * STEP + (BM + wn * (BN / WN) + li) * 64;
+    bf16x8 fa[2][MT], fb[2][NT];
+    auto read = [&](int it, int ks, int b) {
+        const int at = (it & 1) * KG * STEP + (((ks * 2 + lh) ^ sw) << 3);
+#pragma unroll
+        for (int i = 0; i < MT; i++) fa[b][i] = *reinterpret_cast<const bf16x8 *>(la + at + i * 32 * 64);
+#pragma unroll
+        for (int j = 0; j < NT; j++) fb[b][j] = *reinterpret_cast<const bf16x8 *>(lb + at + j * 32 * 64);
+    };
+    auto meet = [&] { // what this wave has requested is in LDS and what it has read has arrived; then everybody's
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    fetch(0);
+    meet();
+    if (its > 1) fetch(1);
+    read(0, 0, 0);
+    for (int it = 0; it < its; it++) {
+        const bool live = KG == 1 || it * KG + kg < kts;
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) {
-            bf16x8 fa[MT], fb[NT];
-#pragma unroll
-            for (int i = 0; i < MT; i++) {
-                const int r = wm * (BM / 2) + i * 32 + li;
-                fa[i] = *reinterpret_cast<const bf16x8 *>(la + r * 64 + (((ks * 2 + lh) ^ (r & 7)) << 3));
+            if (ks < 3) {
+                read(it, ks + 1, (ks + 1) & 1);
+            } else if (it + 1 < its) {
+                meet();
+                if (it + 2 < its) fetch(it + 2);
+                read(it + 1, 0, 0);
             }
+            if (live)
 #pragma unroll
-            for (int j = 0; j < NT; j++) {
-                const int r = wn * (BN / 2) + j * 32 + li;
-                fb[j] = *reinterpret_cast<const bf16x8 *>(lb + r * 64 + (((ks * 2 + lh) ^ (r & 7)) << 3));
-            }
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks & 1][i], fb[ks & 1][j], acc[i][j], 0, 0, 0);
+        }
+    }
+    if constexpr (KG == 2) { // the second group's sums join the first one's, which finishes
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        float *mail = reinterpret_cast<float *>(lds) + gw * PATCH + lane;
+        if (kg == 1)
 #pragma unroll
             for (int i = 0; i < MT; i++)
 #pragma unroll
-                for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        }
-    }
-    if (NT == 2 && p.act == AXQ_ACT_GLU_GELU) { // a wave's two column tiles are a group of gates and its ups
-        const int n = n0 / 2 + wn * 32 + li;
-        if (n >= p.n / 2) return;
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) mail[((i * NT + j) * 16 + r) * 64] = acc[i][j][r];
+        __syncthreads();
+        if (kg == 1) return;
 #pragma unroll
         for (int i = 0; i < MT; i++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int m = m0 + wm * (BM / 2) + i * 32 + acc_row(r, lane);
-                if (m < m1) finish(p, a.parts.cap, m, n, axq_gelu_tanh(acc[i][0][r]) * acc[i][NT - 1][r], true);
-            }
-        return;
-    }
+            for (int j = 0; j < NT; j++)
 #pragma unroll
-    for (int j = 0; j < NT; j++) {
-        const int n = n0 + wn * (BN / 2) + j * 32 + li;
-        if (n >= p.n) continue;
-#pragma unroll
-        for (int i = 0; i < MT; i++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int m = m0 + wm * (BM / 2) + i * 32 + acc_row(r, lane);
-                if (m < m1) finish(p, a.parts.cap, m, n, acc[i][j][r]);
-            }
+                for (int r = 0; r < 16; r++) acc[i][j][r] += mail[((i * NT + j) * 16 + r) * 64];
     }
-    if (!GROUPED && p.avg.out) {
-#pragma clang loop unroll(disable)
-        for (int x = 0; x < NT * MT * 16; x++) {
-            const int n = n0 + wn * (BN / 2) + (x & (NT - 1)) * 32 + li, m = m0 + wm * (BM / 2) + x / (NT * 16) * 32 + acc_row((x / NT) & 15, lane);
-            if (n < p.n && m < m1) finish_mean(p, m, n);
-        }
+    else {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the stages have been read: they take the results' patches
+        __builtin_amdgcn_s_barrier();
     }
+    float *patch = reinterpret_cast<float *>(lds) + gw * PATCH; // a wave's own: it has read its mail
+    write_tile<MT, NT, GROUPED>(p, a.parts.cap, acc, patch, m0 + wm * (BM / WM), m1, n0 + wn * (BN / WN), lane);
 }
 
 // GEMM on f32 rows in true 32-bit: 64 x 64 tiles, 4 x 4 results per thread, K in steps of 16.
@@ -504,6 +628,17 @@ __global__ void __launch_bounds__(256) dense_gemm_f32_kernel(GemmArgs a) {
                 if (!GROUPED && p.avg.out) finish_mean(p, m, n);
             }
         }
+}
+
+template <int BM, int BN, int WM, int WN, int KG, bool GROUPED>
+int launch_gemm(axq_ctx *ctx, const GemmArgs &a) {
+    static std::atomic<uint64_t> lds_allowed{0};
+    constexpr size_t stages = (size_t)2 * KG * (BM + BN) * 64 * 2, out = (size_t)WM * WN * gemm_patch(BM / 32 / WM, BN / 32 / WN, KG) * 4, lds = stages > out ? stages : out;
+    if (lds > 48 * 1024)
+        if (int rc = axq_allow_lds(ctx, reinterpret_cast<const void *>(dense_gemm_kernel<BM, BN, WM, WN, KG, GROUPED>), lds_allowed, lds)) return rc;
+    dense_gemm_kernel<BM, BN, WM, WN, KG, GROUPED><<<a.tiles, 64 * WM * WN * KG, lds, ctx->stream>>>(a);
+    AXQ_LAUNCH_CHECK(ctx, "dense_gemm_kernel");
+    return AXQ_OK;
 }
 
 int count_tiles(GemmArgs &a, int bm, int bn) {
@@ -721,17 +856,55 @@ int axq_dense_gemm(axq_ctx *ctx, axq_parts &parts, int m, int k, int ldx, bool f
     if (f32) {
         count_tiles(a, 64, 64);
         dense_gemm_f32_kernel<false><<<a.tiles, 256, 0, ctx->stream>>>(a);
-    } else if (m > 64 && count_tiles(a, 128, 128) >= ctx->prop.multiProcessorCount) {
-        dense_gemm_kernel<128, 128, false><<<a.tiles, 256, 0, ctx->stream>>>(a);
-    } else if (glu) {
-        count_tiles(a, 64, 128);
-        dense_gemm_kernel<64, 128, false><<<a.tiles, 256, 0, ctx->stream>>>(a);
-    } else {
-        count_tiles(a, 64, 64);
-        dense_gemm_kernel<64, 64, false><<<a.tiles, 256, 0, ctx->stream>>>(a);
+        AXQ_LAUNCH_CHECK(ctx, "dense_gemm_f32_kernel");
+        return AXQ_OK;
     }
-    AXQ_LAUNCH_CHECK(ctx, "dense_gemm_kernel");
-    return AXQ_OK;
+    // Cost of a launch in units of a 128 x 128 tile that has a compute unit to itself: two 128 x 128 workgroups share one, a 256 x 256
+    // tile is four at 1.35 times the rate (2047 rows, K = 2048: 8192 columns 98 against 130 us).  The 256 x 256 tiles get the
+    // widest weights, as many as is cheapest, the others a launch of their own: a few columns more than whole rounds of the
+    // chip (a narrow projection beside wide ones) would cost a round of large tiles.
+    const int cus = ctx->prop.multiProcessorCount;
+    auto square_cost = [&](int tiles) { return 2.0f * (float)((tiles + 2 * cus - 1) / (2 * cus)); };
+    if (m > 128) {
+        int order[AXQ_MAX_PARTS], n = parts.n_parts;
+        for (int i = 0; i < n; i++) {
+            int at = i;
+            for (; at > 0 && parts.p[order[at - 1]].n < parts.p[i].n; at--) order[at] = order[at - 1];
+            order[at] = i;
+        }
+        const int mt2 = (m + 255) / 256, mt1 = (m + 127) / 128;
+        int square = 0, wide = 0, cut = 0;
+        for (int i = 0; i < n; i++) square += mt1 * ((parts.p[i].n + 127) / 128);
+        float best = square_cost(square);
+        for (int i = 0, left = square; i < n; i++) {
+            wide += mt2 * ((parts.p[order[i]].n + 255) / 256);
+            left -= mt1 * ((parts.p[order[i]].n + 127) / 128);
+            const float cost = 3.0f * (float)((wide + cus - 1) / cus) + (left ? 0.2f + square_cost(left) * (left > cus ? 1.0f : 0.5f) : 0.f);
+            if (cost < best) {
+                best = cost;
+                cut = i + 1;
+            }
+        }
+        if (cut > 0) {
+            axq_parts rest = parts;
+            a.parts.n_parts = rest.n_parts = 0;
+            for (int i = 0; i < n; i++)
+                if (i < cut) a.parts.p[a.parts.n_parts++] = parts.p[order[i]];
+                else rest.p[rest.n_parts++] = parts.p[order[i]];
+            count_tiles(a, 256, 256);
+            if (int rc = launch_gemm<256, 256, 2, 4, 1, false>(ctx, a)) return rc;
+            if (!rest.n_parts) return AXQ_OK;
+            a.parts = rest;
+        }
+    }
+    if (m > 64) {
+        const int square = count_tiles(a, 128, 128);
+        if (square > cus) return launch_gemm<128, 128, 2, 2, 1, false>(ctx, a);
+        if (square > cus / 2) return launch_gemm<128, 128, 2, 2, 2, false>(ctx, a);
+    }
+    if (glu)
+        return count_tiles(a, 64, 128) > cus ? launch_gemm<64, 128, 2, 2, 1, false>(ctx, a) : launch_gemm<64, 128, 2, 2, 2, false>(ctx, a);
+    return count_tiles(a, 64, 64) > cus ? launch_gemm<64, 64, 2, 2, 1, false>(ctx, a) : launch_gemm<64, 64, 2, 2, 2, false>(ctx, a);
 }
 
 int axq_dense_gemm_rows_per_tile(int rows, int groups, bool f32) { return !f32 && rows >= 96 * groups ? 128 : 64; }
@@ -750,10 +923,9 @@ int axq_dense_gemm_grouped(axq_ctx *ctx, axq_part &part, const axq_groups &g, in
     const int bn = f32 ? 64 : (g.bm == 128 ? 128 : 64);
     a.mt = g.max_tiles;
     a.tiles = (part.n + bn - 1) / bn * a.mt;
-    if (f32) dense_gemm_f32_kernel<true><<<a.tiles, 256, 0, ctx->stream>>>(a);
-    else if (g.bm == 128) dense_gemm_kernel<128, 128, true><<<a.tiles, 256, 0, ctx->stream>>>(a);
-    else dense_gemm_kernel<64, 64, true><<<a.tiles, 256, 0, ctx->stream>>>(a);
-    AXQ_LAUNCH_CHECK(ctx, "grouped dense_gemm_kernel");
+    if (!f32) return g.bm == 128 ? launch_gemm<128, 128, 2, 2, 1, true>(ctx, a) : launch_gemm<64, 64, 2, 2, 1, true>(ctx, a);
+    dense_gemm_f32_kernel<true><<<a.tiles, 256, 0, ctx->stream>>>(a);
+    AXQ_LAUNCH_CHECK(ctx, "grouped dense_gemm_f32_kernel");
     return AXQ_OK;
 }
 

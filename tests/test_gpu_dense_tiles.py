@@ -1,0 +1,33 @@
+"""The tiles of the products with bfloat16 weights, through models whose one wide product takes them: row and column counts on both
+sides of their edges, odd steps for two groups of waves, columns whose rows are no whole 16 bytes, a few narrow weights beside a
+wide one, and what happens to a result on its way out (softcap, GLU, residual, the mean over the layers)."""
+import pytest
+
+from . import gemosun_common as gc
+from . import lakulix_common as lc
+from .stack_common import close, feed, tokens_of
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,vocab,width", [(300, 22003, 64), (257, 22004, 200), (129, 17000, 72), (150, 8300, 192), (140, 8301, 64), (200, 4400, 130),
+                                              (70, 300, 320)])
+def test_logits_of_every_tile(ctx, rows, vocab, width):
+    cfg = lc.config([lc.wkv(heads=2, dim=8)], width=width, vocab=vocab)
+    t = lc.tensors(cfg, rows + width)
+    tokens = tokens_of(cfg, rows)
+    want = lc.oracle(cfg, t).forward(tokens)[0]
+    m = lc.product(cfg, t, "bfloat16", ctx)
+    assert close(m.forward_rows(tokens, range(rows)), want, "bfloat16")
+    m.close()
+
+
+@pytest.mark.parametrize("rows,ff", [(300, 11000), (270, 10977), (150, 4200)])
+def test_wide_feed_forward_beside_narrow_projections(ctx, rows, ff):
+    cfg = gc.config([gc.attention(heads=3, kv_heads=1, dim=16, mlp=gc.dense(ff)), gc.attention(mlp=gc.dense(40))], width=96, vocab=150)
+    t = gc.tensors(cfg, 5)
+    tokens = tokens_of(cfg, rows)
+    want = gc.oracle(cfg, t).forward(tokens)[0]
+    m = gc.product(cfg, t, "bfloat16", ctx, 400)
+    assert close(feed(m, tokens, [rows]), want, "bfloat16", 2)
+    m.close()
