@@ -912,14 +912,14 @@ bool all_layers_in_small_batch_reach(const axq_model *m, int nb) {
     return true;
 }
 
-// Fewest rows from which the layers' linears go through the GEMM: where all of them are superblock types as soon as the
-// small-batch GEMV would need a second pass over the weights, else PROMPT_GEMM_MIN where that GEMV is the alternative, and eight
+// Fewest rows from which the layers' linears go through the GEMM: where the rows kernel covers all of them as soon as the
+// small-batch GEMV would need a real second pass over the weights, else PROMPT_GEMM_MIN where that GEMV is the alternative, and eight
 // where single-vector passes are.
 int gemm_rows_min(const axq_model *m, int nb) {
     bool rows = true;
     for (int l = 0; l < m->cfg.num_hidden_layers; l++)
         for (const axq_weight *w : {m->w_qkv[l], m->w_o[l], m->w_gu[l], m->w_down[l], m->w_sep[0][l], m->w_sep[1][l], m->w_sep[2][l]})
-            rows = rows && (!w || axq_dev_rows_gemm_covers(w));
+            rows = rows && (!w || axq_dev_rows_gemm_covers(w, nb > AXQ_ROWS_GEMM_MIN ? nb : AXQ_ROWS_GEMM_MIN, false));
     return rows ? AXQ_ROWS_GEMM_MIN : all_layers_in_small_batch_reach(m, nb) ? PROMPT_GEMM_MIN : PROMPT_BATCH;
 }
 
@@ -1196,7 +1196,7 @@ int run_batch_step(axq_model *m, int max_pos_now) {
     int rc;
     if (m->n_seq > PROMPT_BATCH && m->n_seq <= GEMV_GROUPS_MAX && m->n_seq < gemm_rows_min(m, PROMPT_BATCH) &&
         all_layers_in_small_batch_reach(m, PROMPT_BATCH)) {
-        // a few more rows than the small-batch GEMV takes, and not all weights of superblock types: groups of eight sequences,
+        // a few more rows than the small-batch GEMV takes, and not all weights covered by the rows kernel: groups of eight sequences,
         // one after the other; plain launches
         rc = AXQ_OK;
         for (int s = 0; s < m->n_seq && !rc; s += PROMPT_BATCH) {

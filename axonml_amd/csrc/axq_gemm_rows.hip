@@ -1,18 +1,23 @@
-// Rows times a packed weight of a superblock type: y[M, N] = x[M, K] * W[N, K]^T on v_mfma_f32_32x32x16_f16, for f32 rows
-// (nine of them up to a prompt) and bf16 rows.  The reference composition is dequantize_tensor -> f32 sgemm
-// (crates/axonml-quant/src/dequantize.rs:34-54, crates/axonml-core/src/backends/cpu.rs:566-598).
+// Rows times a packed weight of a superblock type or of a type with blocks of 32: y[M, N] = x[M, K] * W[N, K]^T on
+// v_mfma_f32_32x32x16_f16, for f32 rows (ten of them up to a prompt; blocks of 32: up to 64) and bf16 rows (blocks: up to 128).  The
+// reference composition is dequantize_tensor -> f32 sgemm (crates/axonml-quant/src/dequantize.rs:34-54,
+// crates/axonml-core/src/backends/cpu.rs:566-598).
 //
-// Time of a call with f32 rows, Q4_K, before (groups of eight vectors, or two-stage operands in LDS) and now, us:
-//   rows            16          32          64
-//   28672 x 4096    40.5 28.0   81.5 35.9   61.8 54.0
-//   4096 x 4096     21.8 15.3   43.0 18.3   33.0 23.8
-//   4096 x 14336    32.0 26.2   63.2 31.0   63.9 40.0
+// Time of a call with f32 rows, before (groups of eight vectors, or two-stage operands in LDS) and now, us:
+//   rows                  10          16          32          64
+//   Q4_K 28672 x 4096     40.3 35.1   40.5 35.7   81.5 44.2   61.8 56.7
+//   Q4_K 4096 x 4096      22.7 16.9   21.8 18.5   43.0 20.5   33.0 23.8
+//   Q4_K 4096 x 14336     31.7 31.6   32.0 32.0   63.2 37.6   63.9 40.0
+//   Q4_0 11008 x 4096, 21 rows: 41.7 30.3; Q4_0 4096 x 4096, 10 and 39 rows: 22.3 16.0, 56.6 22.7; Q8_0 11008 x 4096, 64 rows: 43.2 34.8;
+//   bf16 rows, Q8_0 4096 x 4096, 16: 26.1 16.2; Q4_0 11008 x 4096, 128: 48.4 36.0
 // What bounds it: at few rows the fixed parts (pre-pass, reduction and the launches around them: 14 us of the 4096 x 4096 calls) and
-// 0.35 us per step of barrier and LDS reads; at many the matrix pipe beside the vector instructions that make operands (2048 bf16 rows
-// x 14336: 320 us, 750 TFLOP/s), which overlap only in part.
+// the LDS reads of x, which every wave makes for its 32 columns (0.35 us per step with one tile of x, 0.6 with two); at many the matrix
+// pipe beside the vector instructions that make operands (2048 bf16 rows x 14336: 320 us, 750 TFLOP/s), which overlap only in part.
 //
-// Numerics.  A bf16 row goes in as f16 under a power-of-two row scale (exact), an f32 row as two f16 rows, leading eleven
-// bits and remainder, whose results are added (22 bits).  A weight goes in without rounding:
+// Numerics.  A bf16 row goes in as f16 under a power-of-two row scale (exact).  An f32 row goes in as two f16 rows, leading eleven
+// bits and remainder, whose results are added (22 bits), from 40 rows on; fewer rows, which the small-batch GEMV with its 28 bits below
+// the row's largest is the alternative for, as three limbs of eleven bits in fixed point: 32 bits below the row's largest, and the
+// first limbs' sums over a block are exact.  A weight goes in without rounding:
 //   Q4_K, Q5_K   w = d (sc (q - C)) + (C d sc - dmin m), C = 8 or 16: sc (q - C) is an integer below 2^10, exact in f16, and is
 //                the operand; sums of them are in units of d.  A step's sum starts from zero and joins the total times d, or, where
 //                registers are short (more than 128 rows), the accumulators of a column hold the running sum and change their
@@ -22,7 +27,17 @@
 //                power of two and the operands are divided by it (exact).
 //   Q6_K         w = d sc (q - 32): sc (q - 32) has 13 bits and goes in as two exact operands, sc times the multiple of eight
 //                and sc times the rest, two products per weight.
-// Centred codes because sums over uncentred ones cancel for rows with a mean.  Accumulation is f32 throughout.
+//   blocks of 32 w = d (q - C) + (m + C d): q - C is the operand, a block's sum starts from zero and joins its superblock's times d; the
+//                offsets of eight blocks, as an f16 pair under a common power of two, meet the blocks' sums of x.
+// Centred codes because sums over uncentred ones cancel for rows with a mean.  Accumulation is f32 throughout: products of a step from
+// zero, steps into a superblock's sum, superblocks into the total.  Root mean square error against 64 bits over that of the result,
+// normal x, K = 1024 / 4096 / 14336, in 1e-8, before and now:
+//   rows       up to 39                       40 and more, f32
+//   Q4_0       7.2 8.6 10.3   6.6 8.2 8.9     8.5 10.6 15.5   8.5 9.7 10.7
+//   Q5_1       9.3 10.4 12.9  7.3 8.7 9.7     9.1 11.2 16.4   8.9 10.1 11.1
+//   Q4_K       9.4 10.5 12.9  7.5 9.0 9.5     13.0 17.7 31.4  10.4 11.3 12.0
+//   Q6_K       8.8 10.0 12.5  5.4 7.2 8.0     15.8 21.6 38.8  10.9 11.7 12.4
+// (limbs in one accumulator: Q4_0 8.6 11.7 16.5; the matrix pipe cuts sums off where it adds small products to large ones.)
 //
 // Shape.  A workgroup of eight waves; a wave computes 32 MI x 32 NJ outputs.  Four waves lie side by side along N; the other
 // factor of two is rows (WM = 2: 64 MI rows) or K (WM = 1: each four waves take half of the workgroup's superblocks, and the
@@ -92,7 +107,7 @@ __device__ inline void barrier() {
 template <bool Q5>
 struct SuperQ45 {
     static constexpr int PAIRS = 2, PRODUCTS = 1, SIDE16 = Q5 ? 3 : 1, SIDE4 = 0;
-    static constexpr bool MIN = true;
+    static constexpr bool MIN = true, BLOCKS = false;
     static constexpr float CENTRE = Q5 ? 16.0f : 8.0f;
     struct Side { u32x4 h, b; };
     struct Raw { u32x4 q; };
@@ -156,7 +171,7 @@ struct SuperQ45 {
             o.off[p] = o.sc[p] * (_Float16)(-(64.0f + CENTRE));
         }
     }
-    __device__ static void make(const Raw &r, const Side &s, const Scales &c, uint32_t mask, int j, int t, half8 (&o)[1]) {
+    __device__ static void make(const Raw &r, const Side &s, const Scales &c, uint32_t mask, int j, int t, int, half8 (&o)[1]) {
         const half2v sc = (t >> 1) ? __builtin_shufflevector(c.sc[j], c.sc[j], 1, 1) : __builtin_shufflevector(c.sc[j], c.sc[j], 0, 0);
         const half2v off = (t >> 1) ? __builtin_shufflevector(c.off[j], c.off[j], 1, 1) : __builtin_shufflevector(c.off[j], c.off[j], 0, 0);
         uint32_t w[4];
@@ -179,7 +194,7 @@ struct SuperQ45 {
 
 struct SuperQ6 {
     static constexpr int PAIRS = 3, PRODUCTS = 2, SIDE16 = 1, SIDE4 = 1;
-    static constexpr bool MIN = false;
+    static constexpr bool MIN = false, BLOCKS = false;
     struct Side { u32x4 sc; uint32_t d; };
     struct Raw { u32x4 ql[2], qh; };
     // a unit is half a superblock, 128 elements: pieces 0 and 1 its 64 bytes of low nibbles, piece 2 its 32 bytes of bit pairs
@@ -218,7 +233,7 @@ struct SuperQ6 {
         }
     }
     // element byte l of the unit: nibble j % 2 of ql[t / 2], bits 2 (2 (j % 2) + t / 2) of qh
-    __device__ static void make(const Raw &r, const Side &, const Scales &c, uint32_t, int j, int t, half8 (&o)[2]) {
+    __device__ static void make(const Raw &r, const Side &, const Scales &c, uint32_t, int j, int t, int, half8 (&o)[2]) {
         const half2v f = (t >> 1) ? __builtin_shufflevector(c.sc[j], c.sc[j], 1, 1) : __builtin_shufflevector(c.sc[j], c.sc[j], 0, 0);
         const half2v c1 = {(_Float16)-1056.0f, (_Float16)-1056.0f}, c0 = {(_Float16)-1024.0f, (_Float16)-1024.0f};
         uint32_t hi[4], lo[4];
@@ -237,25 +252,146 @@ struct SuperQ6 {
     }
 };
 
+// Blocks of 32 with an f16 scale d each (and a minimum m): the operand is the centred code, an integer; a block's sum starts from
+// zero and joins the total times d; m + C d meets the block's sum of x, eight blocks at a time.
+template <int BITS, bool WITH_MIN>
+struct Block32 {
+    static constexpr int PAIRS = BITS == 8 ? 4 : 2, PRODUCTS = 1, REC = WITH_MIN ? 2 : 1, SIDE16 = REC + (BITS == 5 ? 2 : 0), SIDE4 = 0;
+    static constexpr bool MIN = WITH_MIN, BLOCKS = true;
+    static constexpr float CENTRE = BITS == 8 ? 128.0f : BITS == 5 ? 16.0f : 8.0f;
+    struct Side { u32x4 r[REC], b[BITS == 5 ? 2 : 1]; };
+    struct Raw { u32x4 q[2]; }; // of the step's two blocks; Q4: the lane's half, in the first two dwords
+    struct Scales {};
+    __device__ static const uint8_t *piece_src(const RowsArgs &a, int unit, int p) { return a.codes + (size_t)unit * (PAIRS * 32) + p * 32; }
+    __device__ static uint32_t piece_pitch(const RowsArgs &a, int) { return a.codes_pitch; }
+    __device__ static const uint8_t *side_src(const RowsArgs &a, int sb, int c) { // the records, then the fifth bits
+        return c < REC ? a.meta + (size_t)sb * (16 * REC) + c * 16 : a.qh + (size_t)sb * 32 + (c - REC) * 16;
+    }
+    __device__ static uint32_t side_pitch(const RowsArgs &a, int c) { return c < REC ? a.meta_pitch : a.qh_pitch; }
+    template <int N>
+    __device__ static void read_side(const uint8_t *stage, int row, int, int, Side &s) {
+#pragma unroll
+        for (int c = 0; c < REC; c++) s.r[c] = *reinterpret_cast<const u32x4 *>(stage + c * N * 16 + row * 16);
+        if constexpr (BITS == 5)
+#pragma unroll
+            for (int c = 0; c < 2; c++) s.b[c] = *reinterpret_cast<const u32x4 *>(stage + (REC + c) * N * 16 + row * 16);
+    }
+    __device__ static uint32_t record(const Side &s, int b) { // d of block b of the superblock, and m above it
+        return WITH_MIN ? s.r[b >> 2][b & 3] : (s.r[0][b >> 1] >> (16 * (b & 1))) & 0xFFFFu;
+    }
+    __device__ static float scale(const Side &s, int b) { return h2f(record(s, b) & 0xFFFFu); }
+    // Q4, Q5: piece = the step's parity, its halves the step's blocks; Q8: a piece is a block
+    __device__ static void read_raw(const uint8_t *tile, int col, int hh, int j, Raw &r) {
+        const int x = (col >> 3) & 1;
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            if constexpr (BITS == 8) {
+                r.q[b] = *reinterpret_cast<const u32x4 *>(tile + (2 * (j & 1) + b) * 1024 + (col * 2 + (hh ^ x)) * 16);
+            } else if constexpr (BITS == 5) {
+                r.q[b] = *reinterpret_cast<const u32x4 *>(tile + (j & 1) * 1024 + (col * 2 + (b ^ x)) * 16);
+            } else {
+                typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+                const u32x2 v = *reinterpret_cast<const u32x2 *>(tile + (j & 1) * 1024 + (col * 2 + (b ^ x)) * 16 + hh * 8);
+                r.q[b][0] = v[0];
+                r.q[b][1] = v[1];
+            }
+        }
+    }
+    __device__ static void make(const Raw &r, const Side &s, const Scales &, uint32_t mask, int j, int t, int hh, half8 (&o)[1]) {
+        const int b = t >> 1, at = t & 1;
+        uint32_t w[4];
+        if constexpr (BITS == 8) { // signed bytes as unsigned ones + 128; 0x6400 | u is 1024 + u
+            const half2v c = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+#pragma unroll
+            for (int d = 0; d < 2; d++) {
+                const uint32_t v = r.q[b][2 * at + d] ^ 0x80808080u;
+                w[2 * d] = bits(halfs((v & 0x00FF00FFu) | 0x64006400u) + c);
+                w[2 * d + 1] = bits(halfs(((v >> 8) & 0x00FF00FFu) | 0x64006400u) + c);
+            }
+        } else { // a code at bits 4..7 (4..8) of a half with 0x5400 is 64 + q
+            const half2v c = {(_Float16)-(64.0f + CENTRE), (_Float16)-(64.0f + CENTRE)};
+            uint32_t e[4];
+            if constexpr (BITS == 4) { // byte i = elements 2 i (low), 2 i + 1: dword 2 hh + at is the operand's eight
+                const uint32_t p = __builtin_amdgcn_perm(0u, r.q[b][at], 0x03010200u); // bytes 0, 2, 1, 3
+                e[0] = p << 4; e[1] = p; e[2] = p >> 4; e[3] = p >> 8;
+            } else { // byte i = elements i (low), i + 16: lanes of the upper half take the high nibbles
+#pragma unroll
+                for (int d = 0; d < 2; d++) {
+                    const uint32_t v = r.q[b][2 * at + d] << (4 - 4 * hh);
+                    e[2 * d] = v;
+                    e[2 * d + 1] = v >> 8;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) e[i] = (e[i] & mask) | 0x54005400u;
+            if constexpr (BITS == 5) {
+                // bits b0..b3 times (2^8 + 2^22): b0 lands on bit 8 and b2 on bit 24 (of the pair 0, 2), nothing else does
+                const uint32_t f = s.b[j >> 1][2 * (j & 1) + b] >> (16 * hh + 8 * at);
+                e[0] |= ((f & 0xFu) * 0x00400100u) & 0x01000100u;
+                e[1] |= (((f >> 1) & 0x7u) * 0x00400100u) & 0x01000100u;
+                e[2] |= (((f >> 4) & 0xFu) * 0x00400100u) & 0x01000100u;
+                e[3] |= (((f >> 5) & 0x7u) * 0x00400100u) & 0x01000100u;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) w[i] = bits(halfs(e[i]) + c);
+        }
+        o[0] = octet(w);
+    }
+    // m + C d of blocks 4 hh .. 4 hh + 3 as f16 pairs, leading halves and then remainders, times a power of two that brings the
+    // superblock's largest below 2^15: |.| < (1 + 16) 2^(e + 1), e the largest exponent of its d and m.  `f`: what undoes it, and the
+    // 1 / 8 of the sums of x.
+    __device__ static half8 offsets(const Side &s, int hh, float &f) {
+        uint32_t most = 0x0400u; // f16 bits; smallest normal number
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            const uint32_t r = record(s, b), d = r & 0x7FFFu, m = (r >> 16) & 0x7FFFu;
+            most = d > most ? d : most;
+            most = m > most ? m : most;
+        }
+        const int e = (int)(most >> 10) - 15;
+        const float up = __builtin_bit_cast(float, (uint32_t)(127 + 9 - e) << 23);
+        f = __builtin_bit_cast(float, (uint32_t)(127 - 9 + e + 3) << 23);
+        uint32_t o[4];
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            float c[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const uint32_t r = hh ? record(s, 4 + 2 * p + i) : record(s, 2 * p + i);
+                c[i] = fmaf(CENTRE, h2f(r & 0xFFFFu), h2f(r >> 16)) * up;
+            }
+            const half2v h = __builtin_bit_cast(half2v, __builtin_amdgcn_cvt_pkrtz(c[0], c[1]));
+            o[p] = bits(h);
+            o[2 + p] = bits(half2v{(_Float16)(c[0] - (float)h[0]), (_Float16)(c[1] - (float)h[1])});
+        }
+        return octet(o);
+    }
+};
+
 // Stages in LDS: NA K steps of x, NW units of codes, the sides and the sums of x of two superblocks.  Half of a group's waves
 // copy x, the other half codes and sides: a wave's waits are in order of its requests, and x, which comes from L2 shortly before
 // it is used, would otherwise wait for codes that were requested from memory for later.
-template <class T, int MI, int WM, int NJ>
+// AT > 1: x as three limbs (see rows_prep_kernel).  2: up to 16 rows, in two tiles [first | second] and [0 | third] whose products meet in
+// one accumulator tile; 3: 32 rows in three tiles, the second and the third meet.
+template <class T, int MI, int WM, int NJ, int AT>
 struct RowsTile {
     static constexpr int KG = 2 / WM, GW = 4 * WM, CW = GW / 2;     // groups along K, waves of one, waves that copy x (and codes)
-    static constexpr int M = 32 * MI * WM, N = 128 * NJ;
+    static constexpr int M = AT == 2 ? 16 : AT == 3 ? 32 * WM : 32 * MI * WM, N = 128 * NJ, XT = AT > 1 ? AT : MI; // rows, columns, tiles of x of a wave
+    static constexpr int acc_of(int l) { return AT == 3 ? (l > 0 ? 1 : 0) : AT == 2 ? 0 : l; } // accumulator tile of a tile of x
+    static constexpr bool first_of(int l) { return l == XT - 1 || acc_of(l) != acc_of(l + 1); }
     static constexpr bool WHOLE = MI <= 2;                          // the fragments of a whole step ahead in registers
     static constexpr int HB = T::PAIRS * 32;                        // code bytes of a row and unit
-    static constexpr int ABYTES = WM * MI * 4096, WBYTES = N * HB, SBYTES = T::MIN ? WM * MI * 2048 : 0; // of a group's stage
+    static constexpr int ABYTES = WM * XT * 4096, WBYTES = N * HB, SBYTES = T::MIN ? WM * XT * 2048 : 0; // of a group's stage
     static constexpr int DBYTES = N * (16 * T::SIDE16 + 4 * T::SIDE4);
     static constexpr int NA = WHOLE ? 3 : 2;
     static constexpr int FIT = (160 * 1024 - KG * (NA * ABYTES + 2 * SBYTES + 2 * DBYTES)) / (KG * WBYTES), NW = FIT > 4 ? 4 : FIT;
     static constexpr int MAIL = KG == 2 ? 8 * MI * NJ * 8 * 64 * 4 : 0; // the groups' exchange, which reuses the stages
     static constexpr int STAGES = KG * (NA * ABYTES + NW * WBYTES + 2 * SBYTES + 2 * DBYTES), LDS = STAGES > MAIL ? STAGES : MAIL;
     // a copying wave's requests: x of a step, sums of a superblock; codes of a unit, sides of a superblock (small ones some of them twice)
-    static constexpr int XL = 2 * MI, SL = T::MIN ? MI : 0, WT = 4 * NJ / CW, WL = WT * T::PAIRS;
+    static constexpr int XL = 2 * XT, SL = T::MIN ? XT : 0, WT = 4 * NJ / CW, WL = WT * T::PAIRS;
     static constexpr int D16 = (2 * NJ * T::SIDE16 + CW - 1) / CW, D4 = (2 * NJ * T::SIDE4 + CW - 1) / CW;
     static constexpr int FIRST = 7 > 2 * NW - 1 ? 7 : 2 * NW - 1;
+    static_assert(AT == 1 || MI == AT - 1, "limbs");
     static_assert(NW >= 2 && WT * CW == 4 * NJ && NA <= FIRST, "stages");
     // Behind barrier b: x of step b + NA and, where b % 4 = 1, the sums of superblock (b + 3) / 4; codes of unit (b + 1) / 2 + NW - 1
     // where b is odd and the sides of superblock (b + 7) / 4 where b % 4 = 1.  In front of barrier g everything that is read
@@ -291,10 +427,10 @@ struct RowsTile {
     }
 };
 
-template <class T, int MI, int WM, int NJ>
+template <class T, int MI, int WM, int NJ, int AT>
 __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
-    using Tile = RowsTile<T, MI, WM, NJ>;
-    constexpr int KG = Tile::KG, HB = Tile::HB, ABYTES = Tile::ABYTES, WBYTES = Tile::WBYTES, SBYTES = Tile::SBYTES, DBYTES = Tile::DBYTES, NA = Tile::NA, NW = Tile::NW;
+    using Tile = RowsTile<T, MI, WM, NJ, AT>;
+    constexpr int KG = Tile::KG, HB = Tile::HB, ABYTES = Tile::ABYTES, WBYTES = Tile::WBYTES, SBYTES = Tile::SBYTES, DBYTES = Tile::DBYTES, NA = Tile::NA, NW = Tile::NW, XT = Tile::XT;
     extern __shared__ uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, li = lane & 31, hh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -302,7 +438,7 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
     const int nt = (a.n + Tile::N - 1) / Tile::N, total = (int)gridDim.x;
     int tile = blockIdx.x;
     if (total % 8 == 0) tile = (tile & 7) * (total >> 3) + (tile >> 3); // workgroups of one XCD share x tiles
-    const int mt0 = (tile / nt) * (WM * MI), n0 = (tile % nt) * Tile::N;
+    const int mt0 = (tile / nt) * (WM * XT), n0 = (tile % nt) * Tile::N;
     const int nsb_row = a.k >> 8, steps_row = a.k >> 6;
     const int lo = (int)blockIdx.y * a.sb_per_split, hi = lo + a.sb_per_split < nsb_row ? lo + a.sb_per_split : nsb_row;
     // superblocks of this group: `loops` is what every wave of the workgroup walks through, `mine` what this group multiplies
@@ -391,6 +527,7 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
         for (int j = 0; j < NJ; j++) T::template read_side<Tile::N>(dbase + (sb & 1) * DBYTES, (wn * NJ + j) * 32 + li, hh, sb0 + sb, next_side[j]);
     };
     auto new_side = [&](bool last = false) { // what the superblock in `side` asks for; where accumulators change their unit, they do with its first product
+        if constexpr (!T::BLOCKS)
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
             float u, shrink;
@@ -405,11 +542,11 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
             }
         }
     };
-    const uint8_t *my_x = abase + wm * MI * 4096 + lane * 16, *my_codes = wbase + wn * NJ * 32 * HB;
+    const uint8_t *my_x = abase + wm * XT * 4096 + lane * 16, *my_codes = wbase + wn * NJ * 32 * HB;
     int a_rd = 0, w_rd = 0; // stage of the step, of the unit that is read next
-    auto read_x = [&](int t, half8 (&f)[MI]) {
+    auto read_x = [&](int t, half8 (&f)[XT]) {
 #pragma unroll
-        for (int i = 0; i < MI; i++) f[i] = *reinterpret_cast<const half8 *>(my_x + a_rd + i * 4096 + t * 1024);
+        for (int i = 0; i < XT; i++) f[i] = *reinterpret_cast<const half8 *>(my_x + a_rd + i * 4096 + t * 1024);
     };
     auto read_codes = [&](int j4, typename T::Raw (&raw)[NJ]) {
 #pragma unroll
@@ -442,9 +579,9 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
     };
     auto make = [&](const typename T::Raw (&raw)[NJ], int j4, int t, half8 (&f)[NJ][T::PRODUCTS]) {
 #pragma unroll
-        for (int j = 0; j < NJ; j++) T::make(raw[j], side[j], scales[j], mask, j4, t, f[j]);
+        for (int j = 0; j < NJ; j++) T::make(raw[j], side[j], scales[j], mask, j4, t, hh, f[j]);
     };
-    auto multiply = [&](const half8 (&x)[MI], const half8 (&w)[NJ][T::PRODUCTS]) {
+    auto multiply = [&](const half8 (&x)[XT], const half8 (&w)[NJ][T::PRODUCTS]) {
 #pragma unroll
         for (int pr = 0; pr < T::PRODUCTS; pr++)
 #pragma unroll
@@ -452,15 +589,15 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
 #pragma unroll
                 for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[i], w[j][pr], acc[i][j], 0, 0, 0);
     };
-    auto add_offsets = [&](int sb, auto tile_j) { // of a column tile
-        if constexpr (T::MIN) {
+    auto add_offsets = [&](int sb, auto tile_j, float16v (&to)[MI][NJ]) { // of a column tile
+        if constexpr (T::MIN && !T::BLOCKS) {
             constexpr int j = decltype(tile_j)::value;
             const half8 o = T::offsets(side[j], hh, inv[j]);
 #pragma unroll
-            for (int i = 0; i < MI; i++) {
-                const uint8_t *x = sbase + (sb & 1) * SBYTES + (wm * MI + i) * 2048 + lane * 16;
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x), o, acc[i][j], 0, 0, 0);
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x + 1024), o, acc[i][j], 0, 0, 0);
+            for (int i = 0; i < XT; i++) {
+                const uint8_t *x = sbase + (sb & 1) * SBYTES + (wm * XT + i) * 2048 + lane * 16;
+                to[Tile::acc_of(i)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x), o, to[Tile::acc_of(i)][j], 0, 0, 0);
+                to[Tile::acc_of(i)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x + 1024), o, to[Tile::acc_of(i)][j], 0, 0, 0);
             }
         }
     };
@@ -481,66 +618,130 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
     barrier();
     read_sides(0);
     if constexpr (Tile::WHOLE) { // meet, request the next step's fragments, work on this step's
-        half8 af[2][4][MI];
+        constexpr int AHEAD = T::BLOCKS ? 1 : 2; // blocks: the next step's fragments take the place of the products' that are done
+        half8 af[AHEAD][4][XT];
         typename T::Raw raw[2][NJ];
-        // a step's products start from zero and their sum joins the total times d: fewer of the additions that round are of the
-        // total's size.  Error against 64 bits, f32 rows of normal x, K = 1024 / 4096 / 14336, Q4_K: 1.0 / 1.1 / 1.25e-7 (a
-        // superblock's products in one sum: 1.3 / 1.4 / 1.45e-7; the two-stage kernel before it, from 40 rows on: 1.3 / 1.8 / 3.1e-7;
-        // the small-batch GEMV: 0.95 / 1.05 / 1.3e-7)
-        float16v sum[MI][NJ];
-        auto fold = [&]() {
+        // a step's products (a block's, with blocks) start from zero, their sums meet in the superblock's, and that joins the total:
+        // few of the additions that round are of the total's size
+        float16v sum[MI][NJ], total[MI][NJ];
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) total[i][j] = sum[i][j] = acc[i][j];
+        auto each = [&](auto fn) {
 #pragma unroll
             for (int i = 0; i < MI; i++)
 #pragma unroll
                 for (int j = 0; j < NJ; j++)
 #pragma unroll
-                    for (int q = 0; q < 16; q++) {
-                        sum[i][j][q] = fmaf(acc[i][j][q], unit[j], sum[i][j][q]);
-                        acc[i][j][q] = 0.f;
-                    }
+                    for (int q = 0; q < 16; q++) fn(i, j, q);
         };
-#pragma unroll
-        for (int i = 0; i < MI; i++)
-#pragma unroll
-            for (int j = 0; j < NJ; j++) sum[i][j] = acc[i][j];
-        auto read_step = [&](int j4) {
+        const float16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        auto read_step = [&](int j4, bool first = false) {
             read_codes(j4, raw[j4 & 1]);
+            if (!T::BLOCKS || first)
 #pragma unroll
-            for (int t = 0; t < 4; t++) read_x(t, af[j4 & 1][t]);
+                for (int t = 0; t < 4; t++) read_x(t, af[j4 % AHEAD][t]);
             asm volatile("" ::: "memory"); // requested here, not where they are used
         };
+        auto products = [&](auto at, auto t0, auto t1, float16v (&to)[MI][NJ]) { // t0 .. t1 - 1 of a step, from zero
+            constexpr int J = decltype(at)::value, T0 = decltype(t0)::value, T1 = decltype(t1)::value;
+            half8 bf[T1 - T0][NJ][T::PRODUCTS];
+            auto mul = [&](int t, int l) {
+#pragma unroll
+                for (int pr = 0; pr < T::PRODUCTS; pr++)
+#pragma unroll
+                    for (int j = 0; j < NJ; j++)
+                        to[Tile::acc_of(l)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                            af[J % AHEAD][t][l], bf[t - T0][j][pr], Tile::first_of(l) && t == T0 && pr == 0 ? zero : to[Tile::acc_of(l)][j], 0, 0, 0);
+            };
+            if constexpr (AT == 1) {
+#pragma unroll
+                for (int t = T0; t < T1; t++) {
+                    make(raw[J & 1], J, t, bf[t - T0]);
+#pragma unroll
+                    for (int l = XT - 1; l >= 0; l--) mul(t, l);
+                }
+            } else {
+#pragma unroll
+                for (int t = T0; t < T1; t++) make(raw[J & 1], J, t, bf[t - T0]);
+#pragma unroll
+                for (int l = XT - 1; l >= 0; l--) // the third limbs first
+#pragma unroll
+                    for (int t = T0; t < T1; t++) mul(t, l);
+            }
+        };
+        using S4 = std::integral_constant<int, 4>;
         auto step = [&](int sb, auto at) {
             constexpr int J = decltype(at)::value;
+            // the last step's sums are in `sum` here: left to itself the compiler keeps the blocks' sums of a superblock apart
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    if (J == 0) asm volatile("" : "+v"(total[i][j]));
+                    else asm volatile("" : "+v"(sum[i][j]));
+                }
             meet(sb, at);
             read_step((J + 1) & 3);
             if (J == 3) read_sides(sb + 1); // looked at behind the next barrier
-            fold();
             if (J == 0) {
 #pragma unroll
                 for (int j = 0; j < NJ; j++) side[j] = next_side[j];
                 new_side();
             }
+            float16v part[MI][NJ];
+            if constexpr (T::BLOCKS) {
+                auto block = [&](auto half) {
+                    constexpr int B = decltype(half)::value;
+                    float d[NJ];
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                half8 bf[NJ][T::PRODUCTS];
-                make(raw[J & 1], J, t, bf);
-                multiply(af[J & 1][t], bf);
+                    for (int j = 0; j < NJ; j++) d[j] = T::scale(side[j], 2 * J + B);
+                    products(at, std::integral_constant<int, 2 * B>{}, std::integral_constant<int, 2 * B + 2>{}, part);
+                    asm volatile("" ::: "memory");
+                    read_x(2 * B, af[0][2 * B]);
+                    read_x(2 * B + 1, af[0][2 * B + 1]);
+                    asm volatile("" ::: "memory");
+                    each([&](int i, int j, int q) { sum[i][j][q] = J == 0 && B == 0 ? part[i][j][q] * d[j] : fmaf(part[i][j][q], d[j], sum[i][j][q]); });
+                };
+                block(S0{});
+                block(S1{});
+                if constexpr (T::MIN && J == 1) { // the superblock's offsets
+                    float f[NJ];
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) {
+                        const half8 o = T::offsets(side[j], hh, f[j]);
+#pragma unroll
+                        for (int i = XT - 1; i >= 0; i--) {
+                            constexpr auto acc_of = Tile::acc_of;
+                            const uint8_t *x = sbase + (sb & 1) * SBYTES + (wm * XT + i) * 2048 + lane * 16;
+                            part[acc_of(i)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x), o, Tile::first_of(i) ? zero : part[acc_of(i)][j], 0, 0, 0);
+                            part[acc_of(i)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x + 1024), o, part[acc_of(i)][j], 0, 0, 0);
+                        }
+                    }
+                    each([&](int i, int j, int q) { sum[i][j][q] = fmaf(part[i][j][q], f[j], sum[i][j][q]); });
+                }
+                if (J == 3) each([&](int i, int j, int q) { total[i][j][q] += sum[i][j][q]; });
+            } else {
+                products(at, S0{}, S4{}, part);
+                if constexpr (T::MIN && J >= 1 && J <= NJ) add_offsets(sb, std::integral_constant<int, J - 1>{}, part);
+                if (J == 0) each([&](int i, int j, int q) { sum[i][j][q] = part[i][j][q]; });
+                else each([&](int i, int j, int q) { sum[i][j][q] += part[i][j][q]; });
+                if (J == 3) each([&](int i, int j, int q) { total[i][j][q] = fmaf(sum[i][j][q], unit[j], total[i][j][q]); });
             }
-            if constexpr (J >= 1 && J <= NJ) add_offsets(sb, std::integral_constant<int, J - 1>{});
         };
-        read_step(0);
+        read_step(0, true);
         for (int sb = 0; sb < mine; sb++) {
             step(sb, S0{}); step(sb, S1{}); step(sb, S2{}); step(sb, S3{});
         }
-        fold();
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
             unit[j] = 1.0f;
 #pragma unroll
-            for (int i = 0; i < MI; i++) acc[i][j] = sum[i][j];
+            for (int i = 0; i < MI; i++) acc[i][j] = total[i][j];
         }
     } else { // a product's fragments ahead; the barrier in front of the step's last products
-        half8 af[2][MI], bf[2][NJ][T::PRODUCTS];
+        half8 af[2][XT], bf[2][NJ][T::PRODUCTS];
         typename T::Raw raw[NJ];
         auto step = [&](int sb, auto at) {
             constexpr int J = decltype(at)::value;
@@ -558,7 +759,7 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
                 if (J == 0 && t == 0) change_unit();
                 multiply(af[t & 1], bf[t & 1]);
                 if constexpr (J >= 1 && J <= NJ)
-                    if (t == 1) add_offsets(sb, std::integral_constant<int, J - 1>{});
+                    if (t == 1) add_offsets(sb, std::integral_constant<int, J - 1>{}, acc);
                 if (t == 3) {
                     if (J == 3) {
 #pragma unroll
@@ -585,9 +786,15 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
     wait_loads_and_lds<0>(); // nothing of this workgroup may still be on its way into LDS
 
     // ---- results.  D layout: lane -> column li; register r -> row 8 (r / 4) + 4 (lane / 32) + r % 4
+    if constexpr (AT > 1) // the first limbs' results and the others'; the others of sixteen rows lie sixteen rows below
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int r = 0; r < (AT == 2 ? 8 : 16); r++) acc[0][j][r] += AT == 2 ? acc[0][j][r + 8 & 15] : acc[MI - 1][j][r];
+    constexpr int MR = AT > 1 ? 1 : MI;
     auto store = [&](int i, int j, int r, float v, float v2) { // v2: of row r + 1, where rows are pairs
         const int gn = n0 + (wn * NJ + j) * 32 + li;
-        const int gm = (mt0 + wm * MI + i) * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
+        const int gm = (AT > 1 ? mt0 / AT + wm : mt0 + wm * MI + i) * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
         if (gm >= a.m || gn >= a.n) return;
         const size_t row = (size_t)(a.pair ? gm >> 1 : gm), rows = (size_t)(a.pair ? a.m >> 1 : a.m);
         if (a.pair) v += v2;
@@ -603,17 +810,17 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
     const int step_r = a.pair ? 2 : 1;
     if constexpr (KG == 2) { // a group finishes half of the registers and hands the other half over
         barrier();
-        float *mail = reinterpret_cast<float *>(lds) + (kg * 4 + wn) * (MI * NJ * 8 * 64) + lane;
+        float *mail = reinterpret_cast<float *>(lds) + (kg * 4 + wn) * (MR * NJ * 8 * 64) + lane;
 #pragma unroll
-        for (int i = 0; i < MI; i++)
+        for (int i = 0; i < MR; i++)
 #pragma unroll
             for (int j = 0; j < NJ; j++)
 #pragma unroll
                 for (int r = 0; r < 8; r++) mail[((i * NJ + j) * 8 + r) * 64] = (kg ? acc[i][j][r] : acc[i][j][r + 8]) * unit[j];
         __syncthreads();
-        const float *got = reinterpret_cast<const float *>(lds) + ((1 - kg) * 4 + wn) * (MI * NJ * 8 * 64) + lane;
+        const float *got = reinterpret_cast<const float *>(lds) + ((1 - kg) * 4 + wn) * (MR * NJ * 8 * 64) + lane;
 #pragma unroll
-        for (int i = 0; i < MI; i++)
+        for (int i = 0; i < MR; i++)
 #pragma unroll
             for (int j = 0; j < NJ; j++) {
                 float v[8];
@@ -625,7 +832,7 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
             }
     } else {
 #pragma unroll
-        for (int i = 0; i < MI; i++)
+        for (int i = 0; i < MR; i++)
 #pragma unroll
             for (int j = 0; j < NJ; j++)
 #pragma unroll
@@ -638,7 +845,7 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
 // norm_w is given ((x * inv_rms) * norm_w, RMSNorm::forward, llm/src/llama.rs:158-187); 1 f32 rows of 2 k gate/up values, four
 // and four, which become silu(gate) * up; 2 bf16 rows.  f32 rows become two rows each.  A workgroup per row, a thread per
 // eight elements; the row stays in registers (NC times 4096 elements) or, NC = 0, is read once per pass.
-template <int IN, int NC>
+template <int IN, int NC, bool LIMBS>
 __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const float *norm_w, float eps, int k, _Float16 *xa, _Float16 *xs,
                                                         float *rowscale) {
     constexpr int HELD = NC > 0 ? NC : 1;
@@ -745,33 +952,43 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
     int sb = 127 + 11 - (eb - 127);
     sb = sb < 1 ? 1 : (sb > 254 ? 254 : sb);
     const float f = __builtin_bit_cast(float, (uint32_t)sb << 23);
-    constexpr int PARTS = IN == 2 ? 1 : 2;
+    constexpr int PARTS = LIMBS ? 3 : IN == 2 ? 1 : 2;
     const int r0 = row * PARTS, steps = k >> 6, nsb = k >> 8;
-    _Float16 *xt = xa + (size_t)(r0 >> 5) * steps * 2048, *st = xs + (size_t)(r0 >> 5) * nsb * 1024;
+    auto slot = [&](int part) { // of the operand's rows: pairs are neighbours; limbs see RowsTile, part 3 = the zeros
+        if (!LIMBS) return r0 + part;
+        return gridDim.x <= 16 ? (part < 2 ? part : 5 - part) * 16 + row : ((row >> 5) * 3 + part) * 32 + (row & 31);
+    };
     each(false, [&](float (&e)[8], int c) {
         if (NC == 0) normed(e, c);
-        _Float16 p[2][8];
-        float sum[2] = {0.f, 0.f};
+        _Float16 p[PARTS][8];
+        float sum[PARTS];
+#pragma unroll
+        for (int part = 0; part < PARTS; part++) sum[part] = 0.f;
 #pragma unroll
         for (int q = 0; q < 8; q++) {
-            const float s = e[q] * f;
-            p[0][q] = (_Float16)s;
-            sum[0] += (float)p[0][q];
-            if (PARTS == 2) {
-                p[1][q] = (_Float16)(s - (float)p[0][q]);
-                sum[1] += (float)p[1][q];
+            float s = e[q] * f;
+#pragma unroll
+            for (int part = 0; part < PARTS; part++) {
+                // limbs: multiples of 2^2, 2^-9, 2^-20, at most 2^10 of them
+                p[part][q] = LIMBS ? (_Float16)(rintf(s * (part == 0 ? 0x1p-2f : part == 1 ? 0x1p9f : 0x1p20f)) * (part == 0 ? 0x1p2f : part == 1 ? 0x1p-9f : 0x1p-20f))
+                                   : (_Float16)s;
+                sum[part] += (float)p[part][q];
+                s -= (float)p[part][q];
             }
         }
         // chunk c: step c / 8, product t, half of the lanes (see the order of elements above)
         const int at = c & 7, t = (at >> 2) * 2 + (at & 1), h = (at >> 1) & 1;
 #pragma unroll
-        for (int part = 0; part < PARTS; part++) {
-            const int lrow = (r0 + part) & 31;
-            const _Float16 *s = p[part];
+        for (int part = 0; part < PARTS + (LIMBS ? 1 : 0); part++) {
+            if (part == PARTS && gridDim.x > 16) break;
+            const int at_row = slot(part), lrow = at_row & 31;
+            _Float16 *xt = xa + (size_t)(at_row >> 5) * steps * 2048, *st = xs + (size_t)(at_row >> 5) * nsb * 1024;
+            const _Float16 *s = p[part < PARTS ? part : 0];
+            const half8 out = part < PARTS ? half8{s[0], s[2], s[1], s[3], s[4], s[6], s[5], s[7]} : half8{0, 0, 0, 0, 0, 0, 0, 0};
             if (c < chunks)
-                *reinterpret_cast<half8 *>(xt + ((size_t)(c >> 3) * 4 + t) * 512 + (h * 32 + lrow) * 8) = half8{s[0], s[2], s[1], s[3], s[4], s[6], s[5], s[7]};
+                *reinterpret_cast<half8 *>(xt + ((size_t)(c >> 3) * 4 + t) * 512 + (h * 32 + lrow) * 8) = out;
             // the sum of 32 elements: four threads; times 1 / 8 it stays within f16's range
-            float g = sum[part];
+            float g = part < PARTS ? sum[part] : 0.f;
             g += __shfl_xor(g, 1);
             g += __shfl_xor(g, 2);
             if ((tid & 3) == 0 && c < chunks) {
@@ -784,51 +1001,65 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
             }
         }
     });
-    if (tid < PARTS) rowscale[r0 + tid] = 1.0f / f;
+    if (tid < (LIMBS ? 1 : PARTS)) rowscale[(LIMBS ? row : r0) + tid] = 1.0f / f;
 }
 
-template <class T, int MI, int WM, int NJ>
+template <class T, int MI, int WM, int NJ, int AT>
 int launch_tile(axq_ctx *ctx, const RowsArgs &a, int splits) {
-    using Tile = RowsTile<T, MI, WM, NJ>;
+    using Tile = RowsTile<T, MI, WM, NJ, AT>;
     static std::atomic<uint64_t> lds_allowed{0};
-    if (int rc = axq_allow_lds(ctx, reinterpret_cast<const void *>(rows_gemm_kernel<T, MI, WM, NJ>), lds_allowed, Tile::LDS)) return rc;
+    if (int rc = axq_allow_lds(ctx, reinterpret_cast<const void *>(rows_gemm_kernel<T, MI, WM, NJ, AT>), lds_allowed, Tile::LDS)) return rc;
     const unsigned tiles = (unsigned)(((a.n + Tile::N - 1) / Tile::N) * ((a.m + Tile::M - 1) / Tile::M));
-    rows_gemm_kernel<T, MI, WM, NJ><<<dim3(tiles, (unsigned)splits), 512, Tile::LDS, ctx->stream>>>(a);
+    rows_gemm_kernel<T, MI, WM, NJ, AT><<<dim3(tiles, (unsigned)splits), 512, Tile::LDS, ctx->stream>>>(a);
     AXQ_LAUNCH_CHECK(ctx, "rows_gemm_kernel");
     return AXQ_OK;
 }
 
-// The tile of a call.  Up to 32, 64 rows of operands (16, 32 f32 rows): one and two row tiles per wave and the two halves of the
-// waves on two parts of K, since a workgroup's time is then its number of steps.  65 to 128 rows: two times two row tiles (at
-// 64 f32 rows and Q4_K 28672 x 4096 2.5 us ahead of four row tiles per wave and split halves).  Above: 256 x 256 outputs.
+// The tile of a call.  Limbs: up to 16 and 32 rows the two halves of the waves on two parts of K, since a workgroup's time is then its
+// number of steps.  Others: up to 32 and 64 rows of operands the same with one and two row tiles per wave; 65 to 128 rows: two times
+// two row tiles (at 64 f32 rows and Q4_K 28672 x 4096 2.5 us ahead of four row tiles per wave and split halves).  Above: 256 x 256
+// outputs, which blocks do not have: their sums do not fit the registers.
 template <class T>
-int launch_rows(axq_ctx *ctx, const RowsArgs &a, int splits) {
-    if (a.m > 128) return launch_tile<T, 4, 2, 2>(ctx, a, splits);
-    if (a.m > 64) return launch_tile<T, 2, 2, 1>(ctx, a, splits);
-    if (a.m > 32) return launch_tile<T, 2, 1, 1>(ctx, a, splits);
-    return launch_tile<T, 1, 1, 1>(ctx, a, splits);
+int launch_rows(axq_ctx *ctx, const RowsArgs &a, int splits, bool limbs) {
+    if (limbs) {
+        if (a.m > 32) return launch_tile<T, 2, 2, 1, 3>(ctx, a, splits);
+        if (a.m > 16) return launch_tile<T, 2, 1, 1, 3>(ctx, a, splits);
+        return launch_tile<T, 1, 1, 1, 2>(ctx, a, splits);
+    }
+    if constexpr (!T::BLOCKS)
+        if (a.m > 128) return launch_tile<T, 4, 2, 2, 1>(ctx, a, splits);
+    if (a.m > 64) return launch_tile<T, 2, 2, 1, 1>(ctx, a, splits);
+    if (a.m > 32) return launch_tile<T, 2, 1, 1, 1>(ctx, a, splits);
+    return launch_tile<T, 1, 1, 1, 1>(ctx, a, splits);
 }
 
-template <int IN>
+template <int IN, bool LIMBS>
 void launch_prep(hipStream_t st, const void *x, const float *norm_w, float eps, int rows, int k, _Float16 *xa, _Float16 *xs, float *rs) {
-    if (k <= 4096) rows_prep_kernel<IN, 1><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
-    else if (k <= 8192) rows_prep_kernel<IN, 2><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
-    else if (k <= 16384) rows_prep_kernel<IN, 4><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
-    else rows_prep_kernel<IN, 0><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
+    if (k <= 4096) rows_prep_kernel<IN, 1, LIMBS><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
+    else if (k <= 8192) rows_prep_kernel<IN, 2, LIMBS><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
+    else if (k <= 16384) rows_prep_kernel<IN, 4, LIMBS><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
+    else rows_prep_kernel<IN, 0, LIMBS><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
 }
 
 } // namespace
 
-bool axq_dev_rows_gemm_covers(const axq_weight *w) {
-    return (w->type == AXQ_Q4_K || w->type == AXQ_Q5_K || w->type == AXQ_Q6_K) && w->k % 256 == 0 && w->k <= INT32_MAX && w->n_rows <= INT32_MAX;
+// Superblock types at any number of rows; blocks of 32 up to 128 rows of operands (above, gemm_blk32_kernel).  K a multiple of 256.
+bool axq_dev_rows_gemm_covers(const axq_weight *w, int rows, bool bf16) {
+    if (w->k % 256 != 0 || w->k > INT32_MAX || w->n_rows > INT32_MAX || rows < 1) return false;
+    switch (w->type) {
+    case AXQ_Q4_K: case AXQ_Q5_K: case AXQ_Q6_K: return true;
+    case AXQ_Q4_0: case AXQ_Q4_1: case AXQ_Q5_0: case AXQ_Q5_1: case AXQ_Q8_0: return rows <= (bf16 ? 128 : 64);
+    default: return false;
+    }
 }
 
 // Scratch: x in operand order | its sub-block sums | row scales | partial sums of a split K.
 int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, int rows, const float *norm_w, float eps, const float *bias,
                       const float *resid, float *y) {
-    const int parts = in == AXQ_ROWS_BF16 ? 1 : 2, m = rows * parts, n = (int)w->n_rows, k = (int)w->k;
-    const int bm = m <= 32 ? 32 : m <= 64 ? 64 : m <= 128 ? 128 : 256;
-    const int nsb = k >> 8, cus = ctx->prop.multiProcessorCount, groups = m <= 64 ? 2 : 1;
+    const bool limbs = in != AXQ_ROWS_BF16 && rows < AXQ_ROWS_PAIRS_MIN;
+    const int parts = in == AXQ_ROWS_BF16 || limbs ? 1 : 2, m = rows * parts, n = (int)w->n_rows, k = (int)w->k;
+    const int bm = limbs ? (rows <= 32 ? 32 : 64) : m <= 32 ? 32 : m <= 64 ? 64 : m <= 128 ? 128 : 256;
+    const int nsb = k >> 8, cus = ctx->prop.multiProcessorCount, groups = m <= (limbs ? 32 : 64) ? 2 : 1;
     const int bn = m <= 128 ? 128 : 256;
     const long tiles = (long)((n + bn - 1) / bn) * ((m + bm - 1) / bm);
     // K is split over as many workgroups as leave every group of waves a superblock, up to one workgroup per compute unit
@@ -839,7 +1070,7 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
     RowsArgs a;
     a.sb_per_split = (nsb + splits - 1) / splits;
     splits = (nsb + a.sb_per_split - 1) / a.sb_per_split;
-    const size_t mtiles = (size_t)(m + bm - 1) / bm * (bm / 32);
+    const size_t mtiles = limbs ? (rows <= 16 ? 2 : rows <= 32 ? 3 : 6) : (size_t)(m + bm - 1) / bm * (bm / 32);
     const size_t xa_bytes = mtiles * 32 * (size_t)k * 2, xs_bytes = mtiles * (size_t)nsb * 2048;
     const size_t rs_bytes = axq_align_up((size_t)m * 4, 256), part_bytes = splits > 1 ? (size_t)splits * rows * (size_t)n * 4 : 0;
     if (int rc = axq_gemm_reserve(ctx, xa_bytes + xs_bytes + rs_bytes + part_bytes)) return rc;
@@ -847,9 +1078,15 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
     _Float16 *xa = reinterpret_cast<_Float16 *>(base), *xs = reinterpret_cast<_Float16 *>(base + xa_bytes);
     float *rs = reinterpret_cast<float *>(base + xa_bytes + xs_bytes);
     switch (in) {
-    case AXQ_ROWS_BF16: launch_prep<2>(ctx->stream, x, nullptr, 0.f, rows, k, xa, xs, rs); break;
-    case AXQ_ROWS_SWIGLU: launch_prep<1>(ctx->stream, x, nullptr, 0.f, rows, k, xa, xs, rs); break;
-    default: launch_prep<0>(ctx->stream, x, norm_w, eps, rows, k, xa, xs, rs); break;
+    case AXQ_ROWS_BF16: launch_prep<2, false>(ctx->stream, x, nullptr, 0.f, rows, k, xa, xs, rs); break;
+    case AXQ_ROWS_SWIGLU:
+        if (limbs) launch_prep<1, true>(ctx->stream, x, nullptr, 0.f, rows, k, xa, xs, rs);
+        else launch_prep<1, false>(ctx->stream, x, nullptr, 0.f, rows, k, xa, xs, rs);
+        break;
+    default:
+        if (limbs) launch_prep<0, true>(ctx->stream, x, norm_w, eps, rows, k, xa, xs, rs);
+        else launch_prep<0, false>(ctx->stream, x, norm_w, eps, rows, k, xa, xs, rs);
+        break;
     }
     a.codes = w->codes; a.meta = w->meta; a.qh = w->qh;
     a.codes_pitch = (uint32_t)w->codes_pitch; a.meta_pitch = (uint32_t)w->meta_pitch; a.qh_pitch = (uint32_t)w->qh_pitch;
@@ -858,9 +1095,14 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
     a.m = m; a.n = n; a.k = k; a.pair = parts == 2; a.bias = bias; a.resid = resid;
     int rc;
     switch (w->type) {
-    case AXQ_Q4_K: rc = launch_rows<SuperQ45<false>>(ctx, a, splits); break;
-    case AXQ_Q5_K: rc = launch_rows<SuperQ45<true>>(ctx, a, splits); break;
-    default: rc = launch_rows<SuperQ6>(ctx, a, splits); break;
+    case AXQ_Q4_K: rc = launch_rows<SuperQ45<false>>(ctx, a, splits, limbs); break;
+    case AXQ_Q5_K: rc = launch_rows<SuperQ45<true>>(ctx, a, splits, limbs); break;
+    case AXQ_Q6_K: rc = launch_rows<SuperQ6>(ctx, a, splits, limbs); break;
+    case AXQ_Q4_0: rc = launch_rows<Block32<4, false>>(ctx, a, splits, limbs); break;
+    case AXQ_Q4_1: rc = launch_rows<Block32<4, true>>(ctx, a, splits, limbs); break;
+    case AXQ_Q5_0: rc = launch_rows<Block32<5, false>>(ctx, a, splits, limbs); break;
+    case AXQ_Q5_1: rc = launch_rows<Block32<5, true>>(ctx, a, splits, limbs); break;
+    default: rc = launch_rows<Block32<8, false>>(ctx, a, splits, limbs); break;
     }
     if (rc || splits == 1) return rc;
     return axq_gemm_reduce(ctx, a.ypart, rs, rows, n, splits, 1.0f, parts, bias, resid, y);

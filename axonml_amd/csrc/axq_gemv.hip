@@ -664,11 +664,12 @@ int launch(axq_ctx *ctx, const axq_weight *w, const float *x, const float *bias,
 int axq_dev_gemv(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, const float *bias, float *y) {
     if (w->n_rows > INT32_MAX || w->k > INT32_MAX)
         return axq_fail(ctx, AXQ_ERR_SHAPE_MISMATCH, "Shape mismatch: weight dimensions exceed 2^31");
-    // many vectors: through the matrix-pipe GEMM, each f32 row as two f16 rows.  Superblock types from nine rows on (Q4_K 28672 x
-    // 4096: 27.6 us for 9 to 16 rows, groups of eight 35 and 40.5; 4096 x 14336 at nine rows even); the others from about 40
-    // rows where the small-batch kernel below is the alternative, from 8 where single-vector passes are
+    // many vectors: through the matrix-pipe GEMM.  Where the rows kernel covers the weight from ten on (4096 x 4096, ten rows: Q4_0 16.0 us,
+    // groups of eight 22.3; Q4_K 16.9 and 22.7; 256 x 512 10.4 and 15.4; nine rows, which the GEMV does as eight and one, are 1 to 2 us
+    // behind it); the others from about 40 rows where the small-batch kernel below is the alternative, from 8 where single-vector passes are
     static const bool no_gemm = getenv("AXQ_GEMV_GEMM") && getenv("AXQ_GEMV_GEMM")[0] == '0'; // development knob
-    while (!no_gemm && batch >= (axq_dev_rows_gemm_covers(w) ? AXQ_ROWS_GEMM_MIN : axq_dev_gemv_batch_covers(w, 8) ? 40 : 8) && axq_dev_gemm_f32_covers(w, 1)) {
+    while (!no_gemm && axq_dev_gemm_f32_covers(w, 1) &&
+           batch >= (axq_dev_rows_gemm_covers(w, batch, false) ? AXQ_ROWS_GEMM_MIN : axq_dev_gemv_batch_covers(w, 8) ? 40 : 8)) {
         const int nb = batch < AXQ_GEMM_F32_MAX_ROWS ? batch : AXQ_GEMM_F32_MAX_ROWS;
         int rc = axq_dev_gemm_f32(ctx, w, x, nb, nullptr, 0.f, bias, nullptr, y);
         if (rc) return rc;

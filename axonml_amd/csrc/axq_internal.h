@@ -162,10 +162,12 @@ int axq_dev_sample_rows(axq_ctx *ctx, int rows, const float *logits, size_t logi
 int axq_dev_attn_rows_mfma(axq_ctx *ctx, const float *qkv, int qkv_rows, const float *rope_cos, const float *rope_sin,
                            const uint16_t *kcache, const uint16_t *vcache, int pos0, int T, int n_heads, int n_kv, int head_dim,
                            int max_pos, int window, float *att);
-// gemm_rows.hip: rows times a superblock-type weight, K a multiple of 256
+// gemm_rows.hip: rows times a packed weight, K a multiple of 256
 enum { AXQ_ROWS_F32 = 0, AXQ_ROWS_SWIGLU = 1, AXQ_ROWS_BF16 = 2 };
-bool axq_dev_rows_gemm_covers(const axq_weight *w);
-#define AXQ_ROWS_GEMM_MIN 9 // f32 rows from which it is ahead of the small-batch GEMV's groups of eight
+bool axq_dev_rows_gemm_covers(const axq_weight *w, int rows, bool bf16);
+// f32 rows below it go in as three limbs of eleven bits (the small-batch GEMV, which took them before, has 28 bits), from it on as pairs
+#define AXQ_ROWS_PAIRS_MIN 40
+#define AXQ_ROWS_GEMM_MIN 10 // f32 rows from which it is ahead of the small-batch GEMV in groups of eight
 int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, int rows, const float *norm_w, float eps, const float *bias,
                       const float *resid, float *y);
 // gemm.hip

@@ -1,5 +1,5 @@
-"""GPU parity of the many-row product with superblock weights (Q4_K, Q5_K, Q6_K): every tile it has, at its edges, against the
-float64 product of the dequantised weights.
+"""GPU parity of the many-row product with superblock weights (Q4_K, Q5_K, Q6_K) and blocks of 32 (Q4_0, Q4_1, Q5_0, Q5_1, Q8_0):
+every tile it has, at its edges, against the float64 product of the dequantised weights.
 
 Bound: an f32 row keeps 22 bits (2^-23 of each element) and K products are added in f32, in at most 4 K / 256 + 8 parts whose
 sums are rounded: |error| <= (2^-22 + (K / 64 + 8) 2^-24) sum |x w|, and the change of the accumulators' unit rounds them once
@@ -24,18 +24,21 @@ def _check(ctx, qtype, n, k, packed, x, bias=None, bf16=False):
         got = q.quantized_matmul(x, qt, bias, ctx)
     x = x.astype(np.float64)
     want = x @ deq.T + (0 if bias is None else bias.astype(np.float64))
-    # Q4_K and Q5_K are added as two parts, each as large as the codes' range
-    span = 3.0 if qtype != o.Q6_K else 1.0
+    # types with an offset are added as two parts, each as large as the codes' range
+    span = 3.0 if qtype in (o.Q4_K, o.Q5_K, o.Q4_1, o.Q5_1) else 1.0
     bound = 3 * (2.0 ** -22 + (k / 64 + 8) * 2.0 ** -24) * span * (np.abs(x) @ np.abs(deq).T) + 2.0 ** -22 * np.abs(want) + 1e-30
     off = np.abs(got - want) / bound
     assert np.isfinite(got).all() and off.max() <= 1, f"{o.TYPE_NAMES[qtype]} {x.shape[0]} x {n} x {k}: {off.max():.2f} of the bound"
 
 
-@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
-@pytest.mark.parametrize("rows,n,k", [(9, 1, 256), (16, 128, 512), (17, 129, 768), (32, 127, 2304), (33, 260, 256), (48, 64, 4352), (64, 128, 1024),
-                                      (65, 257, 512), (128, 256, 256), (130, 4, 768), (9, 2048, 4096), (40, 1030, 2560)])
+BLOCKS = [o.Q4_0, o.Q4_1, o.Q5_0, o.Q5_1, o.Q8_0]
+
+
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K, *BLOCKS])
+@pytest.mark.parametrize("rows,n,k", [(9, 1, 256), (10, 1, 256), (16, 128, 512), (17, 129, 768), (32, 127, 2304), (33, 260, 256), (39, 132, 1280),
+                                      (48, 64, 4352), (64, 128, 1024), (65, 257, 512), (128, 256, 256), (130, 4, 768), (10, 2048, 4096), (40, 1030, 2560)])
 def test_tiles_and_remainders(ctx, qtype, rows, n, k):
-    """Row counts on both sides of the tiles of 16, 32, 64 and 128 f32 rows, columns around 128 and 256, one superblock, odd counts
+    """Row counts on both sides of the tiles of 16, 32, 39, 64 and 128 f32 rows, columns around 128 and 256, one superblock, odd counts
     of them for the two halves of a workgroup, and K in pieces."""
     rng = np.random.default_rng(rows * 7 + n + k + qtype)
     packed = o.quantize(qtype, gen_weight(rng, n, k))
@@ -57,6 +60,25 @@ def test_superblocks_of_every_scale(ctx, qtype, size, at, rows):
     b[:, at:at + 2] = rng.choice(d, len(b)).view(np.uint8).reshape(-1, 2)
     if qtype != o.Q6_K:
         b[:, 2:4] = rng.choice(m, len(b)).view(np.uint8).reshape(-1, 2)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    x[1] = np.abs(x[1])
+    _check(ctx, qtype, n, k, b.reshape(-1), x)
+
+
+@pytest.mark.parametrize("qtype", BLOCKS)
+@pytest.mark.parametrize("rows", [12, 24, 56])
+def test_blocks_of_every_scale(ctx, qtype, rows):
+    """Blocks without a scale, without a minimum, with neither, from f16's smallest numbers to its largest, of either sign."""
+    rng = np.random.default_rng(rows + qtype)
+    n, k = 140, 1536
+    size = {o.Q4_0: 18, o.Q4_1: 20, o.Q5_0: 22, o.Q5_1: 24, o.Q8_0: 34}[qtype]
+    b = o.quantize(qtype, gen_weight(rng, n, k)).reshape(-1, size).copy()
+    d = np.array([0, 6e-8, 1e-6, 1e-3, 0.5, 300, -1e-3, 65504 if qtype != o.Q5_1 else 2000], np.float16)
+    b[:, :2] = rng.choice(d, len(b)).view(np.uint8).reshape(-1, 2)
+    if qtype in (o.Q4_1, o.Q5_1):
+        m = np.array([0, 0, 6e-8, 1e-4, -0.1, 60, -65504], np.float16)
+        b[:, 2:4] = rng.choice(m, len(b)).view(np.uint8).reshape(-1, 2)
+    b[:k // 32, :2] = 0  # a row of nothing but minima
     x = rng.standard_normal((rows, k)).astype(np.float32)
     x[1] = np.abs(x[1])
     _check(ctx, qtype, n, k, b.reshape(-1), x)
