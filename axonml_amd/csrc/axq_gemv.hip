@@ -659,6 +659,14 @@ int launch(axq_ctx *ctx, const axq_weight *w, const float *x, const float *bias,
     return AXQ_OK;
 }
 
+// Whether the context's stream records into a graph.  The GEMM's scratch grows on demand, which no capture allows, and moves when it
+// grows, under the graphs that were recorded; the small-batch GEMV's stands as long as the context does.
+bool being_captured(axq_ctx *ctx) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess) (void)hipGetLastError();
+    return status == hipStreamCaptureStatusActive;
+}
+
 } // namespace
 
 int axq_dev_gemv(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, const float *bias, float *y) {
@@ -668,10 +676,15 @@ int axq_dev_gemv(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, c
     // groups of eight 22.3; Q4_K 16.9 and 22.7; 256 x 512 10.4 and 15.4; nine rows, which the GEMV does as eight and one, are 1 to 2 us
     // behind it); the others from about 40 rows where the small-batch kernel below is the alternative, from 8 where single-vector passes are
     static const bool no_gemm = getenv("AXQ_GEMV_GEMM") && getenv("AXQ_GEMV_GEMM")[0] == '0'; // development knob
+    const int others_min = axq_dev_gemv_batch_covers(w, 8) ? 40 : 8;
     while (!no_gemm && axq_dev_gemm_f32_covers(w, 1) &&
-           batch >= (axq_dev_rows_gemm_covers(w, batch, false) ? AXQ_ROWS_GEMM_MIN : axq_dev_gemv_batch_covers(w, 8) ? 40 : 8)) {
+           (batch >= others_min || (batch >= AXQ_ROWS_GEMM_MIN && axq_dev_rows_gemm_covers(w, batch, false) && !being_captured(ctx)))) {
         const int nb = batch < AXQ_GEMM_F32_MAX_ROWS ? batch : AXQ_GEMM_F32_MAX_ROWS;
         int rc = axq_dev_gemm_f32(ctx, w, x, nb, nullptr, 0.f, bias, nullptr, y);
+        if (rc == AXQ_ERR_ALLOCATION_FAILED && nb < others_min) { // no room for its scratch: the kernel below needs none
+            (void)hipGetLastError();
+            break;
+        }
         if (rc) return rc;
         x += (size_t)nb * (size_t)w->k;
         y += (size_t)nb * (size_t)w->n_rows;
