@@ -424,23 +424,26 @@ __global__ void __launch_bounds__(128) rope_append_kernel(const float *qkv, int 
     vc[e + half] = __half_as_ushort(__float2half_rn(vh[e + half]));
 }
 
-// attn_prompt_kernel, grid (heads, tokens), 1024 threads: the query of head `head` at position p = pos0 + b
+// attn_prompt_kernel, grid (heads, tokens), TH threads: the query of head `head` at position p = pos0 + b
 // against the cached keys lo..p (causal, llama.rs:420-447; lo > 0 under a sliding window): scores into LDS, their
 // maximum, exponentials and sum, then sum_j e_j v_j / sum.  Keys and values are read 16 bytes per lane,
 // head_dim / 8 lanes per position.  APPEND (rows of different sequences only, pos_arr given): the row's own key and
 // value are not in the cache yet; every workgroup rotates the key itself, uses both from LDS (rounded to f16 as the
 // cache holds them), and the first query head of each KV head writes them to the cache.
-template <int D, bool APPEND>
-__global__ void __launch_bounds__(1024) attn_prompt_kernel(const float *qkv, int qkv_rows, const float *rope_cos,
+// TH is 1024 where workgroups are few (all loads of a short context at once), 256 where they are more than run at once: such a
+// workgroup's time is barriers and latency, and eight of them on a compute unit fill each other's gaps.  32 heads x 64 sequences at
+// position 128: 33 us with 1024 threads, 21.8 us with 256.
+template <int D, bool APPEND, int TH>
+__global__ void __launch_bounds__(TH) attn_prompt_kernel(const float *qkv, int qkv_rows, const float *rope_cos,
                                                            const float *rope_sin, uint16_t *kcache, uint16_t *vcache, int pos0,
                                                            const int32_t *pos_arr, size_t seq_stride, int n_heads, int n_kv,
                                                            int max_pos, int window, float *att, PackOut pk) {
-    constexpr int HALF = D / 2, LP = D / 8, PPB = 1024 / LP; // lanes per position, positions per pass of the workgroup
+    constexpr int HALF = D / 2, LP = D / 8, PPB = TH / LP, WAVES = TH / 64; // lanes per position, positions per pass of the workgroup
     extern __shared__ float sc[];                            // scores, then exp(score - max)
     __shared__ __attribute__((aligned(16))) float qs[D];
     __shared__ __attribute__((aligned(16))) float knew[APPEND ? D : 4], vnew[APPEND ? D : 4];
     __shared__ float red[16];
-    __shared__ __attribute__((aligned(16))) float osum[16 * D];
+    __shared__ __attribute__((aligned(16))) float osum[WAVES * D];
     const int head = blockIdx.x, b = blockIdx.y;
     const int p = pos_arr ? pos_arr[b] : pos0 + b; // as in rope_append_kernel
     if (pos_arr) { kcache += (size_t)b * seq_stride; vcache += (size_t)b * seq_stride; }
@@ -456,8 +459,8 @@ __global__ void __launch_bounds__(1024) attn_prompt_kernel(const float *qkv, int
         const float q1 = qh[tid], q2 = qh[tid + HALF];
         qs[tid] = q1 * c - q2 * s;
         qs[tid + HALF] = q1 * s + q2 * c;
-    } else if (APPEND && tid >= 512 && tid < 512 + HALF) { // other waves: the new key and value (arithmetic of rope_append_kernel)
-        const int e = tid - 512, q_dim = n_heads * D, kv_dim = n_kv * D;
+    } else if (APPEND && tid >= TH / 2 && tid < TH / 2 + HALF) { // other waves: the new key and value (arithmetic of rope_append_kernel)
+        const int e = tid - TH / 2, q_dim = n_heads * D, kv_dim = n_kv * D;
         const float *row = qkv + (size_t)b * qkv_rows;
         const float *kh = row + q_dim + (size_t)kvh * D, *vh = row + q_dim + kv_dim + (size_t)kvh * D;
         const float nc = rope_cos[(size_t)p * HALF + e], ns = rope_sin[(size_t)p * HALF + e];
@@ -507,16 +510,16 @@ __global__ void __launch_bounds__(1024) attn_prompt_kernel(const float *qkv, int
     }
     __syncthreads();
     float mx = -INFINITY;
-    for (int j = tid; j < span; j += 1024) mx = fmaxf(mx, sc[j]);
+    for (int j = tid; j < span; j += TH) mx = fmaxf(mx, sc[j]);
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m));
     if (lane == 0) red[wave] = mx;
     __syncthreads();
     mx = red[0];
 #pragma unroll
-    for (int w = 1; w < 16; w++) mx = fmaxf(mx, red[w]);
+    for (int w = 1; w < WAVES; w++) mx = fmaxf(mx, red[w]);
     float sum = 0.f;
-    for (int j = tid; j < span; j += 1024) {
+    for (int j = tid; j < span; j += TH) {
         const float e = expf(sc[j] - mx);
         sc[j] = e;
         sum += e;
@@ -544,7 +547,7 @@ __global__ void __launch_bounds__(1024) attn_prompt_kernel(const float *qkv, int
             for (int i = 0; i < 8; i++) acc[i] = fmaf(e, vf[i], acc[i]);
         }
     }
-    // lanes of a wave that hold the same dims, then the sixteen waves in order
+    // lanes of a wave that hold the same dims, then the waves in order
 #pragma unroll
     for (int m = LP; m < 64; m <<= 1) {
 #pragma unroll
@@ -559,7 +562,7 @@ __global__ void __launch_bounds__(1024) attn_prompt_kernel(const float *qkv, int
     if (tid < D) {
         float o = 0.f;
 #pragma unroll
-        for (int w = 0; w < 16; w++) o += osum[w * D + tid];
+        for (int w = 0; w < WAVES; w++) o += osum[w * D + tid];
         o /= sum;
         att[(size_t)b * n_heads * D + (size_t)head * D + tid] = o;
         qs[tid] = o; // the query is in registers by now
@@ -962,17 +965,29 @@ struct Rows {
     bool split_attn;     // per_seq: the positions split over workgroups and merged (long contexts) instead of one workgroup per head
 };
 
+template <int D, bool APPEND, int TH>
+void launch_attn_rows_th(axq_model *m, int l, const float *qkv, int nb, int pos0, const int32_t *pos_arr, size_t cache_off, size_t lds,
+                         float *att, hipStream_t st, PackOut pk) {
+    const axq_model_config &c = m->cfg;
+    static std::atomic<uint64_t> lds_allowed{0};
+    if (lds > 48 * 1024) (void)axq_allow_lds(m->ctx, reinterpret_cast<const void *>(&attn_prompt_kernel<D, APPEND, TH>), lds_allowed, 128 * 1024); // a
+    // refusal is the context's error now, and the launch below fails with it
+    const size_t off = (size_t)l * c.num_key_value_heads * c.max_position_embeddings * D + cache_off;
+    attn_prompt_kernel<D, APPEND, TH><<<dim3(c.num_attention_heads, nb), TH, lds, st>>>(
+        qkv, m->qkv_rows, m->rope_cos, m->rope_sin, m->kcache + off, m->vcache + off, pos0, pos_arr, m->seq_stride, c.num_attention_heads,
+        c.num_key_value_heads, c.max_position_embeddings, c.sliding_window, att, pk);
+}
+
+// 256 threads where more workgroups than two per compute unit (what fits of the large ones) would queue and eight of the small ones
+// fit a compute unit's LDS.
 template <int D, bool APPEND>
 void launch_attn_rows_t(axq_model *m, int l, const float *qkv, int nb, int pos0, const int32_t *pos_arr, size_t cache_off, size_t lds,
                         float *att, hipStream_t st, PackOut pk) {
-    const axq_model_config &c = m->cfg;
-    static std::atomic<uint64_t> lds_allowed{0};
-    if (lds > 48 * 1024) (void)axq_allow_lds(m->ctx, reinterpret_cast<const void *>(&attn_prompt_kernel<D, APPEND>), lds_allowed, 128 * 1024); // a
-    // refusal is the context's error now, and the launch below fails with it
-    const size_t off = (size_t)l * c.num_key_value_heads * c.max_position_embeddings * D + cache_off;
-    attn_prompt_kernel<D, APPEND><<<dim3(c.num_attention_heads, nb), 1024, lds, st>>>(
-        qkv, m->qkv_rows, m->rope_cos, m->rope_sin, m->kcache + off, m->vcache + off, pos0, pos_arr, m->seq_stride, c.num_attention_heads,
-        c.num_key_value_heads, c.max_position_embeddings, c.sliding_window, att, pk);
+    const long workgroups = (long)m->cfg.num_attention_heads * nb;
+    if (lds <= 16 * 1024 && workgroups > 2L * m->ctx->prop.multiProcessorCount)
+        launch_attn_rows_th<D, APPEND, 256>(m, l, qkv, nb, pos0, pos_arr, cache_off, lds, att, st, pk);
+    else
+        launch_attn_rows_th<D, APPEND, 1024>(m, l, qkv, nb, pos0, pos_arr, cache_off, lds, att, st, pk);
 }
 
 // Attention of `nb` rows of layer l.  pos_arr == NULL: rows of one sequence (cache at cache_off) at positions pos0.., whose
