@@ -5,9 +5,9 @@
 //
 // Time of a call with f32 rows, before (groups of eight vectors, or two-stage operands in LDS) and now, us:
 //   rows                  10          16          32          64
-//   Q4_K 28672 x 4096     40.3 35.1   40.5 35.7   81.5 44.2   61.8 56.7
-//   Q4_K 4096 x 4096      22.7 16.9   21.8 18.5   43.0 20.5   33.0 23.8
-//   Q4_K 4096 x 14336     31.7 31.6   32.0 32.0   63.2 37.6   63.9 40.0
+//   Q4_K 28672 x 4096     40.3 35.1   40.5 35.7   81.5 44.2   61.8 53.9
+//   Q4_K 4096 x 4096      22.7 16.9   21.8 18.5   43.0 20.5   33.0 23.4
+//   Q4_K 4096 x 14336     31.7 31.6   32.0 32.0   63.2 37.6   63.9 38.4
 //   Q4_0 11008 x 4096, 21 rows: 41.7 30.3; Q4_0 4096 x 4096, 10 and 39 rows: 22.3 16.0, 56.6 22.7; Q8_0 11008 x 4096, 64 rows: 43.2 34.8;
 //   bf16 rows, Q8_0 4096 x 4096, 16: 26.1 16.2; Q4_0 11008 x 4096, 128: 48.4 36.0
 // What bounds it: at few rows the fixed parts (pre-pass, reduction and the launches around them: 14 us of the 4096 x 4096 calls) and
@@ -29,14 +29,14 @@
 //                and sc times the rest, two products per weight.
 //   blocks of 32 w = d (q - C) + (m + C d): q - C is the operand, a block's sum starts from zero and joins its superblock's times d; the
 //                offsets of eight blocks, as an f16 pair under a common power of two, meet the blocks' sums of x.
-// Centred codes because sums over uncentred ones cancel for rows with a mean.  Accumulation is f32 throughout: products of a step from
+// Centred codes because sums over uncentred ones cancel for rows with a mean.  Accumulation is f32 throughout: products of a step (limbs, blocks; else of two) from
 // zero, steps into a superblock's sum, superblocks into the total.  Root mean square error against 64 bits over that of the result,
 // normal x, K = 1024 / 4096 / 14336, in 1e-8, before and now:
 //   rows       up to 39                       40 and more, f32
 //   Q4_0       7.2 8.6 10.3   6.6 8.2 8.9     8.5 10.6 15.5   8.5 9.7 10.7
 //   Q5_1       9.3 10.4 12.9  7.3 8.7 9.7     9.1 11.2 16.4   8.9 10.1 11.1
-//   Q4_K       9.4 10.5 12.9  7.5 9.0 9.5     13.0 17.7 31.4  10.4 11.3 12.0
-//   Q6_K       8.8 10.0 12.5  5.4 7.2 8.0     15.8 21.6 38.8  10.9 11.7 12.4
+//   Q4_K       9.4 10.5 12.9  7.5 9.0 9.5     13.0 17.7 31.4  11.3 12.1 12.7
+//   Q6_K       8.8 10.0 12.5  5.4 7.2 8.0     15.8 21.6 38.8  12.4 13.1 13.7
 // (limbs in one accumulator: Q4_0 8.6 11.7 16.5; the matrix pipe cuts sums off where it adds small products to large ones.)
 //
 // Shape.  A workgroup of eight waves; a wave computes 32 MI x 32 NJ outputs.  Four waves lie side by side along N; the other
@@ -644,7 +644,7 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
                 for (int t = 0; t < 4; t++) read_x(t, af[j4 % AHEAD][t]);
             asm volatile("" ::: "memory"); // requested here, not where they are used
         };
-        auto products = [&](auto at, auto t0, auto t1, float16v (&to)[MI][NJ]) { // t0 .. t1 - 1 of a step, from zero
+        auto products = [&](auto at, auto t0, auto t1, float16v (&to)[MI][NJ], auto fresh) { // t0 .. t1 - 1 of a step, from zero where `fresh`
             constexpr int J = decltype(at)::value, T0 = decltype(t0)::value, T1 = decltype(t1)::value;
             half8 bf[T1 - T0][NJ][T::PRODUCTS];
             auto mul = [&](int t, int l) {
@@ -653,7 +653,7 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
 #pragma unroll
                     for (int j = 0; j < NJ; j++)
                         to[Tile::acc_of(l)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                            af[J % AHEAD][t][l], bf[t - T0][j][pr], Tile::first_of(l) && t == T0 && pr == 0 ? zero : to[Tile::acc_of(l)][j], 0, 0, 0);
+                            af[J % AHEAD][t][l], bf[t - T0][j][pr], decltype(fresh)::value && Tile::first_of(l) && t == T0 && pr == 0 ? zero : to[Tile::acc_of(l)][j], 0, 0, 0);
             };
             if constexpr (AT == 1) {
 #pragma unroll
@@ -672,6 +672,7 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
             }
         };
         using S4 = std::integral_constant<int, 4>;
+        float16v part[MI][NJ];
         auto step = [&](int sb, auto at) {
             constexpr int J = decltype(at)::value;
             // the last step's sums are in `sum` here: left to itself the compiler keeps the blocks' sums of a superblock apart
@@ -690,14 +691,13 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
                 for (int j = 0; j < NJ; j++) side[j] = next_side[j];
                 new_side();
             }
-            float16v part[MI][NJ];
             if constexpr (T::BLOCKS) {
                 auto block = [&](auto half) {
                     constexpr int B = decltype(half)::value;
                     float d[NJ];
 #pragma unroll
                     for (int j = 0; j < NJ; j++) d[j] = T::scale(side[j], 2 * J + B);
-                    products(at, std::integral_constant<int, 2 * B>{}, std::integral_constant<int, 2 * B + 2>{}, part);
+                    products(at, std::integral_constant<int, 2 * B>{}, std::integral_constant<int, 2 * B + 2>{}, part, std::true_type{});
                     asm volatile("" ::: "memory");
                     read_x(2 * B, af[0][2 * B]);
                     read_x(2 * B + 1, af[0][2 * B + 1]);
@@ -723,10 +723,12 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
                 }
                 if (J == 3) each([&](int i, int j, int q) { total[i][j][q] += sum[i][j][q]; });
             } else {
-                products(at, S0{}, S4{}, part);
+                // f32 pairs and bf16 rows: two steps to a sum, half the additions (Q4_K 28672 x 4096, 64 f32 rows 56.4 -> 53.9 us)
+                constexpr int RUN = AT == 1 ? 2 : 1;
+                products(at, S0{}, S4{}, part, std::integral_constant<bool, J % RUN == 0>{});
                 if constexpr (T::MIN && J >= 1 && J <= NJ) add_offsets(sb, std::integral_constant<int, J - 1>{}, part);
-                if (J == 0) each([&](int i, int j, int q) { sum[i][j][q] = part[i][j][q]; });
-                else each([&](int i, int j, int q) { sum[i][j][q] += part[i][j][q]; });
+                if (J == RUN - 1) each([&](int i, int j, int q) { sum[i][j][q] = part[i][j][q]; });
+                else if (J % RUN == RUN - 1) each([&](int i, int j, int q) { sum[i][j][q] += part[i][j][q]; });
                 if (J == 3) each([&](int i, int j, int q) { total[i][j][q] = fmaf(sum[i][j][q], unit[j], total[i][j][q]); });
             }
         };
