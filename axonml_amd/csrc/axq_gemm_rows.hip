@@ -8,7 +8,7 @@
 //   Q4_K 28672 x 4096     40.3 35.1   40.5 35.7   81.5 44.2   61.8 53.9
 //   Q4_K 4096 x 4096      22.7 16.9   21.8 18.5   43.0 20.5   33.0 23.4
 //   Q4_K 4096 x 14336     31.7 31.6   32.0 32.0   63.2 37.6   63.9 38.4
-//   Q4_0 11008 x 4096, 21 rows: 41.7 30.3; Q4_0 4096 x 4096, 10 and 39 rows: 22.3 16.0, 56.6 22.7; Q8_0 11008 x 4096, 64 rows: 43.2 34.8;
+//   Q4_0 4096 x 11008, 21 rows: 41.7 30.3; Q4_0 4096 x 4096, 10 and 39 rows: 22.3 16.0, 56.6 22.7; Q8_0 11008 x 4096, 64 rows: 43.2 34.8;
 //   bf16 rows, Q8_0 4096 x 4096, 16: 26.1 16.2; Q4_0 11008 x 4096, 128: 48.4 36.0
 // What bounds it: at few rows the fixed parts (pre-pass, reduction and the launches around them: 14 us of the 4096 x 4096 calls) and
 // the LDS reads of x, which every wave makes for its 32 columns (0.35 us per step with one tile of x, 0.6 with two); at many the matrix
