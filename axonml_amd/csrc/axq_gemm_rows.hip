@@ -1,5 +1,5 @@
 // Rows times a packed weight of a superblock type or of a type with blocks of 32: y[M, N] = x[M, K] * W[N, K]^T on
-// v_mfma_f32_32x32x16_f16, for f32 rows (ten of them up to a prompt; blocks of 32: up to 64) and bf16 rows (blocks: up to 128).  The
+// v_mfma_f32_32x32x16_f16, for f32 rows (ten of them up to a prompt) and bf16 rows; blocks of 32 up to a tile per compute unit.  The
 // reference composition is dequantize_tensor -> f32 sgemm (crates/axonml-quant/src/dequantize.rs:34-54,
 // crates/axonml-core/src/backends/cpu.rs:566-598).
 //
@@ -1045,12 +1045,18 @@ void launch_prep(hipStream_t st, const void *x, const float *norm_w, float eps, 
 
 } // namespace
 
-// Superblock types at any number of rows; blocks of 32 up to 128 rows of operands (above, gemm_blk32_kernel).  K a multiple of 256.
-bool axq_dev_rows_gemm_covers(const axq_weight *w, int rows, bool bf16) {
+// Superblock types at any number of rows; blocks of 32, whose sums fit the registers of 128 x 128 outputs only, up to 128 rows of
+// operands and while such tiles are at most one per compute unit (bf16 rows, us here and in gemm_blk32_kernel: Q5_1 4096 x 4096, 509
+// rows 52.2 59.1; Q4_0 4096 x 4096, 256 rows 27.9 39.2; Q8_0 11008 x 4096, 256 rows, 172 tiles, 59.4 72.5; Q5_0 11008 x 4096, 512 rows,
+// 344 tiles, 136.8 128.4; Q4_0 14336 x 4096, 1024 rows, 219 217).  K a multiple of 256.
+bool axq_dev_rows_gemm_covers(const axq_ctx *ctx, const axq_weight *w, int rows, bool bf16) {
     if (w->k % 256 != 0 || w->k > INT32_MAX || w->n_rows > INT32_MAX || rows < 1) return false;
     switch (w->type) {
     case AXQ_Q4_K: case AXQ_Q5_K: case AXQ_Q6_K: return true;
-    case AXQ_Q4_0: case AXQ_Q4_1: case AXQ_Q5_0: case AXQ_Q5_1: case AXQ_Q8_0: return rows <= (bf16 ? 128 : 64);
+    case AXQ_Q4_0: case AXQ_Q4_1: case AXQ_Q5_0: case AXQ_Q5_1: case AXQ_Q8_0: {
+        const int64_t m = (int64_t)rows * (bf16 ? 1 : 2);
+        return m <= 128 || (m + 127) / 128 * ((w->n_rows + 127) / 128) <= ctx->prop.multiProcessorCount;
+    }
     default: return false;
     }
 }
@@ -1060,9 +1066,10 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
                       const float *resid, float *y) {
     const bool limbs = in != AXQ_ROWS_BF16 && rows < AXQ_ROWS_PAIRS_MIN;
     const int parts = in == AXQ_ROWS_BF16 || limbs ? 1 : 2, m = rows * parts, n = (int)w->n_rows, k = (int)w->k;
-    const int bm = limbs ? (rows <= 32 ? 32 : 64) : m <= 32 ? 32 : m <= 64 ? 64 : m <= 128 ? 128 : 256;
+    const bool wide = m > 128 && (w->type == AXQ_Q4_K || w->type == AXQ_Q5_K || w->type == AXQ_Q6_K); // 256 x 256 outputs
+    const int bm = limbs ? (rows <= 32 ? 32 : 64) : m <= 32 ? 32 : m <= 64 ? 64 : wide ? 256 : 128;
     const int nsb = k >> 8, cus = ctx->prop.multiProcessorCount, groups = m <= (limbs ? 32 : 64) ? 2 : 1;
-    const int bn = m <= 128 ? 128 : 256;
+    const int bn = wide ? 256 : 128;
     const long tiles = (long)((n + bn - 1) / bn) * ((m + bm - 1) / bm);
     // K is split over as many workgroups as leave every group of waves a superblock, up to one workgroup per compute unit
     int splits = (int)(cus / tiles);

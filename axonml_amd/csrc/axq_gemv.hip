@@ -678,7 +678,7 @@ int axq_dev_gemv(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, c
     static const bool no_gemm = getenv("AXQ_GEMV_GEMM") && getenv("AXQ_GEMV_GEMM")[0] == '0'; // development knob
     const int others_min = axq_dev_gemv_batch_covers(w, 8) ? 40 : 8;
     while (!no_gemm && axq_dev_gemm_f32_covers(w, 1) &&
-           (batch >= others_min || (batch >= AXQ_ROWS_GEMM_MIN && axq_dev_rows_gemm_covers(w, batch, false) && !being_captured(ctx)))) {
+           (batch >= others_min || (batch >= AXQ_ROWS_GEMM_MIN && axq_dev_rows_gemm_covers(ctx, w, batch, false) && !being_captured(ctx)))) {
         const int nb = batch < AXQ_GEMM_F32_MAX_ROWS ? batch : AXQ_GEMM_F32_MAX_ROWS;
         int rc = axq_dev_gemm_f32(ctx, w, x, nb, nullptr, 0.f, bias, nullptr, y);
         if (rc == AXQ_ERR_ALLOCATION_FAILED && nb < others_min) { // no room for its scratch: the kernel below needs none

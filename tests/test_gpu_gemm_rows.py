@@ -66,6 +66,20 @@ def test_superblocks_of_every_scale(ctx, qtype, size, at, rows):
 
 
 @pytest.mark.parametrize("qtype", BLOCKS)
+@pytest.mark.parametrize("rows,n", [(129, 257), (513, 640), (130, 16384), (130, 16385)])
+def test_blocks_in_many_tiles(ctx, qtype, rows, n):
+    """More than one tile of rows, K in pieces or whole; as many tiles as compute units with bf16 rows (2 x 128) and
+    one column more, which the kernel with operands in LDS takes."""
+    k = 256 if n > 10000 else 1536
+    rng = np.random.default_rng(rows + n + qtype)
+    packed = o.quantize(qtype, gen_weight(rng, n, k))
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    _check(ctx, qtype, n, k, packed, x, bf16=True)
+    if n < 10000:
+        _check(ctx, qtype, n, k, packed, x)
+
+
+@pytest.mark.parametrize("qtype", BLOCKS)
 @pytest.mark.parametrize("rows", [12, 24, 56])
 def test_blocks_of_every_scale(ctx, qtype, rows):
     """Blocks without a scale, without a minimum, with neither, from f16's smallest numbers to its largest, of either sign."""
