@@ -127,7 +127,7 @@ struct SuperQ45 {
         if constexpr (Q5) s.b = *reinterpret_cast<const u32x4 *>(stage + (1 + hh) * N * 16 + row * 16);
     }
     // u, the accumulators' unit for a superblock, inv = 1 / u and shrink = d / u: u = d 2^p, p = 0 unless dmin / d >= 64 (p <= 24:
-    // operands stay multiples of f16's smallest number); dmin where d = 0; 0 for a superblock of zeros
+    // operands stay multiples of f16's smallest number, see `excess`); dmin where d = 0; 0 for a superblock of zeros
     __device__ static void unit_of(const Side &s, float &u, float &inv, float &shrink) {
         const float d = h2f(s.h[0] & 0xFFFFu), dm = h2f(s.h[0] >> 16);
         auto expo = [](float v) { return (int)((__builtin_bit_cast(uint32_t, v) >> 23) & 0xFF); };
@@ -137,9 +137,17 @@ struct SuperQ45 {
         shrink = d == 0.f ? 0.f : __builtin_bit_cast(float, (uint32_t)(127 - p) << 23);
         inv = 1.0f / (u == 0.f ? 1.0f : u);
     }
-    // four of the offsets of a superblock, sub-blocks 4 hh .. 4 hh + 3, in units of u and times eight (their sums of x come times
-    // 1 / 8), |.| <= 8 (16 * 63 + 64 * 63): leading halves, then remainders
-    __device__ static half8 offsets(const Side &s, int hh, float inv) {
+    // How many powers of two dmin / d lies beyond what p takes up: up to 10 more (f16's largest over its smallest number), 0 for
+    // anything that comes of values.  The offsets are divided by 2^excess and join accumulators that are divided by it meanwhile.
+    __device__ static int excess(const Side &s) {
+        const float d = h2f(s.h[0] & 0xFFFFu), dm = h2f(s.h[0] >> 16);
+        auto expo = [](float v) { return (int)((__builtin_bit_cast(uint32_t, v) >> 23) & 0xFF); };
+        const int r = expo(dm) - expo(d) - 5 - 24;
+        return d == 0.f || r < 0 ? 0 : r;
+    }
+    // four of the offsets of a superblock, sub-blocks 4 hh .. 4 hh + 3, in units of u 2^excess and times eight (their sums of x come
+    // times 1 / 8), |.| <= 8 (16 * 63 + 64 * 63): leading halves, then remainders
+    __device__ static half8 offsets(const Side &s, int hh, float inv) { // inv = 1 / (u 2^excess)
         // C d sc - dmin m: both products exact (11 x 6 bits), so that their difference loses nothing where they nearly cancel
         const float dc = CENTRE * h2f(s.h[0] & 0xFFFFu), dm = -h2f(s.h[0] >> 16), to_unit = 8.0f * inv;
         const uint32_t sc = hh ? (s.h[3] & 0x0F0F0F0Fu) | ((s.h[1] >> 2) & 0x30303030u) : s.h[1] & 0x3F3F3F3Fu;
@@ -592,13 +600,24 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
     auto add_offsets = [&](int sb, auto tile_j, float16v (&to)[MI][NJ]) { // of a column tile
         if constexpr (T::MIN && !T::BLOCKS) {
             constexpr int j = decltype(tile_j)::value;
-            const half8 o = T::offsets(side[j], hh, inv[j]);
+            const int over = T::excess(side[j]);
+            const bool any_over = __builtin_amdgcn_ballot_w64(over > 0) != 0; // a column's lanes all have its factor; exact, being a power of two
+            auto times_pow2 = [&](int e) {
+                const float f = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
+#pragma unroll
+                for (int i = 0; i < MI; i++)
+#pragma unroll
+                    for (int q = 0; q < 16; q++) to[i][j][q] *= f;
+            };
+            if (any_over) times_pow2(-over);
+            const half8 o = T::offsets(side[j], hh, inv[j] * __builtin_bit_cast(float, (uint32_t)(127 - over) << 23));
 #pragma unroll
             for (int i = 0; i < XT; i++) {
                 const uint8_t *x = sbase + (sb & 1) * SBYTES + (wm * XT + i) * 2048 + lane * 16;
                 to[Tile::acc_of(i)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x), o, to[Tile::acc_of(i)][j], 0, 0, 0);
                 to[Tile::acc_of(i)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x + 1024), o, to[Tile::acc_of(i)][j], 0, 0, 0);
             }
+            if (any_over) times_pow2(over);
         }
     };
     using S0 = std::integral_constant<int, 0>; using S1 = std::integral_constant<int, 1>;

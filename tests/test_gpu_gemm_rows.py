@@ -65,6 +65,25 @@ def test_superblocks_of_every_scale(ctx, qtype, size, at, rows):
     _check(ctx, qtype, n, k, b.reshape(-1), x)
 
 
+@pytest.mark.parametrize("qtype,size", [(o.Q4_K, 144), (o.Q5_K, 176)])
+@pytest.mark.parametrize("rows", [12, 24, 39, 56, 100, 160])
+@pytest.mark.parametrize("k", [256, 768])
+def test_every_pair_of_scale_and_minimum(ctx, qtype, size, rows, k):
+    """Scales and minima of every power of two that f16 has, 2^-24 to 2^15, in all pairs, and of either sign: a column of its own for
+    a pair, and three pairs to a column."""
+    rng = np.random.default_rng(rows + k + qtype)
+    e = np.arange(-24, 16)
+    d, m = (v.ravel() for v in np.meshgrid(e, e))
+    n, per = len(d), k // 256
+    b = o.quantize(qtype, gen_weight(rng, n, k)).reshape(n, per, size).copy()
+    for s in range(per):
+        order = rng.permutation(n) if s else np.arange(n)
+        for at, v in ((0, d[order]), (2, m[order])):
+            f = np.minimum(2.0 ** v * (1 + rng.random(n)), 65504.0) * rng.choice([1.0, 1.0, -1.0], n)
+            b[:, s, at:at + 2] = f.astype(np.float16).view(np.uint8).reshape(n, 2)
+    _check(ctx, qtype, n, k, b.reshape(-1), rng.standard_normal((rows, k)).astype(np.float32))
+
+
 @pytest.mark.parametrize("qtype", BLOCKS)
 @pytest.mark.parametrize("rows,n", [(129, 257), (513, 640), (130, 16384), (130, 16385)])
 def test_blocks_in_many_tiles(ctx, qtype, rows, n):
