@@ -14,10 +14,11 @@
 // the LDS reads of x, which every wave makes for its 32 columns (0.35 us per step with one tile of x, 0.6 with two); at many the matrix
 // pipe beside the vector instructions that make operands (2048 bf16 rows x 14336: 320 us, 750 TFLOP/s), which overlap only in part.
 //
-// Numerics.  A bf16 row goes in as f16 under a power-of-two row scale (exact).  An f32 row goes in as two f16 rows, leading eleven
-// bits and remainder, whose results are added (22 bits), from 40 rows on; fewer rows, which the small-batch GEMV with its 28 bits below
-// the row's largest is the alternative for, as three limbs of eleven bits in fixed point: 32 bits below the row's largest, and the
-// first limbs' sums over a block are exact.  A weight goes in without rounding:
+// Numerics.  A bf16 row goes in as f16 under a power-of-two row scale that puts its largest element right below f16's limit: exact
+// down to 2^-31 of that element, and what is smaller to within 2^-39 of it.  An f32 row goes in as two f16 rows, leading eleven
+// bits and remainder, whose results are added (22 bits, and 2^-39 of the row's largest), from 40 rows on; fewer rows, which the
+// small-batch GEMV with its 28 bits below the largest of every 32 is the alternative for, as three limbs of eleven bits in fixed
+// point: 32 bits below the row's largest, and the first limbs' sums over a block are exact.  A weight goes in without rounding:
 //   Q4_K, Q5_K   w = d (sc (q - C)) + (C d sc - dmin m), C = 8 or 16: sc (q - C) is an integer below 2^10, exact in f16, and is
 //                the operand; sums of them are in units of d.  A step's sum starts from zero and joins the total times d, or, where
 //                registers are short (more than 128 rows), the accumulators of a column hold the running sum and change their
@@ -126,30 +127,31 @@ struct SuperQ45 {
         s.h = *reinterpret_cast<const u32x4 *>(stage + row * 16);
         if constexpr (Q5) s.b = *reinterpret_cast<const u32x4 *>(stage + (1 + hh) * N * 16 + row * 16);
     }
-    // u, the accumulators' unit for a superblock, inv = 1 / u and shrink = d / u: u = d 2^p, p = 0 unless dmin / d >= 64 (p <= 24:
-    // operands stay multiples of f16's smallest number, see `excess`); dmin where d = 0; 0 for a superblock of zeros
+    // u, the accumulators' unit for a superblock, inv = 1 / u and shrink = d / u: u = d 2^p, p = 3 unless dmin / d >= 64 (p <= 24:
+    // operands stay multiples of f16's smallest number, see `excess`); dmin where d = 0; 0 for a superblock of zeros.  Not d itself:
+    // the sums of x come times 1 / 64, and 64 times an offset has to stay within f16
     __device__ static void unit_of(const Side &s, float &u, float &inv, float &shrink) {
         const float d = h2f(s.h[0] & 0xFFFFu), dm = h2f(s.h[0] >> 16);
         auto expo = [](float v) { return (int)((__builtin_bit_cast(uint32_t, v) >> 23) & 0xFF); };
-        int p = expo(dm) - expo(d) - 5;
-        p = p < 0 ? 0 : (p > 24 ? 24 : p);
+        int p = expo(dm) - expo(d) - 2;
+        p = p < 3 ? 3 : (p > 24 ? 24 : p);
         u = d == 0.f ? dm : d * __builtin_bit_cast(float, (uint32_t)(127 + p) << 23);
         shrink = d == 0.f ? 0.f : __builtin_bit_cast(float, (uint32_t)(127 - p) << 23);
         inv = 1.0f / (u == 0.f ? 1.0f : u);
     }
-    // How many powers of two dmin / d lies beyond what p takes up: up to 10 more (f16's largest over its smallest number), 0 for
+    // How many powers of two dmin / d lies beyond what p takes up: up to 13 more (f16's largest over its smallest number), 0 for
     // anything that comes of values.  The offsets are divided by 2^excess and join accumulators that are divided by it meanwhile.
     __device__ static int excess(const Side &s) {
         const float d = h2f(s.h[0] & 0xFFFFu), dm = h2f(s.h[0] >> 16);
         auto expo = [](float v) { return (int)((__builtin_bit_cast(uint32_t, v) >> 23) & 0xFF); };
-        const int r = expo(dm) - expo(d) - 5 - 24;
+        const int r = expo(dm) - expo(d) - 2 - 24;
         return d == 0.f || r < 0 ? 0 : r;
     }
-    // four of the offsets of a superblock, sub-blocks 4 hh .. 4 hh + 3, in units of u 2^excess and times eight (their sums of x come
-    // times 1 / 8), |.| <= 8 (16 * 63 + 64 * 63): leading halves, then remainders
+    // four of the offsets of a superblock, sub-blocks 4 hh .. 4 hh + 3, in units of u 2^excess and times 64 (their sums of x come
+    // times 1 / 64), |.| <= 8 (16 * 63 + 64 * 63): leading halves, then remainders
     __device__ static half8 offsets(const Side &s, int hh, float inv) { // inv = 1 / (u 2^excess)
         // C d sc - dmin m: both products exact (11 x 6 bits), so that their difference loses nothing where they nearly cancel
-        const float dc = CENTRE * h2f(s.h[0] & 0xFFFFu), dm = -h2f(s.h[0] >> 16), to_unit = 8.0f * inv;
+        const float dc = CENTRE * h2f(s.h[0] & 0xFFFFu), dm = -h2f(s.h[0] >> 16), to_unit = 64.0f * inv;
         const uint32_t sc = hh ? (s.h[3] & 0x0F0F0F0Fu) | ((s.h[1] >> 2) & 0x30303030u) : s.h[1] & 0x3F3F3F3Fu;
         const uint32_t mn = hh ? ((s.h[3] >> 4) & 0x0F0F0F0Fu) | ((s.h[2] >> 2) & 0x30303030u) : s.h[2] & 0x3F3F3F3Fu;
         uint32_t o[4];
@@ -347,7 +349,7 @@ struct Block32 {
     }
     // m + C d of blocks 4 hh .. 4 hh + 3 as f16 pairs, leading halves and then remainders, times a power of two that brings the
     // superblock's largest below 2^15: |.| < (1 + 16) 2^(e + 1), e the largest exponent of its d and m.  `f`: what undoes it, and the
-    // 1 / 8 of the sums of x.
+    // 1 / 64 of the sums of x.
     __device__ static half8 offsets(const Side &s, int hh, float &f) {
         uint32_t most = 0x0400u; // f16 bits; smallest normal number
 #pragma unroll
@@ -358,7 +360,7 @@ struct Block32 {
         }
         const int e = (int)(most >> 10) - 15;
         const float up = __builtin_bit_cast(float, (uint32_t)(127 + 9 - e) << 23);
-        f = __builtin_bit_cast(float, (uint32_t)(127 - 9 + e + 3) << 23);
+        f = __builtin_bit_cast(float, (uint32_t)(127 - 9 + e + 6) << 23);
         uint32_t o[4];
 #pragma unroll
         for (int p = 0; p < 2; p++) {
@@ -967,10 +969,11 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
         const uint32_t o = __builtin_bit_cast(uint32_t, red[i]);
         top = o > top ? o : top;
     }
-    // top in [2^e, 2^(e+1)) -> multiply by 2^(11 - e): a sum of 32 stays below 2^17; inf/nan rows are passed through unscaled
+    // top in [2^e, 2^(e+1)) -> multiply by 2^(14 - e), the most that f16 holds: what the smallest elements lose is what lies below
+    // 2^-39 of the row's largest; a sum of 32 stays below 2^20; inf/nan rows are passed through unscaled
     int eb = (int)(top >> 23);
-    if (eb == 0 || eb == 0xFF) eb = 127 + 11;
-    int sb = 127 + 11 - (eb - 127);
+    if (eb == 0 || eb == 0xFF) eb = 127 + 14;
+    int sb = 127 + 14 - (eb - 127);
     sb = sb < 1 ? 1 : (sb > 254 ? 254 : sb);
     const float f = __builtin_bit_cast(float, (uint32_t)sb << 23);
     constexpr int PARTS = LIMBS ? 3 : IN == 2 ? 1 : 2;
@@ -990,8 +993,8 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
             float s = e[q] * f;
 #pragma unroll
             for (int part = 0; part < PARTS; part++) {
-                // limbs: multiples of 2^2, 2^-9, 2^-20, at most 2^10 of them
-                p[part][q] = LIMBS ? (_Float16)(rintf(s * (part == 0 ? 0x1p-2f : part == 1 ? 0x1p9f : 0x1p20f)) * (part == 0 ? 0x1p2f : part == 1 ? 0x1p-9f : 0x1p-20f))
+                // limbs: multiples of 2^5, 2^-6, 2^-17, at most 2^10 of them
+                p[part][q] = LIMBS ? (_Float16)(rintf(s * (part == 0 ? 0x1p-5f : part == 1 ? 0x1p6f : 0x1p17f)) * (part == 0 ? 0x1p5f : part == 1 ? 0x1p-6f : 0x1p-17f))
                                    : (_Float16)s;
                 sum[part] += (float)p[part][q];
                 s -= (float)p[part][q];
@@ -1008,12 +1011,12 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
             const half8 out = part < PARTS ? half8{s[0], s[2], s[1], s[3], s[4], s[6], s[5], s[7]} : half8{0, 0, 0, 0, 0, 0, 0, 0};
             if (c < chunks)
                 *reinterpret_cast<half8 *>(xt + ((size_t)(c >> 3) * 4 + t) * 512 + (h * 32 + lrow) * 8) = out;
-            // the sum of 32 elements: four threads; times 1 / 8 it stays within f16's range
+            // the sum of 32 elements: four threads; times 1 / 64 it stays within f16's range
             float g = part < PARTS ? sum[part] : 0.f;
             g += __shfl_xor(g, 1);
             g += __shfl_xor(g, 2);
             if ((tid & 3) == 0 && c < chunks) {
-                g *= 1.0f / 8.0f;
+                g *= 1.0f / 64.0f;
                 const _Float16 ghi = (_Float16)g, glo = (_Float16)(g - (float)ghi);
                 const int sub = (c >> 2) & 7;
                 _Float16 *d = st + (size_t)(c >> 5) * 1024 + ((sub >> 2) * 32 + lrow) * 8 + (sub & 3);
