@@ -17,8 +17,10 @@
 // Numerics.  A bf16 row goes in as f16 under a power-of-two row scale that puts its largest element right below f16's limit: exact
 // down to 2^-31 of that element, and what is smaller to within 2^-39 of it.  An f32 row goes in as two f16 rows, leading eleven
 // bits and remainder, whose results are added (22 bits, and 2^-39 of the row's largest), from 40 rows on; fewer rows, which the
-// small-batch GEMV with its 28 bits below the largest of every 32 is the alternative for, as three limbs of eleven bits in fixed
-// point: 32 bits below the row's largest, and the first limbs' sums over a block are exact.  A weight goes in without rounding:
+// small-batch GEMV with its 28 bits below the largest of every 32 is the alternative for, as three limbs.  The first is a multiple of
+// 2^-10 of the power of two above its block's largest, so that its sums over a block are exact; the second and the third, f16
+// themselves and 2^11 times as large as they count, hold the next 22 bits of what is left of each element: 33 bits below the
+// block's largest, 22 bits of the element where that is less, down to 2^-50 of the row's largest.  A weight goes in without rounding:
 //   Q4_K, Q5_K   w = d (sc (q - C)) + (C d sc - dmin m), C = 8 or 16: sc (q - C) is an integer below 2^10, exact in f16, and is
 //                the operand; sums of them are in units of d.  A step's sum starts from zero and joins the total times d, or, where
 //                registers are short (more than 128 rows), the accumulators of a column hold the running sum and change their
@@ -809,11 +811,11 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
     wait_loads_and_lds<0>(); // nothing of this workgroup may still be on its way into LDS
 
     // ---- results.  D layout: lane -> column li; register r -> row 8 (r / 4) + 4 (lane / 32) + r % 4
-    if constexpr (AT > 1) // the first limbs' results and the others'; the others of sixteen rows lie sixteen rows below
+    if constexpr (AT > 1) // the first limbs' results and the others', which come times 2^11; the others of sixteen rows lie sixteen rows below
 #pragma unroll
         for (int j = 0; j < NJ; j++)
 #pragma unroll
-            for (int r = 0; r < (AT == 2 ? 8 : 16); r++) acc[0][j][r] += AT == 2 ? acc[0][j][r + 8 & 15] : acc[MI - 1][j][r];
+            for (int r = 0; r < (AT == 2 ? 8 : 16); r++) acc[0][j][r] = fmaf(AT == 2 ? acc[0][j][r + 8 & 15] : acc[MI - 1][j][r], 0x1p-11f, acc[0][j][r]);
     constexpr int MR = AT > 1 ? 1 : MI;
     auto store = [&](int i, int j, int r, float v, float v2) { // v2: of row r + 1, where rows are pairs
         const int gn = n0 + (wn * NJ + j) * 32 + li;
@@ -988,18 +990,38 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
         float sum[PARTS];
 #pragma unroll
         for (int part = 0; part < PARTS; part++) sum[part] = 0.f;
+        // limbs: the first is a multiple of 2^(g - 9), at most 2^10 of it, 2^g the magnitude of the block's largest (a block of 32 is
+        // four threads'); the second and the third, times 2^11, are what that leaves
+        float grid = 0.f, ungrid = 0.f;
+        if (LIMBS) {
+            uint32_t most = 0;
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const uint32_t b = __builtin_bit_cast(uint32_t, e[q] * f) & 0x7FFFFFFFu;
+                most = b > most ? b : most;
+            }
+#pragma unroll
+            for (int m = 1; m <= 2; m <<= 1) {
+                const uint32_t o = (uint32_t)__shfl_xor((int)most, m);
+                most = o > most ? o : most;
+            }
+            int g = (int)(most >> 23) - 127;
+            g = g < -15 ? -15 : g > 14 ? 14 : g; // f16's smallest number is 2^-24
+            grid = __builtin_bit_cast(float, (uint32_t)(127 + g - 9) << 23);
+            ungrid = __builtin_bit_cast(float, (uint32_t)(127 - g + 9) << 23);
+        }
 #pragma unroll
         for (int q = 0; q < 8; q++) {
             float s = e[q] * f;
 #pragma unroll
             for (int part = 0; part < PARTS; part++) {
-                // limbs: multiples of 2^5, 2^-6, 2^-17, at most 2^10 of them
-                p[part][q] = LIMBS ? (_Float16)(rintf(s * (part == 0 ? 0x1p-5f : part == 1 ? 0x1p6f : 0x1p17f)) * (part == 0 ? 0x1p5f : part == 1 ? 0x1p-6f : 0x1p-17f))
-                                   : (_Float16)s;
+                p[part][q] = LIMBS && part == 0 ? (_Float16)(rintf(s * ungrid) * grid) : (_Float16)s;
                 sum[part] += (float)p[part][q];
                 s -= (float)p[part][q];
+                if (LIMBS && part == 0) s *= 0x1p11f;
             }
         }
+        float carry = 0.f; // what a limb's pair of sums does not hold goes to the next limb's
         // chunk c: step c / 8, product t, half of the lanes (see the order of elements above)
         const int at = c & 7, t = (at >> 2) * 2 + (at & 1), h = (at >> 1) & 1;
 #pragma unroll
@@ -1016,8 +1038,9 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
             g += __shfl_xor(g, 1);
             g += __shfl_xor(g, 2);
             if ((tid & 3) == 0 && c < chunks) {
-                g *= 1.0f / 64.0f;
+                g = part < PARTS ? fmaf(g, 1.0f / 64.0f, carry) : 0.f;
                 const _Float16 ghi = (_Float16)g, glo = (_Float16)(g - (float)ghi);
+                if (LIMBS) carry = (g - (float)ghi - (float)glo) * (part == 0 ? 0x1p11f : 1.0f);
                 const int sub = (c >> 2) & 7;
                 _Float16 *d = st + (size_t)(c >> 5) * 1024 + ((sub >> 2) * 32 + lrow) * 8 + (sub & 3);
                 d[0] = ghi; d[4] = ghi;

@@ -6,8 +6,9 @@ in the kernels' operands, plus 3e-7 of the results' for the f32 sums (1e-7 is me
 [2^t, 2^(t + 1)):
   rows of f16 pairs   delta = 2^-22 |x| + 2^(t - 39): f16's smallest number is 2^-38 of the largest power of two
   bf16 rows           delta = 2^(t - 39)
+  rows of limbs       delta = min(2^-22 |x|, 2^(g - 32)) + 2^(t - 50), 2^g the power of two of the largest of the element's 32
 Where weights have an offset, the offset of 32 of them (at most the middle of their range and half a step) meets a sum of x that is
-off by as much as 2^(t - 33)."""
+off by as much as 2^(t - 33), or 2^(t - 44) with limbs."""
 import numpy as np
 import pytest
 
@@ -17,6 +18,7 @@ from tests.util import gen_weight
 
 pytestmark = pytest.mark.gpu
 
+LIMBS = 40  # f32 rows below it are limbs
 TYPES = [o.Q4_K, o.Q5_K, o.Q6_K, o.Q4_0, o.Q5_0, o.Q8_0]
 SYMMETRIC = [o.Q4_0, o.Q5_0, o.Q8_0, o.Q6_K]  # a single weight can be zero exactly
 
@@ -45,6 +47,9 @@ def _check(ctx, qtype, x, n, zero, bf16=False):
     t = _power(np.abs(x).max(1, keepdims=True))
     if bf16:
         delta = np.broadcast_to(2.0 ** (t - 39), x.shape)
+    elif rows < LIMBS:
+        g = np.repeat(_power(np.abs(x).reshape(rows, k // 32, 32).max(2)), 32, axis=1)
+        delta = np.minimum(2.0 ** -22 * np.abs(x), 2.0 ** (g - 32)) + 2.0 ** (t - 50)
     else:
         delta = 2.0 ** -22 * np.abs(x) + 2.0 ** (t - 39)
     square = delta ** 2 @ (w ** 2).T
@@ -52,14 +57,14 @@ def _check(ctx, qtype, x, n, zero, bf16=False):
         b = w.reshape(n, k // 32, 32)
         lo, hi = b.min(2), b.max(2)
         offset = np.abs(lo + hi) / 2 + (hi - lo) / 30
-        square += 4.0 ** (t - 33) * (offset ** 2).sum(1)
+        square += 4.0 ** (t - (33 if bf16 or rows >= LIMBS else 44)) * (offset ** 2).sum(1)
     rms = lambda v: np.sqrt(np.mean(np.square(v)))
     off, bound = rms(got - want), np.sqrt(np.mean(square)) + 3e-7 * rms(want)
     assert off <= bound, f"{o.TYPE_NAMES[qtype]} {rows} x {n} x {k}: {off / rms(want):.2e}, bound {bound / rms(want):.2e}"
 
 
 @pytest.mark.parametrize("qtype", TYPES)
-@pytest.mark.parametrize("rows", [40, 64, 65, 160])
+@pytest.mark.parametrize("rows", [10, 16, 17, 32, 33, 39, 40, 64, 65, 160])
 @pytest.mark.parametrize("top", [14, 23])
 def test_a_large_element_in_a_block_of_its_own(ctx, qtype, rows, top):
     rng = np.random.default_rng(rows + top)
@@ -76,3 +81,24 @@ def test_bf16_rows_with_a_large_element(ctx, qtype, rows, top):
     x = rng.standard_normal((rows, 1024)).astype(np.float32)
     x[np.arange(rows), 256 + rng.integers(0, 32, size=rows)] = 1.5 * 2.0 ** top
     _check(ctx, qtype, x, 384, np.arange(256, 288), bf16=True)
+
+
+@pytest.mark.parametrize("qtype", SYMMETRIC)
+@pytest.mark.parametrize("rows", [10, 16, 17, 32, 33, 39, 40, 64])
+@pytest.mark.parametrize("top", [9, 14])
+def test_a_large_element_in_every_block(ctx, qtype, rows, top):
+    """Below 40 rows the second and the third limb carry the small elements."""
+    rng = np.random.default_rng(rows + top)
+    x = rng.standard_normal((rows, 1024)).astype(np.float32)
+    x[:, 7::32] = 1.5 * 2.0 ** top
+    _check(ctx, qtype, x, 384, np.arange(7, 1024, 32))
+
+
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("rows", [10, 16, 17, 32, 33, 39])
+def test_blocks_of_uneven_magnitude(ctx, qtype, rows):
+    """Blocks of 32 whose magnitudes lie up to 2^20 apart; the larger half meets weights of zero."""
+    rng = np.random.default_rng(rows)
+    x = rng.standard_normal((rows, 1024)).astype(np.float32) * np.repeat(2.0 ** -rng.permuted(np.tile(np.arange(8, 17), 4)[:32]), 32).astype(np.float32)
+    x[:, 512:] *= np.float32(2.0 ** 12)
+    _check(ctx, qtype, x, 384, np.arange(512, 1024))
