@@ -31,7 +31,8 @@
 //   Q6_K         w = d sc (q - 32): sc (q - 32) has 13 bits and goes in as two exact operands, sc times the multiple of eight
 //                and sc times the rest, two products per weight.
 //   blocks of 32 w = d (q - C) + (m + C d): q - C is the operand, a block's sum starts from zero and joins its superblock's times d; the
-//                offsets of eight blocks, as an f16 pair under a common power of two, meet the blocks' sums of x.
+//                offsets of eight blocks, as an f16 pair under a common power of two, meet the blocks' sums of x.  C is the middle
+//                code, or, with a minimum, the code nearest to a weight of zero (see Block32::centre).
 // Centred codes because sums over uncentred ones cancel for rows with a mean.  Accumulation is f32 throughout: products of a step (limbs, blocks; else of two) from
 // zero, steps into a superblock's sum, superblocks into the total.  Root mean square error against 64 bits over that of the result,
 // normal x, K = 1024 / 4096 / 14336, in 1e-8, before and now:
@@ -265,7 +266,9 @@ struct SuperQ6 {
 };
 
 // Blocks of 32 with an f16 scale d each (and a minimum m): the operand is the centred code, an integer; a block's sum starts from
-// zero and joins the total times d; m + C d meets the block's sum of x, eight blocks at a time.
+// zero and joins the total times d; m + C d meets the block's sum of x, eight blocks at a time.  With a minimum the centre is the
+// code that lies nearest to zero: the middle for weights around zero, the lowest one for a block of one value, whose d says nothing
+// about its weights (the quantisers write 1) and would come back 8 or 16 times in both sums.
 template <int BITS, bool WITH_MIN>
 struct Block32 {
     static constexpr int PAIRS = BITS == 8 ? 4 : 2, PRODUCTS = 1, REC = WITH_MIN ? 2 : 1, SIDE16 = REC + (BITS == 5 ? 2 : 0), SIDE4 = 0;
@@ -274,6 +277,10 @@ struct Block32 {
     struct Side { u32x4 r[REC], b[BITS == 5 ? 2 : 1]; };
     struct Raw { u32x4 q[2]; }; // of the step's two blocks; Q4: the lane's half, in the first two dwords
     struct Scales {};
+    __device__ static float centre(uint32_t record) {
+        const float zero = -h2f(record >> 16) * __builtin_amdgcn_rcpf(h2f(record & 0xFFFFu)); // where the weight is zero; not a number: code 0
+        return rintf(fminf(fmaxf(zero, 0.f), BITS == 5 ? 31.0f : 15.0f));
+    }
     __device__ static const uint8_t *piece_src(const RowsArgs &a, int unit, int p) { return a.codes + (size_t)unit * (PAIRS * 32) + p * 32; }
     __device__ static uint32_t piece_pitch(const RowsArgs &a, int) { return a.codes_pitch; }
     __device__ static const uint8_t *side_src(const RowsArgs &a, int sb, int c) { // the records, then the fifth bits
@@ -321,7 +328,7 @@ struct Block32 {
                 w[2 * d + 1] = bits(halfs(((v >> 8) & 0x00FF00FFu) | 0x64006400u) + c);
             }
         } else { // a code at bits 4..7 (4..8) of a half with 0x5400 is 64 + q
-            const half2v c = {(_Float16)-(64.0f + CENTRE), (_Float16)-(64.0f + CENTRE)};
+            const half2v c = pk2(-64.0f - (WITH_MIN ? centre(record(s, 2 * j + b)) : CENTRE));
             uint32_t e[4];
             if constexpr (BITS == 4) { // byte i = elements 2 i (low), 2 i + 1: dword 2 hh + at is the operand's eight
                 const uint32_t p = __builtin_amdgcn_perm(0u, r.q[b][at], 0x03010200u); // bytes 0, 2, 1, 3
@@ -349,8 +356,8 @@ struct Block32 {
         }
         o[0] = octet(w);
     }
-    // m + C d of blocks 4 hh .. 4 hh + 3 as f16 pairs, leading halves and then remainders, times a power of two that brings the
-    // superblock's largest below 2^15: |.| < (1 + 16) 2^(e + 1), e the largest exponent of its d and m.  `f`: what undoes it, and the
+    // m + C d of blocks 4 hh .. 4 hh + 3 as f16 pairs, leading halves and then remainders, times a power of two that keeps the
+    // superblock's largest within f16: |.| <= max(|m|, |d|) < 2^(e + 1), e the largest exponent of its d and m.  `f`: what undoes it, and the
     // 1 / 64 of the sums of x.
     __device__ static half8 offsets(const Side &s, int hh, float &f) {
         uint32_t most = 0x0400u; // f16 bits; smallest normal number
@@ -361,8 +368,8 @@ struct Block32 {
             most = m > most ? m : most;
         }
         const int e = (int)(most >> 10) - 15;
-        const float up = __builtin_bit_cast(float, (uint32_t)(127 + 9 - e) << 23);
-        f = __builtin_bit_cast(float, (uint32_t)(127 - 9 + e + 6) << 23);
+        const float up = __builtin_bit_cast(float, (uint32_t)(127 + 13 - e) << 23);
+        f = __builtin_bit_cast(float, (uint32_t)(127 - 13 + e + 6) << 23);
         uint32_t o[4];
 #pragma unroll
         for (int p = 0; p < 2; p++) {
@@ -370,7 +377,7 @@ struct Block32 {
 #pragma unroll
             for (int i = 0; i < 2; i++) {
                 const uint32_t r = hh ? record(s, 4 + 2 * p + i) : record(s, 2 * p + i);
-                c[i] = fmaf(CENTRE, h2f(r & 0xFFFFu), h2f(r >> 16)) * up;
+                c[i] = fmaf(centre(r), h2f(r & 0xFFFFu), h2f(r >> 16)) * up;
             }
             const half2v h = __builtin_bit_cast(half2v, __builtin_amdgcn_cvt_pkrtz(c[0], c[1]));
             o[p] = bits(h);

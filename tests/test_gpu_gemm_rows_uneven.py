@@ -19,7 +19,7 @@ from tests.util import gen_weight
 pytestmark = pytest.mark.gpu
 
 LIMBS = 40  # f32 rows below it are limbs
-TYPES = [o.Q4_K, o.Q5_K, o.Q6_K, o.Q4_0, o.Q5_0, o.Q8_0]
+TYPES = [o.Q4_K, o.Q5_K, o.Q6_K, o.Q4_0, o.Q4_1, o.Q5_0, o.Q5_1, o.Q8_0]
 SYMMETRIC = [o.Q4_0, o.Q5_0, o.Q8_0, o.Q6_K]  # a single weight can be zero exactly
 
 
