@@ -23,7 +23,7 @@
 // block's largest, 22 bits of the element where that is less, down to 2^-50 of the row's largest.  A weight goes in without rounding:
 //   Q4_K, Q5_K   w = d (sc (q - C)) + (C d sc - dmin m), C = 8 or 16: sc (q - C) is an integer below 2^10, exact in f16, and is
 //                the operand; sums of them are in units of d.  A step's sum starts from zero and joins the total times d, or, where
-//                registers are short (more than 128 rows), the accumulators of a column hold the running sum and change their
+//                registers are short (256 x 256 outputs), the accumulators of a column hold the running sum and change their
 //                unit at a superblock boundary (one multiply per register and 256 k).  The offset, one number per sub-block of
 //                32, joins in the same unit as an f16 pair, against the sub-block's sum of x as an f16 pair: two products more
 //                per superblock.  Where dmin is so large beside d that the pair would leave f16's range, the unit is d times a
@@ -1070,18 +1070,18 @@ int launch_tile(axq_ctx *ctx, const RowsArgs &a, int splits) {
 }
 
 // The tile of a call.  Limbs: up to 16 and 32 rows the two halves of the waves on two parts of K, since a workgroup's time is then its
-// number of steps.  Others: up to 32 and 64 rows of operands the same with one and two row tiles per wave; 65 to 128 rows: two times
-// two row tiles (at 64 f32 rows and Q4_K 28672 x 4096 2.5 us ahead of four row tiles per wave and split halves).  Above: 256 x 256
-// outputs, which blocks do not have: their sums do not fit the registers.
+// number of steps.  Others: up to 32 and 64 rows of operands the same with one and two row tiles per wave; above two times
+// two row tiles (at 64 f32 rows and Q4_K 28672 x 4096 2.5 us ahead of four row tiles per wave and split halves), or 256 x 256
+// outputs (see wide_tiles), which blocks do not have: their sums do not fit the registers.
 template <class T>
-int launch_rows(axq_ctx *ctx, const RowsArgs &a, int splits, bool limbs) {
+int launch_rows(axq_ctx *ctx, const RowsArgs &a, int splits, bool limbs, bool wide) {
     if (limbs) {
         if (a.m > 32) return launch_tile<T, 2, 2, 1, 3>(ctx, a, splits);
         if (a.m > 16) return launch_tile<T, 2, 1, 1, 3>(ctx, a, splits);
         return launch_tile<T, 1, 1, 1, 2>(ctx, a, splits);
     }
     if constexpr (!T::BLOCKS)
-        if (a.m > 128) return launch_tile<T, 4, 2, 2, 1>(ctx, a, splits);
+        if (wide) return launch_tile<T, 4, 2, 2, 1>(ctx, a, splits);
     if (a.m > 64) return launch_tile<T, 2, 2, 1, 1>(ctx, a, splits);
     if (a.m > 32) return launch_tile<T, 2, 1, 1, 1>(ctx, a, splits);
     return launch_tile<T, 1, 1, 1, 1>(ctx, a, splits);
@@ -1095,6 +1095,21 @@ void launch_prep(hipStream_t st, const void *x, const float *norm_w, float eps, 
     else rows_prep_kernel<IN, 0, LIMBS><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
 }
 
+// How many tiles of 128 x 128 outputs a call of m rows of operands has, where 256 x 256 are the alternative.
+int64_t square_tiles(int64_t m, int64_t n) { return m <= 128 ? 0 : (m + 127) / 128 * ((n + 127) / 128); }
+
+// Superblock types: 256 x 256 outputs per workgroup, which make an operand once for twice the rows, where tiles of 128 x 128 are
+// more than one to two compute units, or where K in parts of at least four superblocks (shorter ones are mostly the start and the
+// partial sums) gives the large tiles a workgroup per compute unit.  Else 128 x 128.  Time with large and small tiles, us:
+//   f32 rows   Q4_K 4096 x 4096, 128: 36.8 27.3 (16 large tiles and eight parts are half the chip); 256: 43.0 39.5
+//              Q4_K 1024 x 4096, 128: 34.4 21.3;  Q5_K 4096 x 4096, 128: 38.8 29.4;  Q6_K 4096 x 14336, 128: 102 83
+//              Q4_K 4096 x 14336, 256 (128 small tiles, 32 large ones in eight parts): 93 105;  Q5_K 6144 x 4096, 160 (144): 54 61
+//   bf16 rows  Q4_K 4096 x 4096, 256: 43.0 29.0; 512 (128 small ones): 52 42;  1024 x 4096, 1024: 47 34.5;  4096 x 14336, 700 (192): 141 173
+bool wide_tiles(const axq_ctx *ctx, int64_t m, int64_t n, int64_t k) {
+    const int64_t cus = ctx->prop.multiProcessorCount, parts = k >> 10;
+    return m > 128 && (square_tiles(m, n) > cus / 2 || (m + 255) / 256 * ((n + 255) / 256) * (parts < 8 ? parts : 8) >= cus);
+}
+
 } // namespace
 
 // Superblock types at any number of rows; blocks of 32, whose sums fit the registers of 128 x 128 outputs only, up to 128 rows of
@@ -1105,10 +1120,8 @@ bool axq_dev_rows_gemm_covers(const axq_ctx *ctx, const axq_weight *w, int rows,
     if (w->k % 256 != 0 || w->k > INT32_MAX || w->n_rows > INT32_MAX || rows < 1) return false;
     switch (w->type) {
     case AXQ_Q4_K: case AXQ_Q5_K: case AXQ_Q6_K: return true;
-    case AXQ_Q4_0: case AXQ_Q4_1: case AXQ_Q5_0: case AXQ_Q5_1: case AXQ_Q8_0: {
-        const int64_t m = (int64_t)rows * (bf16 ? 1 : 2);
-        return m <= 128 || (m + 127) / 128 * ((w->n_rows + 127) / 128) <= ctx->prop.multiProcessorCount;
-    }
+    case AXQ_Q4_0: case AXQ_Q4_1: case AXQ_Q5_0: case AXQ_Q5_1: case AXQ_Q8_0:
+        return square_tiles((int64_t)rows * (bf16 ? 1 : 2), w->n_rows) <= ctx->prop.multiProcessorCount;
     default: return false;
     }
 }
@@ -1118,7 +1131,7 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
                       const float *resid, float *y) {
     const bool limbs = in != AXQ_ROWS_BF16 && rows < AXQ_ROWS_PAIRS_MIN;
     const int parts = in == AXQ_ROWS_BF16 || limbs ? 1 : 2, m = rows * parts, n = (int)w->n_rows, k = (int)w->k;
-    const bool wide = m > 128 && (w->type == AXQ_Q4_K || w->type == AXQ_Q5_K || w->type == AXQ_Q6_K); // 256 x 256 outputs
+    const bool wide = !limbs && (w->type == AXQ_Q4_K || w->type == AXQ_Q5_K || w->type == AXQ_Q6_K) && wide_tiles(ctx, m, n, k);
     const int bm = limbs ? (rows <= 32 ? 32 : 64) : m <= 32 ? 32 : m <= 64 ? 64 : wide ? 256 : 128;
     const int nsb = k >> 8, cus = ctx->prop.multiProcessorCount, groups = m <= (limbs ? 32 : 64) ? 2 : 1;
     const int bn = wide ? 256 : 128;
@@ -1156,14 +1169,14 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
     a.m = m; a.n = n; a.k = k; a.pair = parts == 2; a.bias = bias; a.resid = resid;
     int rc;
     switch (w->type) {
-    case AXQ_Q4_K: rc = launch_rows<SuperQ45<false>>(ctx, a, splits, limbs); break;
-    case AXQ_Q5_K: rc = launch_rows<SuperQ45<true>>(ctx, a, splits, limbs); break;
-    case AXQ_Q6_K: rc = launch_rows<SuperQ6>(ctx, a, splits, limbs); break;
-    case AXQ_Q4_0: rc = launch_rows<Block32<4, false>>(ctx, a, splits, limbs); break;
-    case AXQ_Q4_1: rc = launch_rows<Block32<4, true>>(ctx, a, splits, limbs); break;
-    case AXQ_Q5_0: rc = launch_rows<Block32<5, false>>(ctx, a, splits, limbs); break;
-    case AXQ_Q5_1: rc = launch_rows<Block32<5, true>>(ctx, a, splits, limbs); break;
-    default: rc = launch_rows<Block32<8, false>>(ctx, a, splits, limbs); break;
+    case AXQ_Q4_K: rc = launch_rows<SuperQ45<false>>(ctx, a, splits, limbs, wide); break;
+    case AXQ_Q5_K: rc = launch_rows<SuperQ45<true>>(ctx, a, splits, limbs, wide); break;
+    case AXQ_Q6_K: rc = launch_rows<SuperQ6>(ctx, a, splits, limbs, wide); break;
+    case AXQ_Q4_0: rc = launch_rows<Block32<4, false>>(ctx, a, splits, limbs, wide); break;
+    case AXQ_Q4_1: rc = launch_rows<Block32<4, true>>(ctx, a, splits, limbs, wide); break;
+    case AXQ_Q5_0: rc = launch_rows<Block32<5, false>>(ctx, a, splits, limbs, wide); break;
+    case AXQ_Q5_1: rc = launch_rows<Block32<5, true>>(ctx, a, splits, limbs, wide); break;
+    default: rc = launch_rows<Block32<8, false>>(ctx, a, splits, limbs, wide); break;
     }
     if (rc || splits == 1) return rc;
     return axq_gemm_reduce(ctx, a.ypart, rs, rows, n, splits, 1.0f, parts, bias, resid, y);

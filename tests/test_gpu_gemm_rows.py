@@ -98,6 +98,16 @@ def test_blocks_in_many_tiles(ctx, qtype, rows, n):
         _check(ctx, qtype, n, k, packed, x)
 
 
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
+@pytest.mark.parametrize("rows,n,k,bf16", [(129, 8192, 256, True), (129, 8193, 256, True), (257, 8129, 768, True), (300, 5377, 1280, False), (2047, 1000, 8192, True)])
+def test_superblocks_in_large_tiles(ctx, qtype, rows, n, k, bf16):
+    """As many tiles of 128 x 128 as half the compute units, and more, which 256 x 256 outputs take; and few outputs over a K that is
+    long enough for eight parts."""
+    rng = np.random.default_rng(rows + n + qtype)
+    packed = o.quantize(qtype, gen_weight(rng, n, k))
+    _check(ctx, qtype, n, k, packed, rng.standard_normal((rows, k)).astype(np.float32), bf16=bf16)
+
+
 @pytest.mark.parametrize("qtype", BLOCKS)
 @pytest.mark.parametrize("rows", [12, 24, 56])
 def test_blocks_of_every_scale(ctx, qtype, rows):
