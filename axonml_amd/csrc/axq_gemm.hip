@@ -813,14 +813,23 @@ __global__ void __launch_bounds__(256) gemm_reduce_kernel(const float *ypart, co
                                                           float inv_ws, int row_mul, const float *bias, const float *resid, float *y) {
     const size_t i4 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, total4 = (size_t)rows * n / 4;
     if (i4 >= total4) return;
-    float4 acc = reinterpret_cast<const float4 *>(ypart)[i4];
+    const float4 first = reinterpret_cast<const float4 *>(ypart)[i4];
+    float acc[4] = {first.x, first.y, first.z, first.w}, lost[4] = {0.f, 0.f, 0.f, 0.f}; // the sum, and what its additions rounded off (two-sum)
     for (int s = 1; s < splits; s++) {
-        const float4 v = reinterpret_cast<const float4 *>(ypart + (size_t)s * rows * n)[i4];
-        acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
+        const float4 v4 = reinterpret_cast<const float4 *>(ypart + (size_t)s * rows * n)[i4];
+        const float v[4] = {v4.x, v4.y, v4.z, v4.w};
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const float sum = acc[c] + v[c], part = sum - acc[c];
+            lost[c] += (acc[c] - (sum - part)) + (v[c] - part);
+            acc[c] = sum;
+        }
     }
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[c] = lost[c] == lost[c] ? acc[c] + lost[c] : acc[c]; // not a number beside an infinite sum
     const size_t row = (i4 * 4) / (size_t)n, col = (i4 * 4) % (size_t)n; // n is a multiple of 4: the four share a row
     const float f = rowscale[row * row_mul] * inv_ws;
-    float4 out = make_float4(acc.x * f, acc.y * f, acc.z * f, acc.w * f);
+    float4 out = make_float4(acc[0] * f, acc[1] * f, acc[2] * f, acc[3] * f);
     if (bias) {
         out.x += bias[col]; out.y += bias[col + 1]; out.z += bias[col + 2]; out.w += bias[col + 3];
     }

@@ -18,11 +18,12 @@
 // down to 2^-31 of that element, and what is smaller to within 2^-39 of it.  An f32 row goes in as two f16 rows, leading eleven
 // bits and remainder, whose results are added (22 bits, and 2^-39 of the row's largest), from 40 rows on; fewer rows, which the
 // small-batch GEMV with its 28 bits below the largest of every 32 is the alternative for, as three limbs.  The first is a multiple of
-// 2^-10 of the power of two above its block's largest, so that its sums over a block are exact; the second and the third, f16
-// themselves and 2^11 times as large as they count, hold the next 22 bits of what is left of each element: 33 bits below the
-// block's largest, 22 bits of the element where that is less, down to 2^-50 of the row's largest.  A weight goes in without rounding:
+// 2^-8 of the power of two above its block's largest, so that its sums over a block are exact and have few bits (with eight or nine
+// bits below that power in place of seven Q4_0 at K = 4096 has an error of 5.9 and 6.7 instead of 5.0); the second and the third, f16
+// themselves and 2^9 times as large as they count, hold the next 22 bits of what is left of each element: 32 bits below the
+// block's largest, 22 bits of the element where that is less, down to 2^-48 of the row's largest.  A weight goes in without rounding:
 //   Q4_K, Q5_K   w = d (sc (q - C)) + (C d sc - dmin m), C = 8 or 16: sc (q - C) is an integer below 2^10, exact in f16, and is
-//                the operand; sums of them are in units of d.  A step's sum starts from zero and joins the total times d, or, where
+//                the operand; sums of them are in units of d, or 8 d to be exact.  A step's sum starts from zero and joins the total, or, where
 //                registers are short (256 x 256 outputs), the accumulators of a column hold the running sum and change their
 //                unit at a superblock boundary (one multiply per register and 256 k).  The offset, one number per sub-block of
 //                32, joins in the same unit as an f16 pair, against the sub-block's sum of x as an f16 pair: two products more
@@ -37,11 +38,12 @@
 // zero, steps into a superblock's sum, superblocks into the total.  Root mean square error against 64 bits over that of the result,
 // normal x, K = 1024 / 4096 / 14336, in 1e-8, before and now:
 //   rows       up to 39                       40 and more, f32
-//   Q4_0       7.2 8.6 10.3   6.6 8.2 8.9     8.5 10.6 15.5   8.5 9.7 10.7
-//   Q5_1       9.3 10.4 12.9  7.3 8.7 9.7     9.1 11.2 16.4   8.9 10.1 11.1
-//   Q4_K       9.4 10.5 12.9  7.5 9.0 9.5     13.0 17.7 31.4  11.3 12.1 12.7
-//   Q6_K       8.8 10.0 12.5  5.4 7.2 8.0     15.8 21.6 38.8  12.4 13.1 13.7
-// (limbs in one accumulator: Q4_0 8.6 11.7 16.5; the matrix pipe cuts sums off where it adds small products to large ones.)
+//   Q4_0       7.2 8.6 10.3   5.0 5.0 5.5     8.5 10.6 15.5   7.9 8.3 9.5
+//   Q5_1       9.4 10.5 12.9  6.4 6.3 6.8     9.1 11.2 16.4   8.1 8.5 9.6
+//   Q4_K       9.4 10.5 12.8  7.4 7.3 7.5     13.0 17.7 31.4  10.8 11.0 11.7
+//   Q6_K       8.9 10.0 12.4  5.3 5.2 5.5     15.8 21.6 38.8  12.0 12.1 12.7
+// (K in parts, whose sums gemm_reduce_kernel adds together with what their additions round off: without that Q4_0, K = 4096 has 8.4 in
+// place of the 6.7 of nine bits, and 9.7 in place of 8.3.  Limbs in one accumulator: Q4_0 8.6 11.7 16.5; the matrix pipe cuts sums off where it adds small products to large ones.)
 //
 // Shape.  A workgroup of eight waves; a wave computes 32 MI x 32 NJ outputs.  Four waves lie side by side along N; the other
 // factor of two is rows (WM = 2: 64 MI rows) or K (WM = 1: each four waves take half of the workgroup's superblocks, and the
@@ -69,6 +71,8 @@ typedef float float16v __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void gbl_void;
+
+constexpr int LB = 7; // bits of the first limb below its block's largest power of two
 
 struct RowsArgs {
     const uint8_t *codes, *meta, *qh;
@@ -822,7 +826,7 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
 #pragma unroll
         for (int j = 0; j < NJ; j++)
 #pragma unroll
-            for (int r = 0; r < (AT == 2 ? 8 : 16); r++) acc[0][j][r] = fmaf(AT == 2 ? acc[0][j][r + 8 & 15] : acc[MI - 1][j][r], 0x1p-11f, acc[0][j][r]);
+            for (int r = 0; r < (AT == 2 ? 8 : 16); r++) acc[0][j][r] = fmaf(AT == 2 ? acc[0][j][r + 8 & 15] : acc[MI - 1][j][r], 1.0f / (1 << (LB + 2)), acc[0][j][r]);
     constexpr int MR = AT > 1 ? 1 : MI;
     auto store = [&](int i, int j, int r, float v, float v2) { // v2: of row r + 1, where rows are pairs
         const int gn = n0 + (wn * NJ + j) * 32 + li;
@@ -997,8 +1001,8 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
         float sum[PARTS];
 #pragma unroll
         for (int part = 0; part < PARTS; part++) sum[part] = 0.f;
-        // limbs: the first is a multiple of 2^(g - 9), at most 2^10 of it, 2^g the magnitude of the block's largest (a block of 32 is
-        // four threads'); the second and the third, times 2^11, are what that leaves
+        // limbs: the first is a multiple of 2^(g - LB), at most 2^(LB + 1) of it, 2^g the magnitude of the block's largest (a block of 32
+        // is four threads'); the second and the third, times 2^(LB + 2), are what that leaves
         float grid = 0.f, ungrid = 0.f;
         if (LIMBS) {
             uint32_t most = 0;
@@ -1013,9 +1017,9 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
                 most = o > most ? o : most;
             }
             int g = (int)(most >> 23) - 127;
-            g = g < -15 ? -15 : g > 14 ? 14 : g; // f16's smallest number is 2^-24
-            grid = __builtin_bit_cast(float, (uint32_t)(127 + g - 9) << 23);
-            ungrid = __builtin_bit_cast(float, (uint32_t)(127 - g + 9) << 23);
+            g = g < LB - 24 ? LB - 24 : g > 14 ? 14 : g; // f16's smallest number is 2^-24
+            grid = __builtin_bit_cast(float, (uint32_t)(127 + g - LB) << 23);
+            ungrid = __builtin_bit_cast(float, (uint32_t)(127 - g + LB) << 23);
         }
 #pragma unroll
         for (int q = 0; q < 8; q++) {
@@ -1025,7 +1029,7 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
                 p[part][q] = LIMBS && part == 0 ? (_Float16)(rintf(s * ungrid) * grid) : (_Float16)s;
                 sum[part] += (float)p[part][q];
                 s -= (float)p[part][q];
-                if (LIMBS && part == 0) s *= 0x1p11f;
+                if (LIMBS && part == 0) s *= (float)(1 << (LB + 2));
             }
         }
         float carry = 0.f; // what a limb's pair of sums does not hold goes to the next limb's
@@ -1047,7 +1051,7 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
             if ((tid & 3) == 0 && c < chunks) {
                 g = part < PARTS ? fmaf(g, 1.0f / 64.0f, carry) : 0.f;
                 const _Float16 ghi = (_Float16)g, glo = (_Float16)(g - (float)ghi);
-                if (LIMBS) carry = (g - (float)ghi - (float)glo) * (part == 0 ? 0x1p11f : 1.0f);
+                if (LIMBS) carry = (g - (float)ghi - (float)glo) * (part == 0 ? (float)(1 << (LB + 2)) : 1.0f);
                 const int sub = (c >> 2) & 7;
                 _Float16 *d = st + (size_t)(c >> 5) * 1024 + ((sub >> 2) * 32 + lrow) * 8 + (sub & 3);
                 d[0] = ghi; d[4] = ghi;
