@@ -1114,6 +1114,37 @@ bool wide_tiles(const axq_ctx *ctx, int64_t m, int64_t n, int64_t k) {
     return m > 128 && (square_tiles(m, n) > cus / 2 || (m + 255) / 256 * ((n + 255) / 256) * (parts < 8 ? parts : 8) >= cus);
 }
 
+// How a call goes to the workgroups.
+struct RowsPlan {
+    bool limbs, wide;
+    int parts, m, bm;            // rows of the operand per row of x, all of them, and of a tile
+    long tiles;
+    int splits, sb_per_split;    // of K
+};
+
+RowsPlan rows_plan(const axq_ctx *ctx, const axq_weight *w, int in, int rows) {
+    RowsPlan p;
+    p.limbs = in != AXQ_ROWS_BF16 && rows < AXQ_ROWS_PAIRS_MIN;
+    p.parts = in == AXQ_ROWS_BF16 || p.limbs ? 1 : 2;
+    p.m = rows * p.parts;
+    const int n = (int)w->n_rows, nsb = (int)(w->k >> 8), groups = p.m <= (p.limbs ? 32 : 64) ? 2 : 1;
+    p.wide = !p.limbs && (w->type == AXQ_Q4_K || w->type == AXQ_Q5_K || w->type == AXQ_Q6_K) && wide_tiles(ctx, p.m, n, w->k);
+    p.bm = p.limbs ? (rows <= 32 ? 32 : 64) : p.m <= 32 ? 32 : p.m <= 64 ? 64 : p.wide ? 256 : 128;
+    const int bn = p.wide ? 256 : 128;
+    p.tiles = (long)((n + bn - 1) / bn) * ((p.m + p.bm - 1) / p.bm);
+    // K is split over as many workgroups as leave every group of waves a superblock, up to one workgroup per compute unit: into sixteen
+    // parts at most for 17 to 39 rows (eight and sixteen, 1024 x 14336: Q6_K, 39 rows 55.5 42.4 us; Q4_K, 17 rows 33.9 29.6, with
+    // thirty-two 30.4), else eight (2048 x 8192, ten rows: Q4_0 19.6 us, sixteen 20.4; Q4_K 20.8, 21.6)
+    const int most = p.limbs && rows > 16 ? 16 : 8;
+    int splits = (int)(ctx->prop.multiProcessorCount / p.tiles);
+    if (splits > nsb / groups) splits = nsb / groups;
+    if (splits > most) splits = most;
+    if (splits < 2 || n % 4 != 0) splits = 1;
+    p.sb_per_split = (nsb + splits - 1) / splits;
+    p.splits = (nsb + p.sb_per_split - 1) / p.sb_per_split;
+    return p;
+}
+
 } // namespace
 
 // Superblock types at any number of rows; blocks of 32, whose sums fit the registers of 128 x 128 outputs only, up to 128 rows of
@@ -1130,25 +1161,37 @@ bool axq_dev_rows_gemm_covers(const axq_ctx *ctx, const axq_weight *w, int rows,
     }
 }
 
+// Whether axq_gemv_f32 takes this kernel for `rows` f32 rows, of which the small-batch GEMV would make groups of eight.  From 17 on,
+// where those are three passes over the weights or more, always: 1.03 (1024 x 14336) to 2.8 times as fast.  10 to 16 rows are two
+// passes, beside which the pre-pass, a workgroup per row, and the reduction weigh more the longer K is and the fewer weight rows there
+// are.  Speed over two passes with 10 and 16 rows:
+//              Q8_0        Q6_K        Q4_0        Q5_1        Q4_K        Q5_K
+//   4096x14336 1.20 1.18   1.06 1.05   1.05 1.02   1.00 0.98   0.98 0.97   0.93 0.91
+//   1024x14336 0.85 0.78   0.84 0.80   0.87 0.82   0.78 0.73   0.83 0.78   0.77 0.73
+//   4096x8192  1.22 1.17   1.12 1.09   1.12 1.06   1.07 1.02   1.05 1.01   1.04 0.99
+//   2048x8192  1.09 1.02   0.95 0.93   1.18 1.12   0.96 0.90   1.10 1.04   1.00 0.95
+//   4096x4096  1.38 1.30   1.22 1.16   1.50 1.41   1.26 1.17   1.35 1.29   1.27 1.20
+//   6144x4096  1.08 1.04   1.09 1.05   1.06 1.00   1.01 0.97   1.02 0.97   0.96 0.92   (three quarters of the compute units)
+//   9216x4096  1.34 1.32   1.28 1.27   1.21 1.14   1.16 1.13   1.14 1.11   1.15 1.12
+bool axq_dev_rows_gemm_pays(const axq_ctx *ctx, const axq_weight *w, int rows) {
+    if (rows < AXQ_ROWS_GEMM_MIN || !axq_dev_rows_gemm_covers(ctx, w, rows, false)) return false;
+    if (rows > 16) return true;
+    const bool slow_gemv = w->type == AXQ_Q8_0 || w->type == AXQ_Q6_K || w->type == AXQ_Q4_0;
+    if (w->k > 8192) return slow_gemv && w->n_rows >= 4096;
+    if (w->k > 4096) return w->n_rows >= 4096 || (w->n_rows >= 2048 && (w->type == AXQ_Q8_0 || w->type == AXQ_Q4_0 || w->type == AXQ_Q4_K));
+    const RowsPlan p = rows_plan(ctx, w, AXQ_ROWS_F32, rows);
+    return slow_gemv || w->n_rows <= 4096 || p.tiles * p.splits * 5 >= ctx->prop.multiProcessorCount * 4;
+}
+
 // Scratch: x in operand order | its sub-block sums | row scales | partial sums of a split K.
 int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, int rows, const float *norm_w, float eps, const float *bias,
                       const float *resid, float *y) {
-    const bool limbs = in != AXQ_ROWS_BF16 && rows < AXQ_ROWS_PAIRS_MIN;
-    const int parts = in == AXQ_ROWS_BF16 || limbs ? 1 : 2, m = rows * parts, n = (int)w->n_rows, k = (int)w->k;
-    const bool wide = !limbs && (w->type == AXQ_Q4_K || w->type == AXQ_Q5_K || w->type == AXQ_Q6_K) && wide_tiles(ctx, m, n, k);
-    const int bm = limbs ? (rows <= 32 ? 32 : 64) : m <= 32 ? 32 : m <= 64 ? 64 : wide ? 256 : 128;
-    const int nsb = k >> 8, cus = ctx->prop.multiProcessorCount, groups = m <= (limbs ? 32 : 64) ? 2 : 1;
-    const int bn = wide ? 256 : 128;
-    const long tiles = (long)((n + bn - 1) / bn) * ((m + bm - 1) / bm);
-    // K is split over as many workgroups as leave every group of waves a superblock, up to one workgroup per compute unit
-    int splits = (int)(cus / tiles);
-    if (splits > nsb / groups) splits = nsb / groups;
-    if (splits > 8) splits = 8;
-    if (splits < 2 || n % 4 != 0) splits = 1;
+    const RowsPlan p = rows_plan(ctx, w, in, rows);
+    const bool limbs = p.limbs, wide = p.wide;
+    const int m = p.m, n = (int)w->n_rows, k = (int)w->k, nsb = k >> 8, splits = p.splits;
     RowsArgs a;
-    a.sb_per_split = (nsb + splits - 1) / splits;
-    splits = (nsb + a.sb_per_split - 1) / a.sb_per_split;
-    const size_t mtiles = limbs ? (rows <= 16 ? 2 : rows <= 32 ? 3 : 6) : (size_t)(m + bm - 1) / bm * (bm / 32);
+    a.sb_per_split = p.sb_per_split;
+    const size_t mtiles = limbs ? (rows <= 16 ? 2 : rows <= 32 ? 3 : 6) : (size_t)(m + p.bm - 1) / p.bm * (p.bm / 32);
     const size_t xa_bytes = mtiles * 32 * (size_t)k * 2, xs_bytes = mtiles * (size_t)nsb * 2048;
     const size_t rs_bytes = axq_align_up((size_t)m * 4, 256), part_bytes = splits > 1 ? (size_t)splits * rows * (size_t)n * 4 : 0;
     if (int rc = axq_gemm_reserve(ctx, xa_bytes + xs_bytes + rs_bytes + part_bytes)) return rc;
@@ -1170,7 +1213,7 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
     a.codes_pitch = (uint32_t)w->codes_pitch; a.meta_pitch = (uint32_t)w->meta_pitch; a.qh_pitch = (uint32_t)w->qh_pitch;
     a.xa = xa; a.xs = xs; a.rowscale = rs; a.y = y;
     a.ypart = splits > 1 ? reinterpret_cast<float *>(base + xa_bytes + xs_bytes + rs_bytes) : nullptr;
-    a.m = m; a.n = n; a.k = k; a.pair = parts == 2; a.bias = bias; a.resid = resid;
+    a.m = m; a.n = n; a.k = k; a.pair = p.parts == 2; a.bias = bias; a.resid = resid;
     int rc;
     switch (w->type) {
     case AXQ_Q4_K: rc = launch_rows<SuperQ45<false>>(ctx, a, splits, limbs, wide); break;
@@ -1183,5 +1226,5 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
     default: rc = launch_rows<Block32<8, false>>(ctx, a, splits, limbs, wide); break;
     }
     if (rc || splits == 1) return rc;
-    return axq_gemm_reduce(ctx, a.ypart, rs, rows, n, splits, 1.0f, parts, bias, resid, y);
+    return axq_gemm_reduce(ctx, a.ypart, rs, rows, n, splits, 1.0f, p.parts, bias, resid, y);
 }

@@ -672,13 +672,12 @@ bool being_captured(axq_ctx *ctx) {
 int axq_dev_gemv(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, const float *bias, float *y) {
     if (w->n_rows > INT32_MAX || w->k > INT32_MAX)
         return axq_fail(ctx, AXQ_ERR_SHAPE_MISMATCH, "Shape mismatch: weight dimensions exceed 2^31");
-    // many vectors: through the matrix-pipe GEMM.  Where the rows kernel covers the weight from ten on (4096 x 4096, ten rows: Q4_0 16.0 us,
-    // groups of eight 22.3; Q4_K 16.9 and 22.7; 256 x 512 10.4 and 15.4; nine rows, which the GEMV does as eight and one, are 1 to 2 us
-    // behind it); the others from about 40 rows where the small-batch kernel below is the alternative, from 8 where single-vector passes are
+    // many vectors: through the matrix-pipe GEMM.  Where the rows kernel pays (see there; nine rows, which the GEMV does as eight and
+    // one, it never does: 1 to 2 us behind); the others from about 40 rows where the small-batch kernel below is the alternative, from 8 where single-vector passes are
     static const bool no_gemm = getenv("AXQ_GEMV_GEMM") && getenv("AXQ_GEMV_GEMM")[0] == '0'; // development knob
     const int others_min = axq_dev_gemv_batch_covers(w, 8) ? 40 : 8;
     while (!no_gemm && axq_dev_gemm_f32_covers(w, 1) &&
-           (batch >= others_min || (batch >= AXQ_ROWS_GEMM_MIN && axq_dev_rows_gemm_covers(ctx, w, batch, false) && !being_captured(ctx)))) {
+           (batch >= others_min || (axq_dev_rows_gemm_pays(ctx, w, batch) && !being_captured(ctx)))) {
         const int nb = batch < AXQ_GEMM_F32_MAX_ROWS ? batch : AXQ_GEMM_F32_MAX_ROWS;
         int rc = axq_dev_gemm_f32(ctx, w, x, nb, nullptr, 0.f, bias, nullptr, y);
         if (rc == AXQ_ERR_ALLOCATION_FAILED && nb < others_min) { // no room for its scratch: the kernel below needs none

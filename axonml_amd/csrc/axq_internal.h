@@ -168,7 +168,8 @@ bool axq_dev_rows_gemm_covers(const axq_ctx *ctx, const axq_weight *w, int rows,
 // f32 rows below it go in as three limbs, 33 bits below the largest of every 32 elements (the small-batch GEMV, which took them before,
 // has 28), from it on as pairs of f16
 #define AXQ_ROWS_PAIRS_MIN 40
-#define AXQ_ROWS_GEMM_MIN 10 // f32 rows from which it is ahead of the small-batch GEMV in groups of eight
+#define AXQ_ROWS_GEMM_MIN 10 // f32 rows from which it can be ahead of the small-batch GEMV in groups of eight
+bool axq_dev_rows_gemm_pays(const axq_ctx *ctx, const axq_weight *w, int rows); // whether it is, for a call of its own
 int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, int rows, const float *norm_w, float eps, const float *bias,
                       const float *resid, float *y);
 // gemm.hip

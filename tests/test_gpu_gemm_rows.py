@@ -98,6 +98,15 @@ def test_blocks_in_many_tiles(ctx, qtype, rows, n):
         _check(ctx, qtype, n, k, packed, x)
 
 
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K, *BLOCKS])
+@pytest.mark.parametrize("rows,n,k", [(10, 100, 8192), (16, 4096, 4352), (16, 4100, 4096), (17, 100, 8192), (24, 260, 14336), (33, 132, 8192)])
+def test_few_rows_on_both_sides_of_the_gemv(ctx, qtype, rows, n, k):
+    """Ten to sixteen rows that the small-batch GEMV keeps or hands over by type, weight rows and K; K in sixteen parts."""
+    rng = np.random.default_rng(rows + n + qtype)
+    packed = o.quantize(qtype, gen_weight(rng, n, k))
+    _check(ctx, qtype, n, k, packed, rng.standard_normal((rows, k)).astype(np.float32), bias=rng.standard_normal(n).astype(np.float32))
+
+
 @pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
 @pytest.mark.parametrize("rows,n,k,bf16", [(129, 8192, 256, True), (129, 8193, 256, True), (257, 8129, 768, True), (300, 5377, 1280, False), (2047, 1000, 8192, True)])
 def test_superblocks_in_large_tiles(ctx, qtype, rows, n, k, bf16):
