@@ -431,8 +431,8 @@ __global__ void __launch_bounds__(128) rope_append_kernel(const float *qkv, int 
 // value are not in the cache yet; every workgroup rotates the key itself, uses both from LDS (rounded to f16 as the
 // cache holds them), and the first query head of each KV head writes them to the cache.
 // TH is 1024 where workgroups are few (all loads of a short context at once), 256 where they are more than run at once: such a
-// workgroup's time is barriers and latency, and eight of them on a compute unit fill each other's gaps.  32 heads x 64 sequences at
-// position 128: 33 us with 1024 threads, 21.8 us with 256.
+// workgroup's time is barriers and latency, and several of them on a compute unit fill each other's gaps.  32 heads x 64 sequences at
+// position 128: 33 us with 1024 threads, 21.8 us with 256.  (See launch_attn_rows_t for where the line lies.)
 template <int D, bool APPEND, int TH>
 __global__ void __launch_bounds__(TH) attn_prompt_kernel(const float *qkv, int qkv_rows, const float *rope_cos,
                                                            const float *rope_sin, uint16_t *kcache, uint16_t *vcache, int pos0,
@@ -978,13 +978,17 @@ void launch_attn_rows_th(axq_model *m, int l, const float *qkv, int nb, int pos0
         c.num_key_value_heads, c.max_position_embeddings, c.sliding_window, att, pk);
 }
 
-// 256 threads where more workgroups than two per compute unit (what fits of the large ones) would queue and eight of the small ones
-// fit a compute unit's LDS.
+// 256 threads where more workgroups than two per compute unit (what fits of the large ones) would queue.  Beyond 1024 positions a
+// workgroup's time is its keys and values, and three small ones have fewer loads under way than two large ones: there only where the
+// small ones are more than three to a compute unit.  A model of four layers, 32 heads of 128, 1024 threads and 256, us for all of it: steps of 17, 32
+// and 64 sequences at position 8 820 786, 954 904, 1317 1221; at 225 830 822, 978 952, 1376 1333; 24 and 31 tokens (768 and 992
+// workgroups) behind 500 932 914, 960 933; behind 1000 946 950, 994 983; behind 2000 1032 1042, 1082 1076; behind 4000 1200 1225, 1297 1284.
 template <int D, bool APPEND>
 void launch_attn_rows_t(axq_model *m, int l, const float *qkv, int nb, int pos0, const int32_t *pos_arr, size_t cache_off, size_t lds,
                         float *att, hipStream_t st, PackOut pk) {
     const long workgroups = (long)m->cfg.num_attention_heads * nb;
-    if (lds <= 16 * 1024 && workgroups > 2L * m->ctx->prop.multiProcessorCount)
+    const long cus = m->ctx->prop.multiProcessorCount;
+    if (lds <= 16 * 1024 && workgroups > (lds <= 4 * 1024 ? 2 : 3) * cus)
         launch_attn_rows_th<D, APPEND, 256>(m, l, qkv, nb, pos0, pos_arr, cache_off, lds, att, st, pk);
     else
         launch_attn_rows_th<D, APPEND, 1024>(m, l, qkv, nb, pos0, pos_arr, cache_off, lds, att, st, pk);
