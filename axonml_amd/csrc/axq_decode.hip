@@ -1150,7 +1150,7 @@ int wanted_logits(axq_model *m, const Wanted *w, int i, int nb) {
 
 int feed_rows(axq_model *m, int seq, const int32_t *toks, int n, int pos0, int *fed, const Wanted *w = nullptr) {
     static const char *knob = getenv("AXQ_PROMPT_BATCH"); // development knob: 0 = no rows at all, 1 = no GEMM
-    const int allow = knob ? atoi(knob) : 2;
+    int allow = knob ? atoi(knob) : 2;
     int i = 0, rc;
     *fed = 0;
     while (m->stack && i < n) { // rows of any number go through described layers together
@@ -1180,8 +1180,13 @@ int feed_rows(axq_model *m, int seq, const int32_t *toks, int n, int pos0, int *
         }
         if (r.mode == ROWS_NONE) break;
         r.lds = prompt_attn_lds(m, r.pos0 + r.nb);
-        if ((rc = reserve_prompt_rows(m, r.nb))) return rc;
-        if ((rc = enqueue_rows(m, r))) return rc;
+        if (!(rc = reserve_prompt_rows(m, r.nb))) rc = enqueue_rows(m, r);
+        if (rc == AXQ_ERR_ALLOCATION_FAILED && r.mode == ROWS_GEMM && all_layers_in_small_batch_reach(m, left) && r.nb < PROMPT_GEMM_MIN) {
+            allow = 1; // no room for a GEMM's rows or scratch: eight at a time need neither.  What went in before it failed is written again
+            (void)hipGetLastError();
+            continue;
+        }
+        if (rc) return rc;
         if ((rc = wanted_logits(m, w, i, r.nb))) return rc;
         i += r.nb;
         *fed = i;
@@ -1213,8 +1218,18 @@ int run_batch_step(axq_model *m, int max_pos_now) {
     r.lds = prompt_attn_lds(m, r.split_attn ? 1 : m->fused_max);
     static const bool no_graph = getenv("AXQ_DECODE_GRAPH") && getenv("AXQ_DECODE_GRAPH")[0] == '0';
     int rc;
-    if (m->n_seq > PROMPT_BATCH && m->n_seq <= GEMV_GROUPS_MAX && m->n_seq < gemm_rows_min(m, PROMPT_BATCH) &&
-        all_layers_in_small_batch_reach(m, PROMPT_BATCH)) {
+    const bool few = m->n_seq > PROMPT_BATCH && m->n_seq <= GEMV_GROUPS_MAX && all_layers_in_small_batch_reach(m, PROMPT_BATCH);
+    bool groups = few && m->n_seq < gemm_rows_min(m, PROMPT_BATCH);
+    if (few && !groups) { // the linears on the rows kernel; without room for its rows and scratch the step starts again in groups
+        r.mode = ROWS_GEMM;
+        if (!(rc = reserve_prompt_rows(m, r.nb))) rc = enqueue_rows(m, r);
+        if (rc == AXQ_ERR_ALLOCATION_FAILED && !reserve_prompt_rows(m, PROMPT_BATCH)) {
+            (void)hipGetLastError();
+            r.mode = ROWS_GEMV;
+            groups = true;
+        }
+    }
+    if (groups) {
         // a few more rows than the small-batch GEMV takes, and not all weights covered by the rows kernel: groups of eight sequences,
         // one after the other; plain launches
         rc = AXQ_OK;
@@ -1224,6 +1239,8 @@ int run_batch_step(axq_model *m, int max_pos_now) {
             g.nb = m->n_seq - s < PROMPT_BATCH ? m->n_seq - s : PROMPT_BATCH;
             rc = enqueue_rows(m, g);
         }
+    } else if (few) {
+        // done above
     } else if (m->n_seq > PROMPT_BATCH) {
         // many more: the linears are GEMMs on f32 rows (which size their scratch as they go, so no graph: a step of so
         // many rows is long against its launches anyway)

@@ -1008,6 +1008,9 @@ __global__ void __launch_bounds__(256) gemm_prep_x_f32_kernel(const float *x, co
 // The context's GEMM scratch, grown to `need` bytes (work that still uses the old one is waited for first).
 int axq_gemm_reserve(axq_ctx *ctx, size_t need) {
     if (ctx->gemm_scratch_bytes >= need) return AXQ_OK;
+    const char *most = getenv("AXQ_GEMM_SCRATCH_MAX"); // development knob: as if the card had no room for more bytes than this
+    if (most && need > strtoull(most, nullptr, 10))
+        return axq_fail(ctx, AXQ_ERR_ALLOCATION_FAILED, "GEMM scratch of %zu bytes: beyond AXQ_GEMM_SCRATCH_MAX", need);
     AXQ_HIP(ctx, hipStreamSynchronize(ctx->stream), AXQ_ERR_DRIVER);
     if (ctx->gemm_scratch) (void)hipFree(ctx->gemm_scratch);
     ctx->gemm_scratch = nullptr;
