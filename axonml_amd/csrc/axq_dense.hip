@@ -403,11 +403,13 @@ __device__ inline void write_tile(const axq_part &p, float cap, const f32x16 (&a
             f32x4 v[4], o[4];
             bool ok[4];
             size_t at[4];
+            int m[4];
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                const int r = r0 + q * rows_at_once + row_l, m = m_base + i * 32 + r;
-                ok[q] = m < m1 && n < cols;
-                at[q] = (size_t)m * p.ldy + n;
+                const int r = r0 + q * rows_at_once + row_l;
+                m[q] = m_base + i * 32 + r;
+                ok[q] = m[q] < m1 && n < cols;
+                at[q] = (size_t)m[q] * p.ldy + n;
                 if (p.resid && ok[q]) o[q] = load4(p.resid + at[q]);
                 v[q] = *reinterpret_cast<const f32x4 *>(patch + r * P + quad * 4);
                 if (glu || p.act == AXQ_ACT_NONE) v[q] += bias;
@@ -415,7 +417,7 @@ __device__ inline void write_tile(const axq_part &p, float cap, const f32x16 (&a
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 if (!ok[q]) continue;
-                if (p.scale) v[q] *= p.scale[at[q] / (size_t)p.ldy];
+                if (p.scale) v[q] *= p.scale[m[q]];
                 if (p.resid) v[q] += o[q];
                 if (vec && p.out16) {
                     *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(p.y) + at[q]) =

@@ -450,17 +450,17 @@ __device__ inline void wait_vm_and_lds() {
 // (the leading halves twice, then the remainders against the sums' leading halves); the sum is added times 256 and
 // the main term's scales are d * 256 / 64 to match.
 //
-// BM x 128 outputs per workgroup of eight waves (BM = 256: 64 x 64 each; 128: 32 x 64),
-// x tiles straight from memory into three LDS stages, two weight stages, one barrier per K step that waits for LDS only,
-// explicit counts of the loads issued since.  A thread converts half a block (16 weights of one row) per step.  The
-// scale records of the tile's columns lie in LDS too, a superblock of them at a time.
+// 256 x 128 outputs per workgroup of eight waves (64 x 64 each), all of K: the calls that come here have more than half as many of
+// them as the chip has compute units (see axq_dev_rows_gemm_covers).  x tiles straight from memory into three LDS stages, two weight
+// stages, one barrier per K step that waits for LDS only, explicit counts of the loads issued since.  A thread converts half a block
+// (16 weights of one row) per step.  The scale records of the tile's columns lie in LDS too, a superblock of them at a time.
 // ---------------------------------------------------------------------------
-constexpr int PBN = 128; // output columns (weight rows) per workgroup
+constexpr int PBM = 256, PBN = 128;        // rows of x and output columns (weight rows) per workgroup
 constexpr float XSUM_SCALE = 1.0f / 64.0f; // the x pre-pass stores the block sums times this
 
-template <int BITS, bool WITH_MIN, int BM>
+template <int BITS, bool WITH_MIN>
 __global__ void __launch_bounds__(512) gemm_blk32_kernel(GemmArgs a) {
-    constexpr int NW = 8, AROWS = BM / NW, XL = AROWS / 8; // BM = 256 or 128 rows of x per workgroup
+    constexpr int BM = PBM, NW = 8, AROWS = BM / NW, XL = AROWS / 8;
     constexpr int MI = BM / 128;                           // MFMA tiles of a wave along M: the waves lie 4 x 2, (32 MI) x 64 each
     constexpr int ASTAGE = BM * 64, BSTAGE = PBN * 64, BOFF = 3 * ASTAGE; // halfs
     constexpr int F = BITS == 5 ? 2 : 1;   // loads of a weight request: codes (and fifth bits)
@@ -475,11 +475,10 @@ __global__ void __launch_bounds__(512) gemm_blk32_kernel(GemmArgs a) {
     int tile = blockIdx.x;
     if (total % 8 == 0) tile = (tile & 7) * (total >> 3) + (tile >> 3); // workgroups of one XCD share x tiles
     const int m0 = (tile / nt) * BM, n0 = (tile % nt) * PBN;
-    const int kbeg = (int)blockIdx.y * a.steps_per_split; // in steps of 64 k; a multiple of 4 (whole superblocks)
-    const int T = a.k / BK - kbeg < a.steps_per_split ? a.k / BK - kbeg : a.steps_per_split; // a multiple of 4
+    const int T = a.k / BK; // steps of 64 k: a multiple of 4 (whole superblocks)
 
     // ---- x tiles (rows of the scratch buffer are allocated up to a multiple of BM: no clamp)
-    const uint8_t *xbase = reinterpret_cast<const uint8_t *>(a.xh + (size_t)m0 * a.k + (size_t)kbeg * BK);
+    const uint8_t *xbase = reinterpret_cast<const uint8_t *>(a.xh + (size_t)m0 * a.k);
     const uint32_t xrow_l = (uint32_t)(wave * AROWS + (lane >> 3)), xchunk_l = (uint32_t)((lane & 7) ^ (lane >> 4));
     const uint32_t xoff = (xrow_l * (uint32_t)a.k + xchunk_l * 8) * 2;
     const size_t x8rows = (size_t)8 * a.k * 2;
@@ -502,7 +501,7 @@ __global__ void __launch_bounds__(512) gemm_blk32_kernel(GemmArgs a) {
     // 16 of the block's 32 bytes (Q8_0)
     auto fetch = [&](int step, Raw &r) {
         step = step < T ? step : T - 1;
-        const size_t blk = (size_t)(kbeg + step) * 2 + bis;
+        const size_t blk = (size_t)step * 2 + bis;
         r.q = *reinterpret_cast<const u32x4 *>(BITS == 8 ? cp + blk * 32 + half * 16 : cp + blk * 16);
         if (BITS == 5) r.qh = *reinterpret_cast<const uint32_t *>(qp + blk * 4);
         asm volatile("" ::: "memory");
@@ -570,14 +569,14 @@ __global__ void __launch_bounds__(512) gemm_blk32_kernel(GemmArgs a) {
     const int rc0 = WITH_MIN ? (wave & 3) * 32 : (wave & 1) * 64; // first column of this wave's kilobyte
     int rcol = n0 + rc0 + (WITH_MIN ? lane >> 1 : lane);
     rcol = rcol < a.n ? rcol : a.n - 1;
-    const uint8_t *rsrc = a.meta + (size_t)rcol * a.meta_pitch + (size_t)(kbeg >> 2) * (16 * RV) + (WITH_MIN ? (lane & 1) * 16 : 0);
+    const uint8_t *rsrc = a.meta + (size_t)rcol * a.meta_pitch + (WITH_MIN ? (lane & 1) * 16 : 0);
     auto fetch_records = [&](int sb) {
         sb = sb < nsb ? sb : nsb - 1;
         __builtin_amdgcn_global_load_lds((gbl_void *)(rsrc + (size_t)sb * (16 * RV)), (lds_void *)(rec_lds + (sb & 1) * RECB + rc0 * 16 * RV), 16, 0, 0);
         asm volatile("" ::: "memory");
     };
     u32x4 mx[MI];
-    const uint8_t *x3p = reinterpret_cast<const uint8_t *>(a.xs3 + (size_t)(m0 + wm + li) * a.xs3_pitch + (size_t)(kbeg >> 2) * 32 + hh * 16);
+    const uint8_t *x3p = reinterpret_cast<const uint8_t *>(a.xs3 + (size_t)(m0 + wm + li) * a.xs3_pitch + hh * 16);
     auto fetch_sums = [&](int sb) {
 #pragma unroll
         for (int i = 0; i < MI; i++) mx[i] = *reinterpret_cast<const u32x4 *>(x3p + ((size_t)i * 32 * a.xs3_pitch + (size_t)sb * 32) * 2);
@@ -716,10 +715,7 @@ __global__ void __launch_bounds__(512) gemm_blk32_kernel(GemmArgs a) {
             for (int r = 0; r < 16; r++) {
                 const int gm = m0 + wm + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                 if (gm < a.m && gn < a.n) {
-                    if (!a.pair) {
-                        if (a.ypart) a.ypart[((size_t)blockIdx.y * a.m + gm) * a.n + gn] = acc[i][j][r];
-                        else a.y[(size_t)gm * a.n + gn] = acc[i][j][r] * (a.rowscale[gm] * (1.0f / ASCALE));
-                    }
+                    if (!a.pair) a.y[(size_t)gm * a.n + gn] = acc[i][j][r] * (a.rowscale[gm] * (1.0f / ASCALE));
                 }
             }
 #pragma unroll
@@ -728,14 +724,10 @@ __global__ void __launch_bounds__(512) gemm_blk32_kernel(GemmArgs a) {
                 if (a.pair && gm < a.m && gn < a.n) {
                     const size_t t = (size_t)(gm >> 1);
                     const float v = acc[i][j][r] + acc[i][j][r + 1];
-                    if (a.ypart) {
-                        a.ypart[((size_t)blockIdx.y * (a.m >> 1) + t) * a.n + gn] = v;
-                    } else {
-                        float out = v * (a.rowscale[gm] * (1.0f / ASCALE));
-                        if (a.bias) out += a.bias[gn];
-                        if (a.resid) out += a.resid[t * a.n + gn];
-                        a.y[t * a.n + gn] = out;
-                    }
+                    float out = v * (a.rowscale[gm] * (1.0f / ASCALE));
+                    if (a.bias) out += a.bias[gn];
+                    if (a.resid) out += a.resid[t * a.n + gn];
+                    a.y[t * a.n + gn] = out;
                 }
             }
         }
@@ -1038,11 +1030,10 @@ struct GemmPlan {
 };
 
 // Whether gemm_blk32_kernel takes this call.
-bool q5_route(const axq_weight *w, int m, bool in_regs_only) {
+bool q5_route(const axq_weight *w, bool in_regs_only) {
     static const bool off = getenv("AXQ_GEMM_BLK32") && getenv("AXQ_GEMM_BLK32")[0] == '0'; // development knob
     const bool type_ok = w->type == AXQ_Q4_0 || w->type == AXQ_Q4_1 || w->type == AXQ_Q5_0 || w->type == AXQ_Q5_1 || w->type == AXQ_Q8_0;
-    static const int min_rows = getenv("AXQ_GEMM_BLK32_MIN_ROWS") ? atoi(getenv("AXQ_GEMM_BLK32_MIN_ROWS")) : 1; // development knob
-    return !off && type_ok && w->k % 256 == 0 && m >= min_rows && w->meta_pitch % 16 == 0 && (!in_regs_only || w->k <= 16 * 256 * 4);
+    return !off && type_ok && w->k % 256 == 0 && w->meta_pitch % 16 == 0 && (!in_regs_only || w->k <= 16 * 256 * 4);
 }
 
 // Split K when the output tiles alone leave most compute units idle (short prompts): the splits' partial sums go
@@ -1054,18 +1045,17 @@ int plan_gemm(axq_ctx *ctx, const axq_weight *w, int m, bool f32_rows, size_t ex
                         (long long)w->k);
     if (w->n_rows > INT32_MAX || w->k > INT32_MAX)
         return axq_fail(ctx, AXQ_ERR_SHAPE_MISMATCH, "Shape mismatch: weight dimensions exceed 2^31");
-    static const int bm_knob = getenv("AXQ_GEMM_BM") ? atoi(getenv("AXQ_GEMM_BM")) : 0; // development knob: 128 or 256 for every shape
-    const int bm = bm_knob ? bm_knob : (m > 128 ? 256 : 128);
+    static const int bm_knob = getenv("AXQ_GEMM_BM") ? atoi(getenv("AXQ_GEMM_BM")) : 0; // development knob: 128 or 256 for every shape of the two-plane kernel
+    p->q5 = q5_route(w, f32_rows);
+    const int bm = p->q5 ? PBM : bm_knob ? bm_knob : (m > 128 ? 256 : 128);
     p->wm = bm / 128;
-    p->q5 = q5_route(w, m, f32_rows);
     const long tiles = (long)((w->n_rows + BN - 1) / BN) * ((m + bm - 1) / bm);
     const int ksteps = (int)(w->k / BK), cus = ctx->prop.multiProcessorCount;
     int splits = (int)(cus / tiles);
     splits = splits > 8 ? 8 : splits;
     if (splits > ksteps / 4) splits = ksteps / 4;
-    if (splits < 2 || w->n_rows % 4 != 0) splits = 1;
+    if (p->q5 || splits < 2 || w->n_rows % 4 != 0) splits = 1;
     p->steps_per_split = (ksteps + splits - 1) / splits;
-    if (p->q5) p->steps_per_split = (p->steps_per_split + 3) & ~3; // whole superblocks per split
     p->splits = (ksteps + p->steps_per_split - 1) / p->steps_per_split;
     // gemm_blk32_kernel reads whole row tiles without a clamp: its x buffers have rows up to a multiple of the tile
     const size_t mpad = p->q5 ? (size_t)(m + bm - 1) / bm * bm : (size_t)m;
@@ -1087,42 +1077,24 @@ XSums plan_sums(axq_ctx *ctx, const axq_weight *w, const GemmPlan &p) {
 }
 
 template <int BITS, bool WITH_MIN>
-int launch_blk32(axq_ctx *ctx, const GemmArgs &a, dim3 grid, size_t lds) {
-    static std::atomic<uint64_t> lds_allowed[2]; // per kernel: a bit per device
-    int rc;
-    if (a.wm == 2) {
-        if ((rc = axq_allow_lds(ctx, reinterpret_cast<const void *>(gemm_blk32_kernel<BITS, WITH_MIN, 256>), lds_allowed[1], lds))) return rc;
-        gemm_blk32_kernel<BITS, WITH_MIN, 256><<<grid, 512, lds, ctx->stream>>>(a);
-    } else {
-        if ((rc = axq_allow_lds(ctx, reinterpret_cast<const void *>(gemm_blk32_kernel<BITS, WITH_MIN, 128>), lds_allowed[0], lds))) return rc;
-        gemm_blk32_kernel<BITS, WITH_MIN, 128><<<grid, 512, lds, ctx->stream>>>(a);
-    }
+int launch_blk32(axq_ctx *ctx, const GemmArgs &a) {
+    static std::atomic<uint64_t> lds_allowed{0};
+    constexpr size_t lds = (size_t)(3 * PBM * 64 + 2 * PBN * 64) * sizeof(_Float16) + 2 * PBN * 32; // three x stages, two weight stages, scale records
+    if (int rc = axq_allow_lds(ctx, reinterpret_cast<const void *>(gemm_blk32_kernel<BITS, WITH_MIN>), lds_allowed, lds)) return rc;
+    const unsigned tiles = (unsigned)(((a.n + PBN - 1) / PBN) * ((a.m + PBM - 1) / PBM));
+    gemm_blk32_kernel<BITS, WITH_MIN><<<tiles, 512, lds, ctx->stream>>>(a);
+    AXQ_LAUNCH_CHECK(ctx, "gemm_blk32_kernel");
     return AXQ_OK;
 }
 
-int launch_gemm_q5(axq_ctx *ctx, GemmArgs a, int splits, int type) {
-    const int bm = 128 * a.wm;
-    const unsigned tiles = (unsigned)(((a.n + PBN - 1) / PBN) * ((a.m + bm - 1) / bm));
-    const dim3 grid(tiles, (unsigned)splits);
-    const size_t lds = (size_t)(3 * bm * 64 + 2 * PBN * 64) * sizeof(_Float16) + 2 * PBN * 32; // three x stages, two weight stages, scale records
-    int rc;
+int launch_gemm_q5(axq_ctx *ctx, const GemmArgs &a, int type) {
     switch (type) {
-    case AXQ_Q4_0: rc = launch_blk32<4, false>(ctx, a, grid, lds); break;
-    case AXQ_Q4_1: rc = launch_blk32<4, true>(ctx, a, grid, lds); break;
-    case AXQ_Q5_0: rc = launch_blk32<5, false>(ctx, a, grid, lds); break;
-    case AXQ_Q5_1: rc = launch_blk32<5, true>(ctx, a, grid, lds); break;
-    default: rc = launch_blk32<8, false>(ctx, a, grid, lds); break;
+    case AXQ_Q4_0: return launch_blk32<4, false>(ctx, a);
+    case AXQ_Q4_1: return launch_blk32<4, true>(ctx, a);
+    case AXQ_Q5_0: return launch_blk32<5, false>(ctx, a);
+    case AXQ_Q5_1: return launch_blk32<5, true>(ctx, a);
+    default: return launch_blk32<8, false>(ctx, a);
     }
-    if (rc) return rc;
-    AXQ_LAUNCH_CHECK(ctx, "gemm_blk32_kernel");
-    if (splits > 1) {
-        const int rows = a.pair ? a.m / 2 : a.m;
-        const size_t total4 = (size_t)rows * a.n / 4;
-        gemm_reduce_kernel<<<(unsigned)((total4 + 255) / 256), 256, 0, ctx->stream>>>(a.ypart, a.rowscale, rows, a.n, splits,
-                                                                                    1.0f / (WSCALE * XSUM_SCALE), a.pair ? 2 : 1, a.bias, a.resid, a.y);
-        AXQ_LAUNCH_CHECK(ctx, "gemm_reduce_kernel");
-    }
-    return AXQ_OK;
 }
 
 // The GEMM proper over activations that already sit in scratch as scaled f16 rows.
@@ -1139,7 +1111,7 @@ int run_gemm(axq_ctx *ctx, const axq_weight *w, int m, const GemmPlan &p, float 
     a.pair = pair ? 1 : 0; a.bias = bias; a.resid = resid; a.wm = p.wm;
     const XSums xs = plan_sums(ctx, w, p);
     a.xs3 = xs.xs3; a.xs3_pitch = xs.pitch;
-    if (p.q5) return launch_gemm_q5(ctx, a, p.splits, w->type);
+    if (p.q5) return launch_gemm_q5(ctx, a, w->type);
     switch (w->type) {
     case AXQ_Q4_0: return launch_gemm<GQ4x<false>>(ctx, a, p.splits);
     case AXQ_Q4_1: return launch_gemm<GQ4x<true>>(ctx, a, p.splits);

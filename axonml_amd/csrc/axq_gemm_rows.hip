@@ -1095,8 +1095,8 @@ template <int IN, bool LIMBS>
 void launch_prep(hipStream_t st, const void *x, const float *norm_w, float eps, int rows, int k, _Float16 *xa, _Float16 *xs, float *rs) {
     if (k <= 4096) rows_prep_kernel<IN, 1, LIMBS><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
     else if (k <= 8192) rows_prep_kernel<IN, 2, LIMBS><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
-    else if (k <= 16384) rows_prep_kernel<IN, 4, LIMBS><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
-    else rows_prep_kernel<IN, 0, LIMBS><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
+    else if (IN == 1 || k <= 16384) rows_prep_kernel<IN, 4, LIMBS><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs); // SwiGLU rows are no longer
+    else if constexpr (IN != 1) rows_prep_kernel<IN, 0, LIMBS><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs);
 }
 
 // How many tiles of 128 x 128 outputs a call of m rows of operands has, where 256 x 256 are the alternative.
