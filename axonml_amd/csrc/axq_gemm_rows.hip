@@ -395,11 +395,14 @@ struct Block32 {
 // copy x, the other half codes and sides: a wave's waits are in order of its requests, and x, which comes from L2 shortly before
 // it is used, would otherwise wait for codes that were requested from memory for later.
 // AT > 1: x as three limbs (see rows_prep_kernel).  2: up to 16 rows, in two tiles [first | second] and [0 | third] whose products meet in
-// one accumulator tile; 3: 32 rows in three tiles, the second and the third meet.
+// one accumulator tile; 3: 32 rows in three tiles, the second and the third meet; 4: up to 40 rows, 32 of them in three tiles and the
+// limbs of the other eight in a fourth, two tiles to each of the groups along M (37 rows as two times 32, six tiles, and so, us: Q6_K
+// 28672 x 4096 104 84, Q4_K 66 55, Q4_K 4096 x 14336 45 41; f16 pairs, with ten bits less, 81, 51 and 37).
 template <class T, int MI, int WM, int NJ, int AT>
 struct RowsTile {
     static constexpr int KG = 2 / WM, GW = 4 * WM, CW = GW / 2;     // groups along K, waves of one, waves that copy x (and codes)
-    static constexpr int M = AT == 2 ? 16 : AT == 3 ? 32 * WM : 32 * MI * WM, N = 128 * NJ, XT = AT > 1 ? AT : MI; // rows, columns, tiles of x of a wave
+    static constexpr int M = AT == 2 ? 16 : AT == 3 ? 32 : AT == 4 ? 40 : 32 * MI * WM, N = 128 * NJ; // rows, columns
+    static constexpr int XT = AT == 2 || AT == 3 ? AT : MI;         // tiles of x of a wave
     static constexpr int acc_of(int l) { return AT == 3 ? (l > 0 ? 1 : 0) : AT == 2 ? 0 : l; } // accumulator tile of a tile of x
     static constexpr bool first_of(int l) { return l == XT - 1 || acc_of(l) != acc_of(l + 1); }
     static constexpr bool WHOLE = MI <= 2;                          // the fragments of a whole step ahead in registers
@@ -414,7 +417,7 @@ struct RowsTile {
     static constexpr int XL = 2 * XT, SL = T::MIN ? XT : 0, WT = 4 * NJ / CW, WL = WT * T::PAIRS;
     static constexpr int D16 = (2 * NJ * T::SIDE16 + CW - 1) / CW, D4 = (2 * NJ * T::SIDE4 + CW - 1) / CW;
     static constexpr int FIRST = 7 > 2 * NW - 1 ? 7 : 2 * NW - 1;
-    static_assert(AT == 1 || MI == AT - 1, "limbs");
+    static_assert(AT == 1 || (AT == 4 ? MI == 2 && WM == 2 : MI == AT - 1 && WM == 1), "limbs");
     static_assert(NW >= 2 && WT * CW == 4 * NJ && NA <= FIRST, "stages");
     // Behind barrier b: x of step b + NA and, where b % 4 = 1, the sums of superblock (b + 3) / 4; codes of unit (b + 1) / 2 + NW - 1
     // where b is odd and the sides of superblock (b + 7) / 4 where b % 4 = 1.  In front of barrier g everything that is read
@@ -689,7 +692,7 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
                         to[Tile::acc_of(l)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
                             af[J % AHEAD][t][l], bf[t - T0][j][pr], decltype(fresh)::value && Tile::first_of(l) && t == T0 && pr == 0 ? zero : to[Tile::acc_of(l)][j], 0, 0, 0);
             };
-            if constexpr (AT == 1) {
+            if constexpr (XT == MI) { // every tile of x has an accumulator of its own
 #pragma unroll
                 for (int t = T0; t < T1; t++) {
                     make(raw[J & 1], J, t, bf[t - T0]);
@@ -822,11 +825,32 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
     wait_loads_and_lds<0>(); // nothing of this workgroup may still be on its way into LDS
 
     // ---- results.  D layout: lane -> column li; register r -> row 8 (r / 4) + 4 (lane / 32) + r % 4
-    if constexpr (AT > 1) // the first limbs' results and the others', which come times 2^11; the others of sixteen rows lie sixteen rows below
+    // the first limbs' results and the others', which come times 2^(LB + 2); the others of sixteen rows lie sixteen rows below
+    constexpr float BELOW = 1.0f / (1 << (LB + 2));
+    if constexpr (AT == 4) { // the third limbs of 32 rows come from the other group; the eight rows' limbs lie eight rows below each other
+        barrier();
+        float *mail = reinterpret_cast<float *>(lds) + wn * (NJ * 16 * 64) + lane;
+        static_assert(4 * NJ * 16 * 64 * 4 <= Tile::LDS, "mail");
+        if (wm == 1)
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) mail[(j * 16 + r) * 64] = acc[0][j][r];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+            if (wm == 1) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[0][j][r] = fmaf(acc[1][j][r + 4] + acc[1][j][r + 8], BELOW, acc[1][j][r]);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[0][j][r] = fmaf(acc[1][j][r] + mail[(j * 16 + r) * 64], BELOW, acc[0][j][r]);
+            }
+    } else if constexpr (AT > 1)
 #pragma unroll
         for (int j = 0; j < NJ; j++)
 #pragma unroll
-            for (int r = 0; r < (AT == 2 ? 8 : 16); r++) acc[0][j][r] = fmaf(AT == 2 ? acc[0][j][r + 8 & 15] : acc[MI - 1][j][r], 1.0f / (1 << (LB + 2)), acc[0][j][r]);
+            for (int r = 0; r < (AT == 2 ? 8 : 16); r++) acc[0][j][r] = fmaf(AT == 2 ? acc[0][j][r + 8 & 15] : acc[MI - 1][j][r], BELOW, acc[0][j][r]);
     constexpr int MR = AT > 1 ? 1 : MI;
     auto store = [&](int i, int j, int r, float v, float v2) { // v2: of row r + 1, where rows are pairs
         const int gn = n0 + (wn * NJ + j) * 32 + li;
@@ -873,7 +897,7 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
             for (int j = 0; j < NJ; j++)
 #pragma unroll
                 for (int r = 0; r < 16; r++)
-                    if (r % step_r == 0) store(i, j, r, acc[i][j][r] * unit[j], acc[i][j][r | 1] * unit[j]);
+                    if (r % step_r == 0 && (AT != 4 || r < 4 || wm == 0)) store(i, j, r, acc[i][j][r] * unit[j], acc[i][j][r | 1] * unit[j]);
     }
 }
 
@@ -993,7 +1017,7 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
     const int r0 = row * PARTS, steps = k >> 6, nsb = k >> 8;
     auto slot = [&](int part) { // of the operand's rows: pairs are neighbours; limbs see RowsTile, part 3 = the zeros
         if (!LIMBS) return r0 + part;
-        return gridDim.x <= 16 ? (part < 2 ? part : 5 - part) * 16 + row : ((row >> 5) * 3 + part) * 32 + (row & 31);
+        return gridDim.x <= 16 ? (part < 2 ? part : 5 - part) * 16 + row : row < 32 ? part * 32 + row : 96 + part * 8 + (row & 7);
     };
     each(false, [&](float (&e)[8], int c) {
         if (NC == 0) normed(e, c);
@@ -1074,13 +1098,13 @@ int launch_tile(axq_ctx *ctx, const RowsArgs &a, int splits) {
 }
 
 // The tile of a call.  Limbs: up to 16 and 32 rows the two halves of the waves on two parts of K, since a workgroup's time is then its
-// number of steps.  Others: up to 32 and 64 rows of operands the same with one and two row tiles per wave; above two times
+// number of steps; more, which are fewer than 40, see RowsTile.  Others: up to 32 and 64 rows of operands the same with one and two row tiles per wave; above two times
 // two row tiles (at 64 f32 rows and Q4_K 28672 x 4096 2.5 us ahead of four row tiles per wave and split halves), or 256 x 256
 // outputs (see wide_tiles), which blocks do not have: their sums do not fit the registers.
 template <class T>
 int launch_rows(axq_ctx *ctx, const RowsArgs &a, int splits, bool limbs, bool wide) {
     if (limbs) {
-        if (a.m > 32) return launch_tile<T, 2, 2, 1, 3>(ctx, a, splits);
+        if (a.m > 32) return launch_tile<T, 2, 2, 1, 4>(ctx, a, splits);
         if (a.m > 16) return launch_tile<T, 2, 1, 1, 3>(ctx, a, splits);
         return launch_tile<T, 1, 1, 1, 2>(ctx, a, splits);
     }
@@ -1129,12 +1153,13 @@ RowsPlan rows_plan(const axq_ctx *ctx, const axq_weight *w, int in, int rows) {
     p.m = rows * p.parts;
     const int n = (int)w->n_rows, nsb = (int)(w->k >> 8), groups = p.m <= (p.limbs ? 32 : 64) ? 2 : 1;
     p.wide = !p.limbs && (w->type == AXQ_Q4_K || w->type == AXQ_Q5_K || w->type == AXQ_Q6_K) && wide_tiles(ctx, p.m, n, w->k);
-    p.bm = p.limbs ? (rows <= 32 ? 32 : 64) : p.m <= 32 ? 32 : p.m <= 64 ? 64 : p.wide ? 256 : 128;
+    p.bm = p.limbs ? (rows <= 32 ? 32 : 40) : p.m <= 32 ? 32 : p.m <= 64 ? 64 : p.wide ? 256 : 128;
     const int bn = p.wide ? 256 : 128;
     p.tiles = (long)((n + bn - 1) / bn) * ((p.m + p.bm - 1) / p.bm);
     // K is split over as many workgroups as leave every group of waves a superblock, up to one workgroup per compute unit: into sixteen
     // parts at most for 17 to 39 rows (eight and sixteen, 1024 x 14336: Q6_K, 39 rows 55.5 42.4 us; Q4_K, 17 rows 33.9 29.6, with
     // thirty-two 30.4), else eight (2048 x 8192, ten rows: Q4_0 19.6 us, sixteen 20.4; Q4_K 20.8, 21.6)
+    static_assert(AXQ_ROWS_PAIRS_MIN <= 40, "limbs of at most 40 rows");
     const int most = p.limbs && rows > 16 ? 16 : 8;
     int splits = (int)(ctx->prop.multiProcessorCount / p.tiles);
     if (splits > nsb / groups) splits = nsb / groups;
@@ -1191,7 +1216,7 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
     const int m = p.m, n = (int)w->n_rows, k = (int)w->k, nsb = k >> 8, splits = p.splits;
     RowsArgs a;
     a.sb_per_split = p.sb_per_split;
-    const size_t mtiles = limbs ? (rows <= 16 ? 2 : rows <= 32 ? 3 : 6) : (size_t)(m + p.bm - 1) / p.bm * (p.bm / 32);
+    const size_t mtiles = limbs ? (rows <= 16 ? 2 : rows <= 32 ? 3 : 4) : (size_t)(m + p.bm - 1) / p.bm * (p.bm / 32);
     const size_t xa_bytes = mtiles * 32 * (size_t)k * 2, xs_bytes = mtiles * (size_t)nsb * 2048;
     const size_t rs_bytes = axq_align_up((size_t)m * 4, 256), part_bytes = splits > 1 ? (size_t)splits * rows * (size_t)n * 4 : 0;
     if (int rc = axq_gemm_reserve(ctx, xa_bytes + xs_bytes + rs_bytes + part_bytes)) return rc;
