@@ -864,10 +864,12 @@ int axq_dense_gemm(axq_ctx *ctx, axq_parts &parts, int m, int k, int ldx, bool f
     // Cost of a launch in units of a 128 x 128 tile that has a compute unit to itself: two 128 x 128 workgroups share one, a 256 x 256
     // tile is four at 1.35 times the rate (2047 rows, K = 2048: 8192 columns 98 against 130 us).  The 256 x 256 tiles get the
     // widest weights, as many as is cheapest, the others a launch of their own: a few columns more than whole rounds of the
-    // chip (a narrow projection beside wide ones) would cost a round of large tiles.
+    // chip (a narrow projection beside wide ones) would cost a round of large tiles.  Not at short K, where a large tile is mostly its start
+    // and its way out (prompts, us, with large tiles and without: K = 1024, Gemosun, 1200 and 2048 tokens 1100 1075, 1352 1334, Lakulix, 2048
+    // 1043 1038; K = 2048, Lakulix, 1200 and 2048 tokens 1400 1410, 1691 1748, Gemosun, 2048 2377 2417).
     const int cus = ctx->prop.multiProcessorCount;
     auto square_cost = [&](int tiles) { return 2.0f * (float)((tiles + 2 * cus - 1) / (2 * cus)); };
-    if (m > 128) {
+    if (m > 128 && a.k >= 1536) {
         int order[AXQ_MAX_PARTS], n = parts.n_parts;
         for (int i = 0; i < n; i++) {
             int at = i;
