@@ -5,14 +5,15 @@
 //
 // Time of a call with f32 rows, before (groups of eight vectors, or two-stage operands in LDS) and now, us:
 //   rows                  10          16          32          64
-//   Q4_K 28672 x 4096     40.3 35.1   40.5 35.7   81.5 44.2   61.8 53.9
-//   Q4_K 4096 x 4096      22.7 16.9   21.8 18.5   43.0 20.5   33.0 23.4
-//   Q4_K 4096 x 14336     31.7 31.6   32.0 32.0   63.2 37.6   63.9 38.4
-//   Q4_0 4096 x 11008, 21 rows: 41.7 30.3; Q4_0 4096 x 4096, 10 and 39 rows: 22.3 16.0, 56.6 22.7; Q8_0 11008 x 4096, 64 rows: 43.2 34.8;
-//   bf16 rows, Q8_0 4096 x 4096, 16: 26.1 16.2; Q4_0 11008 x 4096, 128: 48.4 36.0
+//   Q4_K 28672 x 4096     41.4 35.7   42.0 36.2   83.7 44.4   61.7 54.7
+//   Q4_K 4096 x 4096      21.9 15.7   21.9 17.2   39.9 20.8   33.0 23.1
+//   Q4_K 4096 x 14336     as before (see axq_dev_rows_gemm_pays)   63.5 36.8   64.0 39.4
+//   Q4_0 4096 x 11008, 21 rows: 41.9 29.2; Q4_0 4096 x 4096, 10 and 39 rows: 21.7 14.4, 54.7 21.2; Q8_0 11008 x 4096, 64 rows: 43.1 34.9;
+//   bf16 rows, Q8_0 4096 x 4096, 16: 26.0 14.5; Q4_0 11008 x 4096, 128: 48.4 36.5; Q4_K 14336 x 4096, 2048: 325 to 328 321
 // What bounds it: at few rows the fixed parts (pre-pass, reduction and the launches around them: 14 us of the 4096 x 4096 calls) and
 // the LDS reads of x, which every wave makes for its 32 columns (0.35 us per step with one tile of x, 0.6 with two); at many the matrix
-// pipe beside the vector instructions that make operands (2048 bf16 rows x 14336: 320 us, 750 TFLOP/s), which overlap only in part.
+// pipe beside the vector instructions that make operands (2048 bf16 rows x 14336: 320 to 330 us from card to card, 730 to 750 TFLOP/s,
+// the pipe busy for 0.46 of it and other vector instructions 0.35), which overlap only in part.
 //
 // Numerics.  A bf16 row goes in as f16 under a power-of-two row scale that puts its largest element right below f16's limit: exact
 // down to 2^-31 of that element, and what is smaller to within 2^-39 of it.  An f32 row goes in as two f16 rows, leading eleven
@@ -1174,7 +1175,7 @@ RowsPlan rows_plan(const axq_ctx *ctx, const axq_weight *w, int in, int rows) {
 
 // Superblock types at any number of rows; blocks of 32, whose sums fit the registers of 128 x 128 outputs only, up to 128 rows of
 // operands and while such tiles are at most one per compute unit (bf16 rows, us here and in gemm_blk32_kernel: Q5_1 4096 x 4096, 509
-// rows 52.2 59.1; Q4_0 4096 x 4096, 256 rows 27.9 39.2; Q8_0 11008 x 4096, 256 rows, 172 tiles, 59.4 72.5; Q5_0 11008 x 4096, 512 rows,
+// rows 54.7 59.2; Q4_0 4096 x 4096, 256 rows 27.9 39.2; Q8_0 11008 x 4096, 256 rows, 172 tiles, 59.4 72.5; Q5_0 11008 x 4096, 512 rows,
 // 344 tiles, 136.8 128.4; Q4_0 14336 x 4096, 1024 rows, 219 217).  K a multiple of 256.
 bool axq_dev_rows_gemm_covers(const axq_ctx *ctx, const axq_weight *w, int rows, bool bf16) {
     if (w->k % 256 != 0 || w->k > INT32_MAX || w->n_rows > INT32_MAX || rows < 1) return false;
