@@ -1,7 +1,9 @@
-"""The logits of a prompt come from its last row, or from a step where the last portion would be one row; described layers take that step
-beside the last rows: both sides of every edge."""
+"""The logits of a prompt come from the step of its last token, behind the rows of the others; described layers take that step beside the last
+rows: both sides of every edge."""
 import numpy as np
 import pytest
+
+import oracle as o
 
 from . import gemosun_common as gc
 from . import lakulix_common as lc
@@ -36,6 +38,22 @@ def test_last_token_of_a_prompt(ctx, monkeypatch, n_tokens):
     assert got == nxt and max_rel_err(logits, lg, DECODE_FLOOR) <= DECODE_RTOL
     gpu.close()
     cpu.close()
+
+
+@pytest.mark.parametrize("qtype,sizes", [(o.Q4_K, {}), (o.F32, {}), (o.Q8_0, dict(hidden_size=320, intermediate_size=448, num_heads=5, num_kv_heads=1))],
+                         ids=["superblocks", "f32 weights", "no whole superblocks"])
+@pytest.mark.parametrize("n_tokens", [2, 9, 10, 11, 33, 41, 65, 71])
+def test_logits_have_the_bits_of_the_step(ctx, qtype, sizes, n_tokens):
+    """The last token of a prompt goes through the layers as the vector that it is, not as a row of a product with fewer bits."""
+    c = tiny_config(max_seq_len=80, **sizes)
+    gpu = load_gpu(ctx, c, random_weights(c, n_tokens, qtype))
+    tokens = np.random.default_rng(n_tokens).integers(0, c["vocab_size"], size=n_tokens)
+    got, logits = gpu.forward_tokens(tokens)
+    hidden = gpu.hidden()
+    gpu.truncate(n_tokens - 1)
+    want, step = gpu.forward(int(tokens[-1]))
+    assert got == want and np.array_equal(logits, step) and np.array_equal(hidden, gpu.hidden())
+    gpu.close()
 
 
 LAKULIX = lc.config([lc.lightning(), lc.attention(), lc.wkv(), lc.attention()], width=96, vocab=150)
