@@ -2,6 +2,7 @@
 #include <stdarg.h>
 #include <stdlib.h>
 #include <strings.h>
+#include <sys/mman.h>
 
 #include "axq_internal.h"
 
@@ -304,16 +305,17 @@ int axq_synchronize(axq_ctx *ctx) {
 int axq_host_alloc(axq_ctx *ctx, size_t bytes, void **hptr) {
     if (!ctx || !hptr) return axq_fail(ctx, AXQ_ERR_INVALID_ARGUMENT, "axq_host_alloc: NULL pointer");
     *hptr = nullptr;
-    AXQ_HIP(ctx, hipSetDevice(ctx->device), AXQ_ERR_DRIVER);
-    const hipError_t e = hipHostMalloc(hptr, bytes ? bytes : 1);
-    if (e == hipSuccess) return AXQ_OK;
-    (void)hipGetLastError(); // the caller goes on without it
-    *hptr = nullptr;
-    return axq_fail(ctx, AXQ_ERR_ALLOCATION_FAILED, "%zu bytes of page-locked memory: %s", bytes, hipGetErrorString(e));
+    const size_t large = 4 << 20; // in pages of 2 MB where there are such
+    if (bytes <= SIZE_MAX - large) {
+        const size_t page = bytes >= large ? 2 << 20 : 4096, whole = axq_align_up(bytes ? bytes : 1, page);
+        *hptr = aligned_alloc(page, whole);
+        if (*hptr && bytes >= large) (void)madvise(*hptr, whole, MADV_HUGEPAGE);
+    }
+    return *hptr ? AXQ_OK : axq_fail(ctx, AXQ_ERR_ALLOCATION_FAILED, "%zu bytes of host memory", bytes);
 }
 
 void axq_host_free(void *hptr) {
-    if (hptr) (void)hipHostFree(hptr);
+    free(hptr);
 }
 
 int axq_set_stream(axq_ctx *ctx, void *hip_stream) {

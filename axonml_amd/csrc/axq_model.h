@@ -40,6 +40,9 @@ struct axq_model {
     // device-side state
     int32_t *pos, *tok, *next, *gen, *prompt, *out;
     int32_t *host_next = nullptr;   // page-locked: the argmax of the last step by sequence
+    uint8_t *host_ring = nullptr;   // page-locked: logits on their way to the caller, two portions of host_portion bytes
+    size_t host_portion = 0;
+    hipEvent_t portion_there[2] = {nullptr, nullptr};
     int32_t *hist;                  // every token fed so far, by position (what a repetition penalty looks at)
     void *sample_scratch;           // scratch of the sampler, allocated when one is set
     bool sampling;                  // next token by axq_sampling_config instead of the plain argmax

@@ -122,7 +122,7 @@ class QuantType(enum.IntEnum):
         return _lib.load_library().axq_type_name(int(self)).decode()
 
 
-# --------------------------------------------------------------------------- page-locked results
+# --------------------------------------------------------------------------- memory for results
 class _HostBlock:
     """One block; the arrays that lie in it keep it, and the last of them gives it back."""
 
@@ -138,10 +138,9 @@ class _HostBlock:
 
 
 class _HostBlocks:
-    """Page-locked memory of a context for results that a call copies to the host: the card writes there itself.  New pageable memory for
-    every call is paged in and filled by way of the runtime's own blocks: of a step of 32 sequences of a small model, 4 MB of
-    logits, that was two thirds.  Blocks that nobody holds are kept up to KEEP bytes, and there are MOST bytes at most: beyond that a result
-    is an ordinary array."""
+    """Memory of a context for results, used again when the last array in it has gone: new memory for every call is paged in by it
+    (8 MB of logits: 360 us so, 660 to new memory).  It is ordinary memory, which may be held for as long as one likes and which forked processes have.  Blocks that
+    nobody holds are kept up to KEEP bytes, and there are MOST bytes at most: beyond that a result is an array of numpy's."""
     KEEP, MOST = 64 << 20, 256 << 20
 
     def __init__(self, ctx):
@@ -206,7 +205,7 @@ class Context:
         self._blocks = _HostBlocks(self)
 
     def host_array(self, *shape):
-        """An uninitialised float32 array for a result, page-locked where there is room."""
+        """An uninitialised float32 array for a result, in memory that has been in use where there is some."""
         return self._blocks.array(shape)
 
     def close(self):

@@ -122,7 +122,7 @@ AXQ_API int axq_free(axq_ctx *ctx, void *dptr);                      /* dealloca
 AXQ_API int axq_copy_to_device(axq_ctx *ctx, void *dst, const void *src, size_t bytes);
 AXQ_API int axq_copy_to_host(axq_ctx *ctx, void *dst, const void *src, size_t bytes);
 AXQ_API int axq_copy_device_to_device(axq_ctx *ctx, void *dst, const void *src, size_t bytes);
-/* Page-locked host memory: copies to and from it need no staging.  Free it when nothing reads or writes it any more. */
+/* Host memory in whole pages, for results that a program reads again and again into the same place.  Any thread may free it, also after the context. */
 AXQ_API int axq_host_alloc(axq_ctx *ctx, size_t bytes, void **hptr);
 AXQ_API void axq_host_free(void *hptr);
 AXQ_API int axq_synchronize(axq_ctx *ctx);                           /* synchronize() */
