@@ -179,7 +179,7 @@ class _HostBlocks:
 
     def drop(self):
         with self.lock:
-            for size, ptrs in self.idle.items():
+            for size, ptrs in list(self.idle.items()):  # a block of another size may come back in here
                 while ptrs:
                     self.lib.axq_host_free(ptrs.pop())
                     self.kept -= size

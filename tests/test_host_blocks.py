@@ -1,4 +1,4 @@
-"""The pool of page-locked blocks that results lie in: what it keeps, gives back and refuses, over a stand-in for the allocator."""
+"""The pool of blocks that results lie in: what it keeps, gives back and refuses, over a stand-in for the allocator."""
 import gc
 import threading
 
@@ -62,6 +62,27 @@ def test_what_is_kept_and_handed_out_is_bounded():
     assert not ctx.lib.blocks and pool.total == 0
     assert pool.array((5,)).shape == (5,) and not ctx.lib.blocks
     assert pool.array((0, 5)).shape == (0, 5)
+
+
+def test_a_block_that_comes_back_while_others_go():
+    """The collector may run anywhere, here in the middle of giving blocks back."""
+    ctx = Ctx()
+    pool = _HostBlocks(ctx)
+    other = [pool.array((3000,))]
+    held = [pool.array((1000,)), pool.array((2000,))]
+    free = ctx.lib.axq_host_free
+
+    def free_and_collect(ptr):
+        free(ptr)
+        other.clear()
+    del held
+    ctx.lib.axq_host_free = free_and_collect
+    pool.MOST = pool.total
+    big = pool.array((1024,) * 2)  # more than there may be: what is idle goes
+    assert big.shape == (1024, 1024) and pool.total == pool.kept == 12288
+    ctx.lib.axq_host_free = free
+    pool.close()
+    assert not ctx.lib.blocks and pool.total == pool.kept == 0
 
 
 def test_no_page_locked_memory():
