@@ -82,8 +82,6 @@ struct axq_stack {
     int32_t *r_route = nullptr;           // ... and the chosen experts, slots, rows by slot and tiles
     int32_t *r_want = nullptr;
     int logits_cap = 0;
-    float *trace = nullptr;
-    int trace_total = 0, trace_row0 = 0;
     hipStream_t beside = nullptr; // a prompt's last token goes through the layers here, behind the rows and beside them
     hipEvent_t ready = nullptr;
 };
@@ -383,7 +381,8 @@ int reserve_rows(axq_model *m, int rows) {
         }
     }
     const size_t es = s.f32 ? 4 : 2, W = s.c.width, C = cap;
-    hipError_t e = dev_alloc(&s.r_h, C * W * 4);
+    const char *most_bytes = getenv("AXQ_GEMM_SCRATCH_MAX"); // development knob, see axq_gemm_reserve
+    hipError_t e = most_bytes && C * W * 4 > strtoull(most_bytes, nullptr, 10) ? hipErrorOutOfMemory : dev_alloc(&s.r_h, C * W * 4);
     if (e == hipSuccess) e = dev_alloc(&s.r_proj, C * proj * 4);
     if (e == hipSuccess) e = dev_alloc(&s.r_o, C * o * 4);
     if (e == hipSuccess) e = dev_alloc(&s.r_z, C * z * 4);
@@ -527,12 +526,6 @@ bool axq_stack_recurrent(const axq_model *m) {
     for (const Layer &l : m->stack->layers)
         if (l.c.mixer != AXQ_MIX_ATTENTION && l.c.mixer != AXQ_MIX_SOFTMAX) return true;
     return false;
-}
-
-void axq_stack_trace(axq_model *m, float *layers, int total_rows, int row0) {
-    m->stack->trace = layers;
-    m->stack->trace_total = total_rows;
-    m->stack->trace_row0 = row0;
 }
 
 int axq_stack_ready(axq_model *m) {
@@ -680,7 +673,7 @@ struct OnStream {
 namespace {
 
 // `then_step`: behind every run's mixer the same run of the step of the next token, on s.beside
-int stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, bool then_step) {
+int stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, float *layers, size_t layer_stride, bool then_step) {
     axq_stack &s = *m->stack;
     axq_ctx *ctx = m->ctx;
     const int W = s.c.width, ldw = pad64(W);
@@ -783,11 +776,9 @@ int stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, bool then_st
             if ((rc = ff_rows(ctx, s, l, ff, parallel ? s.r_x2 : s.r_x, nb, y, avg))) return rc;
         }
         x = s.r_h;
-        if (s.trace)
-            AXQ_HIP(ctx, hipMemcpyAsync(s.trace + ((size_t)run * s.trace_total + s.trace_row0) * W, s.r_h, (size_t)nb * W * 4, hipMemcpyDeviceToHost,
-                                        ctx->stream), AXQ_ERR_COPY_FAILED);
+        if (layers)
+            AXQ_HIP(ctx, hipMemcpyAsync(layers + run * layer_stride, s.r_h, (size_t)nb * W * 4, hipMemcpyDeviceToHost, ctx->stream), AXQ_ERR_COPY_FAILED);
     }
-    s.trace = nullptr;
     if (then_step) return AXQ_OK; // whose residual stream is in m->h
     AXQ_HIP(ctx, hipMemcpyAsync(m->h, s.r_h + (size_t)(nb - 1) * W, (size_t)W * 4, hipMemcpyDeviceToDevice, ctx->stream), AXQ_ERR_COPY_FAILED);
     return AXQ_OK;
@@ -813,7 +804,7 @@ int axq_stack_rows_and_step(axq_model *m, const int32_t *toks, int nb, int pos0)
         OnStream on(ctx, s.beside);
         rc = step_embed(m);
     }
-    if (!rc) rc = stack_rows(m, toks, nb, pos0, true);
+    if (!rc) rc = stack_rows(m, toks, nb, pos0, nullptr, 0, true);
     if (!rc) {
         OnStream on(ctx, s.beside);
         rc = step_head(m);
@@ -827,7 +818,9 @@ int axq_stack_rows_and_step(axq_model *m, const int32_t *toks, int nb, int pos0)
     return rc;
 }
 
-int axq_stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0) { return stack_rows(m, toks, nb, pos0, false); }
+int axq_stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, float *layers, size_t layer_stride) {
+    return stack_rows(m, toks, nb, pos0, layers, layer_stride, false);
+}
 
 int axq_stack_logits_rows(axq_model *m, const int32_t *rows, int n, float *logits) {
     axq_stack &s = *m->stack;

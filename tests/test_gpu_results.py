@@ -3,6 +3,7 @@ keep and that the processes it forks have."""
 import numpy as np
 import pytest
 
+from . import lakulix_common as lc
 from tests.decode_common import load_gpu, load_oracle, random_weights, tiny_config
 from tests.util import DECODE_FLOOR, DECODE_RTOL, max_rel_err
 
@@ -55,3 +56,24 @@ def test_logits_come_by_portions(ctx, n_seq, vocab):
         assert nxt[s] == want and max_rel_err(logits[s], lg, DECODE_FLOOR) <= DECODE_RTOL
     gpu.close()
     cpu.close()
+
+
+def test_layer_outputs_go_to_the_call_that_wants_them(ctx, monkeypatch):
+    """A call that fails leaves no place behind where a later prompt would write its layers' outputs."""
+    cfg = lc.config([lc.attention(), lc.lightning()], width=96, vocab=150)
+    m = lc.product(cfg, lc.tensors(cfg, 3), "bfloat16", ctx)
+    tokens = np.arange(20, dtype=np.int32)
+    layers, logits = np.full((2, 20, 96), 7, np.float32), np.full((1, 150), 7, np.float32)
+    place = np.array([19], np.int32)
+    call = lambda: m.ctx.lib.axq_model_forward_rows(m.handle, tokens.ctypes.data, 20, place.ctypes.data, 1, logits.ctypes.data, layers.ctypes.data)  # noqa: E731
+    monkeypatch.setenv("AXQ_GEMM_SCRATCH_MAX", "0")
+    assert call() != 0
+    monkeypatch.delenv("AXQ_GEMM_SCRATCH_MAX")
+    got = m.forward_tokens(tokens)[1]
+    m.reset()
+    m.forward_rows(tokens, [3])
+    assert (layers == 7).all() and (logits == 7).all()
+    m.reset()
+    assert call() == 0 and not (layers == 7).any() and not (logits == 7).any()
+    assert np.abs(logits[0] - got).max() <= lc.LIMIT["bfloat16"] * np.abs(got).max()
+    m.close()
