@@ -25,7 +25,7 @@ struct axq_ctx {
     int gemv_wgs_per_cu; // GEMV workgroups per compute unit that the rows are spread over
     void *gemm_scratch; // device scratch of the prefill GEMM (scaled f16 activations + row scales), grown on demand
     size_t gemm_scratch_bytes;
-    hipStream_t aux_stream[4]; // benchmarks only: launches that may overlap (created on first use, default priority)
+    hipStream_t aux_stream[4]; // launches that may overlap (created on first use, default priority): the first for prompts of described layers, all for benchmarks
     hipEvent_t aux_event[4], aux_fork;
     char err[512];
 };

@@ -228,8 +228,8 @@ static void launch_read_u(int in_flight, int threads, unsigned grid, hipStream_t
     else launch_read<32, NT>(threads, grid, st, src, n16, sink);
 }
 
-// Streams beside the context's own, for launches that may overlap (benchmarks only; default priority).  The first use
-// creates them; axq_destroy releases them.
+// Streams beside the context's own, for launches that may overlap (default priority).  The first use creates them; axq_destroy
+// releases them.
 int axq_aux_streams(axq_ctx *ctx, int n) {
     if (n > AXQ_AUX_STREAMS) n = AXQ_AUX_STREAMS;
     for (int i = 0; i < n; i++) {
