@@ -1,5 +1,5 @@
 """The tiles of the products with bfloat16 weights, through models whose one wide product takes them: row and column counts on both
-sides of their edges, odd steps for two groups of waves, columns whose rows are no whole 16 bytes, a few narrow weights beside a
+sides of their edges, odd steps for two groups of waves, K beyond the stages in LDS, columns whose rows are no whole 16 bytes, a few narrow weights beside a
 wide one, and what happens to a result on its way out (softcap, GLU, residual, the mean over the layers)."""
 import pytest
 
@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("rows,vocab,width", [(300, 22003, 64), (257, 22004, 200), (129, 17000, 72), (150, 8300, 192), (140, 8301, 64), (200, 4400, 130),
-                                              (70, 300, 320), (300, 22003, 1600), (257, 17004, 1544), (260, 17000, 1536)])
+                                              (70, 300, 320), (300, 22003, 1600), (257, 17004, 1544), (260, 17000, 1536),
+                                              (150, 8300, 384), (150, 8300, 704), (140, 8301, 1000), (129, 8200, 1408)])
 def test_logits_of_every_tile(ctx, rows, vocab, width):
     cfg = lc.config([lc.wkv(heads=2, dim=8)], width=width, vocab=vocab)
     t = lc.tensors(cfg, rows + width)

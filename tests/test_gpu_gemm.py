@@ -52,16 +52,16 @@ def test_many_rows(ctx, qtype, m, n, k):
 @pytest.mark.parametrize("qtype", [o.Q4_0, o.Q4_1, o.Q5_1, o.Q8_0])
 @pytest.mark.parametrize("m", [40, 160])
 def test_llama_ffn_width_with_an_odd_count_of_superblocks(ctx, qtype, m):
-    """K = 11008 (the 7B LLaMA feed-forward width, 43 superblocks of 256): the block-of-32 kernel's two record buffers and
-    its split of K over workgroups at an odd count, on both of its row tiles."""
+    """K = 11008 (the 7B LLaMA feed-forward width, 43 superblocks of 256): an odd count of them over the
+    workgroups that K is split over, on tiles of 64 and of 128 rows."""
     _check(ctx, qtype, m, 96, 11008, seed=m + qtype)
 
 
 @pytest.mark.parametrize("qtype", [o.Q4_0, o.Q4_1, o.Q5_0, o.Q5_1, o.Q8_0])
 @pytest.mark.parametrize("m,n,k", [(1, 1, 256), (127, 31, 768), (129, 129, 256), (257, 255, 512), (300, 130, 2304), (513, 4, 1280)])
 def test_ragged_tiles_of_the_block_of_32_kernel(ctx, qtype, m, n, k):
-    """Row and column counts on both sides of its tile edges (128 and 256 rows, 128 columns, 32 and 64 per wave), one
-    superblock and an odd count of them, every type it takes."""
+    """Row and column counts on both sides of 128 and 256 rows and of 128 columns, one superblock and an odd count of them, every
+    type with blocks of 32."""
     _check(ctx, qtype, m, n, k, seed=m * 3 + n + k + qtype)
 
 
@@ -69,9 +69,8 @@ def test_ragged_tiles_of_the_block_of_32_kernel(ctx, qtype, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(1, 1, 256), (127, 31, 768), (129, 129, 256), (257, 255, 512), (300, 130, 2304), (513, 4, 1280),
                                    (260, 520, 4352)])
 def test_ragged_tiles_of_the_superblock_kernel(ctx, qtype, m, n, k):
-    """Row and column counts on both sides of its tile edges (128 and 256 rows, 256 columns, 64 per wave), one superblock,
-    odd counts of them (the minimum term takes them in pairs) and a K that is split over workgroups unevenly; Q5_K's fifth
-    bits ride along with the codes."""
+    """Row and column counts on both sides of 128 and 256 rows and of 128 columns, one superblock, odd counts of them and a K that is
+    split over workgroups unevenly."""
     _check(ctx, qtype, m, n, k, seed=m * 3 + n + k + qtype)
 
 

@@ -88,7 +88,7 @@ def test_every_pair_of_scale_and_minimum(ctx, qtype, size, rows, k):
 @pytest.mark.parametrize("rows,n", [(129, 257), (513, 640), (130, 16384), (130, 16385)])
 def test_blocks_in_many_tiles(ctx, qtype, rows, n):
     """More than one tile of rows, K in pieces or whole; as many tiles as compute units with bf16 rows (2 x 128) and
-    one column more, which the kernel with operands in LDS takes."""
+    one column more, which the large tiles take (several superblocks of those: test_gpu_gemm_rows_large.py)."""
     k = 256 if n > 10000 else 1536
     rng = np.random.default_rng(rows + n + qtype)
     packed = o.quantize(qtype, gen_weight(rng, n, k))
