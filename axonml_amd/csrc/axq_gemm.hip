@@ -732,7 +732,7 @@ int run_gemm(axq_ctx *ctx, const axq_weight *w, int m, const GemmPlan &p, float 
 } // namespace
 
 int axq_dev_gemm_bf16(axq_ctx *ctx, const axq_weight *w, const uint16_t *x, int m, float *y) {
-    if (axq_dev_rows_gemm_covers(ctx, w, m, true)) return axq_dev_rows_gemm(ctx, w, x, AXQ_ROWS_BF16, m, nullptr, 0.f, nullptr, nullptr, y);
+    if (axq_dev_rows_gemm_covers(w, m)) return axq_dev_rows_gemm(ctx, w, x, AXQ_ROWS_BF16, m, nullptr, 0.f, nullptr, nullptr, y);
     GemmPlan p;
     int rc;
     if ((rc = plan_gemm(ctx, w, m, &p))) return rc;
@@ -763,7 +763,7 @@ int axq_dev_gemm_f32_ex(axq_ctx *ctx, const axq_weight *w, const float *x, bool 
     int rc;
     if (swiglu && (norm_w || !axq_dev_gemm_f32_takes_swiglu(w)))
         return axq_fail(ctx, AXQ_ERR_INVALID_ARGUMENT, "axq_dev_gemm_f32_ex: SwiGLU rows need k %% 4 == 0, k <= 16384 and no norm");
-    if (axq_dev_rows_gemm_covers(ctx, w, m, false))
+    if (axq_dev_rows_gemm_covers(w, m))
         return axq_dev_rows_gemm(ctx, w, x, swiglu ? AXQ_ROWS_SWIGLU : AXQ_ROWS_F32, m, norm_w, eps, bias, resid, y, chain);
     if (chain) chain->ready_for = nullptr;
     if ((rc = plan_gemm(ctx, w, 2 * m, &p))) return rc;

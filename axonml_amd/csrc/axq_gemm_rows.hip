@@ -47,7 +47,7 @@
 // (K in parts, whose sums gemm_reduce_kernel adds together with what their additions round off: without that Q4_0, K = 4096 has 8.4 in
 // place of the 6.7 of nine bits, and 9.7 in place of 8.3.  Limbs in one accumulator: Q4_0 8.6 11.7 16.5; the matrix pipe cuts sums off where it adds small products to large ones.)
 //
-// Shape.  A workgroup of eight waves; a wave computes 32 MI x 32 NJ outputs.  Four waves lie side by side along N; the other
+// Shape (rows_gemm_kernel).  A workgroup of eight waves; a wave computes 32 MI x 32 outputs.  Four waves lie side by side along N; the other
 // factor of two is rows (WM = 2: 64 MI rows) or K (WM = 1: each four waves take half of the workgroup's superblocks, and the
 // two sums meet in LDS).  What the design turns on:
 //   - weights never pass through LDS as operands.  Their packed codes come into LDS as they are (global_load_lds, two K steps
@@ -400,10 +400,10 @@ struct Block32 {
 // one accumulator tile; 3: 32 rows in three tiles, the second and the third meet; 4: up to 40 rows, 32 of them in three tiles and the
 // limbs of the other eight in a fourth, two tiles to each of the groups along M (37 rows as two times 32, six tiles, and so, us: Q6_K
 // 28672 x 4096 104 84, Q4_K 66 55, Q4_K 4096 x 14336 45 41; f16 pairs, with ten bits less, 81, 51 and 37).
-template <class T, int MI, int WM, int NJ, int AT>
+template <class T, int MI, int WM, int AT>
 struct RowsTile {
     static constexpr int KG = 2 / WM, GW = 4 * WM, CW = GW / 2;     // groups along K, waves of one, waves that copy x (and codes)
-    static constexpr int M = AT == 2 ? 16 : AT == 3 ? 32 : AT == 4 ? 40 : 32 * MI * WM, N = 128 * NJ; // rows, columns
+    static constexpr int M = AT == 2 ? 16 : AT == 3 ? 32 : AT == 4 ? 40 : 32 * MI * WM, N = 128; // rows, columns
     static constexpr int XT = AT == 2 || AT == 3 ? AT : MI;         // tiles of x of a wave
     static constexpr int acc_of(int l) { return AT == 3 ? (l > 0 ? 1 : 0) : AT == 2 ? 0 : l; } // accumulator tile of a tile of x
     static constexpr bool first_of(int l) { return l == XT - 1 || acc_of(l) != acc_of(l + 1); }
@@ -412,14 +412,14 @@ struct RowsTile {
     static constexpr int DBYTES = N * (16 * T::SIDE16 + 4 * T::SIDE4);
     static constexpr int NA = 3;
     static constexpr int FIT = (160 * 1024 - KG * (NA * ABYTES + 2 * SBYTES + 2 * DBYTES)) / (KG * WBYTES), NW = FIT > 4 ? 4 : FIT;
-    static constexpr int MAIL = KG == 2 ? 8 * MI * NJ * 8 * 64 * 4 : 0; // the groups' exchange, which reuses the stages
+    static constexpr int MAIL = KG == 2 ? 8 * MI * 8 * 64 * 4 : 0; // the groups' exchange, which reuses the stages
     static constexpr int STAGES = KG * (NA * ABYTES + NW * WBYTES + 2 * SBYTES + 2 * DBYTES), LDS = STAGES > MAIL ? STAGES : MAIL;
     // a copying wave's requests: x of a step, sums of a superblock; codes of a unit, sides of a superblock (small ones some of them twice)
-    static constexpr int XL = 2 * XT, SL = T::MIN ? XT : 0, WT = 4 * NJ / CW, WL = WT * T::PAIRS;
-    static constexpr int D16 = (2 * NJ * T::SIDE16 + CW - 1) / CW, D4 = (2 * NJ * T::SIDE4 + CW - 1) / CW;
+    static constexpr int XL = 2 * XT, SL = T::MIN ? XT : 0, WT = 4 / CW, WL = WT * T::PAIRS;
+    static constexpr int D16 = (2 * T::SIDE16 + CW - 1) / CW, D4 = (2 * T::SIDE4 + CW - 1) / CW;
     static constexpr int FIRST = 7 > 2 * NW - 1 ? 7 : 2 * NW - 1;
     static_assert(AT == 1 || (AT == 4 ? MI == 2 && WM == 2 : MI == AT - 1 && WM == 1), "limbs");
-    static_assert(NW >= 2 && WT * CW == 4 * NJ && NA <= FIRST, "stages");
+    static_assert(NW >= 2 && WT * CW == 4 && NA <= FIRST, "stages");
     // Behind barrier b: x of step b + NA and, where b % 4 = 1, the sums of superblock (b + 3) / 4; codes of unit (b + 1) / 2 + NW - 1
     // where b is odd and the sides of superblock (b + 7) / 4 where b % 4 = 1.  In front of barrier g everything that is read
     // behind it must have come (x and codes of step g + 1, at a superblock's end sums and sides of the next): how many of the wave's
@@ -469,9 +469,9 @@ __device__ inline void store_result(const RowsArgs &a, int gm, int gn, float v, 
     }
 }
 
-template <class T, int MI, int WM, int NJ, int AT>
+template <class T, int MI, int WM, int AT>
 __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
-    using Tile = RowsTile<T, MI, WM, NJ, AT>;
+    using Tile = RowsTile<T, MI, WM, AT>;
     constexpr int KG = Tile::KG, HB = Tile::HB, ABYTES = Tile::ABYTES, WBYTES = Tile::WBYTES, SBYTES = Tile::SBYTES, DBYTES = Tile::DBYTES, NA = Tile::NA, NW = Tile::NW, XT = Tile::XT;
     extern __shared__ uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, li = lane & 31, hh = lane >> 5;
@@ -536,12 +536,12 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
         uint8_t *dst = dbase + (sb & 1) * DBYTES;
 #pragma unroll
         for (int q = 0; q < Tile::D16; q++) {
-            const int ii = (cw + q * Tile::CW) % (2 * NJ * T::SIDE16), c = ii / (2 * NJ), r0 = ii % (2 * NJ) * 64;
+            const int ii = (cw + q * Tile::CW) % (2 * T::SIDE16), c = ii / 2, r0 = ii % 2 * 64;
             copy(T::side_src(a, at, c) + (size_t)n0 * T::side_pitch(a, c) + row_of(r0 + lane) * T::side_pitch(a, c), dst + c * Tile::N * 16 + r0 * 16);
         }
 #pragma unroll
         for (int q = 0; q < Tile::D4; q++) {
-            const int r0 = (cw + q * Tile::CW) % (2 * NJ) * 64;
+            const int r0 = (cw + q * Tile::CW) % 2 * 64;
             __builtin_amdgcn_global_load_lds((gbl_void *)(T::side_src(a, at, T::SIDE16) + (size_t)n0 * T::side_pitch(a, T::SIDE16) +
                                                           row_of(r0 + lane) * T::side_pitch(a, T::SIDE16)),
                                              (lds_void *)(dst + T::SIDE16 * Tile::N * 16 + r0 * 4), 4, 0, 0);
@@ -550,42 +550,17 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
     };
 
     // ---- products
-    float16v acc[MI][NJ];
-#pragma unroll
-    for (int i = 0; i < MI; i++)
-#pragma unroll
-        for (int j = 0; j < NJ; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
-    float unit[NJ], inv[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; j++) unit[j] = 1.0f;
-    typename T::Side side[NJ], next_side[NJ];
-    typename T::Scales scales[NJ];
+    float unit, inv;
+    typename T::Side side, next_side;
+    typename T::Scales scales;
     uint32_t mask; // in a vector register: an instruction takes one scalar operand, and (w & mask) | base has its base there
     asm("v_mov_b32 %0, 0x00f000f0" : "=v"(mask));
-    auto read_sides = [&](int sb) {
-#pragma unroll
-        for (int j = 0; j < NJ; j++) T::template read_side<Tile::N>(dbase + (sb & 1) * DBYTES, (wn * NJ + j) * 32 + li, hh, sb0 + sb, next_side[j]);
-    };
-    auto new_side = [&] { // what the superblock in `side` asks for
-        if constexpr (!T::BLOCKS)
-#pragma unroll
-            for (int j = 0; j < NJ; j++) {
-                float shrink;
-                T::unit_of(side[j], unit[j], inv[j], shrink);
-                T::scales(side[j], shrink, hh, scales[j]);
-            }
-    };
-    const uint8_t *my_x = abase + wm * XT * 4096 + lane * 16, *my_codes = wbase + wn * NJ * 32 * HB;
+    auto read_sides = [&](int sb) { T::template read_side<Tile::N>(dbase + (sb & 1) * DBYTES, wn * 32 + li, hh, sb0 + sb, next_side); };
+    const uint8_t *my_x = abase + wm * XT * 4096 + lane * 16, *my_codes = wbase + wn * 32 * HB;
     int a_rd = 0, w_rd = 0; // stage of the step, of the unit that is read next
     auto read_x = [&](int t, half8 (&f)[XT]) {
 #pragma unroll
         for (int i = 0; i < XT; i++) f[i] = *reinterpret_cast<const half8 *>(my_x + a_rd + i * 4096 + t * 1024);
-    };
-    auto read_codes = [&](int j4, typename T::Raw (&raw)[NJ]) {
-#pragma unroll
-        for (int j = 0; j < NJ; j++) T::read_raw(my_codes + w_rd + j * 32 * HB, li, hh, j4, raw[j]);
     };
     // behind the barrier of step 4 sb + J: the stages of that step have been read by everybody, and what the next one reads is there
     auto meet = [&](int sb, auto step) {
@@ -604,29 +579,24 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
         a_rd = a_rd == (NA - 1) * ABYTES ? 0 : a_rd + ABYTES;
         if (J & 1) w_rd = w_rd == (NW - 1) * WBYTES ? 0 : w_rd + WBYTES;
     };
-    auto make = [&](const typename T::Raw (&raw)[NJ], int j4, int t, half8 (&f)[NJ][T::PRODUCTS]) {
-#pragma unroll
-        for (int j = 0; j < NJ; j++) T::make(raw[j], side[j], scales[j], mask, j4, t, hh, f[j]);
-    };
-    auto add_offsets = [&](int sb, auto tile_j, float16v (&to)[MI][NJ]) { // of a column tile
+    auto add_offsets = [&](int sb, float16v (&to)[MI]) {
         if constexpr (T::MIN && !T::BLOCKS) {
-            constexpr int j = decltype(tile_j)::value;
-            const int over = T::excess(side[j]);
+            const int over = T::excess(side);
             const bool any_over = __builtin_amdgcn_ballot_w64(over > 0) != 0; // a column's lanes all have its factor; exact, being a power of two
             auto times_pow2 = [&](int e) {
                 const float f = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
 #pragma unroll
                 for (int i = 0; i < MI; i++)
 #pragma unroll
-                    for (int q = 0; q < 16; q++) to[i][j][q] *= f;
+                    for (int q = 0; q < 16; q++) to[i][q] *= f;
             };
             if (any_over) times_pow2(-over);
-            const half8 o = T::offsets(side[j], hh, inv[j] * __builtin_bit_cast(float, (uint32_t)(127 - over) << 23));
+            const half8 o = T::offsets(side, hh, inv * __builtin_bit_cast(float, (uint32_t)(127 - over) << 23));
 #pragma unroll
             for (int i = 0; i < XT; i++) {
                 const uint8_t *x = sbase + (sb & 1) * SBYTES + (wm * XT + i) * 2048 + lane * 16;
-                to[Tile::acc_of(i)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x), o, to[Tile::acc_of(i)][j], 0, 0, 0);
-                to[Tile::acc_of(i)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x + 1024), o, to[Tile::acc_of(i)][j], 0, 0, 0);
+                to[Tile::acc_of(i)] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x), o, to[Tile::acc_of(i)], 0, 0, 0);
+                to[Tile::acc_of(i)] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x + 1024), o, to[Tile::acc_of(i)], 0, 0, 0);
             }
             if (any_over) times_pow2(over);
         }
@@ -650,51 +620,45 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
     // meet, request the next step's fragments, work on this step's
     constexpr int AHEAD = T::BLOCKS ? 1 : 2; // blocks: the next step's fragments take the place of the products' that are done
     half8 af[AHEAD][4][XT];
-    typename T::Raw raw[2][NJ];
+    typename T::Raw raw[2];
     // a step's products (a block's, with blocks) start from zero, their sums meet in the superblock's, and that joins the total:
     // few of the additions that round are of the total's size
-    float16v sum[MI][NJ], total[MI][NJ];
+    const float16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float16v part[MI], sum[MI], total[MI];
 #pragma unroll
-    for (int i = 0; i < MI; i++)
-#pragma unroll
-        for (int j = 0; j < NJ; j++) total[i][j] = sum[i][j] = acc[i][j];
+    for (int i = 0; i < MI; i++) total[i] = sum[i] = zero;
     auto each = [&](auto fn) {
 #pragma unroll
         for (int i = 0; i < MI; i++)
 #pragma unroll
-            for (int j = 0; j < NJ; j++)
-#pragma unroll
-                for (int q = 0; q < 16; q++) fn(i, j, q);
+            for (int q = 0; q < 16; q++) fn(i, q);
     };
-    const float16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     auto read_step = [&](int j4, bool first = false) {
-        read_codes(j4, raw[j4 & 1]);
+        T::read_raw(my_codes + w_rd, li, hh, j4, raw[j4 & 1]);
         if (!T::BLOCKS || first)
 #pragma unroll
             for (int t = 0; t < 4; t++) read_x(t, af[j4 % AHEAD][t]);
         asm volatile("" ::: "memory"); // requested here, not where they are used
     };
-    auto products = [&](auto at, auto t0, auto t1, float16v (&to)[MI][NJ], auto fresh) { // t0 .. t1 - 1 of a step, from zero where `fresh`
+    auto products = [&](auto at, auto t0, auto t1, auto fresh) { // t0 .. t1 - 1 of a step, from zero where `fresh`
         constexpr int J = decltype(at)::value, T0 = decltype(t0)::value, T1 = decltype(t1)::value;
-        half8 bf[T1 - T0][NJ][T::PRODUCTS];
+        half8 bf[T1 - T0][T::PRODUCTS];
         auto mul = [&](int t, int l) {
 #pragma unroll
             for (int pr = 0; pr < T::PRODUCTS; pr++)
-#pragma unroll
-                for (int j = 0; j < NJ; j++)
-                    to[Tile::acc_of(l)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                        af[J % AHEAD][t][l], bf[t - T0][j][pr], decltype(fresh)::value && Tile::first_of(l) && t == T0 && pr == 0 ? zero : to[Tile::acc_of(l)][j], 0, 0, 0);
+                part[Tile::acc_of(l)] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                    af[J % AHEAD][t][l], bf[t - T0][pr], decltype(fresh)::value && Tile::first_of(l) && t == T0 && pr == 0 ? zero : part[Tile::acc_of(l)], 0, 0, 0);
         };
         if constexpr (XT == MI) { // every tile of x has an accumulator of its own
 #pragma unroll
             for (int t = T0; t < T1; t++) {
-                make(raw[J & 1], J, t, bf[t - T0]);
+                T::make(raw[J & 1], side, scales, mask, J, t, hh, bf[t - T0]);
 #pragma unroll
                 for (int l = XT - 1; l >= 0; l--) mul(t, l);
             }
         } else {
 #pragma unroll
-            for (int t = T0; t < T1; t++) make(raw[J & 1], J, t, bf[t - T0]);
+            for (int t = T0; t < T1; t++) T::make(raw[J & 1], side, scales, mask, J, t, hh, bf[t - T0]);
 #pragma unroll
             for (int l = XT - 1; l >= 0; l--) // the third limbs first
 #pragma unroll
@@ -702,75 +666,64 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
         }
     };
     using S4 = std::integral_constant<int, 4>;
-    float16v part[MI][NJ];
     auto step = [&](int sb, auto at) {
         constexpr int J = decltype(at)::value;
         // the last step's sums are in `sum` here: left to itself the compiler keeps the blocks' sums of a superblock apart
 #pragma unroll
-        for (int i = 0; i < MI; i++)
-#pragma unroll
-            for (int j = 0; j < NJ; j++) {
-                if (J == 0) asm volatile("" : "+v"(total[i][j]));
-                else asm volatile("" : "+v"(sum[i][j]));
-            }
+        for (int i = 0; i < MI; i++) {
+            if (J == 0) asm volatile("" : "+v"(total[i]));
+            else asm volatile("" : "+v"(sum[i]));
+        }
         meet(sb, at);
         read_step((J + 1) & 3);
         if (J == 3) read_sides(sb + 1); // looked at behind the next barrier
         if (J == 0) {
-#pragma unroll
-            for (int j = 0; j < NJ; j++) side[j] = next_side[j];
-            new_side();
+            side = next_side;
+            if constexpr (!T::BLOCKS) {
+                float shrink;
+                T::unit_of(side, unit, inv, shrink);
+                T::scales(side, shrink, hh, scales);
+            }
         }
         if constexpr (T::BLOCKS) {
             auto block = [&](auto half) {
                 constexpr int B = decltype(half)::value;
-                float d[NJ];
-#pragma unroll
-                for (int j = 0; j < NJ; j++) d[j] = T::scale(side[j], 2 * J + B);
-                products(at, std::integral_constant<int, 2 * B>{}, std::integral_constant<int, 2 * B + 2>{}, part, std::true_type{});
+                const float d = T::scale(side, 2 * J + B);
+                products(at, std::integral_constant<int, 2 * B>{}, std::integral_constant<int, 2 * B + 2>{}, std::true_type{});
                 asm volatile("" ::: "memory");
                 read_x(2 * B, af[0][2 * B]);
                 read_x(2 * B + 1, af[0][2 * B + 1]);
                 asm volatile("" ::: "memory");
-                each([&](int i, int j, int q) { sum[i][j][q] = J == 0 && B == 0 ? part[i][j][q] * d[j] : fmaf(part[i][j][q], d[j], sum[i][j][q]); });
+                each([&](int i, int q) { sum[i][q] = J == 0 && B == 0 ? part[i][q] * d : fmaf(part[i][q], d, sum[i][q]); });
             };
             block(S0{});
             block(S1{});
             if constexpr (T::MIN && J == 1) { // the superblock's offsets
-                float f[NJ];
+                float f;
+                const half8 o = T::offsets(side, hh, f);
 #pragma unroll
-                for (int j = 0; j < NJ; j++) {
-                    const half8 o = T::offsets(side[j], hh, f[j]);
-#pragma unroll
-                    for (int i = XT - 1; i >= 0; i--) {
-                        constexpr auto acc_of = Tile::acc_of;
-                        const uint8_t *x = sbase + (sb & 1) * SBYTES + (wm * XT + i) * 2048 + lane * 16;
-                        part[acc_of(i)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x), o, Tile::first_of(i) ? zero : part[acc_of(i)][j], 0, 0, 0);
-                        part[acc_of(i)][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x + 1024), o, part[acc_of(i)][j], 0, 0, 0);
-                    }
+                for (int i = XT - 1; i >= 0; i--) {
+                    constexpr auto acc_of = Tile::acc_of;
+                    const uint8_t *x = sbase + (sb & 1) * SBYTES + (wm * XT + i) * 2048 + lane * 16;
+                    part[acc_of(i)] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x), o, Tile::first_of(i) ? zero : part[acc_of(i)], 0, 0, 0);
+                    part[acc_of(i)] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8 *>(x + 1024), o, part[acc_of(i)], 0, 0, 0);
                 }
-                each([&](int i, int j, int q) { sum[i][j][q] = fmaf(part[i][j][q], f[j], sum[i][j][q]); });
+                each([&](int i, int q) { sum[i][q] = fmaf(part[i][q], f, sum[i][q]); });
             }
-            if (J == 3) each([&](int i, int j, int q) { total[i][j][q] += sum[i][j][q]; });
+            if (J == 3) each([&](int i, int q) { total[i][q] += sum[i][q]; });
         } else {
             // f32 pairs and bf16 rows: two steps to a sum, half the additions (Q4_K 28672 x 4096, 64 f32 rows 56.4 -> 53.9 us)
             constexpr int RUN = AT == 1 ? 2 : 1;
-            products(at, S0{}, S4{}, part, std::integral_constant<bool, J % RUN == 0>{});
-            if constexpr (T::MIN && J >= 1 && J <= NJ) add_offsets(sb, std::integral_constant<int, J - 1>{}, part);
-            if (J == RUN - 1) each([&](int i, int j, int q) { sum[i][j][q] = part[i][j][q]; });
-            else if (J % RUN == RUN - 1) each([&](int i, int j, int q) { sum[i][j][q] += part[i][j][q]; });
-            if (J == 3) each([&](int i, int j, int q) { total[i][j][q] = fmaf(sum[i][j][q], unit[j], total[i][j][q]); });
+            products(at, S0{}, S4{}, std::integral_constant<bool, J % RUN == 0>{});
+            if constexpr (T::MIN && J == 1) add_offsets(sb, part);
+            if (J == RUN - 1) each([&](int i, int q) { sum[i][q] = part[i][q]; });
+            else if (J % RUN == RUN - 1) each([&](int i, int q) { sum[i][q] += part[i][q]; });
+            if (J == 3) each([&](int i, int q) { total[i][q] = fmaf(sum[i][q], unit, total[i][q]); });
         }
     };
     read_step(0, true);
     for (int sb = 0; sb < mine; sb++) {
         step(sb, S0{}); step(sb, S1{}); step(sb, S2{}); step(sb, S3{});
-    }
-#pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        unit[j] = 1.0f;
-#pragma unroll
-        for (int i = 0; i < MI; i++) acc[i][j] = total[i][j];
     }
     for (int sb = mine; sb < loops; sb++) { // the other group has one more
         meet(sb, S0{}); meet(sb, S1{}); meet(sb, S2{}); meet(sb, S3{});
@@ -782,63 +735,59 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
     constexpr float BELOW = 1.0f / (1 << (LB + 2));
     if constexpr (AT == 4) { // the third limbs of 32 rows come from the other group; the eight rows' limbs lie eight rows below each other
         barrier();
-        float *mail = reinterpret_cast<float *>(lds) + wn * (NJ * 16 * 64) + lane;
-        static_assert(4 * NJ * 16 * 64 * 4 <= Tile::LDS, "mail");
+        float *mail = reinterpret_cast<float *>(lds) + wn * (16 * 64) + lane;
+        static_assert(4 * 16 * 64 * 4 <= Tile::LDS, "mail");
         if (wm == 1)
 #pragma unroll
-            for (int j = 0; j < NJ; j++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) mail[(j * 16 + r) * 64] = acc[0][j][r];
+            for (int r = 0; r < 16; r++) mail[r * 64] = total[0][r];
         __syncthreads();
+        if (wm == 1) {
 #pragma unroll
-        for (int j = 0; j < NJ; j++)
-            if (wm == 1) {
+            for (int r = 0; r < 4; r++) total[0][r] = fmaf(total[1][r + 4] + total[1][r + 8], BELOW, total[1][r]);
+        } else {
 #pragma unroll
-                for (int r = 0; r < 4; r++) acc[0][j][r] = fmaf(acc[1][j][r + 4] + acc[1][j][r + 8], BELOW, acc[1][j][r]);
-            } else {
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[0][j][r] = fmaf(acc[1][j][r] + mail[(j * 16 + r) * 64], BELOW, acc[0][j][r]);
-            }
+            for (int r = 0; r < 16; r++) total[0][r] = fmaf(total[1][r] + mail[r * 64], BELOW, total[0][r]);
+        }
     } else if constexpr (AT > 1)
 #pragma unroll
-        for (int j = 0; j < NJ; j++)
-#pragma unroll
-            for (int r = 0; r < (AT == 2 ? 8 : 16); r++) acc[0][j][r] = fmaf(AT == 2 ? acc[0][j][r + 8 & 15] : acc[MI - 1][j][r], BELOW, acc[0][j][r]);
+        for (int r = 0; r < (AT == 2 ? 8 : 16); r++) total[0][r] = fmaf(AT == 2 ? total[0][r + 8 & 15] : total[MI - 1][r], BELOW, total[0][r]);
     constexpr int MR = AT > 1 ? 1 : MI;
-    auto store = [&](int i, int j, int r, float v, float v2) {
-        store_result(a, (AT > 1 ? mt0 / AT + wm : mt0 + wm * MI + i) * 32 + 8 * (r >> 2) + 4 * hh + (r & 3), n0 + (wn * NJ + j) * 32 + li, v, v2);
+    auto store = [&](int i, int r, float v, float v2) {
+        store_result(a, (AT > 1 ? mt0 / AT + wm : mt0 + wm * MI + i) * 32 + 8 * (r >> 2) + 4 * hh + (r & 3), n0 + wn * 32 + li, v, v2);
     };
     const int step_r = a.pair ? 2 : 1;
     if constexpr (KG == 2) { // a group finishes half of the registers and hands the other half over
         barrier();
-        float *mail = reinterpret_cast<float *>(lds) + (kg * 4 + wn) * (MR * NJ * 8 * 64) + lane;
+        float *mail = reinterpret_cast<float *>(lds) + (kg * 4 + wn) * (MR * 8 * 64) + lane;
 #pragma unroll
         for (int i = 0; i < MR; i++)
 #pragma unroll
-            for (int j = 0; j < NJ; j++)
-#pragma unroll
-                for (int r = 0; r < 8; r++) mail[((i * NJ + j) * 8 + r) * 64] = (kg ? acc[i][j][r] : acc[i][j][r + 8]) * unit[j];
-        __syncthreads();
-        const float *got = reinterpret_cast<const float *>(lds) + ((1 - kg) * 4 + wn) * (MR * NJ * 8 * 64) + lane;
-#pragma unroll
-        for (int i = 0; i < MR; i++)
-#pragma unroll
-            for (int j = 0; j < NJ; j++) {
-                float v[8];
-#pragma unroll
-                for (int r = 0; r < 8; r++) v[r] = (kg ? acc[i][j][r + 8] : acc[i][j][r]) * unit[j] + got[((i * NJ + j) * 8 + r) * 64];
-#pragma unroll
-                for (int r = 0; r < 8; r++)
-                    if (r % step_r == 0) store(i, j, kg * 8 + r, v[r], v[r | 1]);
+            for (int r = 0; r < 8; r++) {
+                float lower = total[i][r], upper = total[i][r + 8];
+                asm("" : "+v"(lower), "+v"(upper)); // a choice between two registers, not of a register's number
+                mail[(i * 8 + r) * 64] = kg ? lower : upper;
             }
+        __syncthreads();
+        const float *got = reinterpret_cast<const float *>(lds) + ((1 - kg) * 4 + wn) * (MR * 8 * 64) + lane;
+#pragma unroll
+        for (int i = 0; i < MR; i++) {
+            float v[8];
+#pragma unroll
+            for (int r = 0; r < 8; r++) {
+                float lower = total[i][r], upper = total[i][r + 8];
+                asm("" : "+v"(lower), "+v"(upper));
+                v[r] = (kg ? upper : lower) + got[(i * 8 + r) * 64];
+            }
+#pragma unroll
+            for (int r = 0; r < 8; r++)
+                if (r % step_r == 0) store(i, kg * 8 + r, v[r], v[r | 1]);
+        }
     } else {
 #pragma unroll
         for (int i = 0; i < MR; i++)
 #pragma unroll
-            for (int j = 0; j < NJ; j++)
-#pragma unroll
-                for (int r = 0; r < 16; r++)
-                    if (r % step_r == 0 && (AT != 4 || r < 4 || wm == 0)) store(i, j, r, acc[i][j][r] * unit[j], acc[i][j][r | 1] * unit[j]);
+            for (int r = 0; r < 16; r++)
+                if (r % step_r == 0 && (AT != 4 || r < 4 || wm == 0)) store(i, r, total[i][r], total[i][r | 1]);
     }
 }
 
@@ -1783,13 +1732,13 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
     if ((NC <= 1 || blockIdx.y == 0) && tid < (LIMBS ? 1 : PARTS)) rowscale[(LIMBS ? row : r0) + tid] = 1.0f / f;
 }
 
-template <class T, int MI, int WM, int NJ, int AT>
+template <class T, int MI, int WM, int AT>
 int launch_tile(axq_ctx *ctx, const RowsArgs &a, int splits) {
-    using Tile = RowsTile<T, MI, WM, NJ, AT>;
+    using Tile = RowsTile<T, MI, WM, AT>;
     static std::atomic<uint64_t> lds_allowed{0};
-    if (int rc = axq_allow_lds(ctx, reinterpret_cast<const void *>(rows_gemm_kernel<T, MI, WM, NJ, AT>), lds_allowed, Tile::LDS)) return rc;
+    if (int rc = axq_allow_lds(ctx, reinterpret_cast<const void *>(rows_gemm_kernel<T, MI, WM, AT>), lds_allowed, Tile::LDS)) return rc;
     const unsigned tiles = (unsigned)(((a.n + Tile::N - 1) / Tile::N) * ((a.m + Tile::M - 1) / Tile::M));
-    rows_gemm_kernel<T, MI, WM, NJ, AT><<<dim3(tiles, (unsigned)splits), 512, Tile::LDS, ctx->stream>>>(a);
+    rows_gemm_kernel<T, MI, WM, AT><<<dim3(tiles, (unsigned)splits), 512, Tile::LDS, ctx->stream>>>(a);
     AXQ_LAUNCH_CHECK(ctx, "rows_gemm_kernel");
     return AXQ_OK;
 }
@@ -1900,9 +1849,9 @@ RowsPlan rows_plan(const axq_ctx *ctx, const axq_weight *w, int in, int rows) {
 template <class T>
 int launch_rows(axq_ctx *ctx, const RowsArgs &a, const RowsPlan &p) {
     if (p.limbs) {
-        if (a.m > 32) return launch_tile<T, 2, 2, 1, 4>(ctx, a, p.splits);
-        if (a.m > 16) return launch_tile<T, 2, 1, 1, 3>(ctx, a, p.splits);
-        return launch_tile<T, 1, 1, 1, 2>(ctx, a, p.splits);
+        if (a.m > 32) return launch_tile<T, 2, 2, 4>(ctx, a, p.splits);
+        if (a.m > 16) return launch_tile<T, 2, 1, 3>(ctx, a, p.splits);
+        return launch_tile<T, 1, 1, 2>(ctx, a, p.splits);
     }
     if constexpr (!T::BLOCKS) {
         if (p.wide) return launch_wide<T>(ctx, a, p.splits);
@@ -1910,15 +1859,15 @@ int launch_rows(axq_ctx *ctx, const RowsArgs &a, const RowsPlan &p) {
     }
     if constexpr (T::BLOCKS)
         if (p.wide) return launch_blocks<T>(ctx, a, p.splits);
-    if (a.m > 64) return launch_tile<T, 2, 2, 1, 1>(ctx, a, p.splits);
-    if (a.m > 32) return launch_tile<T, 2, 1, 1, 1>(ctx, a, p.splits);
-    return launch_tile<T, 1, 1, 1, 1>(ctx, a, p.splits);
+    if (a.m > 64) return launch_tile<T, 2, 2, 1>(ctx, a, p.splits);
+    if (a.m > 32) return launch_tile<T, 2, 1, 1>(ctx, a, p.splits);
+    return launch_tile<T, 1, 1, 1>(ctx, a, p.splits);
 }
 
 } // namespace
 
 // Packed types at any number of rows, K a multiple of 256.
-bool axq_dev_rows_gemm_covers(const axq_ctx *ctx, const axq_weight *w, int rows, bool bf16) {
+bool axq_dev_rows_gemm_covers(const axq_weight *w, int rows) {
     if (w->k % 256 != 0 || w->k > INT32_MAX || w->n_rows > INT32_MAX || rows < 1) return false;
     switch (w->type) {
     case AXQ_Q4_K: case AXQ_Q5_K: case AXQ_Q6_K: case AXQ_Q4_0: case AXQ_Q4_1: case AXQ_Q5_0: case AXQ_Q5_1: case AXQ_Q8_0: return true;
@@ -1939,7 +1888,7 @@ bool axq_dev_rows_gemm_covers(const axq_ctx *ctx, const axq_weight *w, int rows,
 //   6144x4096  1.08 1.04   1.09 1.05   1.06 1.00   1.01 0.97   1.02 0.97   0.96 0.92   (three quarters of the compute units)
 //   9216x4096  1.34 1.32   1.28 1.27   1.21 1.14   1.16 1.13   1.14 1.11   1.15 1.12
 bool axq_dev_rows_gemm_pays(const axq_ctx *ctx, const axq_weight *w, int rows) {
-    if (rows < AXQ_ROWS_GEMM_MIN || !axq_dev_rows_gemm_covers(ctx, w, rows, false)) return false;
+    if (rows < AXQ_ROWS_GEMM_MIN || !axq_dev_rows_gemm_covers(w, rows)) return false;
     if (rows > 16) return true;
     const bool slow_gemv = w->type == AXQ_Q8_0 || w->type == AXQ_Q6_K || w->type == AXQ_Q4_0;
     if (w->k > 8192) return slow_gemv && w->n_rows >= 4096;
@@ -1977,7 +1926,7 @@ static void launch_prep_sums(hipStream_t st, const PartSums &ps, const float *no
 }
 
 // `chain`: the weight that takes y as f32 rows next, RMS-normalised where chain->norm_w is given.  Where K is split, its operands are made with the
-// reduction, in one pass over the sums (64 rows of 4096, eight parts: 10.2 us in two launches, 6.6 in one), and chain->ready says where: the
+// reduction, in one pass over the sums (64 rows of 4096, eight parts: 10.2 us in two launches, 6.8 in one), and chain->ready_at says where: the
 // next call, of that weight and as many rows and with nothing in between, takes them.
 int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, int rows, const float *norm_w, float eps, const float *bias,
                       const float *resid, float *y, axq_rows_chain *chain) {
@@ -1992,7 +1941,7 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
     size_t next_at = 0;
     RowsPlan np;
     RowsRoom nroom = {};
-    if (next && splits > 1 && !bias && next->k == n && next->k <= 16384 && axq_dev_rows_gemm_covers(ctx, next, rows, false)) {
+    if (next && splits > 1 && !bias && next->k == n && next->k <= 16384 && axq_dev_rows_gemm_covers(next, rows)) {
         np = rows_plan(ctx, next, AXQ_ROWS_F32, rows);
         nroom = rows_room(np, rows, next);
         next_at = room.end(at);

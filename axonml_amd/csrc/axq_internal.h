@@ -164,7 +164,7 @@ int axq_dev_attn_rows_mfma(axq_ctx *ctx, const float *qkv, int qkv_rows, const f
                            int max_pos, int window, float *att);
 // gemm_rows.hip: rows times a packed weight, K a multiple of 256
 enum { AXQ_ROWS_F32 = 0, AXQ_ROWS_SWIGLU = 1, AXQ_ROWS_BF16 = 2 };
-bool axq_dev_rows_gemm_covers(const axq_ctx *ctx, const axq_weight *w, int rows, bool bf16);
+bool axq_dev_rows_gemm_covers(const axq_weight *w, int rows);
 // f32 rows below it go in as three limbs, 33 bits below the largest of every 32 elements (the small-batch GEMV, which took them before,
 // has 28), from it on as pairs of f16
 #define AXQ_ROWS_PAIRS_MIN 40
