@@ -36,14 +36,16 @@
 //   blocks of 32 w = d (q - C) + (m + C d): q - C is the operand, a block's sum starts from zero and joins its superblock's times d; the
 //                offsets of eight blocks, as an f16 pair under a common power of two, meet the blocks' sums of x.  C is the middle
 //                code, or, with a minimum, the code nearest to a weight of zero (see Block32::centre).
-// Centred codes because sums over uncentred ones cancel for rows with a mean.  Accumulation is f32 throughout: products of a step (limbs, blocks; else of two) from
-// zero, steps into a superblock's sum, superblocks into the total.  Root mean square error against 64 bits over that of the result,
-// normal x, K = 1024 / 4096 / 14336, in 1e-8, before and now:
-//   rows       up to 39                       40 and more, f32
-//   Q4_0       7.2 8.6 10.3   5.0 5.0 5.5     8.5 10.6 15.5   7.9 8.3 9.5
-//   Q5_1       9.4 10.5 12.9  6.4 6.3 6.8     9.1 11.2 16.4   8.1 8.5 9.6
-//   Q4_K       9.4 10.5 12.8  7.4 7.3 7.5     13.0 17.7 31.4  10.8 11.0 11.7
-//   Q6_K       8.9 10.0 12.4  5.3 5.2 5.5     15.8 21.6 38.8  12.0 12.1 12.7
+// Centred codes because sums over uncentred ones cancel for rows with a mean.  Accumulation is f32 throughout.  rows_gemm_kernel: products of a step (limbs, blocks;
+// else of two) from zero, steps into a superblock's sum, superblocks into the total.  rows_apart_kernel: two steps from zero, into the total of one of two halves.
+// Large tiles have registers for the total only, which a block's sum (rows_blocks_kernel) or every product (rows_wide_kernel) joins.
+// Root mean square error against 64 bits over that of the result, normal x, K = 1024 / 4096 / 14336, in 1e-8, before and now:
+//   rows       up to 39                       40 and more, f32                     f32, large tiles (before the same but for Q5_1)
+//   Q4_0       7.2 8.6 10.3   5.0 5.0 5.5     8.5 10.6 15.5   7.9 8.3 9.5          11.5 21.0 38.3
+//   Q5_1       9.4 10.5 12.9  6.4 6.3 6.8     9.1 11.2 16.4   8.1 8.5 9.6          12.4 22.4 40.7   12.1 22.2 40.7
+//   Q4_K       9.4 10.5 12.8  7.4 7.3 7.5     13.0 17.7 31.4  10.8 11.0 11.7       16.4 31.4 58.6
+//   Q6_K       8.9 10.0 12.4  5.3 5.2 5.5     15.8 21.6 38.8  12.0 12.1 12.7       20.6 40.8 76.7
+// (64 f32 rows times 14336 x 4096 in rows_apart_kernel, Q4_K and Q6_K: 11.9 and 12.9, as in rows_gemm_kernel.)
 // (K in parts, whose sums gemm_reduce_kernel adds together with what their additions round off: without that Q4_0, K = 4096 has 8.4 in
 // place of the 6.7 of nine bits, and 9.7 in place of 8.3.  Limbs in one accumulator: Q4_0 8.6 11.7 16.5; the matrix pipe cuts sums off where it adds small products to large ones.)
 //
@@ -1774,7 +1776,7 @@ int launch_apart(axq_ctx *ctx, const RowsArgs &a, int splits) {
 }
 
 // Up to 64 rows of more than 4096 elements a workgroup for every 4096 of each: as many as there are rows leave most of the chip idle, and what a
-// row costs most is its conversion (21 rows of 11008, limbs: 8.6 us with one, 6.5 so; 64 rows of 14336, SwiGLU: 9.7, 7.2).
+// row costs most is its conversion (21 rows of 11008, limbs: 8.6 us with one, 6.5 so; 64 rows of 14336, SwiGLU: 9.7, 8.1).
 template <int IN, bool LIMBS>
 void launch_prep(hipStream_t st, const void *x, const float *norm_w, float eps, int rows, int k, _Float16 *xa, _Float16 *xs, float *rs) {
     const int parts = rows <= 64 ? (k + 4095) / 4096 : 1;
