@@ -158,3 +158,24 @@ __device__ inline void axq_store_packed(const float (&v)[8], int t, int b, int b
         xsg[(size_t)nblk * 8 + slot] = sum;
     }
 }
+
+// The same for a row that the batch does not have: zeros, without the work on values.
+template <bool EVEN_ODD>
+__device__ inline void axq_store_packed_zeros(int t, int b, int nblk, uint8_t *xa, float *xsg) {
+    const int blk = t >> 2, e0 = (t & 3) * 8;
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+        const int row = 4 * b + l;
+        if (EVEN_ODD) {
+            *reinterpret_cast<uint32_t *>(xa + ((size_t)(blk * 2 + 0) * 32 + row) * 16 + (e0 >> 1)) = 0;
+            *reinterpret_cast<uint32_t *>(xa + ((size_t)(blk * 2 + 1) * 32 + row) * 16 + (e0 >> 1)) = 0;
+        } else {
+            *reinterpret_cast<uint2 *>(xa + ((size_t)(blk * 2 + (e0 >> 4)) * 32 + row) * 16 + (e0 & 15)) = make_uint2(0, 0);
+        }
+    }
+    if ((t & 3) == 0) {
+        const int slot = (blk * 2 + (b & 1)) * 4 + (b >> 1);
+        xsg[slot] = 0.f;
+        xsg[(size_t)nblk * 8 + slot] = 0.f;
+    }
+}
