@@ -397,13 +397,13 @@ __global__ void __launch_bounds__(512) gemm_kernel(GemmArgs a) {
                 const int gm = m0 + wm + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                 if (gm < a.m && gn < a.n) {
                     if (!a.pair) {
-                        if (a.ypart) a.ypart[((size_t)blockIdx.y * a.m + gm) * a.n + gn] = acc[i][j][r];
+                        if (a.ypart) a.ypart[((size_t)blockIdx.y * a.m + gm) * axq_part_pitch(a.n) + gn] = acc[i][j][r];
                         else a.y[(size_t)gm * a.n + gn] = acc[i][j][r] * (a.rowscale[gm] * (1.0f / T::WS));
                     } else if ((r & 1) == 0) { // gm is even: this register and the next hold the two parts of row gm / 2
                         const size_t t = (size_t)(gm >> 1);
                         const float v = acc[i][j][r] + acc[i][j][r + 1];
                         if (a.ypart) {
-                            a.ypart[((size_t)blockIdx.y * (a.m >> 1) + t) * a.n + gn] = v;
+                            a.ypart[((size_t)blockIdx.y * (a.m >> 1) + t) * axq_part_pitch(a.n) + gn] = v;
                         } else {
                             float out = v * (a.rowscale[gm] * (1.0f / T::WS));
                             if (a.bias) out += a.bias[gn];
@@ -456,7 +456,7 @@ template <int S>
 __global__ void __launch_bounds__(256) gemm_reduce_kernel(const float *ypart, const float *rowscale, int rows, int n, int parts,
                                                           float inv_ws, int row_mul, const float *bias, const float *resid, float *y) {
     const int splits = S > 0 ? S : parts;
-    const size_t i4 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, total4 = (size_t)rows * n / 4;
+    const size_t i4 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, quads = (size_t)axq_part_pitch(n) / 4, total4 = (size_t)rows * quads;
     if (i4 >= total4) return;
     const float4 first = reinterpret_cast<const float4 *>(ypart)[i4];
     float acc[4] = {first.x, first.y, first.z, first.w}, lost[4] = {0.f, 0.f, 0.f, 0.f}; // the sum, and what its additions rounded off (two-sum)
@@ -465,7 +465,7 @@ __global__ void __launch_bounds__(256) gemm_reduce_kernel(const float *ypart, co
         float4 v4[AHEAD];
 #pragma unroll
         for (int i = 0; i < AHEAD; i++)
-            if (s0 + i < splits) v4[i] = reinterpret_cast<const float4 *>(ypart + (size_t)(s0 + i) * rows * n)[i4];
+            if (s0 + i < splits) v4[i] = reinterpret_cast<const float4 *>(ypart)[(size_t)(s0 + i) * total4 + i4];
 #pragma unroll
         for (int i = 0; i < AHEAD; i++) {
             if (s0 + i >= splits) break;
@@ -480,17 +480,17 @@ __global__ void __launch_bounds__(256) gemm_reduce_kernel(const float *ypart, co
     }
 #pragma unroll
     for (int c = 0; c < 4; c++) acc[c] = lost[c] == lost[c] ? acc[c] + lost[c] : acc[c]; // not a number beside an infinite sum
-    const size_t row = (i4 * 4) / (size_t)n, col = (i4 * 4) % (size_t)n; // n is a multiple of 4: the four share a row
+    typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+    const size_t row = i4 / quads, col = i4 % quads * 4, at = row * n + col;
     const float f = rowscale[row * row_mul] * inv_ws;
-    float4 out = make_float4(acc[0] * f, acc[1] * f, acc[2] * f, acc[3] * f);
-    if (bias) {
-        out.x += bias[col]; out.y += bias[col + 1]; out.z += bias[col + 2]; out.w += bias[col + 3];
+    if (col + 4 <= (size_t)n) {
+        float4u out = {acc[0] * f, acc[1] * f, acc[2] * f, acc[3] * f};
+        if (bias) out += *reinterpret_cast<const float4u *>(bias + col);
+        if (resid) out += *reinterpret_cast<const float4u *>(resid + at);
+        *reinterpret_cast<float4u *>(y + at) = out;
+    } else {
+        for (int c = 0; c < n % 4; c++) y[at + c] = (acc[c] * f + (bias ? bias[col + c] : 0.f)) + (resid ? resid[at + c] : 0.f);
     }
-    if (resid) {
-        const float4 r = reinterpret_cast<const float4 *>(resid)[i4];
-        out.x += r.x; out.y += r.y; out.z += r.z; out.w += r.w;
-    }
-    reinterpret_cast<float4 *>(y)[i4] = out;
 }
 
 template <class T>
@@ -654,7 +654,7 @@ int axq_gemm_reserve(axq_ctx *ctx, size_t need) {
 // y from the partial sums of a split K, on the context's stream (see gemm_reduce_kernel).
 int axq_gemm_reduce(axq_ctx *ctx, const float *ypart, const float *rowscale, int rows, int n, int splits, float inv_ws, int row_mul,
                     const float *bias, const float *resid, float *y) {
-    const size_t total4 = (size_t)rows * n / 4;
+    const size_t total4 = (size_t)rows * (axq_part_pitch(n) / 4);
     decltype(&gemm_reduce_kernel<0>) kernel;
     switch (splits) {
     case 2: kernel = gemm_reduce_kernel<2>; break;
@@ -695,13 +695,19 @@ int plan_gemm(axq_ctx *ctx, const axq_weight *w, int m, GemmPlan *p) {
     int splits = (int)(cus / tiles);
     splits = splits > 8 ? 8 : splits;
     if (splits > ksteps / 4) splits = ksteps / 4;
-    if (splits < 2 || w->n_rows % 4 != 0) splits = 1;
+    if (splits < 2) splits = 1;
     p->steps_per_split = (ksteps + splits - 1) / splits;
     p->splits = (ksteps + p->steps_per_split - 1) / p->steps_per_split;
     p->xh_bytes = axq_align_up((size_t)m * (size_t)w->k * 2, 256);
     p->rs_bytes = axq_align_up((size_t)m * 4, 256);
-    p->part_bytes = axq_align_up(p->splits > 1 ? (size_t)p->splits * m * (size_t)w->n_rows * 4 : 0, 256);
-    return axq_gemm_reserve(ctx, p->xh_bytes + p->rs_bytes + p->part_bytes);
+    p->part_bytes = axq_align_up(p->splits > 1 ? (size_t)p->splits * m * (size_t)axq_part_pitch((int)w->n_rows) * 4 : 0, 256);
+    const int rc = axq_gemm_reserve(ctx, p->xh_bytes + p->rs_bytes + p->part_bytes);
+    if (rc == AXQ_OK || p->splits == 1 || w->n_rows % 4 == 0) return rc;
+    (void)hipGetLastError(); // no room for parts of K: whole, as calls of so many columns always can
+    p->splits = 1;
+    p->steps_per_split = ksteps;
+    p->part_bytes = 0;
+    return axq_gemm_reserve(ctx, p->xh_bytes + p->rs_bytes);
 }
 
 // The GEMM proper over activations that already sit in scratch as scaled f16 rows.

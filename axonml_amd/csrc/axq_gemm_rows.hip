@@ -84,7 +84,7 @@ struct RowsArgs {
     const _Float16 *xa;    // x in operand order: [tile of 32 rows][step of 64 k][t = 0..3][lane][8]
     const _Float16 *xs;    // its sub-block sums: [tile][superblock][leading halves, remainders][lane][8]: sub-blocks 4 (lane / 32) .., twice
     const float *rowscale; // [m]
-    float *y, *ypart;      // ypart: [splits][rows][n] unscaled sums (NULL: one workgroup covers all of K)
+    float *y, *ypart;      // ypart: [splits][rows][part_pitch] unscaled sums (NULL: one workgroup covers all of K)
     int m, n, k;           // m rows of xa; with `pair` rows 2t and 2t + 1 are the parts of row t, and y has m / 2 rows
     int sb_per_split, pair;
     const float *bias, *resid;
@@ -462,7 +462,7 @@ __device__ inline void store_result(const RowsArgs &a, int gm, int gn, float v, 
     const size_t row = (size_t)(a.pair ? gm >> 1 : gm), rows = (size_t)(a.pair ? a.m >> 1 : a.m);
     if (a.pair) v += v2;
     if (a.ypart) {
-        a.ypart[((size_t)blockIdx.y * rows + row) * a.n + gn] = v;
+        a.ypart[((size_t)blockIdx.y * rows + row) * axq_part_pitch(a.n) + gn] = v;
     } else {
         float out = v * a.rowscale[gm];
         if (a.bias) out += a.bias[gn];
@@ -799,10 +799,12 @@ __global__ void __launch_bounds__(512, 2) rows_gemm_kernel(RowsArgs a) {
 template <int MI, int NJ>
 __device__ inline void write_rows(const RowsArgs &a, const float16v (&acc)[MI][NJ], float *patch, int gm0, int n0, int lane) {
     typedef float float4v __attribute__((ext_vector_type(4)));
+    typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
     constexpr int PITCH = NJ * 32 + 4, QUADS = NJ * 8, AT_ONCE = 64 / QUADS;
     const int li = lane & 31, hh = lane >> 5, quad = lane % QUADS, col = n0 + quad * 4, rows = a.pair ? a.m >> 1 : a.m;
-    float *out = a.ypart ? a.ypart + (size_t)blockIdx.y * rows * a.n : a.y;
-    const bool vec = ((a.n & 3) | ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(a.resid)) & 15)) == 0;
+    const int pitch = a.ypart ? axq_part_pitch(a.n) : a.n;
+    float *out = a.ypart ? a.ypart + (size_t)blockIdx.y * rows * pitch : a.y;
+    const bool whole = col + 3 < pitch; // four columns of y, whose rows lie where they lie: any n takes 16-byte accesses
     float4v bias = {0.f, 0.f, 0.f, 0.f};
     if (a.bias && !a.ypart)
 #pragma unroll
@@ -821,18 +823,18 @@ __device__ inline void write_rows(const RowsArgs &a, const float16v (&acc)[MI][N
             const float *from = patch + (a.pair ? 2 * r : r) * PITCH + quad * 4;
             float4v v = *reinterpret_cast<const float4v *>(from);
             if (a.pair) v += *reinterpret_cast<const float4v *>(from + PITCH);
-            const size_t at = (size_t)row * a.n + col;
+            const size_t at = (size_t)row * pitch + col;
             if (!a.ypart) {
                 v = v * a.rowscale[a.pair ? 2 * row : row];
                 if (a.bias) v += bias;
                 if (a.resid) {
-                    if (vec) v += *reinterpret_cast<const float4v *>(a.resid + at);
+                    if (whole) v += *reinterpret_cast<const float4u *>(a.resid + at);
                     else
                         for (int e = 0; e < 4; e++)
                             if (col + e < a.n) v[e] += a.resid[at + e];
                 }
             }
-            if (vec) *reinterpret_cast<float4v *>(out + at) = v;
+            if (whole) *reinterpret_cast<float4u *>(out + at) = v;
             else
                 for (int e = 0; e < 4; e++)
                     if (col + e < a.n) out[at + e] = v[e];
@@ -1809,7 +1811,7 @@ struct RowsPlan {
     int splits, sb_per_split;    // of K
 };
 
-RowsPlan rows_plan(const axq_ctx *ctx, const axq_weight *w, int in, int rows) {
+RowsPlan rows_plan(const axq_ctx *ctx, const axq_weight *w, int in, int rows, bool whole_k = false) {
     RowsPlan p;
     p.limbs = in != AXQ_ROWS_BF16 && rows < AXQ_ROWS_PAIRS_MIN;
     p.parts = in == AXQ_ROWS_BF16 || p.limbs ? 1 : 2;
@@ -1834,7 +1836,7 @@ RowsPlan rows_plan(const axq_ctx *ctx, const axq_weight *w, int in, int rows) {
     int splits = (int)(ctx->prop.multiProcessorCount / p.tiles);
     if (splits > nsb / groups) splits = nsb / groups;
     if (splits > most) splits = most;
-    if (splits < 2 || n % 4 != 0) splits = 1;
+    if (splits < 2 || whole_k) splits = 1;
     p.sb_per_split = (nsb + splits - 1) / splits;
     p.splits = (nsb + p.sb_per_split - 1) / p.sb_per_split;
     // 128 x 128 outputs whose halves have K of their own: from eight superblocks per workgroup on.  Shorter ones are mostly the start, which
@@ -1916,7 +1918,7 @@ static RowsRoom rows_room(const RowsPlan &p, int rows, const axq_weight *w) {
     r.xa = mtiles * 32 * (size_t)w->k * 2;
     r.xs = mtiles * (size_t)(w->k >> 8) * 2048;
     r.rs = axq_align_up((size_t)p.m * 4, 256);
-    r.part = p.splits > 1 ? (size_t)p.splits * rows * (size_t)w->n_rows * 4 : 0;
+    r.part = p.splits > 1 ? (size_t)p.splits * rows * (size_t)axq_part_pitch((int)w->n_rows) * 4 : 0;
     return r;
 }
 
@@ -1932,11 +1934,16 @@ static void launch_prep_sums(hipStream_t st, const PartSums &ps, const float *no
 // next call, of that weight and as many rows and with nothing in between, takes them.
 int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, int rows, const float *norm_w, float eps, const float *bias,
                       const float *resid, float *y, axq_rows_chain *chain) {
-    const RowsPlan p = rows_plan(ctx, w, in, rows);
+    const size_t at = chain && chain->ready_for == w ? chain->ready_at : 0;
+    RowsPlan p = rows_plan(ctx, w, in, rows);
+    RowsRoom room = rows_room(p, rows, w);
+    if (w->n_rows % 4 != 0 && p.splits > 1 && axq_gemm_reserve(ctx, room.end(at)) != AXQ_OK) { // no room for parts of K: whole, as such calls always can
+        (void)hipGetLastError();
+        p = rows_plan(ctx, w, in, rows, true);
+        room = rows_room(p, rows, w);
+    }
     const bool limbs = p.limbs;
     const int m = p.m, n = (int)w->n_rows, k = (int)w->k, splits = p.splits;
-    const RowsRoom room = rows_room(p, rows, w);
-    const size_t at = chain && chain->ready_for == w ? chain->ready_at : 0;
     const bool ready = at != 0;
     const axq_weight *next = chain ? chain->next : nullptr;
     if (chain) chain->ready_for = nullptr;
