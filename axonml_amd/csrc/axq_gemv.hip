@@ -669,7 +669,7 @@ bool being_captured(axq_ctx *ctx) {
 
 } // namespace
 
-int axq_dev_gemv(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, const float *bias, float *y) {
+int axq_dev_gemv(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, const float *bias, float *y, bool scratch_stands) {
     if (w->n_rows > INT32_MAX || w->k > INT32_MAX)
         return axq_fail(ctx, AXQ_ERR_SHAPE_MISMATCH, "Shape mismatch: weight dimensions exceed 2^31");
     // many vectors: through the matrix-pipe GEMM.  Where the rows kernel pays (see there; nine rows, which the GEMV does as eight and
@@ -677,7 +677,7 @@ int axq_dev_gemv(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, c
     static const bool no_gemm = getenv("AXQ_GEMV_GEMM") && getenv("AXQ_GEMV_GEMM")[0] == '0'; // development knob
     const int others_min = axq_dev_gemv_batch_covers(w, 8) ? 40 : 8;
     while (!no_gemm && axq_dev_gemm_f32_covers(w, 1) &&
-           (batch >= others_min || (axq_dev_rows_gemm_pays(ctx, w, batch) && !being_captured(ctx)))) {
+           (batch >= others_min || (axq_dev_rows_gemm_pays(ctx, w, batch) && (scratch_stands || !being_captured(ctx))))) {
         const int nb = batch < AXQ_GEMM_F32_MAX_ROWS ? batch : AXQ_GEMM_F32_MAX_ROWS;
         int rc = axq_dev_gemm_f32(ctx, w, x, nb, nullptr, 0.f, bias, nullptr, y);
         if (rc == AXQ_ERR_ALLOCATION_FAILED && nb < others_min) { // no room for its scratch: the kernel below needs none

@@ -36,6 +36,9 @@ struct axq_model {
     int32_t *bprompt, *boffsets, *bout; // prompts, their offsets and the generated ids of a batched generate
     hipGraphExec_t graph_b, graph_bf; // batched step: split attention / one attention workgroup per head (short contexts)
     bool graph_b_ok, graph_bf_ok;
+    const void *graph_scratch[2] = {nullptr, nullptr}; // whole, split attention: the GEMM scratch that graph holds the address of,
+    size_t scratch_need[2] = {0, 0};                   // at most how much of it a step takes, and the
+    int plain_steps[2] = {0, 0};                       // steps that have been plain launches
     int max_splits;
     // device-side state
     int32_t *pos, *tok, *next, *gen, *prompt, *out;
