@@ -1494,6 +1494,10 @@ __global__ void __launch_bounds__(512, 2) rows_apart_kernel(RowsArgs a) {
 // eight elements; the row stays in registers (NC times 4096 elements) or, NC = 0, is read once per pass.  Few rows: NC workgroups
 // per row, which all look for its largest element and write 4096 elements each (see launch_prep).  3: as 0, of rows that are still sums of
 // parts of K, which are added up, in gemm_reduce_kernel's order, and written as well.
+// Eight neighbouring rows' pieces fill a line of 128 bytes of the operand (four rows', where rows become two), so they go to one XCD, whose L2
+// puts the line together: workgroups go round the XCDs, and the number of a row is that of its workgroup with the middle digits exchanged
+// (as many workgroups as make whole 64 rows).  2048 bf16 rows of 4096: 18.5 us with row = workgroup, 11.5 so; SwiGLU, 511 rows of 14336: 26.4, 22.5; whole
+// calls: 2048 x 14336 x 4096 291.5 285.3, 509 x 4096 x 4096 54.5 52.7, 33 f32 rows x 4096 x 14336 36.9 35.1.
 struct PartSums {
     const float *part, *scale; // [splits][rows][k]; scale of row t at [t * mul]
     int splits, mul;
@@ -1501,9 +1505,9 @@ struct PartSums {
     float *y;
 };
 struct NoSums {};
-__device__ inline void add_parts(const PartSums &ps, size_t row, int k, int c, float (&e)[8]) {
+__device__ inline void add_parts(const PartSums &ps, size_t row, int rows, int k, int c, float (&e)[8]) {
     typedef float float4v __attribute__((ext_vector_type(4)));
-    const size_t stride = (size_t)gridDim.x * k / 4;
+    const size_t stride = (size_t)rows * k / 4;
     const float4v *from = reinterpret_cast<const float4v *>(ps.part + row * k) + 2 * c;
     float lost[8];
     float4v v[8][2];
@@ -1553,15 +1557,16 @@ __device__ inline void add_parts(const PartSums &ps, size_t row, int k, int c, f
     to[1] = out[1];
 }
 template <int IN, int NC, bool LIMBS>
-__global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const float *norm_w, float eps, int k, _Float16 *xa, _Float16 *xs,
+__global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const float *norm_w, float eps, int rows, int k, _Float16 *xa, _Float16 *xs,
                                                         float *rowscale, std::conditional_t<IN == 3, PartSums, NoSums> sums) {
     constexpr int HELD = NC > 0 ? NC : 1;
     __shared__ float red[8];
-    const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, chunks = k >> 3;
+    const int row = (int)((blockIdx.x & ~63u) | (blockIdx.x & 7) << 3 | (blockIdx.x >> 3 & 7)), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, chunks = k >> 3;
+    if (row >= rows) return;
     float v[HELD][8];
     auto load = [&](int c, float (&e)[8]) {
         if constexpr (IN == 3) {
-            add_parts(sums, row, k, c, e);
+            add_parts(sums, row, rows, k, c, e);
         } else if (IN == 2) {
             const u32x4 r = reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint16_t *>(x) + (size_t)row * k)[c];
 #pragma unroll
@@ -1666,7 +1671,7 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
     const int r0 = row * PARTS, steps = k >> 6, nsb = k >> 8;
     auto slot = [&](int part) { // of the operand's rows: pairs are neighbours; limbs see RowsTile, part 3 = the zeros
         if (!LIMBS) return r0 + part;
-        return gridDim.x <= 16 ? (part < 2 ? part : 5 - part) * 16 + row : row < 32 ? part * 32 + row : 96 + part * 8 + (row & 7);
+        return rows <= 16 ? (part < 2 ? part : 5 - part) * 16 + row : row < 32 ? part * 32 + row : 96 + part * 8 + (row & 7);
     };
     each(false, [&](float (&e)[8], int c) {
         if (NC > 1 && gridDim.y > 1 && (unsigned)(c >> 9) != blockIdx.y) return; // another workgroup's
@@ -1711,7 +1716,7 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
         const int at = c & 7, t = (at >> 2) * 2 + (at & 1), h = (at >> 1) & 1;
 #pragma unroll
         for (int part = 0; part < PARTS + (LIMBS ? 1 : 0); part++) {
-            if (part == PARTS && gridDim.x > 16) break;
+            if (part == PARTS && rows > 16) break;
             const int at_row = slot(part), lrow = at_row & 31;
             _Float16 *xt = xa + (size_t)(at_row >> 5) * steps * 2048, *st = xs + (size_t)(at_row >> 5) * nsb * 1024;
             const _Float16 *s = p[part < PARTS ? part : 0];
@@ -1781,11 +1786,12 @@ int launch_apart(axq_ctx *ctx, const RowsArgs &a, int splits) {
 // row costs most is its conversion (21 rows of 11008, limbs: 8.6 us with one, 6.5 so; 64 rows of 14336, SwiGLU: 9.7, 8.1).
 template <int IN, bool LIMBS>
 void launch_prep(hipStream_t st, const void *x, const float *norm_w, float eps, int rows, int k, _Float16 *xa, _Float16 *xs, float *rs) {
+    const unsigned grid = (unsigned)(rows + 63) / 64 * 64;
     const int parts = rows <= 64 ? (k + 4095) / 4096 : 1;
-    if (k <= 4096) rows_prep_kernel<IN, 1, LIMBS><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs, {});
-    else if (k <= 8192) rows_prep_kernel<IN, 2, LIMBS><<<dim3(rows, parts), 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs, {});
-    else if (IN == 1 || k <= 16384) rows_prep_kernel<IN, 4, LIMBS><<<dim3(rows, parts), 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs, {}); // SwiGLU rows are no longer
-    else if constexpr (IN != 1) rows_prep_kernel<IN, 0, LIMBS><<<rows, 512, 0, st>>>(x, norm_w, eps, k, xa, xs, rs, {});
+    if (k <= 4096) rows_prep_kernel<IN, 1, LIMBS><<<grid, 512, 0, st>>>(x, norm_w, eps, rows, k, xa, xs, rs, {});
+    else if (k <= 8192) rows_prep_kernel<IN, 2, LIMBS><<<dim3(grid, parts), 512, 0, st>>>(x, norm_w, eps, rows, k, xa, xs, rs, {});
+    else if (IN == 1 || k <= 16384) rows_prep_kernel<IN, 4, LIMBS><<<dim3(grid, parts), 512, 0, st>>>(x, norm_w, eps, rows, k, xa, xs, rs, {}); // SwiGLU rows are no longer
+    else if constexpr (IN != 1) rows_prep_kernel<IN, 0, LIMBS><<<grid, 512, 0, st>>>(x, norm_w, eps, rows, k, xa, xs, rs, {});
 }
 
 // How many tiles of 128 x 128 outputs a call of m rows of operands has, where 256 x 256 are the alternative.
@@ -1924,9 +1930,10 @@ static RowsRoom rows_room(const RowsPlan &p, int rows, const axq_weight *w) {
 
 template <bool LIMBS>
 static void launch_prep_sums(hipStream_t st, const PartSums &ps, const float *norm_w, float eps, int rows, int k, _Float16 *xa, _Float16 *xs, float *rs) {
-    if (k <= 4096) rows_prep_kernel<3, 1, LIMBS><<<rows, 512, 0, st>>>(nullptr, norm_w, eps, k, xa, xs, rs, ps);
-    else if (k <= 8192) rows_prep_kernel<3, 2, LIMBS><<<rows, 512, 0, st>>>(nullptr, norm_w, eps, k, xa, xs, rs, ps);
-    else rows_prep_kernel<3, 4, LIMBS><<<rows, 512, 0, st>>>(nullptr, norm_w, eps, k, xa, xs, rs, ps);
+    const unsigned grid = (unsigned)(rows + 63) / 64 * 64;
+    if (k <= 4096) rows_prep_kernel<3, 1, LIMBS><<<grid, 512, 0, st>>>(nullptr, norm_w, eps, rows, k, xa, xs, rs, ps);
+    else if (k <= 8192) rows_prep_kernel<3, 2, LIMBS><<<grid, 512, 0, st>>>(nullptr, norm_w, eps, rows, k, xa, xs, rs, ps);
+    else rows_prep_kernel<3, 4, LIMBS><<<grid, 512, 0, st>>>(nullptr, norm_w, eps, rows, k, xa, xs, rs, ps);
 }
 
 // `chain`: the weight that takes y as f32 rows next, RMS-normalised where chain->norm_w is given.  Where K is split, its operands are made with the
