@@ -35,6 +35,7 @@ struct axq_part {
     int ldy;
     const float *resid;     // where y's are, added; NULL: nothing
     const float *scale;     // row form only: factor of row t at scale[t]; NULL: 1
+    const float *unscale;   // row form only: factor of row t's product, in front of the bias; NULL: 1
     const int32_t *sel;     // vector form only: row r is row sel[r / sel_rows] * sel_rows + r % sel_rows of w
     int sel_rows;
     axq_avg avg;            // avg.out == NULL: none
@@ -87,6 +88,14 @@ int axq_dense_gemv(axq_ctx *ctx, int mode, const axq_in &in, axq_parts &parts);
 // m rows against the parts; k is padded by the caller's rows to ldx = a multiple of 64 with zeros.
 // f32 rows: true 32-bit multiply-adds; bf16 rows: the matrix pipe.
 int axq_dense_gemm(axq_ctx *ctx, axq_parts &parts, int m, int k, int ldx, bool f32);
+// y[m, n] = x W^T for one AXQ_BF16 or (half) AXQ_F16 weight, K a multiple of 64, with rows of the weight's own type that hold `parts` addends of x one
+// behind the other, [m][parts * k]; y = unscale * product + bias + resid.  Few tiles split K: `part` then has axq_dense16_room floats.
+struct axq_dense16 { const void *w; int ldw, n, k, m, parts; bool half; const void *x; const float *unscale, *bias, *resid; float *y, *part; };
+size_t axq_dense16_room(axq_ctx *ctx, int n, int m, int k);
+int axq_dense16_gemm(axq_ctx *ctx, const axq_dense16 &a, bool whole_k);
+// A few f32 rows against an AXQ_BF16 or AXQ_F16 weight, in 32-bit products, every weight read once; whether that pays
+bool axq_dense_few_pays(const axq_weight *w, const float *x, int rows);
+int axq_dense_few(axq_ctx *ctx, const axq_weight *w, const float *x, int rows, const float *bias, float *y);
 // Rows sorted by the weight they go through (a mixture's experts): weight e is part.w + e * stride.  `tiles` is made on the
 // device by axq_moe_sort for the same `bm`: tiles[0] of them, tile i covers slots tiles[4 i + 5] .. tiles[4 i + 6] - 1 and goes
 // through weight tiles[4 i + 4].  Row `slot` of the operand is src[slot] (NULL: slot); results are rows of y by slot.

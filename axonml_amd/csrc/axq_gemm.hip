@@ -1,4 +1,4 @@
-// Prefill-path quantized matmul: y[M, N] = x[M, K] (bf16) * W[N, K]^T, f32 accumulate and output, of plain f16, bf16 and f32 weights
+// Prefill-path quantized matmul: y[M, N] = x[M, K] (bf16) * W[N, K]^T, f32 accumulate and output, of plain f32 weights, some of f16 and bf16 ones
 // and of blocks whose rows are no whole superblocks: packed types with K a multiple of 256 have kernels of their own (axq_gemm_rows.hip).
 //
 // The reference composition is dequantize_tensor -> f32 sgemm (crates/axonml-quant/src/dequantize.rs:34-54,
@@ -23,6 +23,7 @@
 
 #include <type_traits>
 
+#include "axq_dense.h"
 #include "axq_internal.h"
 
 namespace {
@@ -422,9 +423,11 @@ __global__ void __launch_bounds__(256) gemm_prep_x_kernel(const uint16_t *x, int
     const int row = blockIdx.x;
     const uint16_t *xr = x + (size_t)row * k;
     uint32_t amax_bits = 0;
-    for (int i = threadIdx.x; i < k; i += blockDim.x) {
-        uint32_t b = (uint32_t)(xr[i] & 0x7FFF);
-        amax_bits = b > amax_bits ? b : amax_bits;
+    for (int i4 = threadIdx.x; i4 < (k >> 2); i4 += blockDim.x) { // k is a multiple of 64
+        const uint2 raw = reinterpret_cast<const uint2 *>(xr)[i4];
+        const uint32_t b[4] = {raw.x & 0x7FFFu, raw.x >> 16 & 0x7FFFu, raw.y & 0x7FFFu, raw.y >> 16 & 0x7FFFu};
+#pragma unroll
+        for (int j = 0; j < 4; j++) amax_bits = b[j] > amax_bits ? b[j] : amax_bits;
     }
     float amax = __builtin_bit_cast(float, amax_bits << 16);
 #pragma unroll
@@ -439,7 +442,7 @@ __global__ void __launch_bounds__(256) gemm_prep_x_kernel(const uint16_t *x, int
     sb = sb < 1 ? 1 : (sb > 254 ? 254 : sb);
     const float f = __builtin_bit_cast(float, (uint32_t)sb << 23);
     typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-    for (int i4 = threadIdx.x; i4 < (k >> 2); i4 += blockDim.x) { // k is a multiple of 64
+    for (int i4 = threadIdx.x; i4 < (k >> 2); i4 += blockDim.x) {
         const uint2 raw = reinterpret_cast<const uint2 *>(xr)[i4];
         const _Float16 h0 = (_Float16)(__builtin_bit_cast(float, raw.x << 16) * f), h1 = (_Float16)(__builtin_bit_cast(float, raw.x & 0xFFFF0000u) * f);
         const _Float16 h2 = (_Float16)(__builtin_bit_cast(float, raw.y << 16) * f), h3 = (_Float16)(__builtin_bit_cast(float, raw.y & 0xFFFF0000u) * f);
@@ -482,7 +485,7 @@ __global__ void __launch_bounds__(256) gemm_reduce_kernel(const float *ypart, co
     for (int c = 0; c < 4; c++) acc[c] = lost[c] == lost[c] ? acc[c] + lost[c] : acc[c]; // not a number beside an infinite sum
     typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
     const size_t row = i4 / quads, col = i4 % quads * 4, at = row * n + col;
-    const float f = rowscale[row * row_mul] * inv_ws;
+    const float f = rowscale ? rowscale[row * row_mul] * inv_ws : inv_ws;
     if (col + 4 <= (size_t)n) {
         float4u out = {acc[0] * f, acc[1] * f, acc[2] * f, acc[3] * f};
         if (bias) out += *reinterpret_cast<const float4u *>(bias + col);
@@ -517,7 +520,37 @@ int launch_gemm(axq_ctx *ctx, GemmArgs a, int splits) {
 // what those leave, so that their GEMM results add up to the f32 product (the GEMM's epilogue adds them: pair mode).
 // SWIGLU: x holds rows of 2 k gate/up values, four gate values followed by the four up values of the same indices (the row
 // order of the fused gate/up weight), and the row that is split is silu(gate) * up (k a multiple of 4, at most 16384).
-template <bool SWIGLU>
+// FORM: the two f16 rows, or the addends of a row one behind the other, smallest first, so that few additions are of the total's size: two f16
+// ones, or three bf16 ones (all 24 bits, and no scale).
+enum { PREP_TWO_ROWS, PREP_TWO_F16, PREP_THREE_BF16 };
+template <int FORM>
+__device__ inline void put_addends(const float (&e)[4], _Float16 *to, int i4, int k) { // four elements from 4 i4 on of a row; `to`: its addends
+    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+    if constexpr (FORM == PREP_THREE_BF16) {
+        uint32_t p[3][4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            uint32_t b = __builtin_bit_cast(uint32_t, e[j]);
+            const bool finite = (b & 0x7F800000u) != 0x7F800000u;
+            if ((b & 0x7FFFFFFFu) > 0x7F800000u) b |= 0x00400000u; // what says that it is not a number may lie in the lower half
+            const float hi = __builtin_bit_cast(float, b & 0xFFFF0000u), r = finite ? e[j] - hi : 0.f;
+            const float mid = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) & 0xFFFF0000u);
+            p[2][j] = b >> 16;
+            p[1][j] = __builtin_bit_cast(uint32_t, mid) >> 16;
+            p[0][j] = __builtin_bit_cast(uint32_t, r - mid) >> 16;
+        }
+#pragma unroll
+        for (int a = 0; a < 3; a++) reinterpret_cast<uint2 *>(to + (size_t)a * k)[i4] = make_uint2(p[a][0] | p[a][1] << 16, p[a][2] | p[a][3] << 16);
+    } else {
+        _Float16 h[4], l[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) { h[j] = (_Float16)e[j]; l[j] = (_Float16)(e[j] - (float)h[j]); }
+        constexpr bool FIRST = FORM == PREP_TWO_ROWS; // the leading bits' place
+        reinterpret_cast<half4 *>(to + (FIRST ? 0 : k))[i4] = half4{h[0], h[1], h[2], h[3]};
+        reinterpret_cast<half4 *>(to + (FIRST ? k : 0))[i4] = half4{l[0], l[1], l[2], l[3]};
+    }
+}
+template <bool SWIGLU, int FORM>
 __global__ void __launch_bounds__(256) gemm_prep_x_f32_kernel(const float *x, const float *norm_w, float eps, int m, int k,
                                                               _Float16 *xh, float *rowscale) {
     // the row stays in registers between the passes: 16 bytes per thread and step, up to 16 steps (k <= 16384);
@@ -604,33 +637,29 @@ __global__ void __launch_bounds__(256) gemm_prep_x_f32_kernel(const float *x, co
     if (eb == 0 || eb == 0xFF) eb = 127 + 14;
     int sb = 127 + 14 - (eb - 127);
     sb = sb < 1 ? 1 : (sb > 254 ? 254 : sb);
-    const float f = __builtin_bit_cast(float, (uint32_t)sb << 23);
-    _Float16 *hi_row = xh + (size_t)(2 * row) * k, *lo_row = hi_row + k;
+    const float f = FORM == PREP_THREE_BF16 ? 1.0f : __builtin_bit_cast(float, (uint32_t)sb << 23);
+    _Float16 *to = xh + (size_t)(FORM == PREP_THREE_BF16 ? 3 : 2) * row * k;
     if (in_regs) {
 #pragma unroll
         for (int c = 0; c < STEPS; c++) {
             const int i4 = c * 256 + threadIdx.x;
             if (i4 * 4 < k) {
                 const float e[4] = {v[c].x * f, v[c].y * f, v[c].z * f, v[c].w * f};
-                _Float16 h[4], l[4];
-#pragma unroll
-                for (int j = 0; j < 4; j++) { h[j] = (_Float16)e[j]; l[j] = (_Float16)(e[j] - (float)h[j]); }
-                typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-                reinterpret_cast<half4 *>(hi_row)[i4] = half4{h[0], h[1], h[2], h[3]};
-                reinterpret_cast<half4 *>(lo_row)[i4] = half4{l[0], l[1], l[2], l[3]};
+                put_addends<FORM>(e, to, i4, k);
             }
         }
     } else {
-        for (int i = threadIdx.x; i < k; i += blockDim.x) {
-            const float e = (norm_w ? (xr[i] * inv) * norm_w[i] : xr[i]) * f;
-            const _Float16 hi = (_Float16)e;
-            hi_row[i] = hi;
-            lo_row[i] = (_Float16)(e - (float)hi);
+        for (int i4 = threadIdx.x; i4 * 4 < k; i4 += blockDim.x) { // k is a multiple of 64
+            float e[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) e[j] = (norm_w ? (xr[4 * i4 + j] * inv) * norm_w[4 * i4 + j] : xr[4 * i4 + j]) * f;
+            put_addends<FORM>(e, to, i4, k);
         }
     }
-    if (threadIdx.x == 0) {
-        rowscale[2 * row] = 1.0f / f;
-        rowscale[2 * row + 1] = 1.0f / f;
+    if (FORM != PREP_THREE_BF16 && threadIdx.x == 0) {
+        const int mul = FORM == PREP_TWO_ROWS ? 2 : 1;
+        rowscale[mul * row] = 1.0f / f;
+        if (mul == 2) rowscale[2 * row + 1] = 1.0f / f;
     }
 }
 
@@ -737,7 +766,57 @@ int run_gemm(axq_ctx *ctx, const axq_weight *w, int m, const GemmPlan &p, float 
 
 } // namespace
 
+namespace {
+
+// 16-bit weights: rows of the weight's own type, no conversion and one product per weight and addend of x.  us, through the two planes and so:
+//   bf16 rows   BF16 3394 x 4096, 42: 87.7 11.7; 471 x 4096, 1536: 152 22.4; 14336 x 3328, 2048: 473 179
+//               F16 3674 x 4096, 187: 41.9 23.6; 14336 x 1280, 1672: 241 106; 7520 x 1856, 1278: 157 60
+//   f32 rows    F16 4096 x 4096, 64: 24.4 19.4; 20000 x 4096, 64: 90.8 69.7; 20000 x 11008, 64: 220 279
+//               BF16 1024 x 11008, 64: 40.1 28.1; 8192 x 2048, 64: 23.3 22.8; 4096 x 11008, 64: 41.1 55.7
+// Few f32 rows against much of a weight stay with the planes: each addend reads the weight again.
+bool covers16(const axq_weight *w, int m, bool f32) {
+    if ((w->type != AXQ_BF16 && w->type != AXQ_F16) || w->k % BK != 0 || w->n_rows > INT32_MAX || w->k > INT32_MAX / 4) return false;
+    return !f32 || m > 128 || w->n_rows * w->k <= (w->type == AXQ_F16 ? 128 << 20 : 17 << 20);
+}
+
+// Scratch: rows (`addends` times the caller's; 0: none) | row scales | partial sums of a split K.  Without room for the last, K whole.
+struct Room16 { _Float16 *x; float *scale, *part; };
+int room16(axq_ctx *ctx, const axq_weight *w, int m, int addends, Room16 *r) {
+    const size_t xb = axq_align_up((size_t)m * (size_t)w->k * 2 * addends, 256), sb = addends ? axq_align_up((size_t)m * 4, 256) : 0;
+    const size_t pb = axq_dense16_room(ctx, (int)w->n_rows, m, (int)w->k * (addends ? addends : 1)) * 4;
+    int rc = axq_gemm_reserve(ctx, xb + sb + pb);
+    const bool whole = rc != AXQ_OK && pb;
+    if (whole) {
+        (void)hipGetLastError();
+        rc = axq_gemm_reserve(ctx, xb + sb);
+    }
+    uint8_t *base = reinterpret_cast<uint8_t *>(ctx->gemm_scratch);
+    *r = {reinterpret_cast<_Float16 *>(base), reinterpret_cast<float *>(base + xb), whole || !pb ? nullptr : reinterpret_cast<float *>(base + xb + sb)};
+    return rc;
+}
+axq_dense16 dense16_of(const axq_weight *w, int m, int addends, const void *x, float *y, const Room16 &r) {
+    axq_dense16 d = {};
+    d.w = w->codes; d.ldw = (int)(w->codes_pitch / 2); d.n = (int)w->n_rows; d.k = (int)w->k; d.m = m; d.parts = addends; d.half = w->type == AXQ_F16;
+    d.x = x; d.y = y; d.part = r.part;
+    return d;
+}
+
+} // namespace
+
 int axq_dev_gemm_bf16(axq_ctx *ctx, const axq_weight *w, const uint16_t *x, int m, float *y) {
+    if (covers16(w, m, false)) {
+        const bool own_rows = w->type == AXQ_F16 || (reinterpret_cast<uintptr_t>(x) & 15) != 0; // the product takes 16 bytes at a time
+        Room16 r;
+        if (int rc = room16(ctx, w, m, own_rows, &r)) return rc;
+        axq_dense16 d = dense16_of(w, m, 1, own_rows ? static_cast<const void *>(r.x) : x, y, r);
+        if (d.half) {
+            gemm_prep_x_kernel<<<m, 256, 0, ctx->stream>>>(x, m, (int)w->k, r.x, r.scale);
+            d.unscale = r.scale;
+        } else if (own_rows) {
+            AXQ_HIP(ctx, hipMemcpyAsync(r.x, x, (size_t)m * (size_t)w->k * 2, hipMemcpyDeviceToDevice, ctx->stream), AXQ_ERR_COPY_FAILED);
+        }
+        return axq_dense16_gemm(ctx, d, !r.part);
+    }
     if (axq_dev_rows_gemm_covers(w, m)) return axq_dev_rows_gemm(ctx, w, x, AXQ_ROWS_BF16, m, nullptr, 0.f, nullptr, nullptr, y);
     GemmPlan p;
     int rc;
@@ -772,11 +851,25 @@ int axq_dev_gemm_f32_ex(axq_ctx *ctx, const axq_weight *w, const float *x, bool 
     if (axq_dev_rows_gemm_covers(w, m))
         return axq_dev_rows_gemm(ctx, w, x, swiglu ? AXQ_ROWS_SWIGLU : AXQ_ROWS_F32, m, norm_w, eps, bias, resid, y, chain);
     if (chain) chain->ready_for = nullptr;
+    if (covers16(w, m, true)) {
+        const bool half = w->type == AXQ_F16;
+        Room16 r;
+        if ((rc = room16(ctx, w, m, half ? 2 : 3, &r))) return rc;
+        if (half && swiglu) gemm_prep_x_f32_kernel<true, PREP_TWO_F16><<<m, 256, 0, ctx->stream>>>(x, nullptr, eps, m, (int)w->k, r.x, r.scale);
+        else if (half) gemm_prep_x_f32_kernel<false, PREP_TWO_F16><<<m, 256, 0, ctx->stream>>>(x, norm_w, eps, m, (int)w->k, r.x, r.scale);
+        else if (swiglu) gemm_prep_x_f32_kernel<true, PREP_THREE_BF16><<<m, 256, 0, ctx->stream>>>(x, nullptr, eps, m, (int)w->k, r.x, r.scale);
+        else gemm_prep_x_f32_kernel<false, PREP_THREE_BF16><<<m, 256, 0, ctx->stream>>>(x, norm_w, eps, m, (int)w->k, r.x, r.scale);
+        axq_dense16 d = dense16_of(w, m, half ? 2 : 3, r.x, y, r);
+        d.unscale = half ? r.scale : nullptr;
+        d.bias = bias;
+        d.resid = resid;
+        return axq_dense16_gemm(ctx, d, !r.part);
+    }
     if ((rc = plan_gemm(ctx, w, 2 * m, &p))) return rc;
     uint8_t *base = reinterpret_cast<uint8_t *>(ctx->gemm_scratch);
     _Float16 *xh = reinterpret_cast<_Float16 *>(base);
     float *rowscale = reinterpret_cast<float *>(base + p.xh_bytes);
-    if (swiglu) gemm_prep_x_f32_kernel<true><<<m, 256, 0, ctx->stream>>>(x, nullptr, eps, m, (int)w->k, xh, rowscale);
-    else gemm_prep_x_f32_kernel<false><<<m, 256, 0, ctx->stream>>>(x, norm_w, eps, m, (int)w->k, xh, rowscale);
+    if (swiglu) gemm_prep_x_f32_kernel<true, PREP_TWO_ROWS><<<m, 256, 0, ctx->stream>>>(x, nullptr, eps, m, (int)w->k, xh, rowscale);
+    else gemm_prep_x_f32_kernel<false, PREP_TWO_ROWS><<<m, 256, 0, ctx->stream>>>(x, norm_w, eps, m, (int)w->k, xh, rowscale);
     return run_gemm(ctx, w, 2 * m, p, y, true, bias, resid);
 }

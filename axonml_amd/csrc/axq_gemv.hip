@@ -24,6 +24,7 @@
 
 #include <stdlib.h>
 
+#include "axq_dense.h"
 #include "axq_internal.h"
 
 namespace {
@@ -676,6 +677,7 @@ int axq_dev_gemv(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, c
     // one, it never does: 1 to 2 us behind); the others from about 40 rows where the small-batch kernel below is the alternative, from 8 where single-vector passes are
     static const bool no_gemm = getenv("AXQ_GEMV_GEMM") && getenv("AXQ_GEMV_GEMM")[0] == '0'; // development knob
     const int others_min = axq_dev_gemv_batch_covers(w, 8) ? 40 : 8;
+    if (batch >= 2 && axq_dense_few_pays(w, x, batch)) return axq_dense_few(ctx, w, x, batch, bias, y);
     while (!no_gemm && axq_dev_gemm_f32_covers(w, 1) &&
            (batch >= others_min || (axq_dev_rows_gemm_pays(ctx, w, batch) && (scratch_stands || !being_captured(ctx))))) {
         const int nb = batch < AXQ_GEMM_F32_MAX_ROWS ? batch : AXQ_GEMM_F32_MAX_ROWS;
