@@ -46,6 +46,7 @@ struct axq_model {
     uint8_t *host_ring = nullptr;   // page-locked: logits on their way to the caller, two portions of host_portion bytes
     size_t host_portion = 0;
     hipEvent_t portion_there[2] = {nullptr, nullptr};
+    hipEvent_t rows_there = nullptr; // LLaMA shape: what a prompt's last token waits for on the context's aux_stream[0]
     int32_t *hist;                  // every token fed so far, by position (what a repetition penalty looks at)
     void *sample_scratch;           // scratch of the sampler, allocated when one is set
     bool sampling;                  // next token by axq_sampling_config instead of the plain argmax
@@ -61,6 +62,14 @@ struct axq_model {
     int prompt_chunk;               // most prompt rows per pass through the layers
     bool attn_mfma;                 // prompt attention of many rows on the matrix pipe (development knob AXQ_ATTN_MFMA=0: off)
     axq_stack *stack = nullptr;     // layers described one by one (axq_model_create_stack) instead of the LLaMA shape above
+};
+
+// Launches go to another stream while this lives.
+struct OnStream {
+    axq_ctx *ctx;
+    hipStream_t before;
+    OnStream(axq_ctx *c, hipStream_t st) : ctx(c), before(c->stream) { c->stream = st; }
+    ~OnStream() { ctx->stream = before; }
 };
 
 // axq_decode.hip: the buffers every model has (token, position, history, prompt, output, logits), for one sequence.

@@ -659,14 +659,6 @@ int step_head(axq_model *m) {
     return axq_dense_gemv(m->ctx, norm_mode(s), norm_in(s, s.top, "final.norm", m->h), hd);
 }
 
-// Launches go to another stream while this lives.
-struct OnStream {
-    axq_ctx *ctx;
-    hipStream_t before;
-    OnStream(axq_ctx *c, hipStream_t st) : ctx(c), before(c->stream) { c->stream = st; }
-    ~OnStream() { ctx->stream = before; }
-};
-
 } // namespace
 
 namespace {

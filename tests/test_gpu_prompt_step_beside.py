@@ -1,0 +1,80 @@
+"""A prompt's last token goes through the layers beside the rows in front of it: logits, caches, position and what follows against the oracle, prompts in
+several chunks, on top of a context, of a batched model, again and again, and where the rows find no room."""
+import numpy as np
+import pytest
+
+import oracle as o
+from axonml_amd import quant as q
+from tests.decode_common import load_gpu, load_oracle, random_weights, tiny_config
+from tests.util import DECODE_FLOOR, DECODE_RTOL, max_rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _walk(cpu, tokens, pos=0):
+    for t in tokens:
+        nxt, lg = cpu.forward(int(t), pos)
+        pos += 1
+    return nxt, lg
+
+
+@pytest.mark.parametrize("lengths", [(193,), (194, 200), (300, 193, 3), (5, 250)])
+@pytest.mark.parametrize("chunk", ["2048", "96"])
+def test_prompts_on_top_of_each_other(ctx, monkeypatch, lengths, chunk):
+    monkeypatch.setenv("AXQ_PROMPT_CHUNK", chunk)
+    c = tiny_config(max_seq_len=sum(lengths) + 8, num_layers=3)
+    w = random_weights(c, sum(lengths))
+    cpu, gpu = load_oracle(c, w), load_gpu(ctx, c, w)
+    rng = np.random.default_rng(len(lengths))
+    for n_seq in (1, 3):  # with several sequences the first one takes the prompt
+        gpu.set_batch(n_seq)
+        pos = 0
+        for n in lengths:
+            tokens = rng.integers(0, c["vocab_size"], size=n)
+            want = _walk(cpu, tokens, pos)
+            got = gpu.forward_tokens(tokens)
+            pos += n
+            assert got[0] == want[0] and max_rel_err(got[1], want[1], DECODE_FLOOR) <= DECODE_RTOL, n
+        for _ in range(3):  # the steps behind it see its position and its keys
+            want, got = cpu.forward(int(want[0]), pos), gpu.forward(int(got[0]))
+            pos += 1
+            assert got[0] == want[0] and max_rel_err(got[1], want[1], DECODE_FLOOR) <= DECODE_RTOL, pos
+    gpu.close()
+    cpu.close()
+
+
+@pytest.mark.parametrize("n", [10, 14, 33])
+def test_wide_models(ctx, n):
+    c = tiny_config(max_seq_len=n + 4, hidden_size=4096, intermediate_size=512, num_heads=4, num_kv_heads=2, vocab_size=64)
+    w = random_weights(c, n)
+    cpu, gpu = load_oracle(c, w), load_gpu(ctx, c, w)
+    tokens = np.random.default_rng(n).integers(0, c["vocab_size"], size=n)
+    want = _walk(cpu, tokens)
+    first = None
+    for _ in range(5):  # the same bits every time
+        gpu.reset()
+        got = gpu.forward_tokens(tokens)
+        assert got[0] == want[0] and max_rel_err(got[1], want[1], DECODE_FLOOR) <= DECODE_RTOL
+        assert first is None or np.array_equal(first, got[1])
+        first = got[1]
+    gpu.close()
+    cpu.close()
+
+
+def test_without_room_for_the_rows(monkeypatch):
+    ctx = q.Context(0)
+    monkeypatch.setenv("AXQ_GEMM_SCRATCH_MAX", "0")
+    c = tiny_config(max_seq_len=32, hidden_size=4096, intermediate_size=512, vocab_size=64)
+    w = random_weights(c, 9)
+    cpu, gpu = load_oracle(c, w), load_gpu(ctx, c, w)
+    tokens = np.random.default_rng(9).integers(0, c["vocab_size"], size=20)
+    want = _walk(cpu, tokens)
+    for _ in range(2):
+        got = gpu.forward_tokens(tokens)  # the rows fail behind the step's first launches and go in by eights
+        assert got[0] == want[0] and max_rel_err(got[1], want[1], DECODE_FLOOR) <= DECODE_RTOL
+        assert gpu.forward(int(got[0]))[0] == cpu.forward(int(want[0]), 20)[0]
+        gpu.reset()
+        monkeypatch.delenv("AXQ_GEMM_SCRATCH_MAX", raising=False)
+    gpu.close()
+    cpu.close()
+    ctx.close()
