@@ -1557,11 +1557,11 @@ __device__ inline void add_parts(const PartSums &ps, size_t row, int rows, int k
     to[1] = out[1];
 }
 template <int IN, int NC, bool LIMBS>
-__global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const float *norm_w, float eps, int rows, int k, _Float16 *xa, _Float16 *xs,
+__global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const float *norm_w, float eps, int rows, int k, int kp, _Float16 *xa, _Float16 *xs,
                                                         float *rowscale, std::conditional_t<IN == 3, PartSums, NoSums> sums) {
     constexpr int HELD = NC > 0 ? NC : 1;
     __shared__ float red[8];
-    const int row = (int)((blockIdx.x & ~63u) | (blockIdx.x & 7) << 3 | (blockIdx.x >> 3 & 7)), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, chunks = k >> 3;
+    const int row = (int)((blockIdx.x & ~63u) | (blockIdx.x & 7) << 3 | (blockIdx.x >> 3 & 7)), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, chunks = k >> 3, all = kp >> 3; // of eight elements: the row's, the operand's (zeros behind the row)
     if (row >= rows) return;
     float v[HELD][8];
     auto load = [&](int c, float (&e)[8]) {
@@ -1590,7 +1590,7 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
             e[0] = l.x; e[1] = l.y; e[2] = l.z; e[3] = l.w; e[4] = h.x; e[5] = h.y; e[6] = h.z; e[7] = h.w;
         }
     };
-    // all threads go through `chunks` in steps of 512; `fn(e, c, i)`: e the elements of chunk c, the i-th of this thread
+    // all threads go through `all` in steps of 512; `fn(e, c, i)`: e the elements of chunk c, the i-th of this thread
     auto each = [&](bool first, auto fn) {
         if constexpr (NC > 0) {
 #pragma unroll
@@ -1605,7 +1605,7 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
                 fn(v[i], c);
             }
         } else {
-            for (int c = tid; c < (chunks + 511) / 512 * 512; c += 512) {
+            for (int c = tid; c < (all + 511) / 512 * 512; c += 512) {
                 float e[8];
                 if (c < chunks) load(c, e);
                 else
@@ -1668,7 +1668,7 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
     sb = sb < 1 ? 1 : (sb > 254 ? 254 : sb);
     const float f = __builtin_bit_cast(float, (uint32_t)sb << 23);
     constexpr int PARTS = LIMBS ? 3 : IN == 2 ? 1 : 2;
-    const int r0 = row * PARTS, steps = k >> 6, nsb = k >> 8;
+    const int r0 = row * PARTS, steps = kp >> 6, nsb = kp >> 8;
     auto slot = [&](int part) { // of the operand's rows: pairs are neighbours; limbs see RowsTile, part 3 = the zeros
         if (!LIMBS) return r0 + part;
         return rows <= 16 ? (part < 2 ? part : 5 - part) * 16 + row : row < 32 ? part * 32 + row : 96 + part * 8 + (row & 7);
@@ -1721,13 +1721,13 @@ __global__ void __launch_bounds__(512) rows_prep_kernel(const void *x, const flo
             _Float16 *xt = xa + (size_t)(at_row >> 5) * steps * 2048, *st = xs + (size_t)(at_row >> 5) * nsb * 1024;
             const _Float16 *s = p[part < PARTS ? part : 0];
             const half8 out = part < PARTS ? half8{s[0], s[2], s[1], s[3], s[4], s[6], s[5], s[7]} : half8{0, 0, 0, 0, 0, 0, 0, 0};
-            if (c < chunks)
+            if (c < all)
                 *reinterpret_cast<half8 *>(xt + ((size_t)(c >> 3) * 4 + t) * 512 + (h * 32 + lrow) * 8) = out;
             // the sum of 32 elements: four threads; times 1 / 64 it stays within f16's range
             float g = part < PARTS ? sum[part] : 0.f;
             g += __shfl_xor(g, 1);
             g += __shfl_xor(g, 2);
-            if ((tid & 3) == 0 && c < chunks) {
+            if ((tid & 3) == 0 && c < all) {
                 g = part < PARTS ? fmaf(g, 1.0f / 64.0f, carry) : 0.f;
                 const _Float16 ghi = (_Float16)g, glo = (_Float16)(g - (float)ghi);
                 if (LIMBS) carry = (g - (float)ghi - (float)glo) * (part == 0 ? (float)(1 << (LB + 2)) : 1.0f);
@@ -1785,13 +1785,13 @@ int launch_apart(axq_ctx *ctx, const RowsArgs &a, int splits) {
 // Up to 64 rows of more than 4096 elements a workgroup for every 4096 of each: as many as there are rows leave most of the chip idle, and what a
 // row costs most is its conversion (21 rows of 11008, limbs: 8.6 us with one, 6.5 so; 64 rows of 14336, SwiGLU: 9.7, 8.1).
 template <int IN, bool LIMBS>
-void launch_prep(hipStream_t st, const void *x, const float *norm_w, float eps, int rows, int k, _Float16 *xa, _Float16 *xs, float *rs) {
+void launch_prep(hipStream_t st, const void *x, const float *norm_w, float eps, int rows, int k, int kp, _Float16 *xa, _Float16 *xs, float *rs) {
     const unsigned grid = (unsigned)(rows + 63) / 64 * 64;
-    const int parts = rows <= 64 ? (k + 4095) / 4096 : 1;
-    if (k <= 4096) rows_prep_kernel<IN, 1, LIMBS><<<grid, 512, 0, st>>>(x, norm_w, eps, rows, k, xa, xs, rs, {});
-    else if (k <= 8192) rows_prep_kernel<IN, 2, LIMBS><<<dim3(grid, parts), 512, 0, st>>>(x, norm_w, eps, rows, k, xa, xs, rs, {});
-    else if (IN == 1 || k <= 16384) rows_prep_kernel<IN, 4, LIMBS><<<dim3(grid, parts), 512, 0, st>>>(x, norm_w, eps, rows, k, xa, xs, rs, {}); // SwiGLU rows are no longer
-    else if constexpr (IN != 1) rows_prep_kernel<IN, 0, LIMBS><<<grid, 512, 0, st>>>(x, norm_w, eps, rows, k, xa, xs, rs, {});
+    const int parts = rows <= 64 ? (kp + 4095) / 4096 : 1;
+    if (kp <= 4096) rows_prep_kernel<IN, 1, LIMBS><<<grid, 512, 0, st>>>(x, norm_w, eps, rows, k, kp, xa, xs, rs, {});
+    else if (kp <= 8192) rows_prep_kernel<IN, 2, LIMBS><<<dim3(grid, parts), 512, 0, st>>>(x, norm_w, eps, rows, k, kp, xa, xs, rs, {});
+    else if (IN == 1 || kp <= 16384) rows_prep_kernel<IN, 4, LIMBS><<<dim3(grid, parts), 512, 0, st>>>(x, norm_w, eps, rows, k, kp, xa, xs, rs, {}); // SwiGLU rows are no longer
+    else if constexpr (IN != 1) rows_prep_kernel<IN, 0, LIMBS><<<grid, 512, 0, st>>>(x, norm_w, eps, rows, k, kp, xa, xs, rs, {});
 }
 
 // How many tiles of 128 x 128 outputs a call of m rows of operands has, where 256 x 256 are the alternative.
@@ -1823,13 +1823,13 @@ RowsPlan rows_plan(const axq_ctx *ctx, const axq_weight *w, int in, int rows, bo
     p.parts = in == AXQ_ROWS_BF16 || p.limbs ? 1 : 2;
     p.m = rows * p.parts;
     const bool super = w->type == AXQ_Q4_K || w->type == AXQ_Q5_K || w->type == AXQ_Q6_K;
-    const int n = (int)w->n_rows, nsb = (int)(w->k >> 8);
+    const int n = (int)w->n_rows, nsb = (int)(w->kp >> 8);
     // Blocks of 32 take large tiles where the small ones are more than one to a compute unit: their sums of a superblock, which keep additions
     // of the total's size few, fit the registers of 128 x 128 outputs only (Q4_0, K = 4096: an error of 0.83 10^-7 there, 2.0 in large tiles).
     // bf16 rows, us in the former kernel of that range, with operands in LDS, and now: 2048 x 14336 x 4096 Q4_0 414 411, Q4_1 475 451, Q5_0 482 431,
     // Q5_1 557 475, Q8_0 447 414; 700 x 11008 x 2048 Q4_0 119 111, Q5_1 153 126; 130 x 17000 x 1024 Q5_0 42.5 35.7.  (Operands made in the
     // fetch, not between the products: Q4_0 397, Q4_1 471, Q5_1 539.)
-    p.wide = !p.limbs && (super ? wide_tiles(ctx, p.m, n, w->k) : square_tiles(p.m, n) > ctx->prop.multiProcessorCount);
+    p.wide = !p.limbs && (super ? wide_tiles(ctx, p.m, n, w->kp) : square_tiles(p.m, n) > ctx->prop.multiProcessorCount);
     const int groups = p.m <= (p.limbs ? 32 : 64) ? 2 : 1; // of waves along K
     p.bm = p.limbs ? (rows <= 32 ? 32 : 40) : p.m <= 32 ? 32 : p.m <= 64 ? 64 : p.wide ? 256 : 128;
     const int bn = p.wide && super ? 256 : 128;
@@ -1876,9 +1876,9 @@ int launch_rows(axq_ctx *ctx, const RowsArgs &a, const RowsPlan &p) {
 
 } // namespace
 
-// Packed types at any number of rows, K a multiple of 256.
+// Packed types at any number of rows, whole superblocks in the planes.
 bool axq_dev_rows_gemm_covers(const axq_weight *w, int rows) {
-    if (w->k % 256 != 0 || w->k > INT32_MAX || w->n_rows > INT32_MAX || rows < 1) return false;
+    if (w->kp % 256 != 0 || w->kp > INT32_MAX || w->n_rows > INT32_MAX || rows < 1) return false;
     switch (w->type) {
     case AXQ_Q4_K: case AXQ_Q5_K: case AXQ_Q6_K: case AXQ_Q4_0: case AXQ_Q4_1: case AXQ_Q5_0: case AXQ_Q5_1: case AXQ_Q8_0: return true;
     default: return false;
@@ -1921,8 +1921,8 @@ struct RowsRoom {
 static RowsRoom rows_room(const RowsPlan &p, int rows, const axq_weight *w) {
     RowsRoom r;
     const size_t mtiles = p.limbs ? (rows <= 16 ? 2 : rows <= 32 ? 3 : 4) : (size_t)(p.m + p.bm - 1) / p.bm * (p.bm / 32);
-    r.xa = mtiles * 32 * (size_t)w->k * 2;
-    r.xs = mtiles * (size_t)(w->k >> 8) * 2048;
+    r.xa = mtiles * 32 * (size_t)w->kp * 2;
+    r.xs = mtiles * (size_t)(w->kp >> 8) * 2048;
     r.rs = axq_align_up((size_t)p.m * 4, 256);
     r.part = p.splits > 1 ? (size_t)p.splits * rows * (size_t)axq_part_pitch((int)w->n_rows) * 4 : 0;
     return r;
@@ -1931,9 +1931,9 @@ static RowsRoom rows_room(const RowsPlan &p, int rows, const axq_weight *w) {
 template <bool LIMBS>
 static void launch_prep_sums(hipStream_t st, const PartSums &ps, const float *norm_w, float eps, int rows, int k, _Float16 *xa, _Float16 *xs, float *rs) {
     const unsigned grid = (unsigned)(rows + 63) / 64 * 64;
-    if (k <= 4096) rows_prep_kernel<3, 1, LIMBS><<<grid, 512, 0, st>>>(nullptr, norm_w, eps, rows, k, xa, xs, rs, ps);
-    else if (k <= 8192) rows_prep_kernel<3, 2, LIMBS><<<grid, 512, 0, st>>>(nullptr, norm_w, eps, rows, k, xa, xs, rs, ps);
-    else rows_prep_kernel<3, 4, LIMBS><<<grid, 512, 0, st>>>(nullptr, norm_w, eps, rows, k, xa, xs, rs, ps);
+    if (k <= 4096) rows_prep_kernel<3, 1, LIMBS><<<grid, 512, 0, st>>>(nullptr, norm_w, eps, rows, k, k, xa, xs, rs, ps);
+    else if (k <= 8192) rows_prep_kernel<3, 2, LIMBS><<<grid, 512, 0, st>>>(nullptr, norm_w, eps, rows, k, k, xa, xs, rs, ps);
+    else rows_prep_kernel<3, 4, LIMBS><<<grid, 512, 0, st>>>(nullptr, norm_w, eps, rows, k, k, xa, xs, rs, ps);
 }
 
 // `chain`: the weight that takes y as f32 rows next, RMS-normalised where chain->norm_w is given.  Where K is split, its operands are made with the
@@ -1950,14 +1950,14 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
         room = rows_room(p, rows, w);
     }
     const bool limbs = p.limbs;
-    const int m = p.m, n = (int)w->n_rows, k = (int)w->k, splits = p.splits;
+    const int m = p.m, n = (int)w->n_rows, k = (int)w->k, kp = (int)w->kp, splits = p.splits;
     const bool ready = at != 0;
     const axq_weight *next = chain ? chain->next : nullptr;
     if (chain) chain->ready_for = nullptr;
     size_t next_at = 0;
     RowsPlan np;
     RowsRoom nroom = {};
-    if (next && splits > 1 && !bias && next->k == n && next->k <= 16384 && axq_dev_rows_gemm_covers(next, rows)) {
+    if (next && splits > 1 && !bias && next->k == n && next->kp == n && next->k <= 16384 && axq_dev_rows_gemm_covers(next, rows)) {
         np = rows_plan(ctx, next, AXQ_ROWS_F32, rows);
         nroom = rows_room(np, rows, next);
         next_at = room.end(at);
@@ -1980,21 +1980,21 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
     float *rs;
     operands(at, room, xa, xs, rs);
     if (!ready) switch (in) {
-    case AXQ_ROWS_BF16: launch_prep<2, false>(ctx->stream, x, nullptr, 0.f, rows, k, xa, xs, rs); break;
+    case AXQ_ROWS_BF16: launch_prep<2, false>(ctx->stream, x, nullptr, 0.f, rows, k, kp, xa, xs, rs); break;
     case AXQ_ROWS_SWIGLU:
-        if (limbs) launch_prep<1, true>(ctx->stream, x, nullptr, 0.f, rows, k, xa, xs, rs);
-        else launch_prep<1, false>(ctx->stream, x, nullptr, 0.f, rows, k, xa, xs, rs);
+        if (limbs) launch_prep<1, true>(ctx->stream, x, nullptr, 0.f, rows, k, kp, xa, xs, rs);
+        else launch_prep<1, false>(ctx->stream, x, nullptr, 0.f, rows, k, kp, xa, xs, rs);
         break;
     default:
-        if (limbs) launch_prep<0, true>(ctx->stream, x, norm_w, eps, rows, k, xa, xs, rs);
-        else launch_prep<0, false>(ctx->stream, x, norm_w, eps, rows, k, xa, xs, rs);
+        if (limbs) launch_prep<0, true>(ctx->stream, x, norm_w, eps, rows, k, kp, xa, xs, rs);
+        else launch_prep<0, false>(ctx->stream, x, norm_w, eps, rows, k, kp, xa, xs, rs);
         break;
     }
     a.codes = w->codes; a.meta = w->meta; a.qh = w->qh;
     a.codes_pitch = (uint32_t)w->codes_pitch; a.meta_pitch = (uint32_t)w->meta_pitch; a.qh_pitch = (uint32_t)w->qh_pitch;
     a.xa = xa; a.xs = xs; a.rowscale = rs; a.y = y;
     a.ypart = splits > 1 ? reinterpret_cast<float *>(base + room.part_at(at)) : nullptr;
-    a.m = m; a.n = n; a.k = k; a.pair = p.parts == 2; a.bias = bias; a.resid = resid;
+    a.m = m; a.n = n; a.k = kp; a.pair = p.parts == 2; a.bias = bias; a.resid = resid;
     int rc;
     switch (w->type) {
     case AXQ_Q4_K: rc = launch_rows<SuperQ45<false>>(ctx, a, p); break;

@@ -676,10 +676,13 @@ int axq_dev_gemv(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, c
     // many vectors: through the matrix-pipe GEMM.  Where the rows kernel pays (see there; nine rows, which the GEMV does as eight and
     // one, it never does: 1 to 2 us behind); the others from about 40 rows where the small-batch kernel below is the alternative, from 8 where single-vector passes are
     static const bool no_gemm = getenv("AXQ_GEMV_GEMM") && getenv("AXQ_GEMV_GEMM")[0] == '0'; // development knob
-    const int others_min = axq_dev_gemv_batch_covers(w, 8) ? 40 : 8;
+    const int others_min = axq_dev_gemv_batch_takes(w, 8) ? 40 : 8;
+    // the types whose small-batch GEMV does not take ragged rows: four rows and more (Q5_1 19483 x 3648, 4: 52.3 us as single vectors, 43.6 so; Q4_1 1000 x
+    // 4032, 3: 12.4, 15.4)
+    const bool ragged = others_min == 8 && w->kp != w->k;
     if (batch >= 2 && axq_dense_few_pays(w, x, batch)) return axq_dense_few(ctx, w, x, batch, bias, y);
     while (!no_gemm && axq_dev_gemm_f32_covers(w, 1) &&
-           (batch >= others_min || (axq_dev_rows_gemm_pays(ctx, w, batch) && (scratch_stands || !being_captured(ctx))))) {
+           (batch >= others_min || ((axq_dev_rows_gemm_pays(ctx, w, batch) || (ragged && batch >= 4)) && (scratch_stands || !being_captured(ctx))))) {
         const int nb = batch < AXQ_GEMM_F32_MAX_ROWS ? batch : AXQ_GEMM_F32_MAX_ROWS;
         int rc = axq_dev_gemm_f32(ctx, w, x, nb, nullptr, 0.f, bias, nullptr, y);
         if (rc == AXQ_ERR_ALLOCATION_FAILED && nb < others_min) { // no room for its scratch: the kernel below needs none
@@ -692,7 +695,7 @@ int axq_dev_gemv(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, c
         batch -= nb;
     }
     // small batches: eight vectors at a time against one pass over the weights, where that kernel applies
-    while (batch >= 2 && axq_dev_gemv_batch_covers(w, batch < 8 ? batch : 8)) {
+    while (batch >= 2 && axq_dev_gemv_batch_takes(w, batch < 8 ? batch : 8)) {
         const int nb = batch < 8 ? batch : 8;
         int rc = axq_dev_gemv_batch(ctx, w, x, nb, bias, nullptr, y);
         if (rc) return rc;

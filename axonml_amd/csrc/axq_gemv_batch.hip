@@ -42,6 +42,7 @@ struct MbArgs {
     float *y;
     float *ypart; // K split over several workgroups: [split][batch][n_rows] partial sums, added by mb_reduce_kernel
     int n_rows, k, batch;
+    int kx; // columns of x: k, or fewer, where the last superblock of the weight is not whole
     int chunks_per_split; // chunks of a row that one workgroup (blockIdx.y) takes
 };
 
@@ -458,11 +459,11 @@ __global__ void __launch_bounds__(512, 4) gemv_mb_kernel(MbArgs a) {
 // itself); AXQ_X_SWIGLU: x holds [batch, 2k] gate/up values, four gate values followed by the four up values of the
 // same indices, and f = silu(gate) * up.
 template <bool EVEN_ODD, int XMODE>
-__global__ void __launch_bounds__(256) pack_x_kernel(const float *x, const float *aux, float eps, int k, int batch, uint8_t *xa,
+__global__ void __launch_bounds__(256) pack_x_kernel(const float *x, const float *aux, float eps, int k, int kp, int batch, uint8_t *xa,
                                                      float *xsg) {
     __shared__ float red[4];
     const int t = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
-    const int ntask = k >> 3, nblk = k >> 5;
+    const int ntask = kp >> 3, nblk = kp >> 5; // kp: whole superblocks; behind k zeros
     float inv = 1.0f;
     if (XMODE == AXQ_X_RMSNORM && b < batch) { // before any thread leaves: the sum needs the whole workgroup
         const float4 *row = reinterpret_cast<const float4 *>(x + (size_t)b * k);
@@ -478,9 +479,9 @@ __global__ void __launch_bounds__(256) pack_x_kernel(const float *x, const float
         ss = (red[0] + red[1]) + (red[2] + red[3]);
         inv = 1.0f / sqrtf(ss / (float)k + eps);
     }
-    if (t >= ntask) return; // k is a multiple of 256: whole quads of tasks
+    if (t >= ntask) return; // whole quads of tasks
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (b < batch) {
+    if (b < batch && t < k >> 3) {
         if (XMODE == AXQ_X_SWIGLU) {
             const float4 *p = reinterpret_cast<const float4 *>(x + (size_t)b * 2 * k + (size_t)t * 16);
 #pragma unroll
@@ -622,9 +623,9 @@ int launch_mb(axq_ctx *ctx, MbArgs a, uint8_t *sc, const float *x, int xmode, co
     float *xsg = const_cast<float *>(a.xsg);
     if (xmode == AXQ_X_PACKED) {
         // the operands are in place already (the previous call prepared them)
-    } else if (xmode == AXQ_X_RMSNORM) pack_x_kernel<T::EVEN_ODD, AXQ_X_RMSNORM><<<pgrid, 256, 0, ctx->stream>>>(x, aux, eps, a.k, a.batch, xa, xsg);
-    else if (xmode == AXQ_X_SWIGLU) pack_x_kernel<T::EVEN_ODD, AXQ_X_SWIGLU><<<pgrid, 256, 0, ctx->stream>>>(x, aux, eps, a.k, a.batch, xa, xsg);
-    else pack_x_kernel<T::EVEN_ODD, AXQ_X_PLAIN><<<pgrid, 256, 0, ctx->stream>>>(x, aux, eps, a.k, a.batch, xa, xsg);
+    } else if (xmode == AXQ_X_RMSNORM) pack_x_kernel<T::EVEN_ODD, AXQ_X_RMSNORM><<<pgrid, 256, 0, ctx->stream>>>(x, aux, eps, a.kx, a.k, a.batch, xa, xsg);
+    else if (xmode == AXQ_X_SWIGLU) pack_x_kernel<T::EVEN_ODD, AXQ_X_SWIGLU><<<pgrid, 256, 0, ctx->stream>>>(x, aux, eps, a.kx, a.k, a.batch, xa, xsg);
+    else pack_x_kernel<T::EVEN_ODD, AXQ_X_PLAIN><<<pgrid, 256, 0, ctx->stream>>>(x, aux, eps, a.kx, a.k, a.batch, xa, xsg);
     const unsigned chunks = (unsigned)((a.k + WAVE_K - 1) / WAVE_K);
     const unsigned tiles = (unsigned)((a.n_rows + 31) / 32);
     // few row tiles (a narrow output): split K over up to four workgroups per tile so that the chip is full
@@ -668,14 +669,14 @@ int launch_mb(axq_ctx *ctx, MbArgs a, uint8_t *sc, const float *x, int xmode, co
 // the same call, so the buffer needs no clearing between calls.
 int gemv_batch_in(axq_ctx *ctx, uint8_t *sc, const axq_weight *w, const float *x, int xmode, const float *aux, float eps, int batch,
                   const float *bias, const float *resid, float *y, int next_even_odd, const float *next_aux) {
-    const int k = (int)w->k;
+    const int k = (int)w->kp;
     MbArgs a;
     a.codes = w->codes; a.meta = w->meta; a.qh = w->qh;
     a.codes_pitch = w->codes_pitch; a.meta_pitch = w->meta_pitch; a.qh_pitch = w->qh_pitch;
     a.xa = sc; a.xsg = reinterpret_cast<float *>(sc + (size_t)32 * k);
     a.bias = bias; a.resid = resid; a.y = y;
     a.ypart = w->n_rows <= AXQ_BATCH_SPLIT_ROWS ? reinterpret_cast<float *>(sc + (size_t)34 * AXQ_BATCH_MAX_K) : nullptr;
-    a.n_rows = (int)w->n_rows; a.k = k; a.batch = batch;
+    a.n_rows = (int)w->n_rows; a.k = k; a.kx = (int)w->k; a.batch = batch;
     int st;
     switch (w->type) {
     case AXQ_Q4_0: st = launch_mb<MQ4x<false>>(ctx, a, sc, x, xmode, aux, eps, next_even_odd, next_aux); break;
@@ -703,6 +704,14 @@ bool axq_dev_gemv_batch_covers(const axq_weight *w, int batch) {
     case AXQ_Q4_0: case AXQ_Q4_1: case AXQ_Q5_0: case AXQ_Q5_1: case AXQ_Q8_0: case AXQ_Q4_K: case AXQ_Q5_K: case AXQ_Q6_K: return true;
     default: return false;
     }
+}
+
+// Rows of padded superblocks: from three on, or of large weights (two rows, us, as two vectors and so: Q8_0 4096 x 4160 13.1 11.9, Q4_1 4096 x 4032 9.2 11.8, 11008 x
+// 4032 15.0 13.7).  Not of a type with a minimum, whose error is larger here than vector by vector (Q5_1 4954 x 9600: 15.5 and 9.5 10^-8).
+bool axq_dev_gemv_batch_takes(const axq_weight *w, int batch) {
+    if (w->k % 256 == 0) return axq_dev_gemv_batch_covers(w, batch);
+    if (w->kp % 256 != 0 || w->kp > AXQ_BATCH_MAX_K || (w->type != AXQ_Q4_0 && w->type != AXQ_Q5_0 && w->type != AXQ_Q8_0)) return false;
+    return batch <= MAX_BATCH && batch >= (w->n_rows * w->k >= 40 << 20 ? 2 : 3);
 }
 
 // Where a caller that prepares the operands of the call with w itself (axq_store_packed, then xmode = AXQ_X_PACKED) has

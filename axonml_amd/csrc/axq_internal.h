@@ -45,7 +45,7 @@ int axq_aux_join(axq_ctx *ctx, int n);
 //                         Q4_K             : d, dmin, scales[12]   (16 B/superblock)
 //   plane 2 (qh)      : Q5_0/Q5_1 only, the 32 high bits of each block (4 B/block)
 //
-// The bytes are exactly those of the packed (`to_bytes`) image, permuted, so
+// The bytes are exactly those of the packed (`to_bytes`) image, permuted (behind a row's last block zeros, where `kp` is beyond k), so
 // upload -> download is the identity and HBM traffic per matmul equals the
 // packed size.  For Q4_K the 128 code bytes of a superblock are further
 // interleaved inside 16-superblock "slices" so that one wavefront reads two
@@ -54,6 +54,7 @@ int axq_aux_join(axq_ctx *ctx, int n);
 struct axq_weight {
     int type;
     int64_t n_rows, k;
+    int64_t kp;          // columns that the planes' rows hold: k, or with blocks of 32 whole superblocks of 256, the last blocks zeros (see axq_weight_alloc)
     size_t packed_bytes; // size of the to_bytes image
     uint8_t *base;       // device allocation
     size_t alloc_bytes;
@@ -141,6 +142,7 @@ size_t axq_xq_bytes(int64_t k);
 int axq_dev_prep_x(axq_ctx *ctx, const float *x, int64_t k, uint8_t *xq);
 // gemv_batch.hip: batches of 2..8 vectors against one pass over the weights
 bool axq_dev_gemv_batch_covers(const axq_weight *w, int batch);
+bool axq_dev_gemv_batch_takes(const axq_weight *w, int batch); // a call of its own, not in a chain: rows of padded superblocks as well
 int axq_dev_gemv_batch(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, const float *bias, const float *resid, float *y);
 int axq_dev_gemv_batch_ex(axq_ctx *ctx, const axq_weight *w, const float *x, int xmode, const float *aux, float eps, int batch,
                           const float *bias, const float *resid, float *y);

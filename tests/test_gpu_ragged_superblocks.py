@@ -1,0 +1,56 @@
+"""Weights of blocks of 32 whose rows are no whole superblocks of 256: zeros lie behind a row's last block on the device.  Upload and download give the same
+bytes, and products of every number of rows agree with 64 bits.
+
+Bound: 3e-7 of the results' root mean square for the f32 sums, f32 rows from 40 on as pairs of f16: 2^-22 sqrt(2) (see test_gpu_gemm_rows_uneven)."""
+import numpy as np
+import pytest
+
+import oracle as o
+from axonml_amd import quant as q
+from tests.util import gen_weight
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [o.Q4_0, o.Q4_1, o.Q5_0, o.Q5_1, o.Q8_0]
+
+
+def _off(got, want):
+    return float(np.sqrt(np.mean(np.square(got - want)) / np.mean(np.square(want))))
+
+
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("k", [736, 768 + 32, 1024 - 64, 1024 + 64, 4096 + 192, 16384 - 128, 16384 + 64])
+def test_products(ctx, qtype, k):
+    n = 300
+    rng = np.random.default_rng(k + qtype)
+    packed = o.quantize(qtype, gen_weight(rng, n, k))
+    w = o.dequantize(qtype, packed, n * k).reshape(n, k).astype(np.float64)
+    qt = q.QuantizedTensor([n, k], qtype, packed)
+    dw = q.DeviceWeight.upload(qt, ctx)
+    assert np.array_equal(dw.download().data, packed)
+    bias = rng.standard_normal(n).astype(np.float32)
+    for rows in (1, 2, 7, 8, 9, 10, 16, 17, 39, 40, 65, 130):
+        x = rng.standard_normal((rows, k)).astype(np.float32)
+        got = q.quantized_matmul(x, dw, bias, ctx)
+        assert _off(got, x.astype(np.float64) @ w.T + bias) <= 3e-7 + 2.0 ** -22 * 2 ** 0.5, rows
+    if k % 64 == 0:
+        for rows in (1, 24, 100, 300):
+            bits = q.f32_to_bf16_bits(rng.standard_normal((rows, k)).astype(np.float32))
+            got = q.quantized_matmul_bf16(bits, dw, ctx)
+            assert _off(got, q.bf16_bits_to_f32(bits).astype(np.float64) @ w.T) <= 3e-7, rows
+    dw.free()
+
+
+@pytest.mark.parametrize("qtype", TYPES)
+def test_large_elements_in_the_last_block(ctx, qtype):
+    """The block in front of the zeros holds the row's largest elements, and bf16 rows take the large tiles."""
+    n, k, rows = 1500, 1024 + 32 * 2, 600
+    rng = np.random.default_rng(qtype)
+    packed = o.quantize(qtype, gen_weight(rng, n, k))
+    w = o.dequantize(qtype, packed, n * k).reshape(n, k).astype(np.float64)
+    qt = q.QuantizedTensor([n, k], qtype, packed)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    x[:, -32:] *= 1000
+    bits = q.f32_to_bf16_bits(x)
+    assert _off(q.quantized_matmul_bf16(bits, qt, ctx), q.bf16_bits_to_f32(bits).astype(np.float64) @ w.T) <= 4e-7
+    assert _off(q.quantized_matmul(x[:20], qt, None, ctx), x[:20].astype(np.float64) @ w.T) <= 4e-7
