@@ -980,22 +980,36 @@ __global__ void __launch_bounds__(256) embed_pos_kernel(const uint16_t *emb16, c
 
 struct MixPtrs { const float *mu[AXQ_MAX_PARTS]; };
 
+// These kernels are their rows' bytes, so they go 16 bytes of f32 and 8 of bf16 a lane at a time.  2047 rows, us, an element and four at a time: tanh norm
+// of 2048 columns 16.4 and 12.3; poly norm of 7168, kept in registers between its sums and its results, 34.5 and 20.6; root mean square and gate of 2048
+// columns 11.6 and 7.5, in groups of 64 18.7 and 7.5.
 __global__ void __launch_bounds__(256) rows_tanh_norm_kernel(axq_in in, int m, int first, int n_mix, MixPtrs mix, axq_rows_out out) {
-    const int t = blockIdx.x;
+    const int t = blockIdx.x, k = in.k;
     const float alpha = in.alpha[0];
-    const float *h = in.x + (size_t)(in.rows ? in.rows[t] : t) * in.k;
-    for (int e = threadIdx.x; e < out.ldx; e += 256) {
-        const bool in_row = e < in.k;
-        const float nw = in_row ? in.nw[e] : 0.f, nb = in_row ? in.nb[e] : 0.f;
-        const float n = in_row ? tanh_norm(h[e], alpha, nw, nb) : 0.f;
+    const float *h = in.x + (size_t)(in.rows ? in.rows[t] : t) * k;
+    for (int e = threadIdx.x * 4; e < out.ldx; e += 1024) { // past the end everything is zero
+        const f32x4 nw = load_quad(in.nw, e, k), nb = load_quad(in.nb, e, k), x = load_quad(h, e, k);
+        f32x4 n, p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; i++) n[i] = e + i < k ? tanh_norm(x[i], alpha, nw[i], nb[i]) : 0.f;
         if (n_mix == 0) {
-            put(out, t, e, n);
+            put_quad(out, t, e, n);
             continue;
         }
-        float p = 0.f;
-        if (in_row && t > 0) p = tanh_norm(h[e - in.k], alpha, nw, nb);
-        else if (in_row && !first) p = in.prev[e];
-        for (int i = 0; i < n_mix; i++) put(out, (size_t)i * m + t, e, in_row ? fmaf(p - n, mix.mu[i][e], n) : 0.f);
+        if (t > 0) {
+            const f32x4 y = load_quad(h - k, e, k);
+#pragma unroll
+            for (int i = 0; i < 4; i++) p[i] = e + i < k ? tanh_norm(y[i], alpha, nw[i], nb[i]) : 0.f;
+        } else if (!first) {
+            p = load_quad(in.prev, e, k);
+        }
+        for (int j = 0; j < n_mix; j++) {
+            const f32x4 mu = load_quad(mix.mu[j], e, k);
+            f32x4 v;
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = fmaf(p[i] - n[i], mu[i], n[i]);
+            put_quad(out, (size_t)j * m + t, e, v);
+        }
     }
 }
 
@@ -1018,24 +1032,85 @@ __global__ void __launch_bounds__(256) rows_rms_gate_kernel(axq_in in, int group
         for (int e = in.k + threadIdx.x; e < out.ldx; e += blockDim.x) put(out, t, e, 0.f);
 }
 
-__global__ void __launch_bounds__(256) rows_poly_norm_kernel(axq_in in, axq_rows_out out) {
+// The same for groups of 4, 8, .. 256 (a group in as many neighbouring lanes as it has quads) or, GROUP = 0, one group that is the row: one workgroup
+// per row, which keeps up to 4096 elements of it.
+template <bool WHOLE>
+__global__ void __launch_bounds__(256) rows_rms_gate_quads_kernel(axq_in in, int group, axq_rows_out out) {
     __shared__ float scratch[16];
-    const int t = blockIdx.x, k = in.k;
+    constexpr int NR = 4;
+    const int t = blockIdx.x, k = in.k, tid = threadIdx.x;
+    const float *x = in.x + (size_t)t * k, *g = in.gate + (size_t)t * k;
+    auto dot = [](f32x4 v) { return fmaf(v[0], v[0], v[1] * v[1]) + fmaf(v[2], v[2], v[3] * v[3]); };
+    auto write = [&](int e, f32x4 v, float inv) {
+        const f32x4 w = load_quad(in.nw, e, k), y = load_quad(g, e, k);
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = e + i < k ? v[i] * inv * w[i] * y[i] : 0.f;
+        put_quad(out, t, e, v);
+    };
+    if constexpr (WHOLE) {
+        f32x4 r[NR];
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            r[i] = load_quad(x, (tid + i * 256) * 4, k);
+            ss += dot(r[i]);
+        }
+        for (int e = (NR * 256 + tid) * 4; e < k; e += 1024) ss += dot(load_quad(x, e, k));
+        const float inv = 1.0f / sqrtf(axq_block_sum(ss, scratch) / (float)k + in.eps);
+#pragma unroll
+        for (int i = 0; i < NR; i++)
+            if ((tid + i * 256) * 4 < out.ldx) write((tid + i * 256) * 4, r[i], inv);
+        for (int e = (NR * 256 + tid) * 4; e < out.ldx; e += 1024) write(e, load_quad(x, e, k), inv);
+    } else {
+        for (int e0 = 0; e0 < out.ldx; e0 += 1024) { // all lanes of a group together
+            const int e = e0 + tid * 4;
+            const f32x4 v = load_quad(x, e, k);
+            float ss = dot(v);
+            for (int s = 1; s < group / 4; s <<= 1) ss += __shfl_xor(ss, s);
+            if (e < out.ldx) write(e, v, 1.0f / sqrtf(ss / (float)group + in.eps));
+        }
+    }
+}
+
+__global__ void __launch_bounds__(256) rows_poly_norm_kernel(axq_in in, axq_rows_out out) {
+    __shared__ float scratch[3][4];
+    constexpr int NR = 8; // quads of a row that a thread keeps; wider rows are read again
+    const int t = blockIdx.x, k = in.k, tid = threadIdx.x;
     const float *x = in.x + (size_t)t * k;
-    float s1 = 0.f, s2 = 0.f, s3 = 0.f;
-    for (int e = threadIdx.x; e < k; e += 256) {
-        const float z = x[e], z2 = z * z, z3 = z2 * z;
-        s1 += z2; s2 = fmaf(z2, z2, s2); s3 = fmaf(z3, z3, s3);
+    float s[3] = {0.f, 0.f, 0.f};
+    f32x4 r[NR];
+    auto add = [&](f32x4 v) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float z = v[i], z2 = z * z, z3 = z2 * z;
+            s[0] += z2; s[1] = fmaf(z2, z2, s[1]); s[2] = fmaf(z3, z3, s[2]);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < NR; i++) r[i] = load_quad(x, (tid + i * 256) * 4, k);
+#pragma unroll
+    for (int i = 0; i < NR; i++) add(r[i]);
+    for (int e = (NR * 256 + tid) * 4; e < k; e += 1024) add(load_quad(x, e, k));
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        s[i] = axq_wave_sum(s[i]);
+        if ((tid & 63) == 0) scratch[i][tid >> 6] = s[i];
     }
-    s1 = axq_block_sum(s1, scratch);
-    s2 = axq_block_sum(s2, scratch);
-    s3 = axq_block_sum(s3, scratch);
-    const float c1 = in.coef[0] / sqrtf(s1 / (float)k + in.eps), c2 = in.coef[1] / sqrtf(s2 / (float)k + in.eps);
-    const float c3 = in.coef[2] / sqrtf(s3 / (float)k + in.eps), c0 = in.coef[3];
-    for (int e = threadIdx.x; e < out.ldx; e += 256) {
-        const float z = e < k ? x[e] : 0.f;
-        put(out, t, e, e < k ? fmaf(fmaf(fmaf(c3, z, c2), z, c1), z, c0) : 0.f);
-    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 3; i++) s[i] = (scratch[i][0] + scratch[i][1]) + (scratch[i][2] + scratch[i][3]);
+    const float c1 = in.coef[0] / sqrtf(s[0] / (float)k + in.eps), c2 = in.coef[1] / sqrtf(s[1] / (float)k + in.eps);
+    const float c3 = in.coef[2] / sqrtf(s[2] / (float)k + in.eps), c0 = in.coef[3];
+    auto write = [&](int e, f32x4 v) {
+        if (e >= out.ldx) return;
+        f32x4 y;
+#pragma unroll
+        for (int i = 0; i < 4; i++) y[i] = e + i < k ? fmaf(fmaf(fmaf(c3, v[i], c2), v[i], c1), v[i], c0) : 0.f;
+        put_quad(out, t, e, y);
+    };
+#pragma unroll
+    for (int i = 0; i < NR; i++) write((tid + i * 256) * 4, r[i]);
+    for (int e = (NR * 256 + tid) * 4; e < out.ldx; e += 1024) write(e, load_quad(x, e, k));
 }
 
 __global__ void __launch_bounds__(256) rows_layer_norm_kernel(axq_in in, const float *nw1, axq_rows_out out1, const float *nw2, axq_rows_out out2) {
@@ -1081,9 +1156,10 @@ __global__ void __launch_bounds__(256) rows_layer_norm_kernel(axq_in in, const f
 
 __global__ void __launch_bounds__(256) rows_glu_kernel(const float *z, int ldz, int k, axq_rows_out out) {
     const float *row = z + (size_t)blockIdx.x * ldz;
-    for (int e = threadIdx.x; e < out.ldx; e += 256) {
-        const float *g = row + (e / AXQ_GLU_GROUP) * 2 * AXQ_GLU_GROUP + e % AXQ_GLU_GROUP;
-        put(out, blockIdx.x, e, e < k ? g[0] * g[AXQ_GLU_GROUP] : 0.f);
+    static_assert(AXQ_GLU_GROUP % 4 == 0, "a quad lies in one group");
+    for (int e = threadIdx.x * 4; e < out.ldx; e += 1024) {
+        const float *g = row + (e / AXQ_GLU_GROUP) * 2 * AXQ_GLU_GROUP + e % AXQ_GLU_GROUP - e; // g[e]
+        put_quad(out, blockIdx.x, e, load_quad(g, e, k) * load_quad(g + AXQ_GLU_GROUP, e, k));
     }
 }
 
@@ -1372,7 +1448,9 @@ int axq_store_prev(axq_ctx *ctx, const axq_in &in, int m, float *prev) {
 }
 
 int axq_rows_rms_gate(axq_ctx *ctx, const axq_in &in, int m, int group, axq_rows_out out) {
-    rows_rms_gate_kernel<<<dim3(m, in.k / group), group <= 128 ? 64 : 256, 0, ctx->stream>>>(in, group, out);
+    if (group <= 256 && group >= 4 && (group & (group - 1)) == 0) rows_rms_gate_quads_kernel<false><<<m, 256, 0, ctx->stream>>>(in, group, out);
+    else if (group == in.k) rows_rms_gate_quads_kernel<true><<<m, 256, 0, ctx->stream>>>(in, group, out);
+    else rows_rms_gate_kernel<<<dim3(m, in.k / group), group <= 128 ? 64 : 256, 0, ctx->stream>>>(in, group, out);
     AXQ_LAUNCH_CHECK(ctx, "rows_rms_gate_kernel");
     return AXQ_OK;
 }
