@@ -2,8 +2,8 @@
 // decay per head) or, before the update and with a bonus for the current token, with r (time mixing with a decay per
 // token, head and key channel).
 //
-// The columns of S do not depend on each other, so a workgroup takes 16 columns of one head; a column lies across 16
-// lanes, every lane keeping dk / 16 of its elements in registers for the whole prompt.  Tokens come through LDS in
+// The columns of S do not depend on each other, so a workgroup takes 16 or 32 columns of one head; a column lies across 16
+// lanes, every lane keeping dk / 16 of its elements (of one column or two) in registers for the whole prompt.  Tokens come through LDS in
 // blocks; the next block is requested while the current one is worked on.  Where heads x columns do not fill the chip, the
 // prompt is cut into segments: their states from zero, a scan over them (the update is linear in the state), then all
 // segments side by side from the states they start in.
@@ -40,15 +40,18 @@ __device__ inline void load_elems(const float *row, int g, float (&out)[E]) {
 }
 
 // Tokens of a group are independent but for the state: their vectors are read ahead, their outputs reduced together.
-template <int E, bool TOKEN_DECAY, bool STATE_ONLY, bool VEC>
+// Bound by LDS reads (a key and a query, 16 bytes per lane and four elements, for three or four multiply-adds each) about as much as by the vector units:
+// a lane with two columns, C = 2, reads them once for both.  2047 tokens, us, one column and two: 16 heads of 128 x 128 with a decay per head 93 and 77,
+// their states alone 59 and 42; 32 heads of 64 x 64 with a decay per token 75 and 62, states 39 and 31 (the states' pass also no longer multiplies the
+// decays in every wave).
+template <int E, bool TOKEN_DECAY, bool STATE_ONLY, bool VEC, int C>
 __global__ void __launch_bounds__(256) linstate_rows_kernel(axq_linstate a, int m_all, int first, int seg_len) {
     constexpr int DKP = 16 * E, NV = TOKEN_DECAY ? 3 : 2, G = E <= (TOKEN_DECAY ? 5 : 8) ? 4 : 2, TB = E <= 8 ? 16 : (E <= 12 ? 8 : 4);
     constexpr int W = VEC ? 4 : 1, LOADS = (NV * TB * DKP / W + 255) / 256; // per thread and block
     __shared__ __attribute__((aligned(16))) float vec[2][NV][TB][DKP];
-    __shared__ __attribute__((aligned(16))) float val[2][16][TB], os[16][TB + 1]; // by column
+    __shared__ __attribute__((aligned(16))) float val[2][16 * C][TB], os[16 * C][TB + 1]; // by column
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane & 15, cw = lane >> 4;
-    const int head = blockIdx.x, c0 = blockIdx.y * 16, mycol = wave * 4 + cw, col = c0 + mycol;
-    const bool live = col < a.dv;
+    const int head = blockIdx.x, c0 = blockIdx.y * 16 * C, mycol = wave * 4 + cw, col = c0 + mycol; // and every 16th after it
     const int seg = blockIdx.z, t_beg = seg * seg_len, m = m_all - t_beg < seg_len ? m_all - t_beg : seg_len;
     const float *q = a.q + (size_t)t_beg * a.ldq + (size_t)head * a.dk, *k = a.k + (size_t)t_beg * a.ldk + (size_t)head * a.dk;
     const float *v = a.v + (size_t)t_beg * a.ldv + (size_t)head * a.dv;
@@ -59,19 +62,22 @@ __global__ void __launch_bounds__(256) linstate_rows_kernel(axq_linstate a, int 
     float *st = (cut ? a.seg_state + seg * all_states : a.state) + head_state;
     first = STATE_ONLY || (first && !cut); // of several segments each starts in a state of its own
 
-    float S[E], u[E], wp[STATE_ONLY ? E : 1];
+    constexpr int WP = STATE_ONLY && TOKEN_DECAY ? E : 1;
+    const bool product = STATE_ONLY && blockIdx.y == 0 && wave == 0; // the wave that leaves the segment's decay
+    float S[C][E], u[E], wp[WP];
 #pragma unroll
-    for (int i = 0; i < (STATE_ONLY ? E : 1); i++) wp[i] = 1.f;
+    for (int i = 0; i < WP; i++) wp[i] = 1.f;
 #pragma unroll
     for (int i = 0; i < E; i++) {
         const int e = elem_of<E>(g, i);
-        S[i] = (!first && live && e < a.dk) ? st[(size_t)e * a.dv + col] : 0.f;
+#pragma unroll
+        for (int c = 0; c < C; c++) S[c][i] = (!first && col + 16 * c < a.dv && e < a.dk) ? st[(size_t)e * a.dv + col + 16 * c] : 0.f;
         u[i] = (TOKEN_DECAY && e < a.dk) ? a.u[(size_t)head * a.dk + e] : 0.f;
     }
     const float decay = TOKEN_DECAY ? 0.f : a.decay[head];
 
     // tokens beyond the last: k = 0 and a decay of 1 leave the state as it is
-    float pre[LOADS][W], pre_v;
+    float pre[LOADS][W], pre_v[C];
     auto request = [&](int t0) {
 #pragma unroll
         for (int i = 0; i < LOADS; i++) {
@@ -87,8 +93,11 @@ __global__ void __launch_bounds__(256) linstate_rows_kernel(axq_linstate a, int 
                 pre[i][0] = there ? *src : none;
             }
         }
-        const int t = t0 + (tid >> 4), c = c0 + (tid & 15);
-        pre_v = (tid < TB * 16 && t < m && c < a.dv) ? v[(size_t)t * a.ldv + c] : 0.f;
+#pragma unroll
+        for (int i = 0; i < C; i++) {
+            const int idx = tid + i * 256, t = t0 + idx / (16 * C), c = c0 + idx % (16 * C);
+            pre_v[i] = (idx < TB * 16 * C && t < m && c < a.dv) ? v[(size_t)t * a.ldv + c] : 0.f;
+        }
     };
     auto deposit = [&](int stage) {
         float *dst = &vec[stage][0][0][0];
@@ -100,48 +109,67 @@ __global__ void __launch_bounds__(256) linstate_rows_kernel(axq_linstate a, int 
                 else dst[idx] = pre[i][0];
             }
         }
-        if (tid < TB * 16) val[stage][tid & 15][tid >> 4] = pre_v;
+#pragma unroll
+        for (int i = 0; i < C; i++) {
+            const int idx = tid + i * 256;
+            if (idx < TB * 16 * C) val[stage][idx % (16 * C)][idx / (16 * C)] = pre_v[i];
+        }
     };
-    struct Group { float q[G][STATE_ONLY ? 1 : E], k[G][E], w[G][TOKEN_DECAY ? E : 1], v[G]; };
+    struct Group { float q[G][STATE_ONLY ? 1 : E], k[G][E], w[G][TOKEN_DECAY ? E : 1], v[C][G]; };
     auto read = [&](int stage, int t, Group &x) {
 #pragma unroll
         for (int i = 0; i < G; i++) {
             if constexpr (!STATE_ONLY) load_elems<E>(vec[stage][0][t + i], g, x.q[i]);
             load_elems<E>(vec[stage][1][t + i], g, x.k[i]);
             if constexpr (TOKEN_DECAY) load_elems<E>(vec[stage][NV - 1][t + i], g, x.w[i]);
-            x.v[i] = val[stage][mycol][t + i];
+#pragma unroll
+            for (int c = 0; c < C; c++) x.v[c][i] = val[stage][mycol + 16 * c][t + i];
         }
     };
     auto work = [&](int t, int nt, const Group &x) {
-        float o[G];
+        float o[C][G];
 #pragma unroll
         for (int j = 0; j < G; j++) {
-            float s = 0.f;
             const bool token = TOKEN_DECAY || t + j < nt; // a constant decay must not touch the state beyond the last token
 #pragma unroll
-            for (int i = 0; i < E; i++) {
-                const float kv = x.k[j][i] * x.v[j];
-                if constexpr (STATE_ONLY) {
-                    float w = decay; // segments of a state-only pass are whole blocks
+            for (int c = 0; c < C; c++) {
+                float s = 0.f;
+#pragma unroll
+                for (int i = 0; i < E; i++) {
+                    const float kv = x.k[j][i] * x.v[c][j];
+                    if constexpr (STATE_ONLY) {
+                        float w = decay; // segments of a state-only pass are whole blocks
+                        if constexpr (TOKEN_DECAY) w = x.w[j][i];
+                        S[c][i] = fmaf(w, S[c][i], kv);
+                    } else if constexpr (TOKEN_DECAY) {
+                        s = fmaf(x.q[j][i], fmaf(u[i], kv, S[c][i]), s);
+                        S[c][i] = fmaf(x.w[j][i], S[c][i], kv);
+                    } else {
+                        S[c][i] = fmaf(token ? decay : 1.f, S[c][i], kv);
+                        s = fmaf(x.q[j][i], S[c][i], s);
+                    }
+                }
+                o[c][j] = s;
+            }
+            if (product) {
+#pragma unroll
+                for (int i = 0; i < WP; i++) {
+                    float w = decay;
                     if constexpr (TOKEN_DECAY) w = x.w[j][i];
-                    S[i] = fmaf(w, S[i], kv);
                     wp[i] *= w;
-                } else if constexpr (TOKEN_DECAY) {
-                    s = fmaf(x.q[j][i], fmaf(u[i], kv, S[i]), s);
-                    S[i] = fmaf(x.w[j][i], S[i], kv);
-                } else {
-                    S[i] = fmaf(token ? decay : 1.f, S[i], kv);
-                    s = fmaf(x.q[j][i], S[i], s);
                 }
             }
-            o[j] = s;
         }
         if constexpr (!STATE_ONLY) {
 #pragma unroll
-            for (int j = 0; j < G; j++) o[j] = row_sum16(o[j]);
+            for (int c = 0; c < C; c++)
+#pragma unroll
+                for (int j = 0; j < G; j++) o[c][j] = row_sum16(o[c][j]);
             if (g == 0) {
 #pragma unroll
-                for (int j = 0; j < G; j++) os[mycol][t + j] = o[j];
+                for (int c = 0; c < C; c++)
+#pragma unroll
+                    for (int j = 0; j < G; j++) os[mycol + 16 * c][t + j] = o[c][j];
             }
         }
     };
@@ -162,8 +190,13 @@ __global__ void __launch_bounds__(256) linstate_rows_kernel(axq_linstate a, int 
         }
         if (t0 + TB < m) deposit(stage ^ 1);
         __syncthreads(); // the outputs are complete, the next block is in place
-        if (!STATE_ONLY && tid < nt * 16 && c0 + (tid & 15) < a.dv)
-            o_out[(size_t)(t0 + (tid >> 4)) * a.heads * a.dv + (size_t)head * a.dv + c0 + (tid & 15)] = os[tid & 15][tid >> 4];
+        if constexpr (!STATE_ONLY) {
+#pragma unroll
+            for (int i = 0; i < C; i++) {
+                const int idx = tid + i * 256, c = idx % (16 * C), r = idx / (16 * C);
+                if (r < nt && c0 + c < a.dv) o_out[(size_t)(t0 + r) * a.heads * a.dv + (size_t)head * a.dv + c0 + c] = os[c][r];
+            }
+        }
         __syncthreads();
     }
     if (!STATE_ONLY && cut) {
@@ -173,9 +206,10 @@ __global__ void __launch_bounds__(256) linstate_rows_kernel(axq_linstate a, int 
 #pragma unroll
     for (int i = 0; i < E; i++) {
         const int e = elem_of<E>(g, i);
-        if (live && e < a.dk) st[(size_t)e * a.dv + col] = S[i];
-        if constexpr (STATE_ONLY)
-            if (col == 0 && e < a.dk) a.seg_decay[((size_t)seg * a.heads + head) * a.dk + e] = wp[i];
+#pragma unroll
+        for (int c = 0; c < C; c++)
+            if (col + 16 * c < a.dv && e < a.dk) st[(size_t)e * a.dv + col + 16 * c] = S[c][i];
+        if (product && col == 0 && e < a.dk) a.seg_decay[((size_t)seg * a.heads + head) * a.dk + e] = wp[WP > 1 ? i : 0];
     }
 }
 
@@ -192,33 +226,44 @@ __global__ void __launch_bounds__(256) linstate_scan_kernel(axq_linstate a, int 
     }
 }
 
-template <int E, bool TOKEN_DECAY, bool VEC>
+template <int E, bool TOKEN_DECAY, bool VEC, int C>
 int launch_rows_t(axq_ctx *ctx, const axq_linstate &a, int m, bool first, int segs) {
-    const int cols = (a.dv + 15) / 16, len = segs > 1 ? ((m + segs - 1) / segs + 15) / 16 * 16 : m;
+    const int cols = (a.dv + 16 * C - 1) / (16 * C), len = segs > 1 ? ((m + segs - 1) / segs + 15) / 16 * 16 : m;
     segs = (m + len - 1) / len;
     if (segs > 1) {
-        linstate_rows_kernel<E, TOKEN_DECAY, true, VEC><<<dim3(a.heads, cols, segs - 1), 256, 0, ctx->stream>>>(a, m, 1, len);
+        linstate_rows_kernel<E, TOKEN_DECAY, true, VEC, C><<<dim3(a.heads, cols, segs - 1), 256, 0, ctx->stream>>>(a, m, 1, len);
         linstate_scan_kernel<<<(unsigned)(((size_t)a.heads * a.dk * a.dv + 255) / 256), 256, 0, ctx->stream>>>(a, segs, first ? 1 : 0);
     }
-    linstate_rows_kernel<E, TOKEN_DECAY, false, VEC><<<dim3(a.heads, cols, segs), 256, 0, ctx->stream>>>(a, m, first ? 1 : 0, len);
+    linstate_rows_kernel<E, TOKEN_DECAY, false, VEC, C><<<dim3(a.heads, cols, segs), 256, 0, ctx->stream>>>(a, m, first ? 1 : 0, len);
     AXQ_LAUNCH_CHECK(ctx, "linstate_rows_kernel");
     return AXQ_OK;
 }
 
 template <int E>
 int launch_rows(axq_ctx *ctx, const axq_linstate &a, int m, bool first) {
-    const int wgs = a.heads * ((a.dv + 15) / 16);
-    int segs = 1;
-    if (a.seg_state && wgs < ctx->prop.multiProcessorCount) {
-        segs = 2 * ctx->prop.multiProcessorCount / wgs;
-        if (segs > m / 64) segs = m / 64;
-        if (segs > AXQ_LINSTATE_SEGS) segs = AXQ_LINSTATE_SEGS;
-        if (segs < 1) segs = 1;
-    }
+    const int cus = ctx->prop.multiProcessorCount;
     auto aligned = [](const void *p, int ld) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && ld % 4 == 0; };
     const bool vec = a.dk % 4 == 0 && aligned(a.q, a.ldq) && aligned(a.k, a.ldk) && (!a.wt || aligned(a.wt, a.ldw));
-    if (a.wt) return vec ? launch_rows_t<E, true, true>(ctx, a, m, first, segs) : launch_rows_t<E, true, false>(ctx, a, m, first, segs);
-    return vec ? launch_rows_t<E, false, true>(ctx, a, m, first, segs) : launch_rows_t<E, false, false>(ctx, a, m, first, segs);
+    auto segments = [&](int wgs) {
+        int segs = 1;
+        if (a.seg_state && wgs < cus) {
+            segs = 2 * cus / wgs;
+            if (segs > m / 64) segs = m / 64;
+            if (segs > AXQ_LINSTATE_SEGS) segs = AXQ_LINSTATE_SEGS;
+            if (segs < 1) segs = 1;
+        }
+        return segs;
+    };
+    // Two columns where they fill a workgroup's 32 and the registers stand it (checked for key sizes of 49..64 and 97..128, which read 16 bytes at a time;
+    // twice the segments keep two workgroups on each compute unit: half as many took 112, 63, 93 and 53 us).
+    if constexpr (E == 4 || E == 8)
+        if (vec && a.dv >= 32) {
+            const int segs = segments(a.heads * ((a.dv + 31) / 32));
+            return a.wt ? launch_rows_t<E, true, true, 2>(ctx, a, m, first, segs) : launch_rows_t<E, false, true, 2>(ctx, a, m, first, segs);
+        }
+    const int segs = segments(a.heads * ((a.dv + 15) / 16));
+    if (a.wt) return vec ? launch_rows_t<E, true, true, 1>(ctx, a, m, first, segs) : launch_rows_t<E, true, false, 1>(ctx, a, m, first, segs);
+    return vec ? launch_rows_t<E, false, true, 1>(ctx, a, m, first, segs) : launch_rows_t<E, false, false, 1>(ctx, a, m, first, segs);
 }
 
 // One token.  grid (heads, column blocks of CB): thread = (column, group of key elements); with a head norm one
