@@ -342,13 +342,20 @@ __global__ void __launch_bounds__(256) token_partial_kernel(Args g, float *part)
 }
 
 // att[i] = sum over the splits of the newest position, in order; a workgroup takes 64 elements, its four waves every
-// fourth split
+// fourth split, eight of them requested at a time
 __global__ void __launch_bounds__(256) token_combine_kernel(const float *part, const int32_t *pos, int n, float *att) {
     __shared__ float red[4][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = blockIdx.x * 64 + lane, splits = pos[0] / CHUNK + 1;
     float o = 0.f;
     if (i < n)
-        for (int s = wave; s < splits; s += 4) o += part[(size_t)s * n + i];
+        for (int s0 = wave; s0 < splits; s0 += 32) { // eight of them under way at a time
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = part[(size_t)(s0 + 4 * u < splits ? s0 + 4 * u : s0) * n + i];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                if (s0 + 4 * u < splits) o += v[u];
+        }
     red[wave][lane] = o;
     __syncthreads();
     if (wave == 0 && i < n) att[i] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);

@@ -409,9 +409,7 @@ __global__ void __launch_bounds__(256) token_partial_kernel(Args g, float *part)
     const int ldp = a.vdim + 2;
     for (int h = wave; h < rep; h += 4) { // scores of a head -> weights under the split's maximum
         const float s = ws[h * CHUNK + lane];
-        float mx = s;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
+        const float mx = axq_wave_max(s);
         const float w = __builtin_amdgcn_exp2f(s - mx); // a split has keys, so mx is finite
         const float sum = axq_wave_sum(w);
         ws[h * CHUNK + lane] = w;
@@ -449,23 +447,47 @@ __global__ void __launch_bounds__(256) token_partial_kernel(Args g, float *part)
     }
 }
 
-// The splits of the newest position put together: workgroup (head, 64 elements), its four waves every fourth split.
+// The splits of the newest position put together: workgroup (head, 64 elements), its four waves every fourth split.  A chain of latencies (position,
+// maxima and sums, values), in which a split's weight is made once, by the lane that has its maximum, and the values are on their way beside the maxima
+// (with route_lanes_kernel's shorter loops 209.6 to 204.5 us of a step of three layers at position 1200).
 __global__ void __launch_bounds__(256) token_combine_kernel(Args g, const float *part, float *att) {
     __shared__ float red[4][64];
     const axq_soft_attn &a = g.a;
-    const int h = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, e = blockIdx.y * 64 + lane, p = g.pos[0], ldp = a.vdim + 2;
+    const int h = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), e = blockIdx.y * 64 + lane, p = g.pos[0], ldp = a.vdim + 2;
     const int psplits = g.cpp / CHUNK, np = (seen_blocks(a, p) + CHUNK - 1) / CHUNK, n = np + p / CHUNK - first_token(a, p) / CHUNK + 1;
     auto at = [&](int i) { return part + ((size_t)(i < np ? i : psplits + i - np) * a.heads + h) * ldp; };
-    float mx = -1e30f;
-    for (int i = lane; i < n; i += 64) mx = fmaxf(mx, at(i)[a.vdim]);
+    // a lane: the largest score and the sum of one split of 64; the wave's first values are requested beside them
+    constexpr int AHEAD = 8;
+    float first[AHEAD];
+    const int ec = e < a.vdim ? e : 0;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
-    float sum = 0.f;
-    for (int i = lane; i < n; i += 64) sum = fmaf(at(i)[a.vdim + 1], __builtin_amdgcn_exp2f(at(i)[a.vdim] - mx), sum);
+    for (int u = 0; u < AHEAD; u++) first[u] = at(wave + 4 * u < n ? wave + 4 * u : n - 1)[ec];
+    float m = -1e30f, s = 0.f;
+    if (lane < n) {
+        m = at(lane)[a.vdim];
+        s = at(lane)[a.vdim + 1];
+    }
+    float mx = fmaxf(-1e30f, m);
+    for (int i = lane + 64; i < n; i += 64) mx = fmaxf(mx, at(i)[a.vdim]);
+    mx = axq_wave_max(mx);
+    float sum = 0.f, o = 0.f;
+    for (int base = 0; base < n; base += 64) {
+        const int left = n - base < 64 ? n - base : 64;
+        if (base > 0 && lane < left) {
+            m = at(base + lane)[a.vdim];
+            s = at(base + lane)[a.vdim + 1];
+        }
+        const float w = lane < left ? __builtin_amdgcn_exp2f(m - mx) : 0.f;
+        sum = fmaf(lane < left ? s : 0.f, w, sum);
+        auto weight = [&](int i) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), i)); };
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            if (wave + 4 * u >= left) break;
+            o = fmaf(base ? at(base + wave + 4 * u)[ec] : first[u], weight(wave + 4 * u), o);
+        }
+        for (int i = wave + 4 * AHEAD; i < left; i += 4) o = fmaf(at(base + i)[ec], weight(i), o);
+    }
     sum = axq_wave_sum(sum);
-    float o = 0.f;
-    if (e < a.vdim)
-        for (int i = wave; i < n; i += 4) o = fmaf(at(i)[e], __builtin_amdgcn_exp2f(at(i)[a.vdim] - mx), o);
     red[wave][lane] = o;
     __syncthreads();
     if (wave == 0 && e < a.vdim)

@@ -237,9 +237,21 @@ __device__ inline float axq_wave_sum(float s) {
     s += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0x4E, 0xf, 0xf, true));  // quad: lanes ^ 2
     s += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0x141, 0xf, 0xf, true)); // half-row mirror
     s += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0x140, 0xf, 0xf, true)); // row mirror
-    s += __shfl_xor(s, 16);
-    s += __shfl_xor(s, 32);
-    return s;
+    auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, s), __builtin_bit_cast(int, s), false, false); // of each two rows: the first, the second
+    s = __builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]);
+    r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, s), __builtin_bit_cast(int, s), false, false);
+    return __builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]);
+}
+// (the casts to int: __builtin_bit_cast of a vector's element takes the first one) fmaxf ignores a NaN beside a number
+__device__ inline float axq_wave_max(float s) {
+    s = fmaxf(s, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0xB1, 0xf, 0xf, true)));
+    s = fmaxf(s, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0x4E, 0xf, 0xf, true)));
+    s = fmaxf(s, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0x141, 0xf, 0xf, true)));
+    s = fmaxf(s, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0x140, 0xf, 0xf, true)));
+    auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, s), __builtin_bit_cast(int, s), false, false);
+    s = fmaxf(__builtin_bit_cast(float, (int)r[0]), __builtin_bit_cast(float, (int)r[1]));
+    r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, s), __builtin_bit_cast(int, s), false, false);
+    return fmaxf(__builtin_bit_cast(float, (int)r[0]), __builtin_bit_cast(float, (int)r[1]));
 }
 // Sum over a workgroup of whole waves (at most 16); scratch: 16 floats.
 __device__ inline float axq_block_sum(float v, float *scratch) {
@@ -249,7 +261,14 @@ __device__ inline float axq_block_sum(float v, float *scratch) {
     if ((threadIdx.x & 63) == 0) scratch[wave] = v;
     __syncthreads();
     float t = 0.f;
-    for (int i = 0; i < nw; i++) t += scratch[i];
+    for (int i = 0; i < nw; i += 4) { // four of them under way at a time
+        float s[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) s[u] = scratch[i + u < nw ? i + u : i];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (i + u < nw) t += s[u];
+    }
     return t;
 }
 #endif

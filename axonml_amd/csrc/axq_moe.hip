@@ -21,7 +21,7 @@ __device__ inline float lane_of(float v, int lane) { return __builtin_bit_cast(f
 
 // Up to 64 experts: a wave per row, a lane per expert.  Places are counted: how many of the others come before this one.
 __global__ void __launch_bounds__(64) route_lanes_kernel(axq_moe_router r, const float *z, int ldz, int32_t *sel, float *wt) {
-    const int t = blockIdx.x, e = threadIdx.x, per = r.experts / r.groups, group = e / per;
+    const int t = blockIdx.x, e = threadIdx.x, per = r.experts / r.groups, group = e / per, first = group * per;
     float s = e < r.experts ? axq_sigmoid(z[(size_t)t * ldz + e]) : 0.f;
     if (!(s == s)) s = 0.f; // with NaN among them places would not be distinct, and `sel` must hold experts whatever comes
     bool usable = e < r.experts;
@@ -29,7 +29,7 @@ __global__ void __launch_bounds__(64) route_lanes_kernel(axq_moe_router r, const
         float a = 0.f, b = 0.f; // scores are positive; a group of one has no second
         for (int j = 0; j < r.experts; j++) {
             const float v = lane_of(s, j);
-            if (j / per == group) {
+            if (j >= first && j - first < per) {
                 b = fmaxf(b, fminf(a, v));
                 a = fmaxf(a, v);
             }
