@@ -665,9 +665,13 @@ __global__ void __launch_bounds__(256) gemm_prep_x_f32_kernel(const float *x, co
 
 } // namespace
 
-// The context's GEMM scratch, grown to `need` bytes (work that still uses the old one is waited for first).
+// The context's GEMM scratch, grown to `need` bytes (work that still uses the old one is waited for first; not while the stream is captured, which the
+// wait would spoil for good: the stream took no launch any more).
 int axq_gemm_reserve(axq_ctx *ctx, size_t need) {
     if (ctx->gemm_scratch_bytes >= need) return AXQ_OK;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone)
+        return axq_fail(ctx, AXQ_ERR_ALLOCATION_FAILED, "GEMM scratch of %zu bytes: cannot grow while the stream is captured", need);
     const char *most = getenv("AXQ_GEMM_SCRATCH_MAX"); // development knob: as if the card had no room for more bytes than this
     if (most && need > strtoull(most, nullptr, 10))
         return axq_fail(ctx, AXQ_ERR_ALLOCATION_FAILED, "GEMM scratch of %zu bytes: beyond AXQ_GEMM_SCRATCH_MAX", need);
