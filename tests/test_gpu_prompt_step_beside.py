@@ -1,5 +1,5 @@
 """A prompt's last token goes through the layers beside the rows in front of it: logits, caches, position and what follows against the oracle, prompts in
-several chunks, on top of a context, of a batched model, again and again, and where the rows find no room."""
+several chunks, on top of a context, of a batched model, again and again, and where the rows, or the graph of the steps to come, find no room."""
 import numpy as np
 import pytest
 
@@ -78,3 +78,21 @@ def test_without_room_for_the_rows(monkeypatch):
     gpu.close()
     cpu.close()
     ctx.close()
+
+
+def test_without_room_for_the_graph(ctx, monkeypatch):
+    c = tiny_config(max_seq_len=320)
+    w = random_weights(c, 11)
+    cpu, gpu = load_oracle(c, w), load_gpu(ctx, c, w)
+    tokens = np.random.default_rng(11).integers(0, c["vocab_size"], size=300)
+    want = _walk(cpu, tokens)
+    monkeypatch.setenv("AXQ_GRAPH_ROOM", "0")
+    got = gpu.forward_tokens(tokens)  # needs none
+    assert got[0] == want[0] and max_rel_err(got[1], want[1], DECODE_FLOOR) <= DECODE_RTOL
+    with pytest.raises(Exception, match="AXQ_GRAPH_ROOM"):
+        gpu.forward(int(got[0]))  # a step does
+    monkeypatch.delenv("AXQ_GRAPH_ROOM")
+    want, got = cpu.forward(int(want[0]), 300), gpu.forward(int(got[0]))
+    assert got[0] == want[0] and max_rel_err(got[1], want[1], DECODE_FLOOR) <= DECODE_RTOL
+    gpu.close()
+    cpu.close()
