@@ -11,6 +11,12 @@ from tests.util import DECODE_FLOOR, DECODE_RTOL, max_rel_err
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def beside(monkeypatch):
+    """However small the model."""
+    monkeypatch.setenv("AXQ_STEP_BESIDE", "1")
+
+
 def _walk(cpu, tokens, pos=0):
     for t in tokens:
         nxt, lg = cpu.forward(int(t), pos)
@@ -96,3 +102,18 @@ def test_without_room_for_the_graph(ctx, monkeypatch):
     assert got[0] == want[0] and max_rel_err(got[1], want[1], DECODE_FLOOR) <= DECODE_RTOL
     gpu.close()
     cpu.close()
+
+
+@pytest.mark.parametrize("rows,layers,width", [(191, 2, 1024), (192, 2, 256), (1024, 2, 1024)])
+def test_both_sides_of_the_rule(ctx, monkeypatch, rows, layers, width):
+    """The same bits beside the rows and behind them, on both sides of where one gives way to the other."""
+    c = tiny_config(max_seq_len=rows + 2, num_layers=layers, hidden_size=width, intermediate_size=256, vocab_size=64)
+    gpu = load_gpu(ctx, c, random_weights(c, rows))
+    tokens = np.random.default_rng(rows).integers(0, c["vocab_size"], size=rows + 1)
+    got = []
+    for knob in ("0", "1", None):
+        monkeypatch.delenv("AXQ_STEP_BESIDE") if knob is None else monkeypatch.setenv("AXQ_STEP_BESIDE", knob)
+        gpu.reset()
+        got.append(gpu.forward_tokens(tokens)[1])
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    gpu.close()
