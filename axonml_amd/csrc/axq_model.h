@@ -58,7 +58,7 @@ struct axq_model {
     bool graph_ok;
     hipGraphExec_t graph_f;         // the same with one attention workgroup per head (short contexts)
     bool graph_f_ok;
-    int fused_max;                  // contexts up to this many positions take graph_f
+    int fused_max, fused_max_one;   // contexts up to this many positions take graph_bf, and with one sequence graph_f
     int prompt_chunk;               // most prompt rows per pass through the layers
     bool attn_mfma;                 // prompt attention of many rows on the matrix pipe (development knob AXQ_ATTN_MFMA=0: off)
     axq_stack *stack = nullptr;     // layers described one by one (axq_model_create_stack) instead of the LLaMA shape above

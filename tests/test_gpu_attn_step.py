@@ -22,6 +22,10 @@ pytestmark = pytest.mark.gpu
     (48, 256, 8, 2, 0, (16, 65)),
     (64, 128, 4, 2, 37, (36, 37, 150)),
     (1, 128, 4, 2, 130, (129, 130, 300)),
+    (1, 256, 2, 2, 0, (319, 320, 321)),         # where one sequence's positions are split
+    (1, 256, 4, 1, 0, (511, 512, 513)),
+    (1, 128, 4, 2, 0, (639, 640, 641)),
+    (3, 256, 2, 2, 0, (320, 639, 640, 641)),
 ])
 def test_step_attention_at_the_edges_of_its_passes(ctx, n_seq, head_dim, heads, kv, window, lengths):
     c = tiny_config(max_seq_len=max(lengths) + 8, num_heads=heads, num_kv_heads=kv, head_dim=head_dim, sliding_window=window)
