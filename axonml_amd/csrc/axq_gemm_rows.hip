@@ -1876,9 +1876,9 @@ int launch_rows(axq_ctx *ctx, const RowsArgs &a, const RowsPlan &p) {
 
 } // namespace
 
-// Packed types at any number of rows, whole superblocks in the planes.
+// Packed types at any number of rows, whole superblocks in the planes; K a multiple of 64, which every GEMM asks for, whatever its planes hold.
 bool axq_dev_rows_gemm_covers(const axq_weight *w, int rows) {
-    if (w->kp % 256 != 0 || w->kp > INT32_MAX || w->n_rows > INT32_MAX || rows < 1) return false;
+    if (w->kp % 256 != 0 || w->k % 64 != 0 || w->kp > INT32_MAX || w->n_rows > INT32_MAX || rows < 1) return false;
     switch (w->type) {
     case AXQ_Q4_K: case AXQ_Q5_K: case AXQ_Q6_K: case AXQ_Q4_0: case AXQ_Q4_1: case AXQ_Q5_0: case AXQ_Q5_1: case AXQ_Q8_0: return true;
     default: return false;

@@ -189,7 +189,7 @@ AXQ_API int axq_gemv_f32(axq_ctx *ctx, const axq_weight *w, const float *x, int 
  * synchronised.  Every call on a GPU shares that GPU's array (it needs no clearing: each call writes what it
  * reads), so calls that overlap on one GPU -- from two contexts or two streams -- race; serialise them. */
 AXQ_API int axq_gemv_f32_static(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, const float *bias, float *y);
-/* y[m, n_rows] = x[m, k] * W^T, x in bf16 (raw uint16), y f32.  Prefill path. */
+/* y[m, n_rows] = x[m, k] * W^T, x in bf16 (raw uint16), y f32.  Prefill path; k a multiple of 64. */
 AXQ_API int axq_gemm_bf16(axq_ctx *ctx, const axq_weight *w, const uint16_t *x_bf16, int m, float *y, int mem);
 
 /* ---- decode: LLaMA/Mistral-shape model, llm/src/llama.rs:731-762, 900-977 - */

@@ -54,3 +54,17 @@ def test_large_elements_in_the_last_block(ctx, qtype):
     bits = q.f32_to_bf16_bits(x)
     assert _off(q.quantized_matmul_bf16(bits, qt, ctx), q.bf16_bits_to_f32(bits).astype(np.float64) @ w.T) <= 4e-7
     assert _off(q.quantized_matmul(x[:20], qt, None, ctx), x[:20].astype(np.float64) @ w.T) <= 4e-7
+
+
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("k", [736, 992, 1760, 4064, 4128])
+def test_the_gemm_takes_multiples_of_64(ctx, qtype, k):
+    """bf16 rows of another K are refused, whatever the planes hold; f32 rows of it are not."""
+    packed = o.quantize(qtype, gen_weight(np.random.default_rng(k), 40, k))
+    qt = q.QuantizedTensor([40, k], qtype, packed)
+    x = np.random.default_rng(k + 1).standard_normal((9, k)).astype(np.float32)
+    for rows in (1, 9):
+        with pytest.raises(Exception, match="64"):
+            q.quantized_matmul_bf16(q.f32_to_bf16_bits(x[:rows]), qt, ctx)
+    want = x.astype(np.float64) @ o.dequantize(qtype, packed, 40 * k).reshape(40, k).astype(np.float64).T
+    assert _off(q.quantized_matmul(x, qt, None, ctx), want) <= 3e-7
