@@ -47,14 +47,14 @@ int axq_aux_join(axq_ctx *ctx, int n);
 //
 // The bytes are exactly those of the packed (`to_bytes`) image, permuted (behind a row's last block zeros, where `kp` is beyond k), so
 // upload -> download is the identity and HBM traffic per matmul equals the
-// packed size.  For Q4_K the 128 code bytes of a superblock are further
+// packed size (and those zeros).  For Q4_K the 128 code bytes of a superblock are further
 // interleaved inside 16-superblock "slices" so that one wavefront reads two
 // fully contiguous 1 KiB runs per row (see q4k_code_offset).
 // ---------------------------------------------------------------------------
 struct axq_weight {
     int type;
     int64_t n_rows, k;
-    int64_t kp;          // columns that the planes' rows hold: k, or with blocks of 32 whole superblocks of 256, the last blocks zeros (see axq_weight_alloc)
+    int64_t kp;          // columns that rows of scales hold: k, or with blocks of 32 whole superblocks of 256, the last blocks zeros; up to there codes may be read, which behind k may be anything (see axq_weight_alloc)
     size_t packed_bytes; // size of the to_bytes image
     uint8_t *base;       // device allocation
     size_t alloc_bytes;

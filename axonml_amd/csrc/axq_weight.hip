@@ -56,20 +56,24 @@ int axq_weight_alloc(axq_ctx *ctx, int type, int64_t n_rows, int64_t k, axq_weig
     w->n_rows = n_rows;
     w->k = k;
     w->packed_bytes = axq_packed_bytes(type, (size_t)n_rows * (size_t)k);
-    // Blocks of 32: rows of whole superblocks in the planes, zeros behind the last block, so that such weights take the kernels that walk superblocks (at
-    // least 768 columns: a third more memory at most).  us, through two f16 planes or vector by vector before and so: bf16 rows Q5_1 14336 x 3904, 2048: 598
-    // 465; Q4_0 4096 x 4032, 509: 59.8 40.8; f32 rows Q4_0 480 x 1216, 7: 29.3 8.7; Q5_0 673 x 8896, 5: 28.4 13.2; Q4_0 4096 x 4032, 21: 22.4 17.5; one vector, Q4_0 11008 x
-    // 4032: 7.47 7.32
+    // Blocks of 32: rows' scales (and fifth bits) of whole superblocks, zeros behind the last block, so that such weights take the kernels that walk
+    // superblocks (from 768 columns on; fewer were not tried).  The codes of rows below 2304 columns lie without a gap: what those kernels read behind a row's end are
+    // the next row's, finite whatever they are, which meet scales and rows of x of zero.  11008 rows, us, each of many weights in turn, kernels for any K; whole superblocks of
+    // codes too; codes without a gap:
+    //   one vector     Q4_0 1088 4.31 4.68 4.36, 1600 4.66 4.81 4.64, 2112 6.32 6.47 6.37, 2880 6.99 6.69 6.94; Q8_0 1088 5.74 5.96 5.76, 2880 11.7 11.1 11.6; Q5_1 1088
+    //                  5.23 5.42 5.30, 2880 8.92 8.27 8.50 (whole cache lines pay for their zeros in long rows)
+    //   3 f32 rows     Q4_0 832 11.3 6.9 6.9, 1600 13.1 8.5 8.4; Q8_0 1600 18.8 10.1 9.9;  8: Q5_1 832 19.7 16.0 16.2, 1600 28.2 21.1 21.4; 21: Q8_0 1344 24.7 18.5 19.2
+    //   512 bf16 rows  Q4_0 832 49.0 37.6 37.5; Q8_0 1600 71.3 54.6 54.6; Q5_1 2112 93.9 75.0 75.0
     w->kp = bs == 32 && k >= 768 ? (int64_t)axq_align_up((size_t)k, 256) : k;
     size_t nblk = (size_t)w->kp / bs;
+    const size_t kc = (size_t)(k >= 2304 ? w->kp : k); // columns of a row of codes
     size_t meta_per_block = 0, qh_per_block = 0;
-    const size_t kp = (size_t)w->kp;
     switch (type) {
-    case AXQ_Q8_0: w->codes_pitch = kp; meta_per_block = 2; break;
-    case AXQ_Q4_0: w->codes_pitch = kp / 2; meta_per_block = 2; break;
-    case AXQ_Q4_1: w->codes_pitch = kp / 2; meta_per_block = 4; break;
-    case AXQ_Q5_0: w->codes_pitch = kp / 2; meta_per_block = 2; qh_per_block = 4; break;
-    case AXQ_Q5_1: w->codes_pitch = kp / 2; meta_per_block = 4; qh_per_block = 4; break;
+    case AXQ_Q8_0: w->codes_pitch = kc; meta_per_block = 2; break;
+    case AXQ_Q4_0: w->codes_pitch = kc / 2; meta_per_block = 2; break;
+    case AXQ_Q4_1: w->codes_pitch = kc / 2; meta_per_block = 4; break;
+    case AXQ_Q5_0: w->codes_pitch = kc / 2; meta_per_block = 2; qh_per_block = 4; break;
+    case AXQ_Q5_1: w->codes_pitch = kc / 2; meta_per_block = 4; qh_per_block = 4; break;
     case AXQ_Q4_K: w->codes_pitch = (size_t)k / 2; meta_per_block = 16; break;
     case AXQ_Q6_K: w->codes_pitch = (size_t)k / 2; meta_per_block = 18; qh_per_block = 64; break; // scales, then the row's d values
     case AXQ_Q5_K: w->codes_pitch = (size_t)k / 2; meta_per_block = 16; qh_per_block = 32; break; // Q4_K's planes and the fifth bits as they are
@@ -79,7 +83,7 @@ int axq_weight_alloc(axq_ctx *ctx, int type, int64_t n_rows, int64_t k, axq_weig
     }
     w->meta_pitch = type == AXQ_Q6_K ? axq_align_up(nblk * meta_per_block, 16) : nblk * meta_per_block;
     w->qh_pitch = nblk * qh_per_block;
-    size_t codes_bytes = axq_align_up(w->codes_pitch * (size_t)n_rows, 256);
+    size_t codes_bytes = axq_align_up(w->codes_pitch * (size_t)n_rows + ((size_t)w->kp - kc), 256); // and what is read behind the last row
     size_t meta_bytes = axq_align_up(w->meta_pitch * (size_t)n_rows, 256);
     size_t qh_bytes = axq_align_up(w->qh_pitch * (size_t)n_rows, 256);
     // 64 bytes of slack: the GEMV kernels may read (and discard) up to one
