@@ -74,3 +74,17 @@ def test_scratch_that_would_grow_in_the_capture(monkeypatch, most):
     gpu.close()
     cpu.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("fused", ["0", "14"])
+@pytest.mark.parametrize("n_seq", [5, 12, 40])
+def test_steps_whose_positions_are_split(ctx, monkeypatch, n_seq, fused):
+    """A graph of their own, from the first position on or in the middle of steps that were not."""
+    monkeypatch.setenv("AXQ_ATTN_FUSED_MAX", fused)
+    c = tiny_config(max_seq_len=48)
+    w = random_weights(c, 50 + n_seq)
+    cpu, gpu = load_oracle(c, w), load_gpu(ctx, c, w)
+    gpu.set_batch(n_seq)
+    _agree(gpu, cpu, n_seq, 3, 0, 40)
+    gpu.close()
+    cpu.close()

@@ -12,9 +12,9 @@ from tests.util import gen_weight
 pytestmark = pytest.mark.gpu
 
 SIZE = {o.Q4_K: 144, o.Q5_K: 176, o.Q6_K: 210, o.Q4_0: 18, o.Q4_1: 20, o.Q5_0: 22, o.Q5_1: 24, o.Q8_0: 34}
-# rows, columns, K and whether the rows are bf16, of a call for every kernel; the last has no split of K, its columns being no multiple of four
+# rows, columns, K and whether the rows are bf16, of a call for every kernel; APART: K in parts, which are too short for that kernel, and whole, by more than 128 tiles
 WIDE = [(600, 1600, 768, False), (1160, 1600, 1024, True)]
-APART = [(50, 1601, 2048, False), (100, 1601, 2304, True)]
+APART = [(50, 1601, 2048, False), (100, 1601, 2304, True), (50, 16387, 2048, False), (100, 16387, 2304, True)]
 BLOCK32 = [(130, 16500, 768, True), (257, 11009, 1024, True), (130, 16499, 2304, False), (65, 16500, 1024, False)]
 
 

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
 @pytest.mark.parametrize("rows,n,k,bf16", [
-    (40, 129, 2048, False), (64, 127, 2304, False), (41, 1, 2560, False),  # columns that no split of K takes: eight, nine, ten superblocks
+    (40, 129, 2048, False), (64, 127, 2304, False), (41, 1, 2560, False),  # in parts of one superblock, which are too short for it
     (65, 257, 2304, True), (128, 130, 2816, True),
     (48, 8192, 8192, False), (65, 12032, 4608, True),                      # K in four parts of eight and in two of nine
     (130, 2048, 16384, True),                                              # two tiles of rows, eight parts
@@ -21,6 +21,16 @@ pytestmark = pytest.mark.gpu
 def test_halves_with_their_own_k(ctx, qtype, rows, n, k, bf16):
     rng = np.random.default_rng(rows + n + k + qtype)
     packed = o.quantize(qtype, gen_weight(rng, n, k))
+    x = rng.standard_normal((rows, k)).astype(np.float32) * (10.0 ** rng.integers(-3, 4, size=(rows, 1))).astype(np.float32)
+    _check(ctx, qtype, n, k, packed, x, bias=None if bf16 else rng.standard_normal(n).astype(np.float32), bf16=bf16)
+
+
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
+@pytest.mark.parametrize("rows,n,k,bf16", [(40, 16512, 2048, False), (64, 16386, 2304, False), (41, 16385, 2560, False), (65, 16387, 2304, True), (128, 16514, 2816, True)])
+def test_halves_with_their_own_k_and_all_of_it(ctx, qtype, rows, n, k, bf16):
+    """More tiles than half the compute units, so that K is not split: eight to eleven superblocks."""
+    rng = np.random.default_rng(rows + n + k + qtype)
+    packed = o.quantize(qtype, gen_weight(rng, 1009, k)).reshape(1009, -1)[np.arange(n) % 1009].reshape(-1)
     x = rng.standard_normal((rows, k)).astype(np.float32) * (10.0 ** rng.integers(-3, 4, size=(rows, 1))).astype(np.float32)
     _check(ctx, qtype, n, k, packed, x, bias=None if bf16 else rng.standard_normal(n).astype(np.float32), bf16=bf16)
 
