@@ -449,7 +449,7 @@ __global__ void __launch_bounds__(256) token_partial_kernel(Args g, float *part)
 
 // The splits of the newest position put together: workgroup (head, 64 elements), its four waves every fourth split.  A chain of latencies (position,
 // maxima and sums, values), in which a split's weight is made once, by the lane that has its maximum, and the values are on their way beside the maxima
-// (with route_lanes_kernel's shorter loops 209.6 to 204.5 us of a step of three layers at position 1200).
+// (with route_lanes_kernel's and argmax_kernel's shorter chains 210.5 to 207.8 us of a step of three layers at position 1200, where runs differ by 1).
 __global__ void __launch_bounds__(256) token_combine_kernel(Args g, const float *part, float *att) {
     __shared__ float red[4][64];
     const axq_soft_attn &a = g.a;

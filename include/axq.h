@@ -251,7 +251,8 @@ AXQ_API int axq_model_layer_runs(const axq_model *m);
 /* Several sequences side by side (the batch dimension of forward_with_cache's input ids and of KVCache,
  * llama.rs:731-762, attention.rs:28-35): n_seq = 1..64 caches and position counters; a batched step feeds
  * one token of every sequence and reads the weights once for all of them (up to eight sequences through the
- * small-batch GEMV as a replayed graph, more through the GEMM on f32 rows, which needs K a multiple of 64).  Calling it discards every
+ * small-batch GEMV, more through the GEMM on f32 rows, which needs K a multiple of 64; as a replayed graph, with the GEMM
+ * from the ninth such step on, or as plain launches where there is no room for a graph).  Calling it discards every
  * cache and starts all sequences at position 0.  The one-sequence calls above keep working on sequence 0. */
 AXQ_API int axq_model_set_batch(axq_model *m, int n_seq);
 AXQ_API int axq_model_batch(const axq_model *m);
