@@ -21,7 +21,7 @@ template <bool F32>
 __global__ void __launch_bounds__(64) prep_kernel(Args g) {
     const axq_sig_attn &a = g.a;
     const int t = blockIdx.y, lane = threadIdx.x, p = g.pos ? g.pos[0] : g.pos0 + t;
-    int h = blockIdx.x;
+    int h = blockIdx.x + (g.q ? 0 : a.heads);
     if (h < a.heads) {
         const float *q = g.q + (size_t)t * g.ldq + (size_t)h * a.dim;
         float ss = 0.f;
@@ -429,16 +429,17 @@ int axq_sig_attn_rows(axq_ctx *ctx, const axq_sig_attn &a, const float *q, const
     if (m < 1 || pos0 < 0 || pos0 + m > a.cap)
         return axq_fail(ctx, AXQ_ERR_OVERFLOW, "Numerical overflow during quantization: positions %d .. %d beyond the cache of %d", pos0, pos0 + m, a.cap);
     const Args g = make_args(a, q, k, v, ldq, ldk, ldv, m, pos0, nullptr, qscratch);
+    const int queries = q ? a.heads : 0; // without q: the keys and values alone
     if (a.f32) {
-        prep_kernel<true><<<dim3(a.heads + 2 * a.kv_heads, m), 64, 0, ctx->stream>>>(g);
-        rows_f32_kernel<<<dim3(a.heads, m), 256, f32_rows_lds(a), ctx->stream>>>(g, out);
+        prep_kernel<true><<<dim3(queries + 2 * a.kv_heads, m), 64, 0, ctx->stream>>>(g);
+        if (q) rows_f32_kernel<<<dim3(a.heads, m), 256, f32_rows_lds(a), ctx->stream>>>(g, out);
     } else {
-        prep_kernel<false><<<dim3(a.heads + a.kv_heads, m), 64, 0, ctx->stream>>>(g);
+        prep_kernel<false><<<dim3(queries + a.kv_heads, m), 64, 0, ctx->stream>>>(g);
         append_values_kernel<<<dim3((m + 31) / 32, (a.vdim + 31) / 32, a.kv_heads), 256, 0, ctx->stream>>>(g);
-        if ((rc = g.dp == 64 ? launch_mfma_k<4>(ctx, g, out) : (g.dp == 128 ? launch_mfma_k<8>(ctx, g, out) : launch_mfma_k<16>(ctx, g, out)))) return rc;
+        if (q && (rc = g.dp == 64 ? launch_mfma_k<4>(ctx, g, out) : (g.dp == 128 ? launch_mfma_k<8>(ctx, g, out) : launch_mfma_k<16>(ctx, g, out)))) return rc;
     }
     AXQ_LAUNCH_CHECK(ctx, "sigmoid attention of rows");
-    return axq_rows_zero_tail(ctx, m, a.heads * a.vdim, out);
+    return q ? axq_rows_zero_tail(ctx, m, a.heads * a.vdim, out) : AXQ_OK;
 }
 
 int axq_sig_attn_token(axq_ctx *ctx, const axq_sig_attn &a, const float *q, const float *k, const float *v, const int32_t *pos, void *qscratch,

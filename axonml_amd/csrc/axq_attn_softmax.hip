@@ -38,7 +38,7 @@ template <bool F32>
 __global__ void __launch_bounds__(256) prep_kernel(Args g) {
     const axq_soft_attn &a = g.a;
     const int t = blockIdx.y, lane = threadIdx.x & 63, p = g.pos ? g.pos[0] : g.pos0 + t;
-    int h = blockIdx.x * 4 + (threadIdx.x >> 6);
+    int h = blockIdx.x * 4 + (threadIdx.x >> 6) + (g.q ? 0 : a.heads);
     if (h >= a.heads + (F32 ? 2 : 1) * a.kv_heads) return;
     if (h < a.heads) {
         const float *q = g.q + (size_t)t * g.ldq + (size_t)h * a.dim;
@@ -585,18 +585,19 @@ int axq_soft_attn_rows(axq_ctx *ctx, const axq_soft_attn &a, const float *q, con
     if (m < 1 || pos0 < 0 || pos0 + m > a.cap)
         return axq_fail(ctx, AXQ_ERR_OVERFLOW, "Numerical overflow during quantization: positions %d .. %d beyond the cache of %d", pos0, pos0 + m, a.cap);
     const Args g = make_args(a, q, k, v, gate, ldq, ldk, ldv, m, pos0, nullptr, qscratch);
+    const int queries = q ? a.heads : 0; // without q: the keys and values alone
     if (a.f32) {
-        prep_kernel<true><<<dim3((a.heads + 2 * a.kv_heads + 3) / 4, m), 256, 0, ctx->stream>>>(g);
+        prep_kernel<true><<<dim3((queries + 2 * a.kv_heads + 3) / 4, m), 256, 0, ctx->stream>>>(g);
         launch_pool<true>(ctx, g);
-        rows_f32_kernel<<<dim3(a.heads, m), 256, f32_rows_lds(a), ctx->stream>>>(g, out);
+        if (q) rows_f32_kernel<<<dim3(a.heads, m), 256, f32_rows_lds(a), ctx->stream>>>(g, out);
     } else {
-        prep_kernel<false><<<dim3((a.heads + a.kv_heads + 3) / 4, m), 256, 0, ctx->stream>>>(g);
+        prep_kernel<false><<<dim3((queries + a.kv_heads + 3) / 4, m), 256, 0, ctx->stream>>>(g);
         append_values_kernel<<<dim3((m + 31) / 32, (a.vdim + 31) / 32, a.kv_heads), 256, 0, ctx->stream>>>(g);
         launch_pool<false>(ctx, g);
-        if ((rc = g.dp == 64 ? launch_mfma_k<4>(ctx, g, out) : (g.dp == 128 ? launch_mfma_k<8>(ctx, g, out) : launch_mfma_k<16>(ctx, g, out)))) return rc;
+        if (q && (rc = g.dp == 64 ? launch_mfma_k<4>(ctx, g, out) : (g.dp == 128 ? launch_mfma_k<8>(ctx, g, out) : launch_mfma_k<16>(ctx, g, out)))) return rc;
     }
     AXQ_LAUNCH_CHECK(ctx, "softmax attention of rows");
-    return axq_rows_zero_tail(ctx, m, a.heads * a.vdim, out);
+    return q ? axq_rows_zero_tail(ctx, m, a.heads * a.vdim, out) : AXQ_OK;
 }
 
 int axq_soft_attn_token(axq_ctx *ctx, const axq_soft_attn &a, const float *q, const float *k, const float *v, const float *gate,

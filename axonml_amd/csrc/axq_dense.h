@@ -160,7 +160,7 @@ size_t axq_sig_attn_k_bytes(const axq_sig_attn &a);
 size_t axq_sig_attn_v_bytes(const axq_sig_attn &a);
 size_t axq_sig_attn_q_bytes(const axq_sig_attn &a, int m);   // scratch for the prepared queries of m rows
 size_t axq_sig_attn_part_bytes(const axq_sig_attn &a);       // scratch of a decode step
-// rows q [m][ldq], k, v (same row stride) at positions pos0.. -> cache, then attention of every row.
+// rows q [m][ldq], k, v (same row stride) at positions pos0.. -> cache, then attention of every row; without q the cache alone.
 int axq_sig_attn_rows(axq_ctx *ctx, const axq_sig_attn &a, const float *q, const float *k, const float *v, int ldq, int ldk, int ldv, int m,
                       int pos0, void *qscratch, axq_rows_out out);
 // one token at position *pos -> att f32 [heads * vdim]
@@ -186,7 +186,7 @@ size_t axq_soft_attn_pk_bytes(const axq_soft_attn &a);
 size_t axq_soft_attn_pv_bytes(const axq_soft_attn &a);
 size_t axq_soft_attn_q_bytes(const axq_soft_attn &a, int m);
 size_t axq_soft_attn_part_bytes(const axq_soft_attn &a);
-// q [m][ldq], k [m][ldk], v [m][ldv] (v may be k: it is not rotated) at positions pos0.. -> cache, then attention of every row;
+// q [m][ldq], k [m][ldk], v [m][ldv] (v may be k: it is not rotated) at positions pos0.. -> cache, then attention of every row (without q the cache alone);
 // gate [m][heads] (NULL: none) multiplies each head's result
 int axq_soft_attn_rows(axq_ctx *ctx, const axq_soft_attn &a, const float *q, const float *k, const float *v, int ldq, int ldk, int ldv,
                        const float *gate, int m, int pos0, void *qscratch, axq_rows_out out);

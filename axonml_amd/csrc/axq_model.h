@@ -79,9 +79,9 @@ void axq_model_drop_graphs(axq_model *m);
 // axq_stack.hip: what the stepping functions of axq_decode.hip call for a model with m->stack set.
 // One token (m->tok at position *m->pos) through the layers to m->logits; fit for graph capture.
 int axq_stack_step(axq_model *m);
-// nb tokens at positions pos0 .. pos0 + nb - 1; afterwards axq_stack_logits_rows can be asked for any of them.
+// nb tokens at positions pos0 .. pos0 + nb - 1; afterwards axq_stack_logits_rows can be asked for any of them, unless `results` said that nobody will.
 // layers: where the residual stream after layer run 0 goes (host; NULL: nowhere), and `layer_stride` elements on after every next one.
-int axq_stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, float *layers = nullptr, size_t layer_stride = 0);
+int axq_stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, bool results, float *layers, size_t layer_stride);
 // the same, and the step of m->tok at *m->pos = pos0 + nb, to m->logits: as axq_stack_rows and then axq_stack_step leave it
 int axq_stack_rows_and_step(axq_model *m, const int32_t *toks, int nb, int pos0);
 // logits of `n` rows (indices within the last axq_stack_rows, on the host) -> host memory

@@ -663,8 +663,18 @@ int step_head(axq_model *m) {
 
 namespace {
 
-// `then_step`: behind every run's mixer the same run of the step of the next token, on ctx->aux_stream[0]
-int stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, float *layers, size_t layer_stride, bool then_step) {
+// Of the last run's first products over rows whose results nobody reads: what its cache or state takes.
+std::vector<First> cache_firsts(const axq_layer_config &c) {
+    std::vector<First> f = mixer_firsts(c);
+    if (c.mixer == AXQ_MIX_SOFTMAX) return {f.begin() + 1, f.begin() + (c.keys_as_values ? 2 : 3)};
+    if (c.mixer == AXQ_MIX_ATTENTION) return {f.begin() + 1, f.begin() + 3};
+    return f; // the recurrences read all of them
+}
+
+// `then_step`: behind every run's mixer the same run of the step of the next token, on ctx->aux_stream[0].  Without `results` nobody reads the residual
+// stream behind the rows, and the last run ends with its cache or state (2048 tokens, four layers of Lakulix at width 2048 1440 -> 1196 us; 2001, three of
+// Gemosun 1565 -> 1163).
+int stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, bool results, float *layers, size_t layer_stride, bool then_step) {
     axq_stack &s = *m->stack;
     axq_ctx *ctx = m->ctx;
     const int W = s.c.width, ldw = pad64(W);
@@ -681,11 +691,12 @@ int stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, float *layer
         const axq_layer_config &c = l.c;
         float *y = average ? s.r_past + (run + 1) * stride : s.r_h;
         const axq_avg avg = avg_of(s, l, s.r_past, stride, run, s.r_h);
-        const bool parallel = s.c.parallel && c.ff > 0, mix = c.mixer == AXQ_MIX_WKV;
+        const bool cache_only = !results && run + 1 == s.runs.size();
+        const bool parallel = s.c.parallel && c.ff > 0 && !cache_only, mix = c.mixer == AXQ_MIX_WKV;
         axq_in in = norm_in(s, l, "norm1", x);
         in.prev = r.prev;
         Proj p;
-        add_firsts(p, l, mixer_firsts(c), s.r_proj, nb, in.nw);
+        add_firsts(p, l, cache_only ? cache_firsts(c) : mixer_firsts(c), s.r_proj, nb, in.nw);
         const float *mu[AXQ_MAX_PARTS] = {};
         for (int i = 0; i < p.parts.n_parts; i++) {
             mu[i] = p.parts.p[i].mu;
@@ -710,11 +721,19 @@ int stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, float *layer
         const axq_rows_out xo = {s.r_x, ldo, s.f32};
         if (c.mixer == AXQ_MIX_ATTENTION) {
             const axq_sig_attn a = attn_of(s, l, r, m->cfg.max_position_embeddings);
-            if ((rc = axq_sig_attn_rows(ctx, a, p.out[0], p.out[1], p.out[2], p.width(0), p.width(1), p.width(2), nb, pos0, s.r_qs, xo))) return rc;
+            if (cache_only) rc = axq_sig_attn_rows(ctx, a, nullptr, p.out[0], p.out[1], 0, p.width(0), p.width(1), nb, pos0, nullptr, xo);
+            else rc = axq_sig_attn_rows(ctx, a, p.out[0], p.out[1], p.out[2], p.width(0), p.width(1), p.width(2), nb, pos0, s.r_qs, xo);
+            if (rc) return rc;
         } else if (c.mixer == AXQ_MIX_SOFTMAX) {
             const axq_soft_attn a = soft_attn_of(s, l, r, m->cfg.max_position_embeddings);
-            const SoftIn i = soft_in(c, p);
-            if ((rc = axq_soft_attn_rows(ctx, a, i.q, i.k, i.v, i.ldq, i.ldk, i.ldv, i.gate, nb, pos0, s.r_qs, xo))) return rc;
+            const int v = c.keys_as_values ? 0 : 1; // where there are no queries
+            if (cache_only) {
+                rc = axq_soft_attn_rows(ctx, a, nullptr, p.out[0], p.out[v], 0, p.width(0), p.width(v), nullptr, nb, pos0, nullptr, xo);
+            } else {
+                const SoftIn i = soft_in(c, p);
+                rc = axq_soft_attn_rows(ctx, a, i.q, i.k, i.v, i.ldq, i.ldk, i.ldv, i.gate, nb, pos0, s.r_qs, xo);
+            }
+            if (rc) return rc;
         } else {
             axq_linstate a = linstate_of(l, r, p, s.r_o);
             axq_in gate;
@@ -740,7 +759,7 @@ int stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, float *layer
             a.seg_state = s.r_seg;
             a.seg_decay = s.r_segw;
             if ((rc = axq_linstate_rows(ctx, a, nb, first))) return rc;
-            if ((rc = axq_rows_rms_gate(ctx, gate, nb, mix ? c.dim : mo, xo))) return rc;
+            if (!cache_only && (rc = axq_rows_rms_gate(ctx, gate, nb, mix ? c.dim : mo, xo))) return rc;
         }
         if (then_step) {
             AXQ_HIP(ctx, hipEventRecord(s.ready, ctx->stream), AXQ_ERR_DRIVER);
@@ -748,6 +767,7 @@ int stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, float *layer
             OnStream on(ctx, ctx->aux_stream[0]);
             if ((rc = step_run(m, run))) return rc;
         }
+        if (cache_only) return AXQ_OK;
         axq_parts o = {};
         o.n_parts = 1;
         o.p[0] = part_of(l, "mix.o", AXQ_ACT_NONE, y, W, x);
@@ -796,7 +816,7 @@ int axq_stack_rows_and_step(axq_model *m, const int32_t *toks, int nb, int pos0)
         OnStream on(ctx, ctx->aux_stream[0]);
         rc = step_embed(m);
     }
-    if (!rc) rc = stack_rows(m, toks, nb, pos0, nullptr, 0, true);
+    if (!rc) rc = stack_rows(m, toks, nb, pos0, false, nullptr, 0, true);
     if (!rc) {
         OnStream on(ctx, ctx->aux_stream[0]);
         rc = step_head(m);
@@ -810,8 +830,8 @@ int axq_stack_rows_and_step(axq_model *m, const int32_t *toks, int nb, int pos0)
     return rc;
 }
 
-int axq_stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, float *layers, size_t layer_stride) {
-    return stack_rows(m, toks, nb, pos0, layers, layer_stride, false);
+int axq_stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, bool results, float *layers, size_t layer_stride) {
+    return stack_rows(m, toks, nb, pos0, results, layers, layer_stride, false);
 }
 
 int axq_stack_logits_rows(axq_model *m, const int32_t *rows, int n, float *logits) {
