@@ -5,15 +5,16 @@
 //
 // Time of a call with f32 rows, before (groups of eight vectors, or two-stage operands in LDS) and now, us:
 //   rows                  10          16          32          64
-//   Q4_K 28672 x 4096     41.4 35.7   42.0 36.2   83.7 44.4   61.7 50 to 57
-//   Q4_K 4096 x 4096      21.9 15.7   21.9 17.2   39.9 20.8   33.0 23.1
-//   Q4_K 4096 x 14336     as before (see axq_dev_rows_gemm_pays)   63.5 36.8   64.0 39.4
+//   Q4_K 28672 x 4096     41.4 35.7   42.0 36.2   83.7 44.4   61.7 47 to 54
+//   Q4_K 4096 x 4096      21.9 15.7   21.9 17.2   39.9 20.8   33.0 22.7
+//   Q4_K 4096 x 14336     as before (see axq_dev_rows_gemm_pays)   63.5 36.8   64.0 37.7
 //   Q4_0 4096 x 11008, 21 rows: 41.9 26.8; Q4_0 4096 x 4096, 10 and 39 rows: 21.7 14.4, 54.7 21.2; Q8_0 11008 x 4096, 64 rows: 43.1 34.9;
-//   bf16 rows, Q8_0 4096 x 4096, 16: 26.0 14.5; Q4_0 11008 x 4096, 128: 48.4 36.5; Q4_K 14336 x 4096, 2048: 325 to 328 295 to 310
+//   bf16 rows, Q8_0 4096 x 4096, 16: 26.0 14.5; Q4_0 11008 x 4096, 128: 48.4 36.5; Q4_K 14336 x 4096, 2048: 325 to 328 265 to 290
 // What bounds it: at few rows the fixed parts (pre-pass, reduction and the launches around them: 14 us of the 4096 x 4096 calls) and
 // the LDS reads of x, which every wave makes for its 32 columns (0.35 us per step with one tile of x, 0.6 with two); at many the matrix
-// pipe beside the vector instructions that make operands.  2048 bf16 rows x 14336 take 275 to 285 us in the kernel, 840 to 870 TFLOP/s: a
-// product keeps its SIMD's issue for about half of its 33 cycles, four vector instructions fit beside it, and there are five to six; and
+// pipe beside the vector instructions that make operands.  2048 bf16 rows x 14336 take 245 to 260 us in the kernel, 920 to 980 TFLOP/s: a
+// product keeps its SIMD's issue for about half of its 33 cycles, four vector instructions fit beside it, and there are five; a tile's way in and out,
+// 5 and 13 us a round (all workgroups write at once); and
 // the card's power: the same products alone, without operands, copies and results, take 208 us, 167 if every x is zero.
 //
 // Numerics.  A bf16 row goes in as f16 under a power-of-two row scale that puts its largest element right below f16's limit: exact
@@ -211,6 +212,12 @@ struct SuperQ45 {
         }
         o[0] = octet(w);
     }
+    template <int PR>
+    __device__ static void make_part(const Raw &r, const Side &s, const Scales &c, uint32_t mask, int j, int t, half8 &o) {
+        half8 all[1];
+        make(r, s, c, mask, j, t, 0, all);
+        o = all[0];
+    }
 };
 
 struct SuperQ6 {
@@ -270,6 +277,12 @@ struct SuperQ6 {
         }
         o[0] = octet(hi);
         o[1] = octet(lo);
+    }
+    template <int PR>
+    __device__ static void make_part(const Raw &r, const Side &s, const Scales &c, uint32_t mask, int j, int t, half8 &o) {
+        half8 both[2];
+        make(r, s, c, mask, j, t, 0, both);
+        o = both[PR];
     }
 };
 
@@ -846,7 +859,12 @@ __device__ inline void write_rows(const RowsArgs &a, const float16v (&acc)[MI][N
 // other reads x and codes from LDS, makes its next operands of them and requests what comes into LDS after them.  Waves 0 .. 3 (rows 0 ..
 // 127) and 4 .. 7 are half a round apart, with a barrier behind every turn.  A turn is sixteen products (half a K step of 64, twice as many
 // for Q6_K), and so are a superblock's offsets against its sums of x, which lie in the ring of x like half a step.
-// The first half's waves copy x, the second half's codes and sides.
+// The first half's waves copy x, the second half's codes and sides, piece by piece between their products, in a loop of its own for each half: a request
+// keeps its wave for 40 to 50 cycles, beside which the matrix pipe works on, where requests in the fetch kept the whole workgroup, and a branch between
+// products for what only one half copies costs more than the copy.  Cycles of a turn (fetch, products, all; Q4_K, stamped): 993 588 1988 with
+// requests in the fetch, 869 for the products with the branches, 657 692 1657 so.  Half of a turn's x is read between the products as well.
+// 2048 bf16 rows x 14336 x 4096, whole call, requests in the fetch and so, us: Q4_K 302 to 313 276 to 286, Q5_K 338 308, Q6_K 477 440; 512 f32 rows,
+// Q4_K 28672 x 4096 287 265.
 template <class T>
 struct WideTile {
     static constexpr int HB = T::PAIRS * 32, XBYTES = 16384, WBYTES = 256 * HB, DBYTES = 256 * (16 * T::SIDE16 + 4 * T::SIDE4);
@@ -855,7 +873,7 @@ struct WideTile {
     static constexpr int LDS = NX * XBYTES + NW * WBYTES + 2 * DBYTES;
     // a copying wave's requests: half a step of x; codes of a unit, sides of a superblock
     static constexpr int XL = 4, WL = 2 * T::PAIRS, D16 = T::SIDE16, D4 = T::SIDE4, D = D16 + D4;
-    static_assert(NX >= 4 && NW == 3, "stages");
+    static_assert(NX >= 4 && NW == 3 && XL <= 4 && WL <= 8 && D <= 8, "stages, and eight places between products");
 };
 
 template <class T>
@@ -874,51 +892,42 @@ __global__ void __launch_bounds__(512, 2) rows_wide_kernel(RowsArgs a) {
     uint8_t *xbase = lds, *wbase = lds + NX * XBYTES, *dbase = wbase + NW * WBYTES;
 
     // ---- copies into LDS (past the end of the row: its last superblock or unit again, which nobody looks at)
-    auto copy = [&](const void *src, uint8_t *dst) { __builtin_amdgcn_global_load_lds((gbl_void *)src, (lds_void *)dst, 16, 0, 0); };
+    auto copy = [&](const void *base, uint32_t off, uint8_t *dst) { // a wave's place in scalar registers, a lane's in 32 bits: registers are short
+        asm volatile("" : "+v"(off)); // extended where it is used
+        __builtin_amdgcn_global_load_lds((gbl_void *)(reinterpret_cast<const uint8_t *>(base) + off), (lds_void *)dst, 16, 0, 0);
+    };
+    const uint32_t lane16 = lane * 16;
     auto in_order = [] { asm volatile("" ::: "memory"); }; // the waits in front of the barriers count on the order of the requests
-    const _Float16 *xp[2], *sp[2];
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
+    auto copy_x = [&](int sb, int h, int at, int piece) { // of turn h of superblock sb of this workgroup into the place at byte `at`
+        const int g = sb0 + sb < nsb_row ? sb0 + sb : nsb_row - 1, hs = T::MIN && h > Tile::OFFSETS ? h - 1 : h, q = piece >> 1, t = piece & 1;
         const size_t mt = (size_t)(mt0 + wn * 2 + q);
-        xp[q] = a.xa + mt * (size_t)(a.k >> 6) * 2048 + lane * 8;
-        sp[q] = a.xs + mt * (size_t)nsb_row * 1024 + lane * 8;
-    }
-    auto copy_x = [&](int sb, int h, int at) { // turn h of superblock sb of this workgroup into the place at byte `at`
-        const int g = sb0 + sb < nsb_row ? sb0 + sb : nsb_row - 1, hs = T::MIN && h > Tile::OFFSETS ? h - 1 : h;
-#pragma unroll
-        for (int q = 0; q < 2; q++)
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-                copy(h == Tile::OFFSETS ? sp[q] + ((size_t)g * 1024 + t * 512) : xp[q] + ((size_t)(g * 8 + hs) * 1024 + t * 512),
-                     xbase + at + (wn * 2 + q) * 2048 + t * 1024);
+        copy(h == Tile::OFFSETS ? a.xs + ((mt * nsb_row + g) * 1024 + t * 512) : a.xa + ((mt * nsb_row + g) * 8192 + hs * 1024 + t * 512), lane16,
+             xbase + at + (wn * 2 + q) * 2048 + t * 1024);
         in_order();
     };
     const int cr = lane >> 1, cs = (lane & 1) ^ ((cr >> 3) & 1); // see rows_gemm_kernel
     auto row_of = [&](int r) { return (uint32_t)(n0 + r < a.n ? r : a.n - 1 - n0); };
-    auto copy_codes = [&](int u, int at) {
+    auto copy_codes = [&](int u, int at, int piece) {
         int unit = sb0 * 2 + u;
         unit = unit < 2 * nsb_row ? unit : 2 * nsb_row - 1;
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const int ct = wn * 2 + q; // column tile of 32 rows
-            const uint32_t row = row_of(ct * 32 + cr);
-#pragma unroll
-            for (int p = 0; p < T::PAIRS; p++)
-                copy(T::piece_src(a, unit, p) + (size_t)n0 * T::piece_pitch(a, p) + (row * T::piece_pitch(a, p) + cs * 16), wbase + at + ct * 32 * HB + p * 1024);
-        }
+        const int ct = wn * 2 + piece / T::PAIRS, p = piece % T::PAIRS; // column tile of 32 rows
+        const uint32_t row = row_of(ct * 32 + cr);
+        copy(T::piece_src(a, unit, p) + (size_t)n0 * T::piece_pitch(a, p), row * T::piece_pitch(a, p) + cs * 16, wbase + at + ct * 32 * HB + p * 1024);
         in_order();
     };
-    auto copy_sides = [&](int sb) { // 64 rows of every piece
+    auto copy_sides = [&](int sb, int c) { // 64 rows of piece c
         const int at = sb0 + sb < nsb_row ? sb0 + sb : nsb_row - 1, r0 = wn * 64;
         uint8_t *dst = dbase + (sb & 1) * DBYTES;
-#pragma unroll
-        for (int c = 0; c < T::SIDE16; c++)
-            copy(T::side_src(a, at, c) + (size_t)n0 * T::side_pitch(a, c) + row_of(r0 + lane) * T::side_pitch(a, c), dst + c * 256 * 16 + r0 * 16);
-        if constexpr (T::SIDE4 > 0)
-            __builtin_amdgcn_global_load_lds((gbl_void *)(T::side_src(a, at, T::SIDE16) + (size_t)n0 * T::side_pitch(a, T::SIDE16) +
-                                                          row_of(r0 + lane) * T::side_pitch(a, T::SIDE16)),
-                                             (lds_void *)(dst + T::SIDE16 * 256 * 16 + r0 * 4), 4, 0, 0);
+        const uint8_t *src = T::side_src(a, at, c) + (size_t)n0 * T::side_pitch(a, c);
+        uint32_t off = row_of(r0 + lane) * T::side_pitch(a, c);
+        asm volatile("" : "+v"(off));
+        if (c < T::SIDE16) copy(src, off, dst + c * 256 * 16 + r0 * 16);
+        else __builtin_amdgcn_global_load_lds((gbl_void *)(src + off), (lds_void *)(dst + T::SIDE16 * 256 * 16 + r0 * 4), 4, 0, 0);
         in_order();
+    };
+    auto all = [](int n, auto fn) {
+#pragma unroll
+        for (int p = 0; p < n; p++) fn(p);
     };
     auto turn_over = [] {
         __builtin_amdgcn_sched_barrier(0);
@@ -964,14 +973,14 @@ __global__ void __launch_bounds__(512, 2) rows_wide_kernel(RowsArgs a) {
     // ---- the requests in front of the first turn, in the order of the later ones
     if (half == 0) {
 #pragma unroll
-        for (int g = 0; g < NX - 1; g++) copy_x(0, g, g * XBYTES);
+        for (int g = 0; g < NX - 1; g++) all(Tile::XL, [&](int p) { copy_x(0, g, g * XBYTES, p); });
         wait_loads_and_lds<(NX - 2) * Tile::XL>();
     } else {
-        copy_sides(0);
-        copy_codes(0, 0);
-        copy_sides(1);
-        copy_codes(1, WBYTES);
-        copy_codes(2, 2 * WBYTES);
+        all(Tile::D, [&](int p) { copy_sides(0, p); });
+        all(Tile::WL, [&](int p) { copy_codes(0, 0, p); });
+        all(Tile::D, [&](int p) { copy_sides(1, p); });
+        all(Tile::WL, [&](int p) { copy_codes(1, WBYTES, p); });
+        all(Tile::WL, [&](int p) { copy_codes(2, 2 * WBYTES, p); });
         wait_loads_and_lds<Tile::D + 2 * Tile::WL>();
     }
     static_assert(NX - 1 <= TURNS, "turns");
@@ -980,27 +989,28 @@ __global__ void __launch_bounds__(512, 2) rows_wide_kernel(RowsArgs a) {
     read_codes(0);
     read_sides(0, side);
     int w_to = 0; // where the next unit of codes goes: the place of the one that has been read
-    auto turn = [&](int sb, auto which) {
+    auto turn = [&](int sb, auto which, auto copier) __attribute__((always_inline)) {
+        constexpr int HALF = decltype(copier)::value;
         constexpr int h = decltype(which)::value, hs = T::MIN && h > Tile::OFFSETS ? h - 1 : h, J = hs >> 1, P = hs & 1;
         constexpr bool OFFS = h == Tile::OFFSETS;
-        half8 xf[2][MI], wf[2][NJ][T::PRODUCTS];
+        // Operands are made in the fetch, while x is on its way.  LATE: of its products t = 1 between the ones before, in the place of what those are done
+        // with: two operands per weight leave no registers for the others (Q6_K, 2048 x 14336 x 4096: 453 us with thirteen of them spilt, 442 so; with
+        // one operand per weight it is the longer way: Q4_K 292 and 303).
+        constexpr bool LATE = T::PRODUCTS == 2;
+        half8 xf[MI], wf[LATE ? 1 : 2][NJ][T::PRODUCTS];
+        auto operand = [&](int t, int j, int pr) -> half8 & { return wf[LATE ? 0 : t][j][pr]; };
+        auto make = [&](auto tt, int j, auto part) {
+            constexpr int t = decltype(tt)::value, pr = decltype(part)::value;
+            T::template make_part<pr>(raw[j], side[j], scales[j], mask, J, 2 * P + t, operand(t, j, pr));
+            asm volatile("" : "+v"(operand(t, j, pr)));
+        };
+        using C0 = std::integral_constant<int, 0>; using C1 = std::integral_constant<int, 1>;
+        auto read_x = [&](int t, int i) { xf[i] = *reinterpret_cast<const half8 *>(my_x + x_at + i * 2048 + t * 1024); };
         int over[NJ] = {0, 0};
         // ---- fetch
 #pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int i = 0; i < MI; i++) xf[t][i] = *reinterpret_cast<const half8 *>(my_x + x_at + i * 2048 + t * 1024);
+        for (int i = 0; i < MI; i++) read_x(0, i);
         in_order();
-        if (half == 0) {
-            constexpr int ahead = h + NX - 1;
-            copy_x(ahead >= TURNS ? sb + 1 : sb, ahead >= TURNS ? ahead - TURNS : ahead, x_at == 0 ? (NX - 1) * XBYTES : x_at - XBYTES);
-        } else {
-            if (h == 0) copy_sides(sb + 2);
-            if (h == 2 || h == TURNS - 2) {
-                copy_codes(2 * sb + (h == 2 ? 0 : 1) + NW, w_to);
-                w_to = w_to == (NW - 1) * WBYTES ? 0 : w_to + WBYTES;
-            }
-        }
         if constexpr (h == 0) new_side();
         if constexpr (OFFS) {
             if constexpr (T::MIN)
@@ -1012,30 +1022,20 @@ __global__ void __launch_bounds__(512, 2) rows_wide_kernel(RowsArgs a) {
             }
         } else {
 #pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int j = 0; j < NJ; j++) {
-                    T::make(raw[j], side[j], scales[j], mask, J, 2 * P + t, hh, wf[t][j]);
-#pragma unroll
-                    for (int pr = 0; pr < T::PRODUCTS; pr++) asm volatile("" : "+v"(wf[t][j][pr])); // made here, while x is on its way, not behind the wait
-                }
+            for (int j = 0; j < NJ; j++) {
+                make(C0{}, j, C0{});
+                if constexpr (LATE) make(C0{}, j, C1{});
+                else make(C1{}, j, C0{});
+            }
         }
-        if constexpr (!OFFS && P == 1) read_codes((J + 1) & 3);
+        if constexpr (!LATE && !OFFS && P == 1) read_codes((J + 1) & 3);
         if constexpr (h == TURNS - 1) read_sides(sb + 1, side);
-        if (half == 0) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        else if (h == 2 || h == TURNS - 2) wait_loads_and_lds<Tile::D + 2 * Tile::WL>(); // what the next turns read first, sides included
+        // what the next turns read first, sides included; here, since the first half reads it in the next phase
+        if (HALF && (h == 2 || h == TURNS - 2)) wait_loads_and_lds<Tile::D + Tile::WL>();
         else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         turn_over();
         // ---- multiply
         __builtin_amdgcn_s_setprio(1);
-        if constexpr (h == 0) {
-#pragma unroll
-            for (int i = 0; i < MI; i++)
-#pragma unroll
-                for (int j = 0; j < NJ; j++)
-#pragma unroll
-                    for (int q = 0; q < 16; q++) acc[i][j][q] *= ratio[j];
-        }
         auto times_pow2 = [&](int j, int e) { // a column's lanes all have its factor; exact, being a power of two
             if (__builtin_amdgcn_ballot_w64(over[j] > 0) == 0) return;
             const float f = __builtin_bit_cast(float, (uint32_t)(127 + e * over[j]) << 23);
@@ -1046,34 +1046,67 @@ __global__ void __launch_bounds__(512, 2) rows_wide_kernel(RowsArgs a) {
         };
         if constexpr (OFFS)
             for (int j = 0; j < NJ; j++) times_pow2(j, -1);
+        // what this wave copies in this turn
+        auto between = [&](int slot) {
+            constexpr int ahead = h + NX - 1;
+            __builtin_amdgcn_sched_barrier(0);
+            if (HALF == 0) {
+                if (slot % 2 == 0) copy_x(ahead >= TURNS ? sb + 1 : sb, ahead >= TURNS ? ahead - TURNS : ahead, x_at == 0 ? (NX - 1) * XBYTES : x_at - XBYTES, slot / 2);
+            } else {
+                if (h == 0 && slot < Tile::D) copy_sides(sb + 2, slot);
+                if ((h == 2 || h == TURNS - 2) && slot < Tile::WL) copy_codes(2 * sb + (h == 2 ? 0 : 1) + NW, w_to, slot);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
 #pragma unroll
         for (int t = 0; t < 2; t++)
 #pragma unroll
             for (int pr = 0; pr < T::PRODUCTS; pr++)
 #pragma unroll
-                for (int i = 0; i < MI; i++)
+                for (int i = 0; i < MI; i++) {
+                    if constexpr (h == 0)
+                        if (t == 0 && pr == 0)
 #pragma unroll
-                    for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[t][i], wf[OFFS ? 0 : t][j][pr], acc[i][j], 0, 0, 0);
+                            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                                for (int q = 0; q < 16; q++) acc[i][j][q] *= ratio[j];
+                    if constexpr (LATE) {
+                        if (t == 0 && pr == 1 && i % 2 == 0) make(C1{}, i / 2, C0{});
+                        if (t == 1 && pr == 0 && i % 2 == 0) make(C1{}, i / 2, C1{});
+                    }
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[i], operand(OFFS ? 0 : t, j, pr), acc[i][j], 0, 0, 0);
+                    if constexpr (h == 0)
+                        if (t == 0 && pr == 0) // a tile changes its unit right in front of its first product
+#pragma unroll
+                            for (int j = 0; j < NJ; j++) {
+                                __builtin_amdgcn_sched_group_barrier(2, 16, 0);
+                                __builtin_amdgcn_sched_group_barrier(8, 1, 0);
+                            }
+                    if (pr == 0) between(t * MI + i);
+                    if (t == 0 && pr == T::PRODUCTS - 1) read_x(1, i); // in the place of what the products are done with: sixteen registers fewer, and the fetch reads half as much
+                }
+        if constexpr (LATE && P == 1) read_codes((J + 1) & 3);
         if constexpr (OFFS)
             for (int j = 0; j < NJ; j++) times_pow2(j, 1);
-        if constexpr (h == 0) // a tile changes its unit right in front of its first product
-#pragma unroll
-            for (int q = 0; q < MI * NJ; q++) {
-                __builtin_amdgcn_sched_group_barrier(2, 16, 0);
-                __builtin_amdgcn_sched_group_barrier(8, 1, 0);
-            }
         __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
-        if (half == 0) wait_loads_and_lds<(NX - 2) * Tile::XL>(); // the next turn's x
+        if (HALF == 0) wait_loads_and_lds<(NX - 2) * Tile::XL>(); // the next turn's x
+        else if (h == 2 || h == TURNS - 2) w_to = w_to == (NW - 1) * WBYTES ? 0 : w_to + WBYTES;
         turn_over();
         x_at = x_at == (NX - 1) * XBYTES ? 0 : x_at + XBYTES;
     };
-    for (int sb = 0; sb < mine; sb++) {
-        turn(sb, std::integral_constant<int, 0>{}); turn(sb, std::integral_constant<int, 1>{}); turn(sb, std::integral_constant<int, 2>{});
-        turn(sb, std::integral_constant<int, 3>{}); turn(sb, std::integral_constant<int, 4>{}); turn(sb, std::integral_constant<int, 5>{});
-        turn(sb, std::integral_constant<int, 6>{}); turn(sb, std::integral_constant<int, 7>{});
-        if constexpr (TURNS == 9) turn(sb, std::integral_constant<int, 8>{});
-    }
+    // a loop for each half: what a half copies is no branch between the products, which would cost more than the copy
+    auto run = [&](auto copier) __attribute__((always_inline)) {
+        for (int sb = 0; sb < mine; sb++) {
+            turn(sb, std::integral_constant<int, 0>{}, copier); turn(sb, std::integral_constant<int, 1>{}, copier); turn(sb, std::integral_constant<int, 2>{}, copier);
+            turn(sb, std::integral_constant<int, 3>{}, copier); turn(sb, std::integral_constant<int, 4>{}, copier); turn(sb, std::integral_constant<int, 5>{}, copier);
+            turn(sb, std::integral_constant<int, 6>{}, copier); turn(sb, std::integral_constant<int, 7>{}, copier);
+            if constexpr (TURNS == 9) turn(sb, std::integral_constant<int, 8>{}, copier);
+        }
+    };
+    if (half == 0) run(std::integral_constant<int, 0>{});
+    else run(std::integral_constant<int, 1>{});
     if (!half) barrier();
     wait_loads_and_lds<0>(); // nothing of this workgroup may still be on its way into LDS
 
@@ -1090,7 +1123,8 @@ __global__ void __launch_bounds__(512, 2) rows_wide_kernel(RowsArgs a) {
 
 // 256 x 128 outputs of a type with blocks of 32, 128 x 32 per wave, with the waves taking turns as above: a turn is a block's eight products,
 // which start from zero and join the total times the block's d in the next fetch, beside the other half's products.  What bounds it is
-// that work, 64 multiply-adds per eight products, and the making of operands.
+// that work, 64 multiply-adds per eight products, and the making of operands.  Copies go between the products (see rows_wide_kernel; in the fetch 2048 bf16
+// rows x 14336 x 4096 take, and so, us: Q4_0 402 331, Q5_0 425 365, Q8_0 402 354, Q5_1 464 414).
 template <class T>
 struct BlocksTile {
     static constexpr int HB = T::PAIRS * 32, XBYTES = 16384, WBYTES = 128 * HB, DBYTES = 128 * 16 * T::SIDE16;
@@ -1099,7 +1133,7 @@ struct BlocksTile {
     static constexpr int LDS = NX * XBYTES + NW * WBYTES + 2 * DBYTES;
     // a copying wave's requests: half a step of x; codes of a unit, sides of a superblock
     static constexpr int XL = 4, WL = T::PAIRS, D = T::SIDE16;
-    static_assert(NX >= 4 && NW == 3, "stages");
+    static_assert(NX >= 4 && NW == 3 && XL <= 4 && WL <= 8 && D <= 8, "stages, and eight places between products");
 };
 
 template <class T>
@@ -1118,43 +1152,36 @@ __global__ void __launch_bounds__(512, 2) rows_blocks_kernel(RowsArgs a) {
     uint8_t *xbase = lds, *wbase = lds + NX * XBYTES, *dbase = wbase + NW * WBYTES;
 
     // ---- copies into LDS (past the end of the row: its last superblock or unit again, which nobody looks at)
-    auto copy = [&](const void *src, uint8_t *dst) { __builtin_amdgcn_global_load_lds((gbl_void *)src, (lds_void *)dst, 16, 0, 0); };
+    auto copy = [&](const void *base, uint32_t off, uint8_t *dst) { // a wave's place in scalar registers, a lane's in 32 bits: registers are short
+        asm volatile("" : "+v"(off)); // extended where it is used
+        __builtin_amdgcn_global_load_lds((gbl_void *)(reinterpret_cast<const uint8_t *>(base) + off), (lds_void *)dst, 16, 0, 0);
+    };
+    const uint32_t lane16 = lane * 16;
     auto in_order = [] { asm volatile("" ::: "memory"); }; // the waits in front of the barriers count on the order of the requests
-    const _Float16 *xp[2], *sp[2];
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
+    auto copy_x = [&](int sb, int h, int at, int piece) { // of turn h of superblock sb of this workgroup into the place at byte `at`
+        const int g = sb0 + sb < nsb_row ? sb0 + sb : nsb_row - 1, hs = T::MIN && h > Tile::OFFSETS ? h - 1 : h, q = piece >> 1, t = piece & 1;
         const size_t mt = (size_t)(mt0 + wn * 2 + q);
-        xp[q] = a.xa + mt * (size_t)(a.k >> 6) * 2048 + lane * 8;
-        sp[q] = a.xs + mt * (size_t)nsb_row * 1024 + lane * 8;
-    }
-    auto copy_x = [&](int sb, int h, int at) { // turn h of superblock sb of this workgroup into the place at byte `at`
-        const int g = sb0 + sb < nsb_row ? sb0 + sb : nsb_row - 1, hs = T::MIN && h > Tile::OFFSETS ? h - 1 : h;
-#pragma unroll
-        for (int q = 0; q < 2; q++)
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-                copy(h == Tile::OFFSETS ? sp[q] + ((size_t)g * 1024 + t * 512) : xp[q] + ((size_t)(g * 8 + hs) * 1024 + t * 512),
-                     xbase + at + (wn * 2 + q) * 2048 + t * 1024);
+        copy(h == Tile::OFFSETS ? a.xs + ((mt * nsb_row + g) * 1024 + t * 512) : a.xa + ((mt * nsb_row + g) * 8192 + hs * 1024 + t * 512), lane16,
+             xbase + at + (wn * 2 + q) * 2048 + t * 1024);
         in_order();
     };
     const int cr = lane >> 1, cs = (lane & 1) ^ ((cr >> 3) & 1); // see rows_gemm_kernel
     auto row_of = [&](int r) { return (uint32_t)(n0 + r < a.n ? r : a.n - 1 - n0); };
-    auto copy_codes = [&](int u, int at) {
+    auto copy_codes = [&](int u, int at, int p) {
         int unit = sb0 * 2 + u;
         unit = unit < 2 * nsb_row ? unit : 2 * nsb_row - 1;
         const uint32_t row = row_of(wn * 32 + cr);
-#pragma unroll
-        for (int p = 0; p < T::PAIRS; p++)
-            copy(T::piece_src(a, unit, p) + (size_t)n0 * T::piece_pitch(a, p) + (row * T::piece_pitch(a, p) + cs * 16), wbase + at + wn * 32 * HB + p * 1024);
+        copy(T::piece_src(a, unit, p) + (size_t)n0 * T::piece_pitch(a, p), row * T::piece_pitch(a, p) + cs * 16, wbase + at + wn * 32 * HB + p * 1024);
         in_order();
     };
-    auto copy_sides = [&](int sb) { // 64 rows of every piece, twice
+    auto copy_sides = [&](int sb, int c) { // 64 rows of piece c, twice
         const int at = sb0 + sb < nsb_row ? sb0 + sb : nsb_row - 1, r0 = (wn & 1) * 64;
-        uint8_t *dst = dbase + (sb & 1) * DBYTES;
-#pragma unroll
-        for (int c = 0; c < T::SIDE16; c++)
-            copy(T::side_src(a, at, c) + (size_t)n0 * T::side_pitch(a, c) + row_of(r0 + lane) * T::side_pitch(a, c), dst + c * 128 * 16 + r0 * 16);
+        copy(T::side_src(a, at, c) + (size_t)n0 * T::side_pitch(a, c), row_of(r0 + lane) * T::side_pitch(a, c), dbase + (sb & 1) * DBYTES + c * 128 * 16 + r0 * 16);
         in_order();
+    };
+    auto all = [](int n, auto fn) {
+#pragma unroll
+        for (int p = 0; p < n; p++) fn(p);
     };
     auto turn_over = [] {
         __builtin_amdgcn_sched_barrier(0);
@@ -1191,21 +1218,22 @@ __global__ void __launch_bounds__(512, 2) rows_blocks_kernel(RowsArgs a) {
     // ---- the requests in front of the first turn, in the order of the later ones
     if (half == 0) {
 #pragma unroll
-        for (int g = 0; g < NX - 1; g++) copy_x(0, g, g * XBYTES);
+        for (int g = 0; g < NX - 1; g++) all(Tile::XL, [&](int p) { copy_x(0, g, g * XBYTES, p); });
         wait_loads_and_lds<(NX - 2) * Tile::XL>();
     } else {
-        copy_sides(0);
-        copy_codes(0, 0);
-        copy_sides(1);
-        copy_codes(1, WBYTES);
-        copy_codes(2, 2 * WBYTES);
+        all(Tile::D, [&](int p) { copy_sides(0, p); });
+        all(Tile::WL, [&](int p) { copy_codes(0, 0, p); });
+        all(Tile::D, [&](int p) { copy_sides(1, p); });
+        all(Tile::WL, [&](int p) { copy_codes(1, WBYTES, p); });
+        all(Tile::WL, [&](int p) { copy_codes(2, 2 * WBYTES, p); });
         wait_loads_and_lds<Tile::D + 2 * Tile::WL>();
     }
     static_assert(NX - 1 <= TURNS, "turns");
     barrier();
     if (half) turn_over(); // the second half is a turn behind
     int w_to = 0; // where the next unit of codes goes: the place of the one that has been read
-    auto turn = [&](int sb, auto which) {
+    auto turn = [&](int sb, auto which, auto copier) __attribute__((always_inline)) {
+        constexpr int HALF = decltype(copier)::value;
         constexpr int h = decltype(which)::value, hs = T::MIN && h > Tile::OFFSETS ? h - 1 : h, J = hs >> 1, P = hs & 1;
         constexpr bool OFFS = h == Tile::OFFSETS;
         half8 xf[2][MI];
@@ -1217,19 +1245,8 @@ __global__ void __launch_bounds__(512, 2) rows_blocks_kernel(RowsArgs a) {
         if (h == 0) read_sides(sb);
         if (!OFFS && P == 0) read_codes(J);
         in_order();
-        if (half == 0) {
-            constexpr int ahead = h + NX - 1;
-            copy_x(ahead >= TURNS ? sb + 1 : sb, ahead >= TURNS ? ahead - TURNS : ahead, x_at == 0 ? (NX - 1) * XBYTES : x_at - XBYTES);
-        } else {
-            if (h == 1) copy_sides(sb + 2);
-            if (h == 3 || h == TURNS - 1) {
-                copy_codes(2 * sb + (h == 3 ? 0 : 1) + NW, w_to);
-                w_to = w_to == (NW - 1) * WBYTES ? 0 : w_to + WBYTES;
-            }
-        }
         if (h != 0 || sb > 0) fold();
-        if (half == 0) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        else if (h == 3 || h == TURNS - 1) wait_loads_and_lds<Tile::D + 2 * Tile::WL>(); // what the next turns read first, sides included
+        if (HALF && (h == 3 || h == TURNS - 1)) wait_loads_and_lds<Tile::D + Tile::WL>(); // what the next turns read first, sides included
         else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         turn_over();
         // ---- multiply
@@ -1241,24 +1258,44 @@ __global__ void __launch_bounds__(512, 2) rows_blocks_kernel(RowsArgs a) {
         } else {
             d = T::scale(side, hs);
         }
+        auto between = [&](int slot) { // copies, piece by piece between the products (see rows_wide_kernel)
+            constexpr int ahead = h + NX - 1;
+            __builtin_amdgcn_sched_barrier(0);
+            if (HALF == 0) {
+                if (slot % 2 == 0) copy_x(ahead >= TURNS ? sb + 1 : sb, ahead >= TURNS ? ahead - TURNS : ahead, x_at == 0 ? (NX - 1) * XBYTES : x_at - XBYTES, slot / 2);
+            } else {
+                if (h == 1 && slot < Tile::D) copy_sides(sb + 2, slot);
+                if ((h == 3 || h == TURNS - 1) && slot < Tile::WL) copy_codes(2 * sb + (h == 3 ? 0 : 1) + NW, w_to, slot);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
 #pragma unroll
         for (int t = 0; t < 2; t++) {
             if constexpr (!OFFS) T::make(raw, side, typename T::Scales(), mask, J, 2 * P + t, hh, wf);
 #pragma unroll
-            for (int i = 0; i < MI; i++) part[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[t][i], wf[0], t == 0 ? zero : part[i], 0, 0, 0);
+            for (int i = 0; i < MI; i++) {
+                part[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[t][i], wf[0], t == 0 ? zero : part[i], 0, 0, 0);
+                between(t * MI + i);
+            }
         }
         __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
-        if (half == 0) wait_loads_and_lds<(NX - 2) * Tile::XL>(); // the next turn's x
+        if (HALF == 0) wait_loads_and_lds<(NX - 2) * Tile::XL>(); // the next turn's x
+        else if (h == 3 || h == TURNS - 1) w_to = w_to == (NW - 1) * WBYTES ? 0 : w_to + WBYTES;
         turn_over();
         x_at = x_at == (NX - 1) * XBYTES ? 0 : x_at + XBYTES;
     };
-    for (int sb = 0; sb < mine; sb++) {
-        turn(sb, std::integral_constant<int, 0>{}); turn(sb, std::integral_constant<int, 1>{}); turn(sb, std::integral_constant<int, 2>{});
-        turn(sb, std::integral_constant<int, 3>{}); turn(sb, std::integral_constant<int, 4>{}); turn(sb, std::integral_constant<int, 5>{});
-        turn(sb, std::integral_constant<int, 6>{}); turn(sb, std::integral_constant<int, 7>{});
-        if constexpr (TURNS == 9) turn(sb, std::integral_constant<int, 8>{});
-    }
+    // a loop for each half: what a half copies is no branch between the products, which would cost more than the copy
+    auto run = [&](auto copier) __attribute__((always_inline)) {
+        for (int sb = 0; sb < mine; sb++) {
+            turn(sb, std::integral_constant<int, 0>{}, copier); turn(sb, std::integral_constant<int, 1>{}, copier); turn(sb, std::integral_constant<int, 2>{}, copier);
+            turn(sb, std::integral_constant<int, 3>{}, copier); turn(sb, std::integral_constant<int, 4>{}, copier); turn(sb, std::integral_constant<int, 5>{}, copier);
+            turn(sb, std::integral_constant<int, 6>{}, copier); turn(sb, std::integral_constant<int, 7>{}, copier);
+            if constexpr (TURNS == 9) turn(sb, std::integral_constant<int, 8>{}, copier);
+        }
+    };
+    if (half == 0) run(std::integral_constant<int, 0>{});
+    else run(std::integral_constant<int, 1>{});
     fold();
     if (!half) barrier();
     wait_loads_and_lds<0>(); // nothing of this workgroup may still be on its way into LDS
@@ -1270,7 +1307,9 @@ __global__ void __launch_bounds__(512, 2) rows_blocks_kernel(RowsArgs a) {
 // 128 x 128 outputs of a superblock type with the waves taking turns as above; the halves of the workgroup have every other half of its
 // superblocks, each with stages of its own, and their sums meet in LDS.  A wave computes 128 x 32, so that an operand is made for four
 // products (64 x 32 per wave and halves that share K make it for two, and that work is what the kernel waited for: 64 f32 rows, Q4_K
-// 28672 x 4096, 55.8 us).  Operands are made between the products; a turn is a K step of 64, sixteen products.  Sums of two steps start from
+// 28672 x 4096, 55.8 us).  A turn is a K step of 64, sixteen products.  Copies go between the products (see rows_wide_kernel), and so do the reads of x and
+// the making of operands for a turn's second half, so that fetch and products take as long: cycles of a turn, stamped, 1290 881 2616 with all of them in
+// the fetch but the operands, 844 855 2105 so; that call 53 to 59 us, 47 to 53 so.  Sums of two steps start from
 // zero and join the total times the superblock's unit: as many additions of the total's size as superblocks, since each half has half of them.
 template <class T>
 struct ApartTile {
@@ -1278,7 +1317,7 @@ struct ApartTile {
     static constexpr int NX = 3, NW = 2, GROUP = NX * XBYTES + NW * WBYTES + SBYTES + DBYTES, LDS = 2 * GROUP;
     // a copying wave's requests: x of a step; codes of a unit, sums and sides of a superblock
     static constexpr int XL = 8, WL = 2 * T::PAIRS, SL = T::MIN ? 4 : 0, D = T::SIDE16 + T::SIDE4;
-    static_assert(LDS <= 160 * 1024 && LDS >= 8 * 32 * 64 * 4, "stages");
+    static_assert(LDS <= 160 * 1024 && LDS >= 8 * 32 * 64 * 4 && XL <= 8 && WL <= 16 && SL <= 16 && D <= 16, "stages, and sixteen places between products");
 };
 
 template <class T>
@@ -1301,53 +1340,47 @@ __global__ void __launch_bounds__(512, 2) rows_apart_kernel(RowsArgs a) {
     const int cw = wn & 1;
 
     // ---- copies into LDS (past the end of the row: its last step, unit or superblock again, which nobody looks at)
-    auto copy = [&](const void *src, uint8_t *dst) { __builtin_amdgcn_global_load_lds((gbl_void *)src, (lds_void *)dst, 16, 0, 0); };
+    auto copy = [&](const void *base, uint32_t off, uint8_t *dst) { // a wave's place in scalar registers, a lane's in 32 bits: registers are short
+        asm volatile("" : "+v"(off)); // extended where it is used
+        __builtin_amdgcn_global_load_lds((gbl_void *)(reinterpret_cast<const uint8_t *>(base) + off), (lds_void *)dst, 16, 0, 0);
+    };
+    const uint32_t lane16 = lane * 16;
     auto in_order = [] { asm volatile("" ::: "memory"); }; // the waits in front of the barriers count on the order of the requests
-    auto copy_x = [&](int g, int at) {
+    auto copy_x = [&](int g, int at, int piece) {
         int step = sb0 * 4 + g;
         step = step < steps_row ? step : steps_row - 1;
-#pragma unroll
-        for (int q = 0; q < 2; q++)
-#pragma unroll
-            for (int t = 0; t < 4; t++)
-                copy(a.xa + ((size_t)(mt0 + cw * 2 + q) * steps_row + step) * 2048 + t * 512 + lane * 8, xbase + at + (cw * 2 + q) * 4096 + t * 1024);
+        const int q = piece >> 2, t = piece & 3;
+        copy(a.xa + ((size_t)(mt0 + cw * 2 + q) * steps_row + step) * 2048 + t * 512, lane16, xbase + at + (cw * 2 + q) * 4096 + t * 1024);
         in_order();
     };
-    auto copy_sums = [&](int sb) {
+    auto copy_sums = [&](int sb, int piece) {
         const int at = sb0 + sb < nsb_row ? sb0 + sb : nsb_row - 1;
-        if constexpr (T::MIN)
-#pragma unroll
-            for (int q = 0; q < 2; q++)
-#pragma unroll
-                for (int t = 0; t < 2; t++)
-                    copy(a.xs + ((size_t)(mt0 + cw * 2 + q) * nsb_row + at) * 1024 + t * 512 + lane * 8, sbase + (cw * 2 + q) * 2048 + t * 1024);
+        const int q = piece >> 1, t = piece & 1;
+        if constexpr (T::MIN) copy(a.xs + ((size_t)(mt0 + cw * 2 + q) * nsb_row + at) * 1024 + t * 512, lane16, sbase + (cw * 2 + q) * 2048 + t * 1024);
         in_order();
     };
     const int cr = lane >> 1, cs = (lane & 1) ^ ((cr >> 3) & 1); // see rows_gemm_kernel
     auto row_of = [&](int r) { return (uint32_t)(n0 + r < a.n ? r : a.n - 1 - n0); };
-    auto copy_codes = [&](int u, int at) {
+    auto copy_codes = [&](int u, int at, int piece) {
         int unit = sb0 * 2 + u;
         unit = unit < 2 * nsb_row ? unit : 2 * nsb_row - 1;
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const int ct = cw * 2 + q; // column tile of 32 rows
-            const uint32_t row = row_of(ct * 32 + cr);
-#pragma unroll
-            for (int p = 0; p < T::PAIRS; p++)
-                copy(T::piece_src(a, unit, p) + (size_t)n0 * T::piece_pitch(a, p) + (row * T::piece_pitch(a, p) + cs * 16), wbase + at + ct * 32 * HB + p * 1024);
-        }
+        const int ct = cw * 2 + piece / T::PAIRS, p = piece % T::PAIRS; // column tile of 32 rows
+        const uint32_t row = row_of(ct * 32 + cr);
+        copy(T::piece_src(a, unit, p) + (size_t)n0 * T::piece_pitch(a, p), row * T::piece_pitch(a, p) + cs * 16, wbase + at + ct * 32 * HB + p * 1024);
         in_order();
     };
-    auto copy_sides = [&](int sb) { // 64 rows of every piece
+    auto copy_sides = [&](int sb, int c) { // 64 rows of piece c
         const int at = sb0 + sb < nsb_row ? sb0 + sb : nsb_row - 1, r0 = cw * 64;
-#pragma unroll
-        for (int c = 0; c < T::SIDE16; c++)
-            copy(T::side_src(a, at, c) + (size_t)n0 * T::side_pitch(a, c) + row_of(r0 + lane) * T::side_pitch(a, c), dbase + c * 128 * 16 + r0 * 16);
-        if constexpr (T::SIDE4 > 0)
-            __builtin_amdgcn_global_load_lds((gbl_void *)(T::side_src(a, at, T::SIDE16) + (size_t)n0 * T::side_pitch(a, T::SIDE16) +
-                                                          row_of(r0 + lane) * T::side_pitch(a, T::SIDE16)),
-                                             (lds_void *)(dbase + T::SIDE16 * 128 * 16 + r0 * 4), 4, 0, 0);
+        const uint8_t *src = T::side_src(a, at, c) + (size_t)n0 * T::side_pitch(a, c);
+        uint32_t off = row_of(r0 + lane) * T::side_pitch(a, c);
+        asm volatile("" : "+v"(off));
+        if (c < T::SIDE16) copy(src, off, dbase + c * 128 * 16 + r0 * 16);
+        else __builtin_amdgcn_global_load_lds((gbl_void *)(src + off), (lds_void *)(dbase + T::SIDE16 * 128 * 16 + r0 * 4), 4, 0, 0);
         in_order();
+    };
+    auto all = [](int n, auto fn) {
+#pragma unroll
+        for (int p = 0; p < n; p++) fn(p);
     };
     auto turn_over = [] {
         __builtin_amdgcn_sched_barrier(0);
@@ -1374,36 +1407,38 @@ __global__ void __launch_bounds__(512, 2) rows_apart_kernel(RowsArgs a) {
     };
     // ---- the requests in front of the first turn, in the order of the later ones
     if (x_wave) {
-        copy_x(0, 0);
-        copy_x(1, XBYTES);
+        all(Tile::XL, [&](int p) { copy_x(0, 0, p); });
+        all(Tile::XL, [&](int p) { copy_x(1, XBYTES, p); });
         wait_loads_and_lds<Tile::XL>();
     } else {
-        copy_sides(0);
-        copy_codes(0, 0);
-        copy_sums(0);
-        copy_codes(1, WBYTES);
+        all(Tile::D, [&](int p) { copy_sides(0, p); });
+        all(Tile::WL, [&](int p) { copy_codes(0, 0, p); });
+        all(Tile::SL, [&](int p) { copy_sums(0, p); });
+        all(Tile::WL, [&](int p) { copy_codes(1, WBYTES, p); });
         wait_loads_and_lds<Tile::SL + Tile::WL>();
     }
     barrier();
     T::template read_side<128>(dbase, wn * 32 + li, hh, sb0, next_side);
     if (half) turn_over(); // the second half is a turn behind
     int x_at = 0;
-    auto turn = [&](int sb, auto which) {
+    auto turn = [&](int sb, auto which, auto copier) __attribute__((always_inline)) {
+        constexpr bool COPIES_X = decltype(copier)::value;
         constexpr int J = decltype(which)::value;
         const bool live = sb < mine;
-        half8 xf[4][MI];
+        // x and operands of the products t = 0 and 1; those of 2 and 3 take their place when they are done with
+        half8 xf[2][MI], wf[2][T::PRODUCTS];
+        auto read_x = [&](int t, int i) { xf[t & 1][i] = *reinterpret_cast<const half8 *>(my_x + x_at + i * 4096 + t * 1024); };
         typename T::Raw raw;
         half8 offs;
         int over = 0;
         // ---- fetch
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-            for (int i = 0; i < MI; i++) xf[t][i] = *reinterpret_cast<const half8 *>(my_x + x_at + i * 4096 + t * 1024);
         T::read_raw(my_codes + (J >> 1) * WBYTES, li, hh, J, raw);
         in_order();
-        if (x_wave) copy_x(4 * sb + J + 2, x_at == 0 ? (NX - 1) * XBYTES : x_at - XBYTES); // the place of the step that everybody has read
-        else if (J == 2) copy_sums(sb + 1);
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int i = 0; i < MI; i++) read_x(t, i);
+        in_order();
         if (J == 0) {
             if (sb > 0) fold(); // of the superblock before
             side = next_side;
@@ -1420,24 +1455,40 @@ __global__ void __launch_bounds__(512, 2) rows_apart_kernel(RowsArgs a) {
         if (J == 3) T::template read_side<128>(dbase, wn * 32 + li, hh, sb0 + sb + 1, next_side);
 #pragma unroll
         for (int i = 0; i < MI; i++) asm volatile("" : "+v"(total[i][0])); // added here, while x is on its way, not behind the wait
+        auto make = [&](int t) {
+            T::make(raw, side, scales, mask, J, t, hh, wf[t & 1]);
+#pragma unroll
+            for (int pr = 0; pr < T::PRODUCTS; pr++) asm volatile("" : "+v"(wf[t & 1][pr]));
+        };
+        make(0);
+        make(1);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         turn_over();
         // ---- multiply
-        if (!x_wave) {
-            if (J == 0) copy_sides(sb + 1);
-            if (J & 1) copy_codes(2 * sb + (J >> 1) + 2, (J >> 1) * WBYTES);
-        }
+        auto between = [&](int slot) { // copies, piece by piece between the products (see rows_wide_kernel)
+            __builtin_amdgcn_sched_barrier(0);
+            if (COPIES_X) {
+                if (slot % 2 == 0) copy_x(4 * sb + J + 2, x_at == 0 ? (NX - 1) * XBYTES : x_at - XBYTES, slot / 2); // the place of the step that everybody has read
+            } else {
+                if (J == 0 && slot < Tile::D) copy_sides(sb + 1, slot);
+                if (J == 2 && slot < Tile::SL) copy_sums(sb + 1, slot);
+                if ((J & 1) && slot < Tile::WL) copy_codes(2 * sb + (J >> 1) + 2, (J >> 1) * WBYTES, slot);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
         __builtin_amdgcn_s_setprio(1);
         const float16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            half8 wf[T::PRODUCTS];
-            T::make(raw, side, scales, mask, J, t, hh, wf);
+        for (int t = 0; t < 4; t++)
 #pragma unroll
             for (int pr = 0; pr < T::PRODUCTS; pr++)
 #pragma unroll
-                for (int i = 0; i < MI; i++) part[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[t][i], wf[pr], J % 2 == 0 && t == 0 && pr == 0 ? zero : part[i], 0, 0, 0);
-        }
+                for (int i = 0; i < MI; i++) {
+                    if (pr == 0 && i == 1 && (t == 1 || t == 2)) make(t + 1);
+                    part[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[t & 1][i], wf[t & 1][pr], J % 2 == 0 && t == 0 && pr == 0 ? zero : part[i], 0, 0, 0);
+                    if (pr == 0) between(t * MI + i);
+                    if (t < 2 && pr == T::PRODUCTS - 1) read_x(t + 2, i);
+                }
         if constexpr (T::MIN && J == 1) {
             auto times_pow2 = [&](int e) { // a column's lanes all have its factor; exact, being a power of two
                 if (__builtin_amdgcn_ballot_w64(over > 0) == 0) return;
@@ -1457,16 +1508,20 @@ __global__ void __launch_bounds__(512, 2) rows_apart_kernel(RowsArgs a) {
         }
         __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
-        if (x_wave) wait_loads_and_lds<Tile::XL>(); // what the next turns read
+        if (COPIES_X) wait_loads_and_lds<Tile::XL>(); // what the next turns read
         else if (J == 0 || J == 1) wait_loads_and_lds<Tile::WL + Tile::D>();
         else wait_loads_and_lds<Tile::WL + Tile::SL>();
         turn_over();
         x_at = x_at == (NX - 1) * XBYTES ? 0 : x_at + XBYTES;
     };
-    for (int sb = 0; sb < loops; sb++) {
-        turn(sb, std::integral_constant<int, 0>{}); turn(sb, std::integral_constant<int, 1>{});
-        turn(sb, std::integral_constant<int, 2>{}); turn(sb, std::integral_constant<int, 3>{});
-    }
+    auto run = [&](auto copier) __attribute__((always_inline)) { // a loop for each kind of wave, see rows_wide_kernel
+        for (int sb = 0; sb < loops; sb++) {
+            turn(sb, std::integral_constant<int, 0>{}, copier); turn(sb, std::integral_constant<int, 1>{}, copier);
+            turn(sb, std::integral_constant<int, 2>{}, copier); turn(sb, std::integral_constant<int, 3>{}, copier);
+        }
+    };
+    if (x_wave) run(std::true_type{});
+    else run(std::false_type{});
     if (mine == loops) fold(); // else the last one was not this half's
     if (!half) barrier();
     wait_loads_and_lds<0>(); // nothing of this workgroup may still be on its way into LDS
@@ -1826,9 +1881,8 @@ RowsPlan rows_plan(const axq_ctx *ctx, const axq_weight *w, int in, int rows, bo
     const int n = (int)w->n_rows, nsb = (int)(w->kp >> 8);
     // Blocks of 32 take large tiles where the small ones are more than one to a compute unit: their sums of a superblock, which keep additions
     // of the total's size few, fit the registers of 128 x 128 outputs only (Q4_0, K = 4096: an error of 0.83 10^-7 there, 2.0 in large tiles).
-    // bf16 rows, us in the former kernel of that range, with operands in LDS, and now: 2048 x 14336 x 4096 Q4_0 414 411, Q4_1 475 451, Q5_0 482 431,
-    // Q5_1 557 475, Q8_0 447 414; 700 x 11008 x 2048 Q4_0 119 111, Q5_1 153 126; 130 x 17000 x 1024 Q5_0 42.5 35.7.  (Operands made in the
-    // fetch, not between the products: Q4_0 397, Q4_1 471, Q5_1 539.)
+    // bf16 rows, us in the former kernel of that range, with operands in LDS, and now: 2048 x 14336 x 4096 Q4_0 414 331, Q5_0 482 365,
+    // Q5_1 557 414, Q8_0 447 354.
     p.wide = !p.limbs && (super ? wide_tiles(ctx, p.m, n, w->kp) : square_tiles(p.m, n) > ctx->prop.multiProcessorCount);
     const int groups = p.m <= (p.limbs ? 32 : 64) ? 2 : 1; // of waves along K
     p.bm = p.limbs ? (rows <= 32 ? 32 : 40) : p.m <= 32 ? 32 : p.m <= 64 ? 64 : p.wide ? 256 : 128;
@@ -1846,9 +1900,8 @@ RowsPlan rows_plan(const axq_ctx *ctx, const axq_weight *w, int in, int rows, bo
     p.sb_per_split = (nsb + splits - 1) / splits;
     p.splits = (nsb + p.sb_per_split - 1) / p.sb_per_split;
     // 128 x 128 outputs whose halves have K of their own: from eight superblocks per workgroup on.  Shorter ones are mostly the start, which
-    // two parts of K make longer.  f32 rows, us so and with shared K: 64 rows, Q4_K 28672 x 4096 (sixteen) 57.2 62.7, Q5_K and Q6_K
-    // 14336 x 4096 (eight) 38.8 43.7 and 45.2 52.0, Q4_K 6144 x 4096 (four) 25.9 25.9, 4096 x 14336 (seven) 41.5 40.2, 4096 x 4096 (two)
-    // 24.2 23.5; bf16 rows: 128, Q4_K 14336 x 4096 (eight) 37.7 39.0; 100, Q5_K 11008 x 4096 (eight) 35.4 40.2
+    // two parts of K make longer.  f32 rows, us so and with shared K: 64 rows, Q4_K 28672 x 4096 (sixteen) 52.5 62.7, Q5_K and Q6_K
+    // 14336 x 4096 (eight) 36.5 43.7 and 44.0 52.0; bf16 rows: 128, Q4_K 14336 x 4096 (eight) 37.7 39.0; 100, Q5_K 11008 x 4096 (eight) 35.4 40.2
     p.apart = super && !p.limbs && !p.wide && p.m > 64 && p.sb_per_split >= 8;
     return p;
 }
