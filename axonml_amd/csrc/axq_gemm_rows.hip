@@ -1899,10 +1899,12 @@ RowsPlan rows_plan(const axq_ctx *ctx, const axq_weight *w, int in, int rows, bo
     if (splits < 2 || whole_k) splits = 1;
     p.sb_per_split = (nsb + splits - 1) / splits;
     p.splits = (nsb + p.sb_per_split - 1) / p.sb_per_split;
-    // 128 x 128 outputs whose halves have K of their own: from eight superblocks per workgroup on.  Shorter ones are mostly the start, which
-    // two parts of K make longer.  f32 rows, us so and with shared K: 64 rows, Q4_K 28672 x 4096 (sixteen) 52.5 62.7, Q5_K and Q6_K
-    // 14336 x 4096 (eight) 36.5 43.7 and 44.0 52.0; bf16 rows: 128, Q4_K 14336 x 4096 (eight) 37.7 39.0; 100, Q5_K 11008 x 4096 (eight) 35.4 40.2
-    p.apart = super && !p.limbs && !p.wide && p.m > 64 && p.sb_per_split >= 8;
+    // 128 x 128 outputs whose halves have K of their own, a superblock each at least.  f32 rows, us so and with shared K: 64 rows, Q4_K 28672 x 4096
+    // (sixteen per workgroup) 52.5 62.7, Q5_K and Q6_K 14336 x 4096 (eight) 36.5 43.7 and 44.0 52.0, 4096 x 14336 (seven) Q4_K 36.5 36.8, Q5_K
+    // 41.3 43.8, Q6_K 48.6 50.8, 6144 x 4096 (four) Q4_K 24.3 26.4, Q6_K 27.9 31.1, Q4_K 4096 x 4096 (two) 21.5 23.1; 100 bf16 rows, Q4_K 4096 x
+    // 14336 36.1 37.0.  Error against 64 bits, 64 rows, three seeds, 1e-8: Q4_K 6144 x 4096 11.29 11.34 11.30 and 11.26 11.32 11.30, 4096 x 14336
+    // 11.75 11.76 11.74 and 11.71 11.72 11.70, Q6_K 6144 x 4096 12.31 12.33 12.33 and 12.31 12.34 12.33: the same additions in another order.
+    p.apart = super && !p.limbs && !p.wide && p.m > 64 && p.sb_per_split >= 2;
     return p;
 }
 

@@ -35,6 +35,17 @@ def test_halves_with_their_own_k_and_all_of_it(ctx, qtype, rows, n, k, bf16):
     _check(ctx, qtype, n, k, packed, x, bias=None if bf16 else rng.standard_normal(n).astype(np.float32), bf16=bf16)
 
 
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
+@pytest.mark.parametrize("rows,n,k,bf16", [(40, 16385, 256, False), (64, 16386, 512, False), (41, 16387, 768, False), (65, 16512, 1024, True), (128, 16390, 1280, True),
+                                           (33, 4096, 1536, True), (50, 513, 4096, False), (64, 6144, 7168, False)])
+def test_halves_of_few_superblocks(ctx, qtype, rows, n, k, bf16):
+    """One superblock (which shares its K), two, three .. seven, alone and in parts; 33 bf16 rows are no large tile."""
+    rng = np.random.default_rng(rows + n + k + qtype)
+    packed = o.quantize(qtype, gen_weight(rng, 509, k)).reshape(509, -1)[np.arange(n) % 509].reshape(-1)
+    x = rng.standard_normal((rows, k)).astype(np.float32) * (10.0 ** rng.integers(-3, 4, size=(rows, 1))).astype(np.float32)
+    _check(ctx, qtype, n, k, packed, x, bias=None if bf16 else rng.standard_normal(n).astype(np.float32), bf16=bf16)
+
+
 @pytest.mark.parametrize("qtype", [o.Q4_K, o.Q6_K, o.Q8_0])
 @pytest.mark.parametrize("rows", [10, 17, 33, 40, 64, 65])
 @pytest.mark.parametrize("sizes", [dict(hidden_size=512, intermediate_size=4352, num_heads=8, num_kv_heads=4),
