@@ -333,11 +333,13 @@ __global__ void __launch_bounds__(64 * WM * WN * KG, 2) dense_gemm_kernel(GemmAr
     write_tile<MT, NT, GROUPED>(p, a.parts.cap, acc, patch, below + m0 + wm * (BM / WM), below + m1, n0 + wn * (BN / WN), lane);
 }
 
-// The same product with the two waves of a SIMD taking turns: while one multiplies, the other fetches the operands of its next
-// products from LDS and requests what comes into LDS after them.  Waves 0 .. 3 are one half of the workgroup and 4 .. 7 the other, half a
+// The same product with the two waves of a SIMD taking turns: while one multiplies, and between its products requests what comes into LDS
+// after them (a request keeps its wave for 40 to 50 cycles, the matrix pipe works on; among the reads, before and so, us: BF16 2048 bf16 rows x
+// 14336 x 4096 250 240, 2047 x 2048 x 2048 30.5 27.6, 2047 x 8192 x 2048 75 74, F16 1278 x 7520 x 1856 65 61.6), the other reads the operands of
+// its next products from LDS.  Waves 0 .. 3 are one half of the workgroup and 4 .. 7 the other, half a
 // round apart, with a barrier behind every turn: a turn is sixteen products (0.26 us of the matrix pipe), the other half's reads hide
 // behind it whole, and no wave has its reads, their latency and its products in one line.
-// LDS is a ring of five units of 32 KB, filled four ahead: every request has three turns of each half (1.5 us) on its way.
+// LDS is a ring of five units of 32 KB, filled four ahead: every request has two and a half turns of each half (1.3 us) on its way.
 //   SPLIT = false: 256 x 256 outputs, a unit is 32 of K, which both halves (128 x 64 per wave) read.
 //   SPLIT = true: 128 x 128 outputs, a unit is 64 of K; the halves take every other one, and their sums meet in LDS.
 // A row of a unit is 64 or 128 bytes whose 16-byte pieces are exchanged so that sixteen consecutive rows' reads touch all banks.
@@ -371,15 +373,17 @@ __global__ void __launch_bounds__(512, 2) dense_turns_kernel(GemmArgs a) {
         gb[i] = p.w + (size_t)row * p.ldw + c * 8;
     }
     const int units = a.k / KU, its = SPLIT ? (units + 1) / 2 : units;
-    auto fetch = [&](int u, int at) { // unit u (past the end the last one again, which nobody multiplies) to element `at` of LDS
+    auto request = [&](int u, int at, int piece) { // of unit u (past the end the last one again, which nobody multiplies) to element `at` of LDS
         u = u < units ? u : units - 1;
-        const int wu = weight_step(u, a.wk / KU);
-        uint16_t *to = lds + at + gw * 512;
-#pragma unroll
-        for (int i = 0; i < L; i++) __builtin_amdgcn_global_load_lds((gbl_void *)(ga[i] + (size_t)u * KU), (lds_void *)(to + i * LW * 512), 16, 0, 0);
-#pragma unroll
-        for (int i = 0; i < L; i++) __builtin_amdgcn_global_load_lds((gbl_void *)(gb[i] + (size_t)wu * KU), (lds_void *)(to + UNIT / 2 + i * LW * 512), 16, 0, 0);
+        const int wu = weight_step(u, a.wk / KU), i = piece % L;
+        uint16_t *to = lds + at + gw * 512 + i * LW * 512;
+        if (piece < L) __builtin_amdgcn_global_load_lds((gbl_void *)(ga[i] + (size_t)u * KU), (lds_void *)to, 16, 0, 0);
+        else __builtin_amdgcn_global_load_lds((gbl_void *)(gb[i] + (size_t)wu * KU), (lds_void *)(to + UNIT / 2), 16, 0, 0);
         asm volatile("" ::: "memory");
+    };
+    auto fetch = [&](int u, int at) {
+#pragma unroll
+        for (int q = 0; q < 2 * L; q++) request(u, at, q);
     };
     auto barrier = [] {
         __builtin_amdgcn_sched_barrier(0);
@@ -436,24 +440,28 @@ __global__ void __launch_bounds__(512, 2) dense_turns_kernel(GemmArgs a) {
             for (int i = 0; i < MT; i++) fa[ks][i] = *reinterpret_cast<const u32x4 *>(la + c + i * 32 * KU);
         }
         asm volatile("" ::: "memory");
-        // unit u + 4 takes the place of unit u - 1, which both halves have read; what the next turns read has come behind the barriers:
-        // of a shared unit both halves' requests in front of the first half's turn
-        fetch(u + 4, at == 0 ? (RING - 1) * UNIT : at - UNIT);
         if (it > 0) fold();
+        // what the next turns read has come behind the barriers: of a shared unit both halves' requests in front of the first half's turn
         if (SPLIT) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
         barrier();
         if (!SPLIT || u < units) {
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
             for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-                for (int i = 0; i < MT; i++)
+                for (int i = 0; i < MT; i++) {
 #pragma unroll
                     for (int j = 0; j < NT; j++) {
                         if constexpr (FOLD) part[i][j] = mma<HALF>(fa[ks][i], fb[ks][j], ks ? part[i][j] : zero);
                         else acc[i][j] = mma<HALF>(fa[ks][i], fb[ks][j], acc[i][j]);
                     }
+                    // unit u + 4 takes the place of unit u - 1, which both halves have read; a piece of it behind every pair of products, or every other
+                    __builtin_amdgcn_sched_barrier(0);
+                    const int slot = ks * MT + i, every = KS * MT / (2 * L);
+                    if (slot % every == 0) request(u + 4, at == 0 ? (RING - 1) * UNIT : at - UNIT, slot / every);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             __builtin_amdgcn_s_setprio(0);
         }
         if (SPLIT) {
