@@ -180,9 +180,12 @@ struct axq_rows_chain {
     const float *norm_w = nullptr;
     const axq_weight *ready_for = nullptr;
     size_t ready_at = 0;
+    bool swiglu = false; // y takes silu(gate) * up of columns that alternate in groups of four (see axq_dev_rows_gemm_makes_swiglu)
 };
 int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, int rows, const float *norm_w, float eps, const float *bias,
                       const float *resid, float *y, axq_rows_chain *chain = nullptr);
+// Whether a call of `rows` f32 rows can leave silu(gate) * up of its columns, which alternate in groups of four, in place of them
+bool axq_dev_rows_gemm_makes_swiglu(const axq_ctx *ctx, const axq_weight *w, int rows);
 // gemm.hip
 int axq_gemm_reserve(axq_ctx *ctx, size_t need);
 // Row pitch of the partial sums of a split K: whole groups of four columns, which the reduction takes (K of an odd number of columns used

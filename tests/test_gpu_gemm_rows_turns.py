@@ -67,3 +67,27 @@ def test_operands_made_with_the_reduction(ctx, qtype, rows, sizes):
     assert max_rel_err(logits, step, DECODE_FLOOR) <= DECODE_RTOL
     gpu.close()
     cpu.close()
+
+
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q6_K, o.Q4_1])
+@pytest.mark.parametrize("inter", [8256, 8320], ids=["half a large tile left", "whole tiles"])
+@pytest.mark.parametrize("rows", [40, 64, 65, 129])
+def test_gate_and_up_leave_their_product(ctx, qtype, inter, rows):
+    """More column tiles than half the compute units, so that a workgroup has all of K: tiles of 128 and of 256 rows of operands, and those of blocks."""
+    c = tiny_config(max_seq_len=rows + 8, vocab_size=64, num_layers=2)  # of a prompt the last layer ends with its keys and values
+    w = random_weights(c, rows, qtype, std=0.02)
+    c["intermediate_size"] = inter
+    rng = np.random.default_rng([rows, inter])
+    w["types"] = {}
+    for l, L in enumerate(w["layers"]):
+        for name, t, shape in (("gate", qtype, (inter, 256)), ("up", qtype, (inter, 256)), ("down", o.Q8_0, (256, inter))):
+            L[name] = o.quantize(t, (rng.standard_normal(shape) * 0.05).astype(np.float32))
+            w["types"][(l, name)] = t
+    cpu, gpu = load_oracle(c, w), load_gpu(ctx, c, w)
+    tokens = rng.integers(0, c["vocab_size"], size=rows + 1)
+    for pos, t in enumerate(tokens):
+        _, lg = cpu.forward(int(t), pos)
+    _, logits = gpu.forward_tokens(tokens)
+    assert max_rel_err(logits, lg, DECODE_FLOOR) <= DECODE_RTOL
+    gpu.close()
+    cpu.close()
