@@ -207,7 +207,7 @@ int axq_init(int device, axq_ctx **out) {
     ctx->fp8_unit_inv = 1.0f / h[0];
     {
         // one vector split, or a small batch packed plus the partial sums of its split K
-        size_t xq_bytes = axq_xq_bytes(AXQ_XQ_MAX_K), mb_bytes = AXQ_BATCH_SCRATCH_BYTES;
+        size_t xq_bytes = axq_xq_bytes(AXQ_XQ_MAX_K), mb_bytes = AXQ_BATCH_SCRATCH_BYTES + (size_t)34 * AXQ_BATCH_MAX_K; // and the operands that a call leaves while it reads its own
         INIT_HIP(hipMalloc((void **)&ctx->xq, xq_bytes > mb_bytes ? xq_bytes : mb_bytes));
     }
     // this device's copy of the scratch of axq_gemv_f32_static; a device the table has no place for (or a failed

@@ -44,6 +44,9 @@ struct MbArgs {
     int n_rows, k, batch;
     int kx; // columns of x: k, or fewer, where the last superblock of the weight is not whole
     int chunks_per_split; // chunks of a row that one workgroup (blockIdx.y) takes
+    uint8_t *next_xa;     // rows of gate and up, four and four: where silu(gate) * up goes as the next GEMV's operands
+    float *next_xsg;
+    int next_even_odd;
 };
 
 __device__ inline float f16lo(uint32_t v) { return __half2float(__ushort_as_half((unsigned short)(v & 0xFFFF))); }
@@ -313,25 +316,28 @@ struct MQ5x {
     }
 };
 
-template <class T>
+// ACT: 64 rows of gate and up, 32 to each half of the waves, whose 32 activations per vector are one block of the next GEMV's operands: the workgroup
+// leaves them as such, in place of its rows.  Four steps of eight sequences at the 7B shape 9378 -> 9200 us: the kernel takes 23.6 in place of 22.2, the
+// one that made the operands took 4.9.  (With eight waves to a tile, 1024 threads, 9471; with a chunk's codes requested a chunk ahead 9430.)
+template <class T, bool ACT>
 __global__ void __launch_bounds__(512, 4) gemv_mb_kernel(MbArgs a) {
     extern __shared__ float lds_f[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int S = (int)blockDim.x >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, waves = (int)blockDim.x >> 6, S = ACT ? waves >> 1 : waves;
+    const int all_wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = ACT && all_wave >= S, wave = all_wave - half * S;
     const int n = lane & 31, h = lane >> 5;
     const int nblk = a.k >> 5;
     float *sgs = lds_f;                    // [block of the row][h][4]: group scales of vectors h, h+2, h+4, h+6
     float *xss = sgs + (size_t)nblk * 8;   // same layout: plain sums of x over the group (contiguous with sgs)
     float *red = xss + (size_t)nblk * 8;   // [wave][vector][row]
-    u32x4 *patch = reinterpret_cast<u32x4 *>(red + (size_t)S * MAX_BATCH * 32) + (size_t)wave * 32 * (T::NP + T::NP2); // this wave's 32 x NP pieces
-    u32x4 *patch2 = patch + 32 * T::NP;                                                                              // and 32 x NP2 of the qh plane
+    u32x4 *patch = reinterpret_cast<u32x4 *>(red + (size_t)waves * MAX_BATCH * 32) + (size_t)all_wave * 32 * (T::NP + T::NP2); // this wave's 32 x NP pieces
+    u32x4 *patch2 = patch + 32 * T::NP;                                                                                      // and 32 x NP2 of the qh plane
 
     // scales and sums of all vectors -> LDS (already in the order the lanes read them).  Requesting the waves' first
     // chunks before this barrier instead of after it was slower (2.70 against 2.54 ms per batched 7B step): nobody
     // multiplies until the slowest wave's chunk has arrived.
     for (int t = tid; t < nblk * 4; t += (int)blockDim.x)
         reinterpret_cast<float4 *>(lds_f)[t] = reinterpret_cast<const float4 *>(a.xsg)[t];
-    const int row0 = blockIdx.x * 32;
+    const int row0 = ACT ? blockIdx.x * 64 + half * 32 : blockIdx.x * 32;
     int row = row0 + n;
     row = row < a.n_rows ? row : a.n_rows - 1;
     __syncthreads();
@@ -435,8 +441,37 @@ __global__ void __launch_bounds__(512, 4) gemv_mb_kernel(MbArgs a) {
     }
     // 4. partial sums of the waves -> y, in wave order
 #pragma unroll
-    for (int bi = 0; bi < 4; bi++) red[((size_t)wave * MAX_BATCH + (2 * bi + h)) * 32 + n] = acc[bi];
+    for (int bi = 0; bi < 4; bi++) red[((size_t)all_wave * MAX_BATCH + (2 * bi + h)) * 32 + n] = acc[bi];
     __syncthreads();
+    if constexpr (ACT) { // a thread per vector and activation, then one per vector and eight of them
+        float *act_of = red + (size_t)waves * MAX_BATCH * 32; // [vector][32], where the patches were
+        const int b0 = tid >> 5, o = tid & 31;
+        if (b0 < MAX_BATCH) {
+            const float *from = red + ((size_t)(o >> 4) * S * MAX_BATCH + b0) * 32 + ((o >> 2) & 3) * 8 + (o & 3); // four gates, four ups, and so again
+            float g = 0.f, u = 0.f;
+            for (int w = 0; w < S; w++) {
+                g += from[(size_t)w * MAX_BATCH * 32];
+                u += from[(size_t)w * MAX_BATCH * 32 + 4];
+            }
+            act_of[tid] = (g * (1.0f / (1.0f + expf(-g)))) * u; // as pack_x_kernel
+        }
+        __syncthreads();
+        if (tid >= 4 * MAX_BATCH) return;
+        const int t = tid & 3, b = tid >> 2;
+        float act[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) act[i] = act_of[b * 32 + t * 8 + i];
+        const int next_nblk = a.n_rows >> 6, task = blockIdx.x * 4 + t;
+        if (b >= a.batch) {
+            if (a.next_even_odd) axq_store_packed_zeros<true>(task, b, next_nblk, a.next_xa, a.next_xsg);
+            else axq_store_packed_zeros<false>(task, b, next_nblk, a.next_xa, a.next_xsg);
+        } else if (a.next_even_odd) {
+            axq_store_packed<true>(act, task, b, a.batch, next_nblk, a.next_xa, a.next_xsg);
+        } else {
+            axq_store_packed<false>(act, task, b, a.batch, next_nblk, a.next_xa, a.next_xsg);
+        }
+        return;
+    }
     for (int t = tid; t < a.batch * 32; t += (int)blockDim.x) {
         const int b = t >> 5, r = t & 31;
         if (row0 + r < a.n_rows) {
@@ -617,6 +652,16 @@ unsigned mb_max_waves() {
 }
 
 template <class T>
+constexpr size_t act_lds(int64_t k, unsigned S) {
+    return ((size_t)(k / 32) * 16 + (size_t)2 * S * MAX_BATCH * 32) * sizeof(float) + (size_t)2 * S * 32 * (T::NP + T::NP2) * 16;
+}
+template <class T>
+std::atomic<uint64_t> &act_lds_mask() {
+    static std::atomic<uint64_t> mask{0};
+    return mask;
+}
+
+template <class T>
 int launch_mb(axq_ctx *ctx, MbArgs a, uint8_t *sc, const float *x, int xmode, const float *aux, float eps, int next_even_odd, const float *next_aux) {
     const dim3 pgrid((unsigned)((a.k / 8 + 255) / 256), MAX_BATCH);
     uint8_t *xa = const_cast<uint8_t *>(a.xa);
@@ -627,6 +672,14 @@ int launch_mb(axq_ctx *ctx, MbArgs a, uint8_t *sc, const float *x, int xmode, co
     else if (xmode == AXQ_X_SWIGLU) pack_x_kernel<T::EVEN_ODD, AXQ_X_SWIGLU><<<pgrid, 256, 0, ctx->stream>>>(x, aux, eps, a.kx, a.k, a.batch, xa, xsg);
     else pack_x_kernel<T::EVEN_ODD, AXQ_X_PLAIN><<<pgrid, 256, 0, ctx->stream>>>(x, aux, eps, a.kx, a.k, a.batch, xa, xsg);
     const unsigned chunks = (unsigned)((a.k + WAVE_K - 1) / WAVE_K);
+    if (a.next_xa) {
+        a.chunks_per_split = (int)chunks;
+        const unsigned S = chunks < 4 ? chunks : 4;
+        const int st = axq_allow_lds(ctx, reinterpret_cast<const void *>(&gemv_mb_kernel<T, true>), act_lds_mask<T>(), 160 * 1024);
+        if (st != AXQ_OK) return st;
+        gemv_mb_kernel<T, true><<<a.n_rows / 64, 128 * S, act_lds<T>(a.k, S), ctx->stream>>>(a);
+        return AXQ_OK;
+    }
     const unsigned tiles = (unsigned)((a.n_rows + 31) / 32);
     // few row tiles (a narrow output): split K over up to four workgroups per tile so that the chip is full
     // (twice as many, for two workgroups per compute unit, was slower: 2.36 against 2.32 ms per batched 7B step; so were
@@ -642,10 +695,10 @@ int launch_mb(axq_ctx *ctx, MbArgs a, uint8_t *sc, const float *x, int xmode, co
     const unsigned S = (unsigned)a.chunks_per_split < smax ? (unsigned)a.chunks_per_split : smax;
     const size_t lds = ((size_t)(a.k / 32) * 16 + (size_t)S * MAX_BATCH * 32) * sizeof(float) + (size_t)S * 32 * (T::NP + T::NP2) * 16;
     if (lds > 64 * 1024) {
-        const int st = axq_allow_lds(ctx, reinterpret_cast<const void *>(&gemv_mb_kernel<T>), mb_lds_mask<T>(), 160 * 1024);
+        const int st = axq_allow_lds(ctx, reinterpret_cast<const void *>(&gemv_mb_kernel<T, false>), mb_lds_mask<T>(), 160 * 1024);
         if (st != AXQ_OK) return st; // the refusal is the call's error: nothing is launched into it
     }
-    gemv_mb_kernel<T><<<dim3(tiles, splits), 64 * S, lds, ctx->stream>>>(a);
+    gemv_mb_kernel<T, false><<<dim3(tiles, splits), 64 * S, lds, ctx->stream>>>(a);
     if (next_even_odd >= 0) {
         // y's operands for the next GEMV (k' = n_rows): the scratch layout of that call
         uint8_t *nxa = sc;
@@ -667,13 +720,19 @@ int launch_mb(axq_ctx *ctx, MbArgs a, uint8_t *sc, const float *x, int xmode, co
 // then 2 * (k / 32) * 8 floats of scales and sums; behind AXQ_BATCH_MAX_K's worth of those the partial sums of a split
 // K (splits only happen below AXQ_BATCH_SPLIT_ROWS rows).  Every byte that a kernel reads there is written earlier in
 // the same call, so the buffer needs no clearing between calls.
+// act_at: where the activations of a weight of gate and up go as the operands of the next GEMV (NULL: y takes the rows); at: where the operands of an
+// AXQ_X_PACKED call lie (NULL: in the scratch).
 int gemv_batch_in(axq_ctx *ctx, uint8_t *sc, const axq_weight *w, const float *x, int xmode, const float *aux, float eps, int batch,
-                  const float *bias, const float *resid, float *y, int next_even_odd, const float *next_aux) {
+                  const float *bias, const float *resid, float *y, int next_even_odd, const float *next_aux, uint8_t *act_at = nullptr, int act_even_odd = 0,
+                  const uint8_t *at = nullptr) {
     const int k = (int)w->kp;
     MbArgs a;
+    a.next_xa = act_at;
+    a.next_xsg = reinterpret_cast<float *>(act_at + (act_at ? (size_t)32 * (w->n_rows / 2) : 0));
+    a.next_even_odd = act_even_odd;
     a.codes = w->codes; a.meta = w->meta; a.qh = w->qh;
     a.codes_pitch = w->codes_pitch; a.meta_pitch = w->meta_pitch; a.qh_pitch = w->qh_pitch;
-    a.xa = sc; a.xsg = reinterpret_cast<float *>(sc + (size_t)32 * k);
+    a.xa = at ? at : sc; a.xsg = reinterpret_cast<const float *>(a.xa + (size_t)32 * k);
     a.bias = bias; a.resid = resid; a.y = y;
     a.ypart = w->n_rows <= AXQ_BATCH_SPLIT_ROWS ? reinterpret_cast<float *>(sc + (size_t)34 * AXQ_BATCH_MAX_K) : nullptr;
     a.n_rows = (int)w->n_rows; a.k = k; a.kx = (int)w->k; a.batch = batch;
@@ -714,6 +773,28 @@ bool axq_dev_gemv_batch_takes(const axq_weight *w, int batch) {
     return batch <= MAX_BATCH && batch >= (w->n_rows * w->k >= 40 << 20 ? 2 : 3);
 }
 
+// Whether a call of `w`, gate and up rows in groups of four, can leave silu(gate) * up as the operands of the call with `down`: all of K in a workgroup (as
+// where 32-row tiles are more than half the compute units), whose 64 rows' pieces and sums fit LDS.
+bool axq_dev_gemv_batch_makes_act(const axq_ctx *ctx, const axq_weight *w, const axq_weight *down, int batch) {
+    if (!axq_dev_gemv_batch_covers(w, batch) || !axq_dev_gemv_batch_covers(down, batch) || w->n_rows != 2 * down->k) return false;
+    if (w->n_rows / 32 <= ctx->prop.multiProcessorCount / 2 || mb_max_waves() != 8) return false;
+    switch (w->type) {
+    case AXQ_Q8_0: return act_lds<MQ80>(w->kp, 8) <= 160 * 1024;
+    case AXQ_Q6_K: return act_lds<MQ6K>(w->kp, 8) <= 160 * 1024;
+    default: return act_lds<MQ5K>(w->kp, 8) <= 160 * 1024; // of the others the largest
+    }
+}
+
+// ... those operands, behind the scratch that the call itself reads
+static uint8_t *act_operands(axq_ctx *ctx) { return ctx->xq + AXQ_BATCH_SCRATCH_BYTES; }
+
+int axq_dev_gemv_batch_act(axq_ctx *ctx, const axq_weight *w, const float *x, int xmode, const float *aux, float eps, int batch, const axq_weight *down) {
+    if (!axq_dev_gemv_batch_makes_act(ctx, w, down, batch))
+        return axq_fail(ctx, AXQ_ERR_SHAPE_MISMATCH, "Shape mismatch: the next weight does not take these rows' activations");
+    return gemv_batch_in(ctx, ctx->xq, w, x, xmode, aux, eps, batch, nullptr, nullptr, nullptr, -1, nullptr, act_operands(ctx),
+                         down->type == AXQ_Q4_0 || down->type == AXQ_Q4_1);
+}
+
 // Where a caller that prepares the operands of the call with w itself (axq_store_packed, then xmode = AXQ_X_PACKED) has
 // to put them; returns whether w takes the even and the odd elements of a block in separate halves.
 bool axq_dev_gemv_batch_operands(axq_ctx *ctx, const axq_weight *w, uint8_t **xa, float **xsg) {
@@ -744,7 +825,9 @@ int axq_dev_gemv_batch_chain(axq_ctx *ctx, const axq_weight *w, const float *x, 
             return axq_fail(ctx, AXQ_ERR_SHAPE_MISMATCH, "Shape mismatch: the next weight does not take this one's output");
         next_even_odd = (next->type == AXQ_Q4_0 || next->type == AXQ_Q4_1) ? 1 : 0;
     }
-    return gemv_batch_in(ctx, ctx->xq, w, x, xmode, aux, eps, batch, bias, resid, y, next_even_odd, next_aux);
+    const bool act = xmode == AXQ_X_ACT;
+    return gemv_batch_in(ctx, ctx->xq, w, x, act ? AXQ_X_PACKED : xmode, aux, eps, batch, bias, resid, y, next_even_odd, next_aux, nullptr, 0,
+                         act ? act_operands(ctx) : nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -773,10 +856,10 @@ int axq_gemv_static_setup(axq_ctx *ctx) {
     if (!ptr) return axq_fail(ctx, AXQ_ERR_DRIVER, "hipGetSymbolAddress gave no address for the static GEMV scratch");
     // Dynamic LDS beyond 64 KB has to be asked for once per kernel and device, and the development knob is read once: both
     // here, through the very masks the launch code consults, so that the entry point itself only launches.
-    int st = axq_allow_lds(ctx, reinterpret_cast<const void *>(&gemv_mb_kernel<MQ4x<false>>), mb_lds_mask<MQ4x<false>>(), 160 * 1024);
-    if (st == AXQ_OK) st = axq_allow_lds(ctx, reinterpret_cast<const void *>(&gemv_mb_kernel<MQ4x<true>>), mb_lds_mask<MQ4x<true>>(), 160 * 1024);
-    if (st == AXQ_OK) st = axq_allow_lds(ctx, reinterpret_cast<const void *>(&gemv_mb_kernel<MQ80>), mb_lds_mask<MQ80>(), 160 * 1024);
-    if (st == AXQ_OK) st = axq_allow_lds(ctx, reinterpret_cast<const void *>(&gemv_mb_kernel<MQ4K>), mb_lds_mask<MQ4K>(), 160 * 1024);
+    int st = axq_allow_lds(ctx, reinterpret_cast<const void *>(&gemv_mb_kernel<MQ4x<false>, false>), mb_lds_mask<MQ4x<false>>(), 160 * 1024);
+    if (st == AXQ_OK) st = axq_allow_lds(ctx, reinterpret_cast<const void *>(&gemv_mb_kernel<MQ4x<true>, false>), mb_lds_mask<MQ4x<true>>(), 160 * 1024);
+    if (st == AXQ_OK) st = axq_allow_lds(ctx, reinterpret_cast<const void *>(&gemv_mb_kernel<MQ80, false>), mb_lds_mask<MQ80>(), 160 * 1024);
+    if (st == AXQ_OK) st = axq_allow_lds(ctx, reinterpret_cast<const void *>(&gemv_mb_kernel<MQ4K, false>), mb_lds_mask<MQ4K>(), 160 * 1024);
     if (st != AXQ_OK) return st;
     (void)mb_max_waves();
     g_scratch_ptr[ctx->device] = ptr;

@@ -130,7 +130,8 @@ int axq_dev_gemv_dp(axq_ctx *ctx, const axq_weight *w, const float *x, const uin
 enum { AXQ_X_PLAIN = 0,    // nothing
        AXQ_X_RMSNORM = 1,  // x <- x / sqrt(mean(x^2) + eps) * aux   (aux = norm weights, K floats)
        AXQ_X_SWIGLU = 2,   // small-batch GEMV only: x holds 2K gate/up values (groups of four and four), x <- silu(gate) * up
-       AXQ_X_PACKED = 3 }; // small-batch GEMV only: the previous call of a chain has prepared this call's operands
+       AXQ_X_PACKED = 3,  // small-batch GEMV only: the previous call of a chain has prepared this call's operands
+       AXQ_X_ACT = 4 };   // ... which was axq_dev_gemv_batch_act
 // ... and to its result before it writes it:
 enum { AXQ_Y_PLAIN = 0,    // y[row] = dot (+ bias[row])
        AXQ_Y_SWIGLU = 1 }; // rows come in groups of four "gate" rows followed by their four "up" rows:
@@ -146,6 +147,8 @@ bool axq_dev_gemv_batch_takes(const axq_weight *w, int batch); // a call of its 
 int axq_dev_gemv_batch(axq_ctx *ctx, const axq_weight *w, const float *x, int batch, const float *bias, const float *resid, float *y);
 int axq_dev_gemv_batch_ex(axq_ctx *ctx, const axq_weight *w, const float *x, int xmode, const float *aux, float eps, int batch,
                           const float *bias, const float *resid, float *y);
+bool axq_dev_gemv_batch_makes_act(const axq_ctx *ctx, const axq_weight *w, const axq_weight *down, int batch);
+int axq_dev_gemv_batch_act(axq_ctx *ctx, const axq_weight *w, const float *x, int xmode, const float *aux, float eps, int batch, const axq_weight *down);
 int axq_dev_gemv_batch_chain(axq_ctx *ctx, const axq_weight *w, const float *x, int xmode, const float *aux, float eps, int batch,
                              const float *bias, const float *resid, float *y, const axq_weight *next, const float *next_aux);
 bool axq_dev_gemv_batch_operands(axq_ctx *ctx, const axq_weight *w, uint8_t **xa, float **xsg);

@@ -1,0 +1,29 @@
+"""Batched steps of up to eight sequences: gate and up leave the operands of the down projection, where their rows fill the chip without K in parts."""
+import numpy as np
+import pytest
+
+import oracle as o
+from tests.decode_common import load_gpu, load_oracle, random_weights, requantize, tiny_config
+from tests.util import DECODE_FLOOR, DECODE_RTOL, max_rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("gate,down", [(o.Q4_K, o.Q4_K), (o.Q4_K, o.Q4_0), (o.Q5_K, o.Q6_K), (o.Q6_K, o.Q4_1), (o.Q8_0, o.Q8_0), (o.Q5_1, o.Q5_0), (o.Q4_0, o.Q4_K)])
+@pytest.mark.parametrize("n_seq,hidden,inter", [(2, 256, 2304), (5, 768, 2304), (8, 1280, 2304), (8, 256, 2048)],
+                         ids=["one chunk", "three chunks", "five chunks", "too few rows"])
+def test_steps_of_several_sequences(ctx, gate, down, n_seq, hidden, inter):
+    c = tiny_config(hidden_size=hidden, intermediate_size=inter, num_layers=2, max_seq_len=16)
+    w = random_weights(c, n_seq, gate, std=0.03)
+    w = requantize(c, w, {(l, "down"): down for l in range(2)}, 7)
+    cpu, gpu = load_oracle(c, w), load_gpu(ctx, c, w)
+    gpu.set_batch(n_seq)
+    rng = np.random.default_rng([n_seq, hidden])
+    steps = rng.integers(0, c["vocab_size"], size=(3, n_seq))
+    got = [gpu.forward_batch(t)[1] for t in steps]
+    for s in range(n_seq):
+        for i in range(3):
+            _, lg = cpu.forward(int(steps[i, s]), i)
+            assert max_rel_err(got[i][s], lg, DECODE_FLOOR) <= DECODE_RTOL, (s, i)
+    gpu.close()
+    cpu.close()
