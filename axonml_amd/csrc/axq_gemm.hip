@@ -854,7 +854,10 @@ int axq_dev_gemm_f32_ex(axq_ctx *ctx, const axq_weight *w, const float *x, bool 
         return axq_fail(ctx, AXQ_ERR_INVALID_ARGUMENT, "axq_dev_gemm_f32_ex: SwiGLU rows need k %% 4 == 0, k <= 16384 and no norm");
     if (axq_dev_rows_gemm_covers(w, m))
         return axq_dev_rows_gemm(ctx, w, x, swiglu ? AXQ_ROWS_SWIGLU : AXQ_ROWS_F32, m, norm_w, eps, bias, resid, y, chain);
-    if (chain) chain->ready_for = nullptr;
+    if (chain) {
+        chain->ready_for = nullptr;
+        chain->sums = {};
+    }
     if (covers16(w, m, true)) {
         const bool half = w->type == AXQ_F16;
         Room16 r;

@@ -2041,7 +2041,10 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
     const int m = p.m, n = (int)w->n_rows, k = (int)w->k, kp = (int)w->kp, splits = p.splits;
     const bool ready = at != 0;
     const axq_weight *next = chain ? chain->next : nullptr;
-    if (chain) chain->ready_for = nullptr;
+    if (chain) {
+        chain->ready_for = nullptr;
+        chain->sums = {};
+    }
     size_t next_at = 0;
     RowsPlan np;
     RowsRoom nroom = {};
@@ -2098,6 +2101,15 @@ int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, 
     default: rc = launch_rows<Block32<8, false>>(ctx, a, p); break;
     }
     if (rc || splits == 1) return rc;
+    if (chain && chain->leave_sums && !bias && !resid) {
+        chain->sums.part = a.ypart;
+        chain->sums.scale = rs;
+        chain->sums.splits = splits;
+        chain->sums.row_mul = p.parts;
+        chain->sums.pitch = axq_part_pitch(n);
+        chain->sums.stride = (size_t)rows * axq_part_pitch(n);
+        return AXQ_OK;
+    }
     if (next_at) {
         const PartSums ps = {a.ypart, rs, splits, p.parts, resid, y};
         _Float16 *nxa, *nxs;

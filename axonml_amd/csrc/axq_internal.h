@@ -176,6 +176,13 @@ bool axq_dev_rows_gemm_covers(const axq_weight *w, int rows);
 #define AXQ_ROWS_PAIRS_MIN 40
 #define AXQ_ROWS_GEMM_MIN 10 // f32 rows from which it can be ahead of the small-batch GEMV in groups of eight
 bool axq_dev_rows_gemm_pays(const axq_ctx *ctx, const axq_weight *w, int rows); // whether it is, for a call of its own
+// The sums of parts of K that a call has left in the context's GEMM scratch for the next kernel of its stream: a value is scale[row * row_mul] times the sum
+// over the parts, added up as gemm_reduce_kernel does; none (splits = 0): they have been added up.
+struct axq_part_sums {
+    const float *part = nullptr, *scale = nullptr;
+    int splits = 0, row_mul = 1, pitch = 0; // elements from row to row
+    size_t stride = 0;                      // elements from part to part
+};
 // One after the other: `next` takes the rows that a call leaves (norm_w: RMS-normalised), with the context's GEMM scratch untouched in
 // between; `ready_for` is the weight whose operands are there, at ready_at.  Kept by the caller for its own chain of calls.
 struct axq_rows_chain {
@@ -184,6 +191,8 @@ struct axq_rows_chain {
     const axq_weight *ready_for = nullptr;
     size_t ready_at = 0;
     bool swiglu = false; // y takes silu(gate) * up of columns that alternate in groups of four (see axq_dev_rows_gemm_makes_swiglu)
+    bool leave_sums = false; // whoever takes y adds up the parts of a K that was split: y is not written where `sums` says so
+    axq_part_sums sums;
 };
 int axq_dev_rows_gemm(axq_ctx *ctx, const axq_weight *w, const void *x, int in, int rows, const float *norm_w, float eps, const float *bias,
                       const float *resid, float *y, axq_rows_chain *chain = nullptr);
