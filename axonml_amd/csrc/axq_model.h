@@ -1,5 +1,6 @@
 // The decode model's state, shared by the LLaMA-shape layers (axq_decode.hip) and the described layers (axq_stack.hip).
 #pragma once
+#include <functional>
 #include <vector>
 
 #include "axq_internal.h"
@@ -82,8 +83,9 @@ int axq_stack_step(axq_model *m);
 // nb tokens at positions pos0 .. pos0 + nb - 1; afterwards axq_stack_logits_rows can be asked for any of them, unless `results` said that nobody will.
 // layers: where the residual stream after layer run 0 goes (host; NULL: nowhere), and `layer_stride` elements on after every next one.
 int axq_stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, bool results, float *layers, size_t layer_stride);
-// the same, and the step of m->tok at *m->pos = pos0 + nb, to m->logits: as axq_stack_rows and then axq_stack_step leave it
-int axq_stack_rows_and_step(axq_model *m, const int32_t *toks, int nb, int pos0);
+// the same, and the step of m->tok at *m->pos = pos0 + nb, to m->logits: as axq_stack_rows and then axq_stack_step leave it.  `token` puts the two there, on the
+// context's stream of the moment.
+int axq_stack_rows_and_step(axq_model *m, const int32_t *toks, int nb, int pos0, const std::function<void()> &token);
 // logits of `n` rows (indices within the last axq_stack_rows, on the host) -> host memory
 int axq_stack_logits_rows(axq_model *m, const int32_t *rows, int n, float *logits);
 int axq_stack_layer_runs(const axq_model *m);

@@ -554,9 +554,16 @@ int step_embed(axq_model *m) {
 
 // rows: the event behind what a run takes of a prompt's rows, its cache or state; its first products wait for it only where they read the previous token's
 // input (the last run has nothing beside it: prompts of 2001 tokens through three layers of Gemosun 1.5 % shorter, 2048 through four of Lakulix 0.7).
-int step_run(axq_model *m, size_t run, hipEvent_t rows = nullptr) {
+// The last run goes on on the rows' stream, `back`, from there: what follows would wait for that stream, and the prompt's end for what follows.
+int step_run(axq_model *m, size_t run, hipEvent_t rows = nullptr, hipStream_t back = nullptr) {
     axq_stack &s = *m->stack;
     axq_ctx *ctx = m->ctx;
+    auto meet_rows = [&]() -> int {
+        if (back) AXQ_HIP(ctx, hipEventRecord(rows, ctx->stream), AXQ_ERR_DRIVER);
+        AXQ_HIP(ctx, hipStreamWaitEvent(back ? back : ctx->stream, rows, 0), AXQ_ERR_DRIVER);
+        if (back) ctx->stream = back; // (the caller puts its own in place again)
+        return AXQ_OK;
+    };
     const int W = s.c.width;
     const bool average = s.c.depth_average && !s.runs.empty();
     float *x = average && run == 0 ? s.past : m->h;
@@ -580,9 +587,9 @@ int step_run(axq_model *m, size_t run, hipEvent_t rows = nullptr) {
     in.prev = r.prev;
     in.pos = m->pos;
     const bool mix = c.mixer == AXQ_MIX_WKV;
-    if (rows && mix) AXQ_HIP(ctx, hipStreamWaitEvent(ctx->stream, rows, 0), AXQ_ERR_DRIVER);
+    if (rows && mix && (rc = meet_rows())) return rc;
     if ((rc = axq_dense_gemv(ctx, mix ? AXQ_IN_TANH_NORM_MIX : norm_mode(s), in, p.parts))) return rc;
-    if (rows && !mix) AXQ_HIP(ctx, hipStreamWaitEvent(ctx->stream, rows, 0), AXQ_ERR_DRIVER);
+    if (rows && !mix && (rc = meet_rows())) return rc;
     out_in.x = s.o;
     out_in.k = mixer_out(c);
     out_in.eps = s.c.norm_eps;
@@ -676,12 +683,14 @@ std::vector<First> cache_firsts(const axq_layer_config &c) {
     return f; // the recurrences read all of them
 }
 
-// `then_step`: behind every run's mixer the same run of the step of the next token, on ctx->aux_stream[0].  Without `results` nobody reads the residual
+// `then_step`: behind every run's mixer the same run of the step of the next token, on ctx->aux_stream[0], in front of the first one what this has to do there; the
+// rows' first product is launched before it, and the last run comes back to the rows' stream.  Without `results` nobody reads the residual
 // stream behind the rows, and the last run ends with its cache or state (2048 tokens, four layers of Lakulix at width 2048 1440 -> 1196 us; 2001, three of
 // Gemosun 1565 -> 1163).
-int stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, bool results, float *layers, size_t layer_stride, bool then_step) {
+int stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, bool results, float *layers, size_t layer_stride, const std::function<int()> *then_step) {
     axq_stack &s = *m->stack;
     axq_ctx *ctx = m->ctx;
+    hipStream_t st = ctx->stream;
     const int W = s.c.width, ldw = pad64(W);
     const size_t es = s.f32 ? 4 : 2;
     const bool first = pos0 == 0, average = s.c.depth_average && !s.runs.empty();
@@ -767,9 +776,10 @@ int stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, bool results
             if (!cache_only && (rc = axq_rows_rms_gate(ctx, gate, nb, mix ? c.dim : mo, xo))) return rc;
         }
         if (then_step) {
-            AXQ_HIP(ctx, hipEventRecord(s.ready, ctx->stream), AXQ_ERR_DRIVER);
+            AXQ_HIP(ctx, hipEventRecord(s.ready, st), AXQ_ERR_DRIVER);
             OnStream on(ctx, ctx->aux_stream[0]);
-            if ((rc = step_run(m, run, s.ready))) return rc;
+            if (run == 0 && (rc = (*then_step)())) return rc;
+            if ((rc = step_run(m, run, s.ready, cache_only ? st : nullptr))) return rc;
         }
         if (cache_only) return AXQ_OK;
         axq_parts o = {};
@@ -809,33 +819,39 @@ int axq_stack_step(axq_model *m) {
 
 // The step behind rows, a layer run of it as soon as the rows have left that run's cache or state, on a stream of its own: the step's kernels
 // are short and few workgroups wide, and the rows' later layers need nothing of them (nor do the two share scratch).
-int axq_stack_rows_and_step(axq_model *m, const int32_t *toks, int nb, int pos0) {
+// At a prompt's start the GPU has nothing to do but what the host has launched: the rows' way to their first product comes first.  At its end the step's last run
+// and the head are on the rows' stream, whose wait for the other stream is over by then.
+int axq_stack_rows_and_step(axq_model *m, const int32_t *toks, int nb, int pos0, const std::function<void()> &token) {
     axq_stack &s = *m->stack;
     axq_ctx *ctx = m->ctx;
     int rc = reserve_rows(m, nb); // in front of the step's first launch: allocations take longer beside one
-    if (rc) return rc;
-    AXQ_HIP(ctx, hipEventRecord(s.ready, ctx->stream), AXQ_ERR_DRIVER); // the token and its position
-    AXQ_HIP(ctx, hipStreamWaitEvent(ctx->aux_stream[0], s.ready, 0), AXQ_ERR_DRIVER);
-    {
-        OnStream on(ctx, ctx->aux_stream[0]);
-        rc = step_embed(m);
+    bool begun = false;
+    const std::function<int()> begin = [&] {
+        begun = true;
+        token();
+        return step_embed(m);
+    };
+    auto fork = [&]() -> int { // what the context's stream has done before
+        AXQ_HIP(ctx, hipEventRecord(s.ready, ctx->stream), AXQ_ERR_DRIVER);
+        AXQ_HIP(ctx, hipStreamWaitEvent(ctx->aux_stream[0], s.ready, 0), AXQ_ERR_DRIVER);
+        return AXQ_OK;
+    };
+    if (!rc && !s.runs.empty() && !(rc = fork())) {
+        rc = stack_rows(m, toks, nb, pos0, false, nullptr, 0, &begin);
+        if (rc) { // whatever has happened, what comes on the context's stream comes behind the step
+            const hipError_t e = hipEventRecord(s.ready, ctx->aux_stream[0]);
+            if (e != hipSuccess || hipStreamWaitEvent(ctx->stream, s.ready, 0) != hipSuccess) (void)hipStreamSynchronize(ctx->aux_stream[0]);
+        }
     }
-    if (!rc) rc = stack_rows(m, toks, nb, pos0, false, nullptr, 0, true);
-    if (!rc) {
-        OnStream on(ctx, ctx->aux_stream[0]);
-        rc = step_head(m);
+    if (!begun) { // no layers, or not as far as the first of them
+        const int e = begin();
+        if (!rc) rc = e;
     }
-    // whatever has happened, what comes on the context's stream comes behind the step
-    const hipError_t e = hipEventRecord(s.ready, ctx->aux_stream[0]), w = e == hipSuccess ? hipStreamWaitEvent(ctx->stream, s.ready, 0) : e;
-    if (w != hipSuccess) {
-        (void)hipStreamSynchronize(ctx->aux_stream[0]);
-        if (!rc) rc = axq_fail(ctx, AXQ_ERR_DRIVER, "a step beside rows: %s", hipGetErrorString(w));
-    }
-    return rc;
+    return rc ? rc : step_head(m);
 }
 
 int axq_stack_rows(axq_model *m, const int32_t *toks, int nb, int pos0, bool results, float *layers, size_t layer_stride) {
-    return stack_rows(m, toks, nb, pos0, results, layers, layer_stride, false);
+    return stack_rows(m, toks, nb, pos0, results, layers, layer_stride, nullptr);
 }
 
 int axq_stack_logits_rows(axq_model *m, const int32_t *rows, int n, float *logits) {
