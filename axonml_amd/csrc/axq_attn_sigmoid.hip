@@ -16,8 +16,7 @@ struct Args {
     void *qs;           // prepared queries: f16 [m][heads][dp] or f32 [m][heads][dim]
 };
 
-// grid (heads + 2 kv_heads, rows), one wave: query head -> normed, scaled by position; key head -> normed, cache; value -> cache
-template <bool F32>
+// f32 cache: grid (heads + 2 kv_heads, rows), one wave: query head -> normed, scaled by position; key head -> normed, cache; value -> cache
 __global__ void __launch_bounds__(64) prep_kernel(Args g) {
     const axq_sig_attn &a = g.a;
     const int t = blockIdx.y, lane = threadIdx.x, p = g.pos ? g.pos[0] : g.pos0 + t;
@@ -28,13 +27,8 @@ __global__ void __launch_bounds__(64) prep_kernel(Args g) {
         for (int e = lane; e < a.dim; e += 64) ss = fmaf(q[e], q[e], ss);
         ss = axq_wave_sum(ss);
         const float inv = 1.0f / sqrtf(ss / (float)a.dim + a.eps), temp = a.temp[p];
-        if (F32) {
-            float *o = reinterpret_cast<float *>(g.qs) + ((size_t)t * a.heads + h) * a.dim;
-            for (int e = lane; e < a.dim; e += 64) o[e] = q[e] * inv * a.qn[e] * temp;
-        } else {
-            _Float16 *o = reinterpret_cast<_Float16 *>(g.qs) + ((size_t)t * a.heads + h) * g.dp;
-            for (int e = lane; e < g.dp; e += 64) o[e] = e < a.dim ? to_half(q[e] * inv * a.qn[e] * temp) : (_Float16)0.f;
-        }
+        float *o = reinterpret_cast<float *>(g.qs) + ((size_t)t * a.heads + h) * a.dim;
+        for (int e = lane; e < a.dim; e += 64) o[e] = q[e] * inv * a.qn[e] * temp;
         return;
     }
     h -= a.heads;
@@ -44,27 +38,52 @@ __global__ void __launch_bounds__(64) prep_kernel(Args g) {
         for (int e = lane; e < a.dim; e += 64) ss = fmaf(k[e], k[e], ss);
         ss = axq_wave_sum(ss);
         const float inv = 1.0f / sqrtf(ss / (float)a.dim + a.eps);
-        if (F32) {
-            float *o = reinterpret_cast<float *>(a.kc) + ((size_t)h * a.cap + p) * a.dim;
-            for (int e = lane; e < a.dim; e += 64) o[e] = k[e] * inv * a.kn[e];
-        } else {
-            _Float16 *o = reinterpret_cast<_Float16 *>(a.kc) + ((size_t)h * g.capp + p) * g.dp;
-            for (int e = lane; e < a.dim; e += 64) o[e] = to_half(k[e] * inv * a.kn[e]); // the padding stays zero
-        }
+        float *o = reinterpret_cast<float *>(a.kc) + ((size_t)h * a.cap + p) * a.dim;
+        for (int e = lane; e < a.dim; e += 64) o[e] = k[e] * inv * a.kn[e];
         return;
     }
     h -= a.kv_heads;
     const float *v = g.v + (size_t)t * g.ldv + (size_t)h * a.vdim;
-    if (F32) {
-        float *o = reinterpret_cast<float *>(a.vc) + ((size_t)h * a.cap + p) * a.vdim;
-        for (int e = lane; e < a.vdim; e += 64) o[e] = v[e];
-    } else {
-        _Float16 *o = reinterpret_cast<_Float16 *>(a.vc) + (size_t)h * g.dvp * g.capp + value_slot(p);
-        for (int e = lane; e < a.vdim; e += 64) o[(size_t)e * g.capp] = to_half(v[e]);
-    }
+    float *o = reinterpret_cast<float *>(a.vc) + ((size_t)h * a.cap + p) * a.vdim;
+    for (int e = lane; e < a.vdim; e += 64) o[e] = v[e];
 }
 
-__global__ void __launch_bounds__(256) append_values_kernel(Args g) { append_values(g.v, g.ldv, g.a.vdim, g.m, g.pos0, g.a.vc, g.dvp, g.capp); }
+// f16 cache: the same of a prompt's rows (prep_grid)
+__global__ void __launch_bounds__(256) prep_rows_kernel(Args g, int values) {
+    const axq_sig_attn &a = g.a;
+    if ((int)blockIdx.x < values) return append_values(blockIdx.x, g.v, g.ldv, a.vdim, g.m, g.pos0, a.vc, g.dvp, g.capp);
+    const int lane = threadIdx.x & 63, queries = g.q ? a.heads : 0;
+    int h, t0;
+    prep_place(values, queries + a.kv_heads, h, t0);
+    if (h >= queries + a.kv_heads) return;
+    const bool query = h < queries;
+    const int kvh = h - queries;
+    const float *norm = query ? a.qn : a.kn;
+    float v[PREP_ROWS][PREP_CHUNKS], n[PREP_CHUNKS], temp[PREP_ROWS];
+    prep_load(query ? g.q + (size_t)h * a.dim : g.k + (size_t)kvh * a.dim, query ? g.ldq : g.ldk, a.dim, t0, g.m, v);
+#pragma unroll
+    for (int i = 0; i < PREP_CHUNKS; i++) n[i] = i * 64 < a.dim && i * 64 + lane < a.dim ? norm[i * 64 + lane] : 0.f;
+#pragma unroll
+    for (int r = 0; r < PREP_ROWS; r++) temp[r] = query && t0 + r < g.m ? a.temp[g.pos0 + t0 + r] : 1.f;
+#pragma unroll
+    for (int r = 0; r < PREP_ROWS; r++) {
+        if (t0 + r >= g.m) break;
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < PREP_CHUNKS; i++) ss = fmaf(v[r][i], v[r][i], ss);
+        ss = axq_wave_sum(ss);
+        const float inv = 1.0f / sqrtf(ss / (float)a.dim + a.eps);
+        _Float16 *o = query ? reinterpret_cast<_Float16 *>(g.qs) + ((size_t)(t0 + r) * a.heads + h) * g.dp
+                            : reinterpret_cast<_Float16 *>(a.kc) + ((size_t)kvh * g.capp + g.pos0 + t0 + r) * g.dp;
+#pragma unroll
+        for (int i = 0; i < PREP_CHUNKS; i++) {
+            if (i * 64 >= g.dp) break;
+            const int e = i * 64 + lane;
+            if (e < a.dim) o[e] = to_half(v[r][i] * inv * n[i] * temp[r]);
+            else if (query) o[e] = (_Float16)0.f; // the keys' padding stays zero
+        }
+    }
+}
 
 // Rows against the f32 cache: grid (heads, rows).  256 keys at a time: scores by thread, then the value sum by element.
 __global__ void __launch_bounds__(256) rows_f32_kernel(Args g, axq_rows_out out) {
@@ -431,11 +450,11 @@ int axq_sig_attn_rows(axq_ctx *ctx, const axq_sig_attn &a, const float *q, const
     const Args g = make_args(a, q, k, v, ldq, ldk, ldv, m, pos0, nullptr, qscratch);
     const int queries = q ? a.heads : 0; // without q: the keys and values alone
     if (a.f32) {
-        prep_kernel<true><<<dim3(queries + 2 * a.kv_heads, m), 64, 0, ctx->stream>>>(g);
+        prep_kernel<<<dim3(queries + 2 * a.kv_heads, m), 64, 0, ctx->stream>>>(g);
         if (q) rows_f32_kernel<<<dim3(a.heads, m), 256, f32_rows_lds(a), ctx->stream>>>(g, out);
     } else {
-        prep_kernel<false><<<dim3(queries + a.kv_heads, m), 64, 0, ctx->stream>>>(g);
-        append_values_kernel<<<dim3((m + 31) / 32, (a.vdim + 31) / 32, a.kv_heads), 256, 0, ctx->stream>>>(g);
+        const int values = value_tiles(m, a.vdim, a.kv_heads);
+        prep_rows_kernel<<<prep_grid(m, queries + a.kv_heads, values), 256, 0, ctx->stream>>>(g, values);
         if (q && (rc = g.dp == 64 ? launch_mfma_k<4>(ctx, g, out) : (g.dp == 128 ? launch_mfma_k<8>(ctx, g, out) : launch_mfma_k<16>(ctx, g, out)))) return rc;
     }
     AXQ_LAUNCH_CHECK(ctx, "sigmoid attention of rows");
@@ -448,7 +467,7 @@ int axq_sig_attn_token(axq_ctx *ctx, const axq_sig_attn &a, const float *q, cons
     if ((rc = check_shape(ctx, a))) return rc;
     const Args g = make_args(a, q, k, v, 0, 0, 0, 1, 0, pos, qscratch);
     if (a.f32) {
-        prep_kernel<true><<<dim3(a.heads + 2 * a.kv_heads, 1), 64, 0, ctx->stream>>>(g);
+        prep_kernel<<<dim3(a.heads + 2 * a.kv_heads, 1), 64, 0, ctx->stream>>>(g);
         axq_rows_out out = {att, a.heads * a.vdim, true};
         rows_f32_kernel<<<dim3(a.heads, 1), 256, f32_rows_lds(a), ctx->stream>>>(g, out);
     } else {

@@ -33,34 +33,23 @@ __device__ inline float rotated(const axq_soft_attn &a, const float *x, int e, i
     return (e & 1) ? fmaf(v, c, w * s) : fmaf(v, c, -(w * s));
 }
 
-// grid (heads + kv_heads (+ kv_heads of values in f32) in fours, rows), a wave each: rotated queries, keys into the cache
-template <bool F32>
+// f32 cache: grid (heads + 2 kv_heads in fours, rows), a wave each: rotated queries, keys and values into the cache
 __global__ void __launch_bounds__(256) prep_kernel(Args g) {
     const axq_soft_attn &a = g.a;
     const int t = blockIdx.y, lane = threadIdx.x & 63, p = g.pos ? g.pos[0] : g.pos0 + t;
     int h = blockIdx.x * 4 + (threadIdx.x >> 6) + (g.q ? 0 : a.heads);
-    if (h >= a.heads + (F32 ? 2 : 1) * a.kv_heads) return;
+    if (h >= a.heads + 2 * a.kv_heads) return;
     if (h < a.heads) {
         const float *q = g.q + (size_t)t * g.ldq + (size_t)h * a.dim;
-        if (F32) {
-            float *o = reinterpret_cast<float *>(g.qs) + ((size_t)t * a.heads + h) * a.dim;
-            for (int e = lane; e < a.dim; e += 64) o[e] = rotated(a, q, e, p);
-        } else {
-            _Float16 *o = reinterpret_cast<_Float16 *>(g.qs) + ((size_t)t * a.heads + h) * g.dp;
-            for (int e = lane; e < g.dp; e += 64) o[e] = e < a.dim ? to_half(rotated(a, q, e, p)) : (_Float16)0.f;
-        }
+        float *o = reinterpret_cast<float *>(g.qs) + ((size_t)t * a.heads + h) * a.dim;
+        for (int e = lane; e < a.dim; e += 64) o[e] = rotated(a, q, e, p);
         return;
     }
     h -= a.heads;
     if (h < a.kv_heads) {
         const float *k = g.k + (size_t)t * g.ldk + (size_t)h * a.dim;
-        if (F32) {
-            float *o = reinterpret_cast<float *>(a.kc) + ((size_t)h * a.cap + p) * a.dim;
-            for (int e = lane; e < a.dim; e += 64) o[e] = rotated(a, k, e, p);
-        } else {
-            _Float16 *o = reinterpret_cast<_Float16 *>(a.kc) + ((size_t)h * g.capp + p) * g.dp;
-            for (int e = lane; e < a.dim; e += 64) o[e] = to_half(rotated(a, k, e, p)); // the padding stays zero
-        }
+        float *o = reinterpret_cast<float *>(a.kc) + ((size_t)h * a.cap + p) * a.dim;
+        for (int e = lane; e < a.dim; e += 64) o[e] = rotated(a, k, e, p);
         return;
     }
     h -= a.kv_heads;
@@ -69,7 +58,47 @@ __global__ void __launch_bounds__(256) prep_kernel(Args g) {
     for (int e = lane; e < a.vdim; e += 64) o[e] = v[e];
 }
 
-__global__ void __launch_bounds__(256) append_values_kernel(Args g) { append_values(g.v, g.ldv, g.a.vdim, g.m, g.pos0, g.a.vc, g.dvp, g.capp); }
+// f16 cache: rotated queries, keys and values into the cache (prep_grid)
+__global__ void __launch_bounds__(256) prep_rows_kernel(Args g, int values) {
+    const axq_soft_attn &a = g.a;
+    if ((int)blockIdx.x < values) return append_values(blockIdx.x, g.v, g.ldv, a.vdim, g.m, g.pos0, a.vc, g.dvp, g.capp);
+    const int lane = threadIdx.x & 63, queries = g.q ? a.heads : 0;
+    int h, t0;
+    prep_place(values, queries + a.kv_heads, h, t0);
+    if (h >= queries + a.kv_heads) return;
+    const bool query = h < queries;
+    const int kvh = h - queries, half = a.rot_dims >> 1;
+    float v[PREP_ROWS][PREP_CHUNKS], c[PREP_ROWS][PREP_CHUNKS], s[PREP_ROWS][PREP_CHUNKS];
+    prep_load(query ? g.q + (size_t)h * a.dim : g.k + (size_t)kvh * a.dim, query ? g.ldq : g.ldk, a.dim, t0, g.m, v);
+#pragma unroll
+    for (int r = 0; r < PREP_ROWS; r++)
+#pragma unroll
+        for (int i = 0; i < PREP_CHUNKS; i++) {
+            const int e = i * 64 + lane;
+            c[r][i] = 1.f;
+            s[r][i] = 0.f;
+            if (i * 64 < a.rot_dims && t0 + r < g.m && e < a.rot_dims) {
+                const size_t at = (size_t)(g.pos0 + t0 + r) * half + (e >> 1);
+                c[r][i] = a.rc[at];
+                s[r][i] = a.rs[at];
+            }
+        }
+#pragma unroll
+    for (int r = 0; r < PREP_ROWS; r++) {
+        if (t0 + r >= g.m) break;
+        _Float16 *o = query ? reinterpret_cast<_Float16 *>(g.qs) + ((size_t)(t0 + r) * a.heads + h) * g.dp
+                            : reinterpret_cast<_Float16 *>(a.kc) + ((size_t)kvh * g.capp + g.pos0 + t0 + r) * g.dp;
+#pragma unroll
+        for (int i = 0; i < PREP_CHUNKS; i++) {
+            if (i * 64 >= g.dp) break;
+            const int e = i * 64 + lane;
+            const float x = v[r][i], w = __shfl_xor(x, 1); // rotated() above
+            const float y = e >= a.rot_dims ? x : (e & 1) ? fmaf(x, c[r][i], w * s[r][i]) : fmaf(x, c[r][i], -(w * s[r][i]));
+            if (e < a.dim) o[e] = to_half(y);
+            else if (query) o[e] = (_Float16)0.f; // the keys' padding stays zero
+        }
+    }
+}
 
 // The means of block b for kv head h, by the threads tid, tid + n, ... of n.
 template <bool F32>
@@ -587,12 +616,12 @@ int axq_soft_attn_rows(axq_ctx *ctx, const axq_soft_attn &a, const float *q, con
     const Args g = make_args(a, q, k, v, gate, ldq, ldk, ldv, m, pos0, nullptr, qscratch);
     const int queries = q ? a.heads : 0; // without q: the keys and values alone
     if (a.f32) {
-        prep_kernel<true><<<dim3((queries + 2 * a.kv_heads + 3) / 4, m), 256, 0, ctx->stream>>>(g);
+        prep_kernel<<<dim3((queries + 2 * a.kv_heads + 3) / 4, m), 256, 0, ctx->stream>>>(g);
         launch_pool<true>(ctx, g);
         if (q) rows_f32_kernel<<<dim3(a.heads, m), 256, f32_rows_lds(a), ctx->stream>>>(g, out);
     } else {
-        prep_kernel<false><<<dim3((queries + a.kv_heads + 3) / 4, m), 256, 0, ctx->stream>>>(g);
-        append_values_kernel<<<dim3((m + 31) / 32, (a.vdim + 31) / 32, a.kv_heads), 256, 0, ctx->stream>>>(g);
+        const int values = value_tiles(m, a.vdim, a.kv_heads);
+        prep_rows_kernel<<<prep_grid(m, queries + a.kv_heads, values), 256, 0, ctx->stream>>>(g, values);
         launch_pool<false>(ctx, g);
         if (q && (rc = g.dp == 64 ? launch_mfma_k<4>(ctx, g, out) : (g.dp == 128 ? launch_mfma_k<8>(ctx, g, out) : launch_mfma_k<16>(ctx, g, out)))) return rc;
     }
@@ -606,7 +635,7 @@ int axq_soft_attn_token(axq_ctx *ctx, const axq_soft_attn &a, const float *q, co
     if ((rc = check_shape(ctx, a))) return rc;
     const Args g = make_args(a, q, k, v, gate, 0, 0, 0, 1, 0, pos, qscratch);
     if (a.f32) {
-        prep_kernel<true><<<dim3((a.heads + 2 * a.kv_heads + 3) / 4, 1), 256, 0, ctx->stream>>>(g);
+        prep_kernel<<<dim3((a.heads + 2 * a.kv_heads + 3) / 4, 1), 256, 0, ctx->stream>>>(g);
         launch_pool<true>(ctx, g);
         axq_rows_out out = {att, a.heads * a.vdim, true};
         rows_f32_kernel<<<dim3(a.heads, 1), 256, f32_rows_lds(a), ctx->stream>>>(g, out);
