@@ -118,13 +118,22 @@ __device__ void pool_block(const Args &g, int h, int b, int tid, int n) {
             reinterpret_cast<float *>(key ? a.pkc : a.pvc)[((size_t)h * g.cap_blocks + b) * d + e] = s * inv;
         } else if (key) {
             const _Float16 *x = reinterpret_cast<const _Float16 *>(a.kc) + ((size_t)h * g.capp + p0) * g.dp + e;
-#pragma unroll 16
+#pragma unroll 32
             for (int j = 0; j < a.pool; j++) s += (float)x[(size_t)j * g.dp];
             reinterpret_cast<_Float16 *>(a.pkc)[((size_t)h * g.cpp + b) * g.dp + e] = (_Float16)(s * inv);
         } else {
             const _Float16 *x = reinterpret_cast<const _Float16 *>(a.vc) + ((size_t)h * g.dvp + e) * g.capp;
+            if (a.pool % 16 == 0) { // sixteen neighbouring positions are 32 bytes
+#pragma unroll 4
+                for (int j = 0; j < a.pool; j += 16) {
+                    const half8 lo = *reinterpret_cast<const half8 *>(x + p0 + j), hi = *reinterpret_cast<const half8 *>(x + p0 + j + 8);
+#pragma unroll
+                    for (int k = 0; k < 16; k++) s += (float)(value_slot(k) < 8 ? lo[value_slot(k) & 7] : hi[value_slot(k) & 7]);
+                }
+            } else {
 #pragma unroll 16
-            for (int j = 0; j < a.pool; j++) s += (float)x[value_slot((int)p0 + j)];
+                for (int j = 0; j < a.pool; j++) s += (float)x[value_slot((int)p0 + j)];
+            }
             reinterpret_cast<_Float16 *>(a.pvc)[((size_t)h * g.dvp + e) * g.cpp + value_slot(b)] = (_Float16)(s * inv);
         }
     }
