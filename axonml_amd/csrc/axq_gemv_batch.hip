@@ -443,17 +443,17 @@ __global__ void __launch_bounds__(512, 4) gemv_mb_kernel(MbArgs a) {
 #pragma unroll
     for (int bi = 0; bi < 4; bi++) red[((size_t)all_wave * MAX_BATCH + (2 * bi + h)) * 32 + n] = acc[bi];
     __syncthreads();
-    if constexpr (ACT) { // a thread per vector and activation, then one per vector and eight of them
+    if constexpr (ACT) { // the 256 activations by as many threads as there are (128 at one chunk), then a thread per vector and eight of them
         float *act_of = red + (size_t)waves * MAX_BATCH * 32; // [vector][32], where the patches were
-        const int b0 = tid >> 5, o = tid & 31;
-        if (b0 < MAX_BATCH) {
-            const float *from = red + ((size_t)(o >> 4) * S * MAX_BATCH + b0) * 32 + ((o >> 2) & 3) * 8 + (o & 3); // four gates, four ups, and so again
+        for (int i = tid; i < MAX_BATCH * 32; i += (int)blockDim.x) {
+            const int b = i >> 5, o = i & 31;
+            const float *from = red + ((size_t)(o >> 4) * S * MAX_BATCH + b) * 32 + ((o >> 2) & 3) * 8 + (o & 3); // four gates, four ups, and so again
             float g = 0.f, u = 0.f;
             for (int w = 0; w < S; w++) {
                 g += from[(size_t)w * MAX_BATCH * 32];
                 u += from[(size_t)w * MAX_BATCH * 32 + 4];
             }
-            act_of[tid] = (g * (1.0f / (1.0f + expf(-g)))) * u; // as pack_x_kernel
+            act_of[i] = (g * (1.0f / (1.0f + expf(-g)))) * u; // as pack_x_kernel
         }
         __syncthreads();
         if (tid >= 4 * MAX_BATCH) return;

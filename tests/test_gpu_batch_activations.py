@@ -10,8 +10,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("gate,down", [(o.Q4_K, o.Q4_K), (o.Q4_K, o.Q4_0), (o.Q5_K, o.Q6_K), (o.Q6_K, o.Q4_1), (o.Q8_0, o.Q8_0), (o.Q5_1, o.Q5_0), (o.Q4_0, o.Q4_K)])
-@pytest.mark.parametrize("n_seq,hidden,inter", [(2, 256, 2304), (5, 768, 2304), (8, 1280, 2304), (8, 256, 2048)],
-                         ids=["one chunk", "three chunks", "five chunks", "too few rows"])
+@pytest.mark.parametrize("n_seq,hidden,inter", [(2, 256, 2304), (5, 256, 2304), (8, 256, 2304), (8, 512, 2304), (5, 768, 2304), (8, 1280, 2304), (8, 256, 2048)],
+                         ids=["one chunk", "one chunk, five", "one chunk, eight", "two chunks", "three chunks", "five chunks", "too few rows"])
 def test_steps_of_several_sequences(ctx, gate, down, n_seq, hidden, inter):
     c = tiny_config(hidden_size=hidden, intermediate_size=inter, num_layers=2, max_seq_len=16)
     w = random_weights(c, n_seq, gate, std=0.03)
@@ -25,5 +25,21 @@ def test_steps_of_several_sequences(ctx, gate, down, n_seq, hidden, inter):
         for i in range(3):
             _, lg = cpu.forward(int(steps[i, s]), i)
             assert max_rel_err(got[i][s], lg, DECODE_FLOOR) <= DECODE_RTOL, (s, i)
+    gpu.close()
+    cpu.close()
+
+
+@pytest.mark.parametrize("n_tokens", [6, 9])
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q4_0, o.Q8_0])
+def test_rows_of_a_short_prompt(ctx, qtype, n_tokens):
+    """Five and eight rows of one chunk, whose first layer's activations the second layer's keys and values are made of."""
+    c = tiny_config(intermediate_size=2304, num_layers=2, max_seq_len=16)
+    w = random_weights(c, n_tokens, qtype)
+    cpu, gpu = load_oracle(c, w), load_gpu(ctx, c, w)
+    tokens = np.random.default_rng(n_tokens).integers(0, c["vocab_size"], size=n_tokens)
+    for pos, t in enumerate(tokens):
+        _, lg = cpu.forward(int(t), pos)
+    _, logits = gpu.forward_tokens(tokens)
+    assert max_rel_err(logits, lg, DECODE_FLOOR) <= DECODE_RTOL
     gpu.close()
     cpu.close()
