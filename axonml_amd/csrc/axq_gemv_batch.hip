@@ -651,9 +651,10 @@ unsigned mb_max_waves() {
     return smax < 1 ? 1 : (smax > 8 ? 8 : smax);
 }
 
+constexpr unsigned act_waves(int64_t k) { return k >= 4 * WAVE_K ? 4 : (unsigned)((k + WAVE_K - 1) / WAVE_K); } // of each half of a workgroup
 template <class T>
-constexpr size_t act_lds(int64_t k, unsigned S) {
-    return ((size_t)(k / 32) * 16 + (size_t)2 * S * MAX_BATCH * 32) * sizeof(float) + (size_t)2 * S * 32 * (T::NP + T::NP2) * 16;
+constexpr size_t act_lds(int64_t k) {
+    return ((size_t)(k / 32) * 16 + (size_t)2 * act_waves(k) * MAX_BATCH * 32) * sizeof(float) + (size_t)2 * act_waves(k) * 32 * (T::NP + T::NP2) * 16;
 }
 template <class T>
 std::atomic<uint64_t> &act_lds_mask() {
@@ -674,10 +675,10 @@ int launch_mb(axq_ctx *ctx, MbArgs a, uint8_t *sc, const float *x, int xmode, co
     const unsigned chunks = (unsigned)((a.k + WAVE_K - 1) / WAVE_K);
     if (a.next_xa) {
         a.chunks_per_split = (int)chunks;
-        const unsigned S = chunks < 4 ? chunks : 4;
+        static_assert(act_lds<T>(AXQ_BATCH_MAX_K) <= 160 * 1024, "any K that is covered fits LDS");
         const int st = axq_allow_lds(ctx, reinterpret_cast<const void *>(&gemv_mb_kernel<T, true>), act_lds_mask<T>(), 160 * 1024);
         if (st != AXQ_OK) return st;
-        gemv_mb_kernel<T, true><<<a.n_rows / 64, 128 * S, act_lds<T>(a.k, S), ctx->stream>>>(a);
+        gemv_mb_kernel<T, true><<<a.n_rows / 64, 128 * act_waves(a.k), act_lds<T>(a.k), ctx->stream>>>(a);
         return AXQ_OK;
     }
     const unsigned tiles = (unsigned)((a.n_rows + 31) / 32);
@@ -773,15 +774,23 @@ bool axq_dev_gemv_batch_takes(const axq_weight *w, int batch) {
     return batch <= MAX_BATCH && batch >= (w->n_rows * w->k >= 40 << 20 ? 2 : 3);
 }
 
-// Whether a call of `w`, gate and up rows in groups of four, can leave silu(gate) * up as the operands of the call with `down`: all of K in a workgroup (as
-// where 32-row tiles are more than half the compute units), whose 64 rows' pieces and sums fit LDS.
+// Whether a call of `w`, gate and up rows in groups of four, leaves silu(gate) * up as the operands of the call with `down`: all of K in a workgroup, as where
+// 32-row tiles are more than half the compute units.  It is a launch less, but the workgroups are half as many and take twice as long, which costs half a
+// round where that makes their last round no fuller.  us of a layer of eight sequences without and with it, by tiles per 256 compute units and K:
+//   two or four rounds of either   448 to 1024 tiles  K 1024: Q4_K -1.1, Q6_K -2.2, Q4_0 -3.4;  4096: Q4_K -0.5 to -3.4, Q8_0 -2.5, Q6_K +0.9 to -2.8;
+//                                  8192: Q4_K 0 to -2.2, Q8_0 -2.3 to -4.1, Q5_1 -0.2 to -1.2, Q6_K +3.0 (more than two rounds -1.9);
+//                                  16384: Q8_0 -10 to -25, Q4_K, Q5_K, Q5_1 up to +2.5
+//   one against two, three against four   144, 256 and 528 to 768 tiles  K 256 to 1024: -0.3 to -3.5;  2048: +0.9 to -1.9;  4096: Q4_0 +0.9 to -0.7, Q4_K +1.1 to
+//                                  +3.2, Q8_0 +1.1 to +2.7, Q6_K +2.9 to +5.0;  8192: Q4_K +3.5 to +5.0, Q8_0 +6 to +8, Q6_K +9 to +13
 bool axq_dev_gemv_batch_makes_act(const axq_ctx *ctx, const axq_weight *w, const axq_weight *down, int batch) {
     if (!axq_dev_gemv_batch_covers(w, batch) || !axq_dev_gemv_batch_covers(down, batch) || w->n_rows != 2 * down->k) return false;
-    if (w->n_rows / 32 <= ctx->prop.multiProcessorCount / 2 || mb_max_waves() != 8) return false;
+    const int64_t cus = ctx->prop.multiProcessorCount, tiles = w->n_rows / 32;
+    if (tiles <= cus / 2 || mb_max_waves() != 8) return false;
+    if (2 * ((tiles / 2 + cus - 1) / cus) > (tiles + cus - 1) / cus) return w->k <= 1024;
     switch (w->type) {
-    case AXQ_Q8_0: return act_lds<MQ80>(w->kp, 8) <= 160 * 1024;
-    case AXQ_Q6_K: return act_lds<MQ6K>(w->kp, 8) <= 160 * 1024;
-    default: return act_lds<MQ5K>(w->kp, 8) <= 160 * 1024; // of the others the largest
+    case AXQ_Q8_0: return true;
+    case AXQ_Q6_K: return w->k <= 4096 || tiles > 2 * cus;
+    default: return w->k <= 12288;
     }
 }
 

@@ -43,3 +43,25 @@ def test_rows_of_a_short_prompt(ctx, qtype, n_tokens):
     assert max_rel_err(logits, lg, DECODE_FLOOR) <= DECODE_RTOL
     gpu.close()
     cpu.close()
+
+
+@pytest.mark.parametrize("gate,hidden,inter", [(o.Q8_0, 8448, 4352), (o.Q8_0, 16384, 4352), (o.Q6_K, 4096, 4352), (o.Q6_K, 4352, 8448), (o.Q6_K, 4352, 4352),
+                                               (o.Q5_K, 12288, 4352), (o.Q5_K, 12544, 4352), (o.Q4_K, 1024, 8448), (o.Q4_K, 1280, 8448)])
+def test_long_rows_and_uneven_rounds(ctx, gate, hidden, inter):
+    """Rows of 33 chunks and of the most there are, and either side of each line between a launch that leaves operands and one of their own."""
+    c = tiny_config(hidden_size=hidden, intermediate_size=inter, num_layers=1, vocab_size=64, max_seq_len=16)
+    rng = np.random.default_rng(hidden)
+    w = random_weights(dict(c, intermediate_size=256), hidden, gate, std=0.01)
+    L = w["layers"][0]
+    for name, n, k in (("gate", inter, hidden), ("up", inter, hidden), ("down", hidden, inter)):  # few different rows: the model is large
+        L[name] = o.quantize(gate, (rng.standard_normal((251, k)) * 0.01).astype(np.float32)).reshape(251, -1)[np.arange(n) % 251].reshape(-1)
+    cpu, gpu = load_oracle(c, w), load_gpu(ctx, c, w)
+    gpu.set_batch(8)
+    steps = rng.integers(0, c["vocab_size"], size=(2, 8))
+    got = [gpu.forward_batch(t)[1] for t in steps]
+    for s in (0, 7):
+        for i in range(2):
+            _, lg = cpu.forward(int(steps[i, s]), i)
+            assert max_rel_err(got[i][s], lg, DECODE_FLOOR) <= DECODE_RTOL, (s, i)
+    gpu.close()
+    cpu.close()
