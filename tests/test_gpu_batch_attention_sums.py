@@ -1,5 +1,5 @@
-"""Batched steps whose q, k and v reach the attention as sums of parts of K: fewer parts than it requests at once, as many, and more, rows as limbs and as
-pairs, one and two heads to a workgroup, against the CPU decode oracle."""
+"""Batched steps whose q, k and v reach the attention as sums of parts of K: fewer parts than the eight it requests at once (2, 4, 3, 4), as many, and more
+(9, 11, 16), rows as limbs and as pairs, one and two heads to a workgroup, against the CPU decode oracle."""
 import numpy as np
 import pytest
 
@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("hidden,n_seq,head_dim,heads,kv,qtype", [(512, 44, 64, 8, 2, o.Q4_K), (1024, 64, 128, 24, 8, o.Q5_K), (1536, 10, 32, 4, 4, o.Q8_0), (2048, 12, 128, 6, 2, o.Q4_K),
-                                                                 (2048, 50, 64, 12, 3, o.Q6_K), (2048, 33, 256, 10, 2, o.Q4_0)])
+                                                                 (2048, 50, 64, 12, 3, o.Q6_K), (2048, 33, 256, 10, 2, o.Q4_0),
+                                                                 (2304, 39, 64, 16, 8, o.Q8_0), (2816, 34, 128, 8, 4, o.Q6_K), (4096, 35, 128, 8, 4, o.Q4_K)])
 def test_steps_over_parts_of_k(ctx, hidden, n_seq, head_dim, heads, kv, qtype):
     c = tiny_config(hidden_size=hidden, num_heads=heads, num_kv_heads=kv, head_dim=head_dim, num_layers=2, max_seq_len=16)
     w = random_weights(c, n_seq, qtype, std=0.03)
