@@ -1925,7 +1925,8 @@ RowsPlan rows_plan(const axq_ctx *ctx, const axq_weight *w, int in, int rows, bo
     if (splits < 2 || whole_k) splits = 1;
     p.sb_per_split = (nsb + splits - 1) / splits;
     p.splits = (nsb + p.sb_per_split - 1) / p.sb_per_split;
-    // 128 x 128 outputs whose halves have K of their own, a superblock each at least.  f32 rows, us so and with shared K: 64 rows, Q4_K 28672 x 4096
+    // 128 x 128 outputs whose halves have K of their own, from two superblocks per workgroup on (a last part may have one: its second half then only
+    // keeps step).  f32 rows, us so and with shared K: 64 rows, Q4_K 28672 x 4096
     // (sixteen per workgroup) 52.5 62.7, Q5_K and Q6_K 14336 x 4096 (eight) 36.5 43.7 and 44.0 52.0, 4096 x 14336 (seven) Q4_K 36.5 36.8, Q5_K
     // 41.3 43.8, Q6_K 48.6 50.8, 6144 x 4096 (four) Q4_K 24.3 26.4, Q6_K 27.9 31.1, Q4_K 4096 x 4096 (two) 21.5 23.1; 100 bf16 rows, Q4_K 4096 x
     // 14336 36.1 37.0.  Error against 64 bits, 64 rows, three seeds, 1e-8: Q4_K 6144 x 4096 11.29 11.34 11.30 and 11.26 11.32 11.30, 4096 x 14336

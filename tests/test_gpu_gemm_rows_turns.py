@@ -37,9 +37,11 @@ def test_halves_with_their_own_k_and_all_of_it(ctx, qtype, rows, n, k, bf16):
 
 @pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
 @pytest.mark.parametrize("rows,n,k,bf16", [(40, 16385, 256, False), (64, 16386, 512, False), (41, 16387, 768, False), (65, 16512, 1024, True), (128, 16390, 1280, True),
-                                           (33, 4096, 1536, True), (50, 513, 4096, False), (64, 6144, 7168, False)])
+                                           (33, 4096, 1536, True), (50, 513, 4096, False), (64, 6144, 7168, False),
+                                           (40, 8192, 1280, False), (64, 12288, 768, False), (66, 8190, 1280, True), (100, 12288, 768, True)])
 def test_halves_of_few_superblocks(ctx, qtype, rows, n, k, bf16):
-    """One superblock (which shares its K), two, three .. seven, alone and in parts; 33 bf16 rows are no large tile."""
+    """One superblock (which shares its K), two, three .. seven, alone and in parts; 33 bf16 rows are no large tile; parts of two of which the last one has
+    one, so that its second half has none."""
     rng = np.random.default_rng(rows + n + k + qtype)
     packed = o.quantize(qtype, gen_weight(rng, 509, k)).reshape(509, -1)[np.arange(n) % 509].reshape(-1)
     x = rng.standard_normal((rows, k)).astype(np.float32) * (10.0 ** rng.integers(-3, 4, size=(rows, 1))).astype(np.float32)
