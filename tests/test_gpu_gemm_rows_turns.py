@@ -71,25 +71,45 @@ def test_operands_made_with_the_reduction(ctx, qtype, rows, sizes):
     cpu.close()
 
 
-@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q6_K, o.Q4_1])
-@pytest.mark.parametrize("inter", [8256, 8320], ids=["half a large tile left", "whole tiles"])
-@pytest.mark.parametrize("rows", [40, 64, 65, 129])
-def test_gate_and_up_leave_their_product(ctx, qtype, inter, rows):
-    """More column tiles than half the compute units, so that a workgroup has all of K: tiles of 128 and of 256 rows of operands, and those of blocks."""
-    c = tiny_config(max_seq_len=rows + 8, vocab_size=64, num_layers=2)  # of a prompt the last layer ends with its keys and values
+def _gate_and_up(ctx, qtype, inter, hidden, rows):
+    c = tiny_config(max_seq_len=rows + 8, vocab_size=64, num_layers=2, hidden_size=hidden)  # of a prompt the last layer ends with its keys and values
     w = random_weights(c, rows, qtype, std=0.02)
     c["intermediate_size"] = inter
     rng = np.random.default_rng([rows, inter])
     w["types"] = {}
     for l, L in enumerate(w["layers"]):
-        for name, t, shape in (("gate", qtype, (inter, 256)), ("up", qtype, (inter, 256)), ("down", o.Q8_0, (256, inter))):
+        for name, t, shape in (("gate", qtype, (inter, hidden)), ("up", qtype, (inter, hidden)), ("down", o.Q8_0, (hidden, inter))):
             L[name] = o.quantize(t, (rng.standard_normal(shape) * 0.05).astype(np.float32))
             w["types"][(l, name)] = t
-    cpu, gpu = load_oracle(c, w), load_gpu(ctx, c, w)
+    return c, load_oracle(c, w), load_gpu(ctx, c, w), rng
+
+
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q6_K, o.Q4_1])
+@pytest.mark.parametrize("inter", [8256, 8320], ids=["half a large tile left", "whole tiles"])
+@pytest.mark.parametrize("hidden,rows", [(256, 40), (256, 64), (256, 65), (256, 129), (512, 40), (512, 64), (512, 129), (768, 40), (768, 64)])
+def test_gate_and_up_leave_their_product(ctx, qtype, inter, hidden, rows):
+    """More column tiles than half the compute units, so that a workgroup has all of K: tiles of 256 rows of operands, those of blocks, and tiles of 128, which
+    need two superblocks (up to 64 rows of one superblock are activated by the product behind them)."""
+    c, cpu, gpu, rng = _gate_and_up(ctx, qtype, inter, hidden, rows)
     tokens = rng.integers(0, c["vocab_size"], size=rows + 1)
     for pos, t in enumerate(tokens):
         _, lg = cpu.forward(int(t), pos)
     _, logits = gpu.forward_tokens(tokens)
     assert max_rel_err(logits, lg, DECODE_FLOOR) <= DECODE_RTOL
+    gpu.close()
+    cpu.close()
+
+
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
+@pytest.mark.parametrize("hidden,rows", [(512, 40), (768, 64)])
+def test_steps_whose_gate_and_up_leave_their_product(ctx, qtype, hidden, rows):
+    c, cpu, gpu, rng = _gate_and_up(ctx, qtype, 8320, hidden, rows)
+    gpu.set_batch(rows)
+    steps = rng.integers(0, c["vocab_size"], size=(2, rows))
+    got = [gpu.forward_batch(t)[1] for t in steps]
+    for s in (0, 1, rows // 2, rows - 1):
+        for i in range(2):
+            _, lg = cpu.forward(int(steps[i, s]), i)
+            assert max_rel_err(got[i][s], lg, DECODE_FLOOR) <= DECODE_RTOL, (s, i)
     gpu.close()
     cpu.close()
