@@ -221,9 +221,18 @@ def test_copy_sequence_copies_whole_caches(ctx, n):
 
 def test_one_layer_at_the_7b_shape(ctx):
     """The real layer shape (hidden 4096, intermediate 14336, 32 query heads over 8 KV heads of 128, Q4_K) with a
-    small vocabulary and one layer, so that the CPU oracle finishes in seconds: the one-token step, a prompt
-    through the GEMM rows, the small-batch rows, and batched steps of eight sequences, all against the oracle."""
-    c = tiny_config(vocab_size=1024, hidden_size=4096, intermediate_size=14336, num_layers=1, num_heads=32, num_kv_heads=8,
+    small vocabulary and one layer, so that the CPU oracle finishes in seconds: the one-token step, the keys and values of a prompt
+    through the GEMM rows and the small-batch rows, and batched steps of eight sequences, all against the oracle."""
+    _walk_at_the_7b_shape(ctx, 1)
+
+
+def test_two_layers_at_the_7b_shape(ctx):
+    """The same with a layer in front whose rows go through attention and all products: of a prompt's rows the last layer makes keys and values only."""
+    _walk_at_the_7b_shape(ctx, 2)
+
+
+def _walk_at_the_7b_shape(ctx, layers):
+    c = tiny_config(vocab_size=1024, hidden_size=4096, intermediate_size=14336, num_layers=layers, num_heads=32, num_kv_heads=8,
                     head_dim=128, max_seq_len=96)
     w = random_weights(c, 400, std=0.02)
     cpu, gpu = load_oracle(c, w), load_gpu(ctx, c, w)
