@@ -12,9 +12,9 @@
 //   bf16 rows, Q8_0 4096 x 4096, 16: 26.0 14.5; Q4_0 11008 x 4096, 128: 48.4 36.5; Q4_K 14336 x 4096, 2048: 325 to 328 265 to 290
 // What bounds it: at few rows the fixed parts (pre-pass, reduction and the launches around them: 14 us of the 4096 x 4096 calls) and
 // the LDS reads of x, which every wave makes for its 32 columns (0.35 us per step with one tile of x, 0.6 with two); at many the matrix
-// pipe beside the vector instructions that make operands.  2048 bf16 rows x 14336 take 245 to 260 us in the kernel, 920 to 980 TFLOP/s: a
-// product keeps its SIMD's issue for about half of its 33 cycles, four vector instructions fit beside it, and there are five; a tile's way in and out,
-// 5 and 13 us a round (all workgroups write at once); and
+// pipe beside the vector instructions that make operands.  2048 bf16 rows x 14336 take 254 to 285 us in the kernel as the clock goes (273 in the
+// first passes, 256 behind hundreds of others), 845 to 945 TFLOP/s: a product keeps its SIMD's issue for about half of its 33 cycles, four vector
+// instructions fit beside it, and there are five; a tile's way in and out, 5 and 13 us a round (all workgroups write at once); and
 // the card's power: the same products alone, without operands, copies and results, take 208 us, 167 if every x is zero.
 //
 // Numerics.  A bf16 row goes in as f16 under a power-of-two row scale that puts its largest element right below f16's limit: exact
