@@ -777,11 +777,11 @@ bool axq_dev_gemv_batch_takes(const axq_weight *w, int batch) {
 // Whether a call of `w`, gate and up rows in groups of four, leaves silu(gate) * up as the operands of the call with `down`: all of K in a workgroup, as where
 // 32-row tiles are more than half the compute units.  It is a launch less, but the workgroups are half as many and take twice as long, which costs half a
 // round where that makes their last round no fuller.  us of a layer of eight sequences without and with it, by tiles per 256 compute units and K:
-//   two or four rounds of either   448 to 1024 tiles  K 1024: Q4_K -1.1, Q6_K -2.2, Q4_0 -3.4;  4096: Q4_K -0.5 to -3.4, Q8_0 -2.5, Q6_K +0.9 to -2.8;
-//                                  8192: Q4_K 0 to -2.2, Q8_0 -2.3 to -4.1, Q5_1 -0.2 to -1.2, Q6_K +3.0 (more than two rounds -1.9);
-//                                  16384: Q8_0 -10 to -25, Q4_K, Q5_K, Q5_1 up to +2.5
-//   one against two, three against four   144, 256 and 528 to 768 tiles  K 256 to 1024: -0.3 to -3.5;  2048: +0.9 to -1.9;  4096: Q4_0 +0.9 to -0.7, Q4_K +1.1 to
-//                                  +3.2, Q8_0 +1.1 to +2.7, Q6_K +2.9 to +5.0;  8192: Q4_K +3.5 to +5.0, Q8_0 +6 to +8, Q6_K +9 to +13
+//   two or four rounds of either   448 to 1024 tiles  K 1024: Q4_K -1.1, Q6_K -2.2, Q4_0 -3.4;  4096: Q4_K -0.5 to -3.4, Q8_0 -1.5 to -2.6, Q6_K +0.9 to
+//                                  -2.8;  8192: Q4_K +0.2 to -2.2, Q8_0 -2.0 to -4.1, Q5_1 -0.2 to -1.2, Q6_K +2.8 to +3.0 (more than two rounds -1.9);
+//                                  16384: Q8_0 -10 to -25, Q4_K, Q5_K, Q5_1 -1.3 to +2.5
+//   one against two, three against four   144, 256 and 528 to 768 tiles  K 256 to 1024: +0.1 to -3.5;  2048: +1.1 to -2.1;  4096: Q4_0 +0.9 to -0.7, Q4_K -0.1 to
+//                                  +3.2, Q8_0 +1.1 to +2.7, Q6_K +1.2 to +5.0;  8192: Q4_K +3.5 to +5.0, Q8_0 +6 to +8, Q6_K +9 to +13
 bool axq_dev_gemv_batch_makes_act(const axq_ctx *ctx, const axq_weight *w, const axq_weight *down, int batch) {
     if (!axq_dev_gemv_batch_covers(w, batch) || !axq_dev_gemv_batch_covers(down, batch) || w->n_rows != 2 * down->k) return false;
     const int64_t cus = ctx->prop.multiProcessorCount, tiles = w->n_rows / 32;
